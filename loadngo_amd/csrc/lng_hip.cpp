@@ -77,6 +77,7 @@ struct Knobs {
     int prefill_upfront = -1;      // LNG_PREFILL_UPFRONT: 0 narrow windows on the tile-by-tile kernel
     int table_in_place = 8192;     // LNG_TABLE_IN_PLACE: row tables of this many bytes or more are read from pinned host memory; 0 never
     int prefill_splits = 0;        // LNG_PREFILL_SPLITS: workgroups per (query tile, kv head) of a split prompt pass; 0 planner
+    int q8_mid = -1;               // LNG_Q8_MID: Q8_0 products of 32 positions or more: 0 never the kernel whose wavefronts share the columns, 1 whenever it can run, -1 planner
     int checksum_wgs = 0;          // LNG_CHECKSUM_WGS: workgroups per compute unit of the streaming read; 0 default (2)
     bool count_second_passes = false; // LNG_COUNT_SECOND_PASSES: long causal passes count the query tiles they repeat
     long decode_wgs = 0;           // LNG_DECODE_WGS: workgroups a decode dispatch aims for; 0 default
@@ -96,6 +97,7 @@ struct Cmd {
     const char *name = "";
     unsigned grid[3] = {1, 1, 1};
     unsigned block = 256;
+    unsigned lds = 0; // bytes of LDS beyond what the kernel declares
     std::vector<char> args;
 };
 
@@ -123,7 +125,8 @@ struct lng_gpu {
     hipFunction_t copy_rows = nullptr, fill_synthetic = nullptr, add_rows = nullptr, rotate_halves = nullptr, rmsnorm_rows = nullptr, rmsnorm_row_wg = nullptr;
     hipFunction_t prepare_v4 = nullptr, prepare_v1 = nullptr;
     hipFunction_t q8_split_x = nullptr, q8_stream = nullptr, q8_stream_one = nullptr, q8_stream_one_w8 = nullptr, q8_stream_bf16 = nullptr, q8_tiled = nullptr,
-                  q8_tiled_bf16 = nullptr;
+                  q8_tiled_bf16 = nullptr, q8_frag_x = nullptr;
+    hipFunction_t q8_mid[2][4] = {}; // [bf16 positions][tile, see q8_mid_tile]
     std::string name;
     unsigned cus = 256;
 
@@ -271,7 +274,7 @@ int check_shape(const lng_grouped_shape &s, bool tiled) {
 
 // One development switch by its environment name; value NULL puts the default back. Returns false for an unknown name.
 const char *const knob_names[] = {"LNG_WIDE_GENERIC", "LNG_F32_GENERIC", "LNG_PLAIN_ROW_BY_ROW", "LNG_DECODE_O3", "LNG_MERGE_WIDE",
-                                  "LNG_Q8_W16", "LNG_WIDE_ROW_BY_ROW", "LNG_PREFILL_STREAM", "LNG_PREFILL_PAIR", "LNG_PREFILL_UPFRONT",
+                                  "LNG_Q8_W16", "LNG_Q8_MID", "LNG_WIDE_ROW_BY_ROW", "LNG_PREFILL_STREAM", "LNG_PREFILL_PAIR", "LNG_PREFILL_UPFRONT",
                                   "LNG_PREFILL_SPLITS", "LNG_DECODE_WGS", "LNG_FUSE_WGS", "LNG_COUNT_SECOND_PASSES", "LNG_CHECKSUM_WGS", "LNG_TABLE_IN_PLACE"};
 bool set_knob(lng_gpu *g, const char *name, const char *value) {
     Knobs &k = g->knobs;
@@ -290,6 +293,7 @@ bool set_knob(lng_gpu *g, const char *name, const char *value) {
     if (!strcmp(name, "LNG_PREFILL_STREAM")) return choice(k.prefill_stream, defaults.prefill_stream);
     if (!strcmp(name, "LNG_PREFILL_PAIR")) return choice(k.prefill_pair, defaults.prefill_pair);
     if (!strcmp(name, "LNG_PREFILL_UPFRONT")) return choice(k.prefill_upfront, defaults.prefill_upfront);
+    if (!strcmp(name, "LNG_Q8_MID")) return choice(k.q8_mid, defaults.q8_mid);
     if (!strcmp(name, "LNG_CHECKSUM_WGS")) return choice(k.checksum_wgs, defaults.checksum_wgs);
     if (!strcmp(name, "LNG_TABLE_IN_PLACE")) {
         k.table_in_place = value ? (int)std::max(0l, std::min(n, 1l << 30)) : defaults.table_in_place;
@@ -1052,6 +1056,12 @@ extern "C" int lng_hip_open(int device, lng_gpu **out) {
         {"lng_q8_tiled", &g->q8_tiled, true},
         {"lng_q8_tiled_bf16", &g->q8_tiled_bf16, true},
         {"lng_q8_stream_bf16", &g->q8_stream_bf16, true},
+        {"lng_q8_frag_x", &g->q8_frag_x, true},
+        {"lng_q8_mid_r32p32", &g->q8_mid[0][1], true},
+        {"lng_q8_mid_r64p64", &g->q8_mid[0][3], true},
+        {"lng_q8_mid_bf16_r16p32", &g->q8_mid[1][0], true},
+        {"lng_q8_mid_bf16_r32p64", &g->q8_mid[1][2], true},
+        {"lng_q8_mid_bf16_r64p64", &g->q8_mid[1][3], true},
         {"lng_rmsnorm_rows", &g->rmsnorm_rows, true},
         {"lng_rmsnorm_row_wg", &g->rmsnorm_row_wg, true},
     };
@@ -1310,7 +1320,7 @@ extern "C" int lng_hip_batch_commit(lng_batch *b, lng_on_done on_done, void *use
         size_t size = c.args.size();
         void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, c.args.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
                           HIP_LAUNCH_PARAM_END};
-        e = hipModuleLaunchKernel(c.fn, c.grid[0], c.grid[1], c.grid[2], c.block, 1, 1, 0, g->stream, nullptr, config);
+        e = hipModuleLaunchKernel(c.fn, c.grid[0], c.grid[1], c.grid[2], c.block, 1, 1, c.lds, g->stream, nullptr, config);
         if (e == hipSuccess && b->timing) {
             hipEvent_t mark = nullptr;
             e = take_event(g, &mark);
@@ -1934,6 +1944,68 @@ void q8_record_stream(lng_batch *b, const lng_k_q8 &a, uint64_t row_tiles, bool 
     b->dispatches += 1;
 }
 
+// The tiles of lng_q8_mid*: rows, positions, wavefronts that share the columns.
+struct Q8MidTile {
+    unsigned rows, pos, waves;
+    const char *name[2]; // f32, bf16 positions
+};
+const Q8MidTile q8_mid_tiles[4] = {{16, 32, 8, {nullptr, "lng_q8_mid_bf16_r16p32"}},
+                                   {32, 32, 8, {"lng_q8_mid_r32p32", nullptr}},
+                                   {32, 64, 4, {nullptr, "lng_q8_mid_bf16_r32p64"}},
+                                   {64, 64, 4, {"lng_q8_mid_r64p64", "lng_q8_mid_bf16_r64p64"}}};
+
+// The tile a product of 32 positions or more takes; -1: lng_q8_tiled. It depends on nothing that differs between a
+// product alone and among several matrices, so that its sums keep their order.
+// Measured (2,880 x 4,096 bf16 / the 5,120 x 2,880 of q, k and v), us: tiles 16 x 32, 32 x 32, 32 x 64, 64 x 64 at 32
+// positions 8.7, 11, 15, 22 / 14, 12, 16, 22; at 77 20, 19, 16, 24 / 24, 19, 26, 25; at 192 33, 28, 27, 25 / 44, 33, 29, 28.
+// Against lng_q8_tiled: 1,280 positions 82 / 135 against 91 / 297, 1,536 99 / 169 against 92 / 305 (one matrix of 4,096
+// rows 133 against 113): x no longer stays in the L2 caches between the row tiles.
+int q8_mid_tile(const lng_gpu *g, uint64_t n, uint64_t cols, bool x_bf16) {
+    if (g->knobs.q8_mid == 0 || cols > 32 * 512) return -1; // a tile's scales are held in LDS: at most 64 KB of them
+    if (g->knobs.q8_mid < 0 && n > 1280) return -1;
+    if (x_bf16) return n <= 48 ? 0 : n <= 128 ? 2 : 3;
+    return n <= 128 ? 1 : 3;
+}
+
+// A chunk of positions: too few tiles of lng_q8_tiled to fill the device.
+// `a` may name further matrices of the same dispatch (first_tile in row tiles, a.tiles of all of them).
+int q8_record_mid(lng_batch *b, lng_k_q8 a, bool x_bf16, int tile) {
+    const Q8MidTile &t = q8_mid_tiles[tile];
+    const uint64_t n = a.n, cols = a.cols, pos = t.pos;
+    const uint64_t pos_tiles = (n + pos - 1) / pos, n_pad = pos_tiles * pos;
+    const uint64_t ids = 8 * ((uint64_t)(a.tiles + 7) / 8) * pos_tiles;
+    if (ids > 0x7fffffffull || !fits_u32(n_pad * cols)) return fail(LNG_ERR_DISPATCH, "too large");
+    if (!x_bf16) {
+        char *planes = nullptr;
+        if (int rc = reserve_x(b->gpu, 2 * n_pad * cols * 2, &planes)) return rc;
+        lng_k_q8_split sp{};
+        sp.x = a.x;
+        sp.hi = (uint16_t *)planes;
+        sp.n = (uint32_t)n;
+        sp.n_pad = (uint32_t)n_pad;
+        sp.cols = (uint32_t)cols;
+        sp.x_stride = a.x_stride;
+        Cmd c0;
+        c0.fn = b->gpu->q8_frag_x;
+        c0.name = "lng_q8_frag_x";
+        c0.grid[0] = (unsigned)((n_pad / 16 * (cols / 32) * 64 + 255) / 256);
+        c0.block = 256;
+        set_args(c0, sp);
+        b->cmds.push_back(std::move(c0));
+        a.x_hi = sp.hi;
+    }
+    Cmd c;
+    c.fn = b->gpu->q8_mid[x_bf16][tile];
+    c.name = t.name[x_bf16];
+    c.grid[0] = (unsigned)ids;
+    c.block = 64 * t.waves;
+    // the wavefronts' partial tiles at the end; before that the scales and the wavefronts' turning buffers
+    c.lds = (unsigned)std::max<uint64_t>(t.waves * t.rows * pos * 4, t.rows * (cols / 32) * 2 + (x_bf16 ? t.waves * pos * 80 : 0));
+    set_args(c, a);
+    b->cmds.push_back(std::move(c));
+    return LNG_OK;
+}
+
 // Many positions: bound by the matrix unit.
 int q8_record_tiled(lng_batch *b, lng_k_q8 a, bool x_bf16) {
     const uint64_t n = a.n, cols = a.cols, rows = a.rows;
@@ -1994,7 +2066,12 @@ int q8_product(lng_batch *b, const lng_slice &codes, const lng_slice &scales, co
         q8_record_stream(b, q.a, (rows + 15) / 16, x_bf16);
         return LNG_OK;
     }
-    return q8_record_tiled(b, q.a, x_bf16);
+    const int tile = q8_mid_tile(b->gpu, n, cols, x_bf16);
+    if (tile < 0) return q8_record_tiled(b, q.a, x_bf16);
+    q.a.tiles = (uint32_t)((rows + q8_mid_tiles[tile].rows - 1) / q8_mid_tiles[tile].rows);
+    if (int rc = q8_record_mid(b, q.a, x_bf16, tile)) return rc;
+    b->dispatches += 1;
+    return LNG_OK;
 }
 
 } // namespace
@@ -2089,7 +2166,8 @@ int q8_many(lng_batch *b, const lng_q8_matrix *matrices, size_t n_matrices, lng_
             if (overlaps(q[i].y, onw)) return fail(LNG_ERR_DISPATCH, "output overlaps an input");
         }
     }
-    if (n >= 32) { // the matrix unit is the bound there, not the launches: one product after the other
+    const int tile = n >= 32 ? q8_mid_tile(b->gpu, n, cols, false) : -1;
+    if (n >= 32 && tile < 0) { // the matrix unit is the bound there, not the launches: one product after the other
         const size_t cmds = b->cmds.size(), dispatches = b->dispatches;
         for (size_t i = 0; i < n_matrices; ++i) {
             if (int rc = q8_record_tiled(b, q[i].a, false)) {
@@ -2100,8 +2178,9 @@ int q8_many(lng_batch *b, const lng_q8_matrix *matrices, size_t n_matrices, lng_
         }
         return LNG_OK;
     }
+    const uint64_t tile_rows = tile < 0 ? 16 : q8_mid_tiles[tile].rows;
     lng_k_q8 a = q[0].a;
-    uint64_t tiles = (a.rows + 15) / 16;
+    uint64_t tiles = (a.rows + tile_rows - 1) / tile_rows;
     a.n_more = (uint32_t)(n_matrices - 1);
     for (size_t i = 1; i < n_matrices; ++i) {
         auto &m = a.more[i - 1];
@@ -2111,9 +2190,15 @@ int q8_many(lng_batch *b, const lng_q8_matrix *matrices, size_t n_matrices, lng_
         m.rows = q[i].a.rows;
         m.y_stride = q[i].a.y_stride;
         m.first_tile = (uint32_t)tiles;
-        tiles += (q[i].a.rows + 15) / 16;
+        tiles += (q[i].a.rows + tile_rows - 1) / tile_rows;
     }
     if (!fits_u32(tiles) || tiles > 0x7fffffffull) return fail(LNG_ERR_DISPATCH, "too large");
+    if (tile >= 0) { // one split of the positions, one product of all matrices; counted as the products it stands for
+        a.tiles = (uint32_t)tiles;
+        if (int rc = q8_record_mid(b, a, false, tile)) return rc;
+        b->dispatches += n_matrices;
+        return LNG_OK;
+    }
     if (norm_w) {
         a.norm_w = (const float *)((const char *)onw.buf->ptr + norm_w->offset);
         a.eps = eps;

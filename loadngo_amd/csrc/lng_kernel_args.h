@@ -182,7 +182,7 @@ typedef struct lng_k_q8 {
     const float *norm_w;
     const float *bias;
     uint32_t accumulate;
-    uint32_t pad_;
+    uint32_t tiles;          /* row tiles of all matrices of the dispatch (lng_q8_mid*) */
     struct lng_k_q8_more {
         const int8_t *codes;
         const uint16_t *scales;

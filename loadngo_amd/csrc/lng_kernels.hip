@@ -2175,6 +2175,8 @@ extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16(lng_k_q8 a) 
     q8_tiled_body<8, 1>(a);
 }
 
+#include "lng_q8_mid.h"
+
 // Synthetic data (see LNG_SYNTH_STD in lng_kernel_args.h for the exact integers).
 // A plain streaming read: the XOR of every 16-byte word of a buffer. Consecutive lanes read consecutive 16-byte
 // words (a wavefront instruction = eight whole 128-byte lines), four loads in flight per lane and turn; the yardstick

@@ -385,3 +385,45 @@ def test_output_projection_with_bias_and_residual_folded_in(gpu, n, bf16):
         assert not np.isnan(together).any() and np.array_equal(together, apart)
         assert not np.array_equal(together.reshape(n, h_stride)[:, :rows], h[:, :rows])
         assert np.array_equal(together.reshape(n, h_stride)[:, rows:], h[:, rows:])
+
+
+@pytest.mark.parametrize("rows,cols,n,bf16", [
+    (64, 32, 32, False), (37, 96, 33, False), (300, 160, 64, False), (100, 64, 128, False), (129, 2880, 129, False), (65, 224, 1281, False),
+    (64, 16384, 40, False), (64, 16416, 40, False),
+    (64, 32, 32, True), (37, 96, 48, True), (300, 160, 49, True), (100, 64, 128, True), (129, 4096, 129, True), (65, 224, 1281, True),
+    (64, 16384, 130, True)])
+def test_products_whose_wavefronts_share_the_columns(gpu, rows, cols, n, bf16):
+    """32 positions or more: the tiles' edges in rows and positions, the positions at which the tile changes, one block,
+    an odd number of blocks (a last pair of one), fewer pairs than wavefronts, the widest matrix whose scales LDS holds and
+    one wider; scales off a 4-byte boundary; gaps of y untouched. The reference's bound (glue.rs:171), and the kernel of
+    256 x 128 tiles within twice the distance of either from float64."""
+    from tests.helpers import from_bf16_bits, to_bf16_bits
+    codes, bits, elements = q8_test_matrix(rows, cols, 80 + rows)
+    x = xorshift_values(23, n * cols).reshape(n, cols)
+    xin = to_bf16_bits(x) if bf16 else x
+    want = (from_bf16_bits(xin) if bf16 else x).astype(np.float64) @ elements.T
+    y_stride = rows + 4
+    y_len = ((n - 1) * y_stride + rows) * 4
+    bufs = [gpu.upload(codes), gpu.upload(np.concatenate([np.array([0x7E00], np.uint16), bits])), gpu.upload(xin), gpu.buffer(y_len)]
+    outs = []
+    try:
+        for force in ("1", "0"):
+            gpu.debug_set("LNG_Q8_MID", force)
+            bufs[3].fill(0xFF)
+            batch = gpu.batch(bufs)
+            m = (C.Slice(0, 0, codes.nbytes), C.Slice(1, 2, bits.nbytes))
+            (batch.gemm_q8_0_bf16 if bf16 else batch.gemm_q8_0)(m, C.Slice(2, 0, xin.nbytes), C.Slice(3, 0, y_len), rows, cols, n, (cols, y_stride))
+            done = batch.run()
+            assert not isinstance(done.gpu_time, Exception), done.gpu_time
+            batch.drop()
+            out = np.full(n * y_stride, np.nan, np.float32)
+            out[:y_len // 4] = bufs[3].read(np.float32)
+            outs.append(out.reshape(n, y_stride))
+    finally:
+        gpu.debug_set("LNG_Q8_MID", None)
+    for b in bufs:
+        b.free()
+    for out in outs:
+        assert not np.isnan(out[:, :rows]).any() and np.isnan(out[:-1, rows:]).all()
+        assert np.abs(out[:, :rows] - want).max() / np.abs(want).max() < 1e-5
+    assert np.abs(outs[0][:, :rows] - outs[1][:, :rows]).max() / np.abs(want).max() < 2e-5
