@@ -112,7 +112,6 @@ int lng_hip_device_name(lng_gpu *gpu, char *name, size_t cap);
  *   LNG_PREFILL_PAIR 0|1     never / whenever possible the prompt-pass kernel of one workgroup per (query tile, kv head, pair of heads)
  *   LNG_PREFILL_UPFRONT 0    narrow windows on the tile-by-tile kernel
  *   LNG_PREFILL_SPLITS n     workgroups per (query tile, kv head) of a prompt pass with fewer workgroups than compute units
- *   LNG_Q8_W16               the one-position Q8_0 kernel always as 16-wavefront workgroups
  *   LNG_Q8_MID 0|1           never / whenever possible the Q8_0 kernel whose wavefronts share the columns of a tile (32 positions or more)
  *   LNG_CHECKSUM_WGS n       workgroups per compute unit of lng_hip_checksum's streaming read (default 2)
  *   LNG_TABLE_IN_PLACE n     row tables of n bytes or more stay in pinned host memory, where the kernels read them,

@@ -70,7 +70,6 @@ struct Knobs {
     bool plain_row_by_row = false; // LNG_PLAIN_ROW_BY_ROW: the row-by-row operator never takes a prompt-pass kernel
     bool decode_o3 = false;        // LNG_DECODE_O3: never the four-wavefront build of the decode kernel
     bool merge_wide = false;       // LNG_MERGE_WIDE: always the merge of one workgroup per query head
-    bool q8_w16 = false;           // LNG_Q8_W16: the one-position Q8_0 kernel always as 16-wavefront workgroups
     bool wide_row_by_row = false;  // LNG_WIDE_ROW_BY_ROW: prompt passes of head widths 128-512 row by row on the decode kernels
     int prefill_stream = -1;       // LNG_PREFILL_STREAM: 0 never the resident prompt-pass kernel, 1 whenever it can run, -1 planner
     int prefill_pair = -1;         // LNG_PREFILL_PAIR: 0 never the head-pair prompt-pass kernel, 1 whenever it can run, -1 planner
@@ -124,8 +123,9 @@ struct lng_gpu {
     hipFunction_t checksum = nullptr, checksum_fold = nullptr;
     hipFunction_t copy_rows = nullptr, fill_synthetic = nullptr, add_rows = nullptr, rotate_halves = nullptr, rmsnorm_rows = nullptr, rmsnorm_row_wg = nullptr;
     hipFunction_t prepare_v4 = nullptr, prepare_v1 = nullptr;
-    hipFunction_t q8_split_x = nullptr, q8_stream = nullptr, q8_stream_one = nullptr, q8_stream_one_w8 = nullptr, q8_stream_bf16 = nullptr, q8_tiled = nullptr,
+    hipFunction_t q8_split_x = nullptr, q8_tiled = nullptr,
                   q8_tiled_bf16 = nullptr, q8_frag_x = nullptr;
+    hipFunction_t q8_norm_frag = nullptr, q8_few[2] = {}, q8_one[2] = {}; // [bf16 positions]
     hipFunction_t q8_mid[2][4] = {}; // [bf16 positions][tile, see q8_mid_tile]
     std::string name;
     unsigned cus = 256;
@@ -274,7 +274,7 @@ int check_shape(const lng_grouped_shape &s, bool tiled) {
 
 // One development switch by its environment name; value NULL puts the default back. Returns false for an unknown name.
 const char *const knob_names[] = {"LNG_WIDE_GENERIC", "LNG_F32_GENERIC", "LNG_PLAIN_ROW_BY_ROW", "LNG_DECODE_O3", "LNG_MERGE_WIDE",
-                                  "LNG_Q8_W16", "LNG_Q8_MID", "LNG_WIDE_ROW_BY_ROW", "LNG_PREFILL_STREAM", "LNG_PREFILL_PAIR", "LNG_PREFILL_UPFRONT",
+                                  "LNG_Q8_MID", "LNG_WIDE_ROW_BY_ROW", "LNG_PREFILL_STREAM", "LNG_PREFILL_PAIR", "LNG_PREFILL_UPFRONT",
                                   "LNG_PREFILL_SPLITS", "LNG_DECODE_WGS", "LNG_FUSE_WGS", "LNG_COUNT_SECOND_PASSES", "LNG_CHECKSUM_WGS", "LNG_TABLE_IN_PLACE"};
 bool set_knob(lng_gpu *g, const char *name, const char *value) {
     Knobs &k = g->knobs;
@@ -287,7 +287,6 @@ bool set_knob(lng_gpu *g, const char *name, const char *value) {
     if (!strcmp(name, "LNG_PLAIN_ROW_BY_ROW")) return flag(k.plain_row_by_row);
     if (!strcmp(name, "LNG_DECODE_O3")) return flag(k.decode_o3);
     if (!strcmp(name, "LNG_MERGE_WIDE")) return flag(k.merge_wide);
-    if (!strcmp(name, "LNG_Q8_W16")) return flag(k.q8_w16);
     if (!strcmp(name, "LNG_WIDE_ROW_BY_ROW")) return flag(k.wide_row_by_row);
     if (!strcmp(name, "LNG_COUNT_SECOND_PASSES")) return flag(k.count_second_passes);
     if (!strcmp(name, "LNG_PREFILL_STREAM")) return choice(k.prefill_stream, defaults.prefill_stream);
@@ -1050,13 +1049,14 @@ extern "C" int lng_hip_open(int device, lng_gpu **out) {
         {"lng_prepare_v4", &g->prepare_v4, true},
         {"lng_prepare_v1", &g->prepare_v1, true},
         {"lng_q8_split_x", &g->q8_split_x, true},
-        {"lng_q8_stream", &g->q8_stream, true},
-        {"lng_q8_stream_one", &g->q8_stream_one, true},
-        {"lng_q8_stream_one_w8", &g->q8_stream_one_w8, true},
         {"lng_q8_tiled", &g->q8_tiled, true},
         {"lng_q8_tiled_bf16", &g->q8_tiled_bf16, true},
-        {"lng_q8_stream_bf16", &g->q8_stream_bf16, true},
         {"lng_q8_frag_x", &g->q8_frag_x, true},
+        {"lng_q8_norm_frag", &g->q8_norm_frag, true},
+        {"lng_q8_few", &g->q8_few[0], true},
+        {"lng_q8_few_bf16", &g->q8_few[1], true},
+        {"lng_q8_one", &g->q8_one[0], true},
+        {"lng_q8_one_bf16", &g->q8_one[1], true},
         {"lng_q8_mid_r32p32", &g->q8_mid[0][1], true},
         {"lng_q8_mid_r64p64", &g->q8_mid[0][3], true},
         {"lng_q8_mid_bf16_r16p32", &g->q8_mid[1][0], true},
@@ -1927,23 +1927,6 @@ int q8_check(lng_batch *b, const lng_slice &codes, const lng_slice &scales, cons
     return LNG_OK;
 }
 
-// Few positions (n < 32): bound by reading the matrix, one pass over it per 16 positions, x split in registers.
-// `a` may name further matrices of the same dispatch (a.more); row_tiles counts the tiles of all of them.
-void q8_record_stream(lng_batch *b, const lng_k_q8 &a, uint64_t row_tiles, bool x_bf16) {
-    const bool one = a.n == 1 && a.cols <= 12288 && !x_bf16; // x of a single position is held in LDS (Q8S_X1 floats)
-    // more row tiles than compute units (several matrices): 8-wavefront workgroups, two per unit, one round
-    const bool w8 = one && row_tiles > b->gpu->cus && !b->gpu->knobs.q8_w16;
-    Cmd c;
-    c.fn = x_bf16 ? b->gpu->q8_stream_bf16 : w8 ? b->gpu->q8_stream_one_w8 : one ? b->gpu->q8_stream_one : b->gpu->q8_stream;
-    c.name = x_bf16 ? "lng_q8_stream_bf16" : w8 ? "lng_q8_stream_one_w8" : one ? "lng_q8_stream_one" : "lng_q8_stream";
-    c.grid[0] = (unsigned)row_tiles;
-    c.grid[1] = (unsigned)((a.n + 15) / 16);
-    c.block = w8 ? 512 : 1024;
-    set_args(c, a);
-    b->cmds.push_back(std::move(c));
-    b->dispatches += 1;
-}
-
 // The tiles of lng_q8_mid*: rows, positions, wavefronts that share the columns.
 struct Q8MidTile {
     unsigned rows, pos, waves;
@@ -1954,17 +1937,46 @@ const Q8MidTile q8_mid_tiles[4] = {{16, 32, 8, {nullptr, "lng_q8_mid_bf16_r16p32
                                    {32, 64, 4, {nullptr, "lng_q8_mid_bf16_r32p64"}},
                                    {64, 64, 4, {"lng_q8_mid_r64p64", "lng_q8_mid_bf16_r64p64"}}};
 
-// The tile a product of 32 positions or more takes; -1: lng_q8_tiled. It depends on nothing that differs between a
+// The tile of lng_q8_mid* a product takes; -1: lng_q8_few (fewer than 32 positions) or lng_q8_tiled. It depends on nothing that differs between a
 // product alone and among several matrices, so that its sums keep their order.
 // Measured (2,880 x 4,096 bf16 / the 5,120 x 2,880 of q, k and v), us: tiles 16 x 32, 32 x 32, 32 x 64, 64 x 64 at 32
 // positions 8.7, 11, 15, 22 / 14, 12, 16, 22; at 77 20, 19, 16, 24 / 24, 19, 26, 25; at 192 33, 28, 27, 25 / 44, 33, 29, 28.
 // Against lng_q8_tiled: 1,280 positions 82 / 135 against 91 / 297, 1,536 99 / 169 against 92 / 305 (one matrix of 4,096
 // rows 133 against 113): x no longer stays in the L2 caches between the row tiles.
 int q8_mid_tile(const lng_gpu *g, uint64_t n, uint64_t cols, bool x_bf16) {
-    if (g->knobs.q8_mid == 0 || cols > 32 * 512) return -1; // a tile's scales are held in LDS: at most 64 KB of them
-    if (g->knobs.q8_mid < 0 && n > 1280) return -1;
+    if (n <= 16) return -1; // q8_record_few (17 to 31 as two groups of 16 would read the codes twice)
+    if (cols > 32 * 512) return -1; // a tile's scales are held in LDS: at most 64 KB of them
+    if (n >= 32 && (g->knobs.q8_mid == 0 || (g->knobs.q8_mid < 0 && n > 1280))) return -1;
     if (x_bf16) return n <= 48 ? 0 : n <= 128 ? 2 : 3;
     return n <= 128 ? 1 : 3;
+}
+
+// f32 positions into operand order (a.x_hi): all at once for lng_q8_few, lng_q8_mid and every matrix of the dispatch.
+// Fewer than 32: a workgroup per position, with the RMS norm if a.norm_w is set.
+int q8_record_frag(lng_batch *b, lng_k_q8 *a, uint64_t n_pad) {
+    const uint64_t cols = a->cols;
+    if (!fits_u32(n_pad * cols)) return fail(LNG_ERR_DISPATCH, "too large");
+    char *planes = nullptr;
+    if (int rc = reserve_x(b->gpu, 2 * n_pad * cols * 2, &planes)) return rc;
+    lng_k_q8_split sp{};
+    sp.x = a->x;
+    sp.hi = (uint16_t *)planes;
+    sp.n = a->n;
+    sp.n_pad = (uint32_t)n_pad;
+    sp.cols = a->cols;
+    sp.x_stride = a->x_stride;
+    sp.norm_w = a->norm_w;
+    sp.eps = a->eps;
+    const bool few = a->n < 32;
+    Cmd c;
+    c.fn = few ? b->gpu->q8_norm_frag : b->gpu->q8_frag_x;
+    c.name = few ? "lng_q8_norm_frag" : "lng_q8_frag_x";
+    c.grid[0] = few ? a->n : (unsigned)((n_pad / 16 * (cols / 32) * 64 + 255) / 256);
+    c.block = few ? 512 : 256;
+    set_args(c, sp);
+    b->cmds.push_back(std::move(c));
+    a->x_hi = sp.hi;
+    return LNG_OK;
 }
 
 // A chunk of positions: too few tiles of lng_q8_tiled to fill the device.
@@ -1972,27 +1984,11 @@ int q8_mid_tile(const lng_gpu *g, uint64_t n, uint64_t cols, bool x_bf16) {
 int q8_record_mid(lng_batch *b, lng_k_q8 a, bool x_bf16, int tile) {
     const Q8MidTile &t = q8_mid_tiles[tile];
     const uint64_t n = a.n, cols = a.cols, pos = t.pos;
-    const uint64_t pos_tiles = (n + pos - 1) / pos, n_pad = pos_tiles * pos;
+    const uint64_t pos_tiles = (n + pos - 1) / pos;
     const uint64_t ids = 8 * ((uint64_t)(a.tiles + 7) / 8) * pos_tiles;
-    if (ids > 0x7fffffffull || !fits_u32(n_pad * cols)) return fail(LNG_ERR_DISPATCH, "too large");
+    if (ids > 0x7fffffffull) return fail(LNG_ERR_DISPATCH, "too large");
     if (!x_bf16) {
-        char *planes = nullptr;
-        if (int rc = reserve_x(b->gpu, 2 * n_pad * cols * 2, &planes)) return rc;
-        lng_k_q8_split sp{};
-        sp.x = a.x;
-        sp.hi = (uint16_t *)planes;
-        sp.n = (uint32_t)n;
-        sp.n_pad = (uint32_t)n_pad;
-        sp.cols = (uint32_t)cols;
-        sp.x_stride = a.x_stride;
-        Cmd c0;
-        c0.fn = b->gpu->q8_frag_x;
-        c0.name = "lng_q8_frag_x";
-        c0.grid[0] = (unsigned)((n_pad / 16 * (cols / 32) * 64 + 255) / 256);
-        c0.block = 256;
-        set_args(c0, sp);
-        b->cmds.push_back(std::move(c0));
-        a.x_hi = sp.hi;
+        if (int rc = q8_record_frag(b, &a, pos_tiles * pos)) return rc;
     }
     Cmd c;
     c.fn = b->gpu->q8_mid[x_bf16][tile];
@@ -2001,6 +1997,28 @@ int q8_record_mid(lng_batch *b, lng_k_q8 a, bool x_bf16, int tile) {
     c.block = 64 * t.waves;
     // the wavefronts' partial tiles at the end; before that the scales and the wavefronts' turning buffers
     c.lds = (unsigned)std::max<uint64_t>(t.waves * t.rows * pos * 4, t.rows * (cols / 32) * 2 + (x_bf16 ? t.waves * pos * 80 : 0));
+    set_args(c, a);
+    b->cmds.push_back(std::move(c));
+    return LNG_OK;
+}
+
+// Fewer than 32 positions: bound by reading the matrix, in tiles of 16 rows. One position splits (and normalises) x in
+// the kernel, whose LDS holds up to 48 KB of it; more go through the planes of q8_record_frag.
+// `a` may name further matrices of the same dispatch (first_tile in tiles of 16 rows).
+int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
+    const uint64_t blocks = a.cols / 32, groups = (a.n + 15) / 16;
+    const bool one = a.n == 1 && a.cols <= (x_bf16 ? 24576u : 12288u);
+    if (!one && !x_bf16) {
+        if (int rc = q8_record_frag(b, &a, groups * 16)) return rc;
+    }
+    Cmd c;
+    c.fn = one ? b->gpu->q8_one[x_bf16] : b->gpu->q8_few[x_bf16];
+    c.name = one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
+    c.grid[0] = (unsigned)row_tiles;
+    c.grid[1] = (unsigned)groups;
+    c.block = 512;
+    const uint64_t scales = blocks <= 512 ? 16 * (((blocks + 1) / 2) | 1) * 4 : 0; // both of a pair of blocks in a word
+    c.lds = (unsigned)(scales + (one ? a.cols * (x_bf16 ? 2u : 4u) : x_bf16 ? 8 * 2 * 16 * 80 : 0)); // x's planes, or the turning buffers
     set_args(c, a);
     b->cmds.push_back(std::move(c));
     return LNG_OK;
@@ -2057,21 +2075,23 @@ int q8_record_tiled(lng_batch *b, lng_k_q8 a, bool x_bf16) {
     return LNG_OK;
 }
 
+// A product of one matrix.
+int q8_record(lng_batch *b, lng_k_q8 a, bool x_bf16) {
+    const int tile = q8_mid_tile(b->gpu, a.n, a.cols, x_bf16);
+    if (tile < 0 && a.n >= 32) return q8_record_tiled(b, a, x_bf16);
+    const uint64_t tile_rows = tile < 0 ? 16 : q8_mid_tiles[tile].rows;
+    a.tiles = (uint32_t)((a.rows + tile_rows - 1) / tile_rows);
+    if (int rc = tile < 0 ? q8_record_few(b, a, a.tiles, x_bf16) : q8_record_mid(b, a, x_bf16, tile)) return rc;
+    b->dispatches += 1;
+    return LNG_OK;
+}
+
 int q8_product(lng_batch *b, const lng_slice &codes, const lng_slice &scales, const lng_slice &x, const lng_slice &y,
                uint64_t rows, uint64_t cols, uint64_t n, uint64_t x_stride, uint64_t y_stride, bool gemm, bool tiled,
                bool x_bf16 = false) {
     Q8Checked q;
     if (int rc = q8_check(b, codes, scales, x, y, rows, cols, n, x_stride, y_stride, gemm, tiled, x_bf16, &q)) return rc;
-    if (n < 32) {
-        q8_record_stream(b, q.a, (rows + 15) / 16, x_bf16);
-        return LNG_OK;
-    }
-    const int tile = q8_mid_tile(b->gpu, n, cols, x_bf16);
-    if (tile < 0) return q8_record_tiled(b, q.a, x_bf16);
-    q.a.tiles = (uint32_t)((rows + q8_mid_tiles[tile].rows - 1) / q8_mid_tiles[tile].rows);
-    if (int rc = q8_record_mid(b, q.a, x_bf16, tile)) return rc;
-    b->dispatches += 1;
-    return LNG_OK;
+    return q8_record(b, q.a, x_bf16);
 }
 
 } // namespace
@@ -2129,8 +2149,7 @@ extern "C" int lng_hip_gemm_q8_0_residual(lng_batch *b, lng_slice codes, lng_sli
         q.a.bias = (const float *)((const char *)ob.buf->ptr + bias->offset);
     }
     q.a.accumulate = 1;
-    q8_record_stream(b, q.a, (rows + 15) / 16, x_dtype == LNG_BF16);
-    return LNG_OK;
+    return q8_record(b, q.a, x_dtype == LNG_BF16);
 }
 
 namespace {
@@ -2166,7 +2185,7 @@ int q8_many(lng_batch *b, const lng_q8_matrix *matrices, size_t n_matrices, lng_
             if (overlaps(q[i].y, onw)) return fail(LNG_ERR_DISPATCH, "output overlaps an input");
         }
     }
-    const int tile = n >= 32 ? q8_mid_tile(b->gpu, n, cols, false) : -1;
+    const int tile = q8_mid_tile(b->gpu, n, cols, false);
     if (n >= 32 && tile < 0) { // the matrix unit is the bound there, not the launches: one product after the other
         const size_t cmds = b->cmds.size(), dispatches = b->dispatches;
         for (size_t i = 0; i < n_matrices; ++i) {
@@ -2193,17 +2212,13 @@ int q8_many(lng_batch *b, const lng_q8_matrix *matrices, size_t n_matrices, lng_
         tiles += (q[i].a.rows + tile_rows - 1) / tile_rows;
     }
     if (!fits_u32(tiles) || tiles > 0x7fffffffull) return fail(LNG_ERR_DISPATCH, "too large");
-    if (tile >= 0) { // one split of the positions, one product of all matrices; counted as the products it stands for
-        a.tiles = (uint32_t)tiles;
-        if (int rc = q8_record_mid(b, a, false, tile)) return rc;
-        b->dispatches += n_matrices;
-        return LNG_OK;
-    }
+    a.tiles = (uint32_t)tiles;
     if (norm_w) {
         a.norm_w = (const float *)((const char *)onw.buf->ptr + norm_w->offset);
         a.eps = eps;
     }
-    q8_record_stream(b, a, tiles, false);
+    if (int rc = tile < 0 ? q8_record_few(b, a, tiles, false) : q8_record_mid(b, a, false, tile)) return rc;
+    b->dispatches += n < 32 ? 1 : n_matrices; // from 32 positions on counted as the products it stands for
     return LNG_OK;
 }
 } // namespace

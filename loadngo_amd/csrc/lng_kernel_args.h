@@ -147,7 +147,7 @@ typedef struct lng_k_prepare {
 } lng_k_prepare;
 
 /* x[n][x_stride] f32 -> two bf16 planes [n_pad][cols]: hi = nearest bf16 of x, lo = nearest bf16
- * of x - hi; rows n..n_pad are zero. */
+ * of x - hi; rows n..n_pad are zero (lng_q8_norm_frag: left alone). */
 typedef struct lng_k_q8_split {
     const float *x;
     uint16_t *hi;
@@ -156,14 +156,17 @@ typedef struct lng_k_q8_split {
     uint32_t n_pad;
     uint32_t cols;
     uint32_t x_stride;
+    const float *norm_w;     /* lng_q8_norm_frag: weights of the RMS norm, or NULL */
+    float eps;
+    uint32_t pad_;
 } lng_k_q8_split;
 
 /* y[p][r] = sum over blocks b of scale[r][b] * sum_i codes[r][32b+i] * x[p][32b+i]. */
 typedef struct lng_k_q8 {
     const int8_t *codes;     /* [rows][cols] */
     const uint16_t *scales;  /* [rows][cols/32] binary16 */
-    const float *x;          /* [n][x_stride] (few positions: split in registers) */
-    const uint16_t *x_hi;    /* [n_pad][cols] bf16 (many positions: the planes lng_q8_split_x wrote) */
+    const float *x;          /* [n][x_stride] (one position: split by the kernel) */
+    const uint16_t *x_hi;    /* [n_pad][cols] bf16 (the planes lng_q8_split_x, lng_q8_frag_x or lng_q8_norm_frag wrote) */
     const uint16_t *x_lo;
     float *y;                /* [n][y_stride] */
     uint32_t rows;
@@ -177,7 +180,7 @@ typedef struct lng_k_q8 {
      * Workgroups from `first_tile` (in units of 16 rows) on belong to matrix more[i]; first_tile ascends. */
     uint32_t n_more;         /* 0..LNG_Q8_MORE */
     float eps;               /* of the RMS norm, when norm_w is set */
-    /* Few positions only. norm_w: x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
+    /* Few positions only. norm_w (one position): x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
      * (cols <= 12288). bias: y gets bias[row] added. accumulate: the result is added to what y holds (a residual). */
     const float *norm_w;
     const float *bias;

@@ -1686,20 +1686,6 @@ extern "C" __global__ __launch_bounds__(256) void lng_q8_split_x(lng_k_q8_split 
     *(uint2 *)(a.lo + at) = make_uint2((uint32_t)lo[0] | ((uint32_t)lo[1] << 16), (uint32_t)lo[2] | ((uint32_t)lo[3] << 16));
 }
 
-// Eight signed bytes as eight bf16 values (exact: |code| <= 128 has at most 8 significant bits, so
-// the upper half of its f32 form is the whole number).
-__device__ __forceinline__ bf16x8 q8_codes_to_bf16(uint2 raw) {
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t word = i < 2 ? raw.x : raw.y;
-        const float f0 = (float)(int8_t)(word >> (16 * (i & 1)));
-        const float f1 = (float)(int8_t)(word >> (16 * (i & 1) + 8));
-        w[i] = (__float_as_uint(f0) >> 16) | (__float_as_uint(f1) & 0xffff0000u);
-    }
-    return as_bf16x8(make_uint4(w[0], w[1], w[2], w[3]));
-}
-
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t bits) {
     return (float)__builtin_bit_cast(_Float16, bits);
 }
@@ -1714,20 +1700,6 @@ __device__ __forceinline__ void q8_split8(const float (&x)[8], bf16x8 &hi, bf16x
     }
 }
 
-// Few positions (one pass of the matrix per 16; bound by reading the matrix, in practice by the
-// number of load instructions a compute unit can take: some 40 cycles each): a workgroup takes
-// 16 rows, its sixteen wavefronts take every sixteenth block of the rows and their partial sums
-// meet in LDS. Lane l holds row l % 16 and, of each block, the 8 columns of group l / 16 - the B
-// operand; positions are the A operand, read as f32 and split in registers. All loads of up to
-// eight blocks are issued before the first product; blocks past the end are skipped, loads and
-// all (the test is the same for the whole wavefront); the rows' scales come through LDS. ONE: a
-// single position, whose x the
-// workgroup first copies to LDS with 16-byte loads (a wavefront's two x loads per block become
-// two LDS reads; x must fit Q8S_X1 floats). Grid: x = 16-row tiles, y = 16-position tiles.
-#define Q8S_WAVES 16
-#define Q8S_UNROLL 8 // blocks in flight per wavefront: 128 blocks (4096 columns) in one turn
-#define Q8S_X1 12288 // floats of x held in LDS by the one-position form (48 KB)
-#define Q8S_SC_BLOCKS 512 // rows of up to this many blocks (16,384 columns) have their scales staged through LDS
 // The matrix a workgroup of a several-matrix dispatch works on becomes the one `a` names; returns its row tile.
 __device__ __forceinline__ uint32_t q8_select_matrix(lng_k_q8 &a) {
     uint32_t tile = blockIdx.x;
@@ -1743,188 +1715,6 @@ __device__ __forceinline__ uint32_t q8_select_matrix(lng_k_q8 &a) {
         }
     }
     return tile;
-}
-
-// WAVES wavefronts share the blocks of a row tile (16; 8 for the one-position form when two workgroups per compute
-// unit cover the row tiles in one round instead of two).
-template <bool ONE, bool XBF16 = false, int WAVES = Q8S_WAVES>
-__device__ __forceinline__ void q8_stream_body(const lng_k_q8 &a, uint32_t tile) {
-    static_assert(ONE || WAVES == 16, "the several-position forms map wavefront w to position w of 16");
-    __shared__ float s_part[Q8S_WAVES - 1][4][64];
-    // ONE: the position's x (normalised there, if asked); otherwise the weights of the RMS norm, if asked
-    __shared__ __attribute__((aligned(16))) float s_x1[(ONE || !XBF16) ? Q8S_X1 : 4];
-    __shared__ __attribute__((aligned(4))) uint16_t s_sc[16 * Q8S_SC_BLOCKS];
-    __shared__ float s_norm[16]; // ONE: partial sums of squares; otherwise the 16 positions' scales
-    const bool normed = !XBF16 && a.norm_w != nullptr; // uniform
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t j = lane & 15u, kg = lane >> 4;
-    const uint32_t r0 = tile * 16u, p0 = blockIdx.y * 16u;
-    const uint32_t row = r0 + j < a.rows ? r0 + j : a.rows - 1u;
-    const uint32_t pos = p0 + j < a.n ? p0 + j : a.n - 1u; // rows of the product past n are not stored
-    const uint32_t blocks = a.cols / 32u;
-    const int8_t *wrow = a.codes + (uint64_t)row * a.cols + 8u * kg;
-    const uint16_t *srow = a.scales + (uint64_t)row * blocks;
-    const float *xrow = a.x + (uint64_t)pos * a.x_stride + 8u * kg;
-    const uint16_t *xrow16 = a.x_hi + (uint64_t)pos * a.plane_stride + 8u * kg; // XBF16: positions in bf16
-    floatx4 y = {0.0f, 0.0f, 0.0f, 0.0f};
-    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    // The scales of the workgroup's 16 rows are one contiguous run (rows follow each other): copied to
-    // LDS a dword per thread, instead of 2-byte loads from 16 different rows per block and wavefront.
-    const bool sc_staged = blocks <= Q8S_SC_BLOCKS && r0 + 16u <= a.rows && ((uintptr_t)a.scales & 3u) == 0;
-    if (!ONE && normed) { // wavefront w works out the scale of position p0 + w (there are 16 of each)
-        const uint32_t pw = p0 + wave < a.n ? p0 + wave : a.n - 1u;
-        const float *xp = a.x + (uint64_t)pw * a.x_stride;
-        float ss = 0.0f;
-        for (uint32_t c = 4u * lane; c < a.cols; c += 256u) {
-            const float4 v = *(const float4 *)(xp + c);
-            ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        if (lane == 0) s_norm[wave] = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
-    }
-    bool staged = false;
-    floatx4 y0 = zero4; // stream 0's sum (wavefront 0)
-    for (uint32_t stream = wave; stream < Q8S_WAVES; stream += WAVES) {
-    y = zero4;
-    for (uint32_t b0 = stream; b0 < blocks || !staged; b0 += Q8S_UNROLL * Q8S_WAVES) {
-        uint2 raw[Q8S_UNROLL];
-        uint16_t scale[Q8S_UNROLL];
-        float4 xa[Q8S_UNROLL], xb[Q8S_UNROLL];
-#pragma unroll
-        for (int u = 0; u < Q8S_UNROLL; ++u) {
-            const uint32_t b = b0 + u * Q8S_WAVES;
-            raw[u] = make_uint2(0, 0);
-            scale[u] = 0;
-            xa[u] = xb[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (b < blocks) { // the same for every lane of the wavefront
-                raw[u] = *(const uint2 *)(wrow + 32u * b);
-                if (!sc_staged) scale[u] = srow[b];
-                if (XBF16) {
-                    xa[u] = *(const float4 *)(xrow16 + 32u * b); // eight bf16 values, used as they are
-                } else if (!ONE) {
-                    xa[u] = *(const float4 *)(xrow + 32u * b);
-                    xb[u] = *(const float4 *)(xrow + 32u * b + 4u);
-                }
-            }
-        }
-        if (!staged) { // every wavefront comes here exactly once, in its first turn
-            if (ONE) {
-                float ss = 0.0f;
-                for (uint32_t i = 4u * threadIdx.x; i < a.cols; i += 4u * 64u * WAVES) {
-                    const float4 v = *(const float4 *)(a.x + i);
-                    *(float4 *)(&s_x1[i]) = v;
-                    ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-                }
-                if (normed) { // every thread normalises the elements it has just written
-#pragma unroll
-                    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-                    if (lane == 0) s_norm[wave] = ss;
-                    __syncthreads();
-                    float total = 0.0f;
-#pragma unroll
-                    for (int w = 0; w < WAVES; ++w) total += s_norm[w];
-                    const float scale = 1.0f / sqrtf(total / (float)a.cols + a.eps);
-                    for (uint32_t i = 4u * threadIdx.x; i < a.cols; i += 4u * 64u * WAVES) {
-                        float4 v = *(const float4 *)(&s_x1[i]);
-                        const float4 nw = *(const float4 *)(a.norm_w + i);
-                        v.x = v.x * scale * nw.x;
-                        v.y = v.y * scale * nw.y;
-                        v.z = v.z * scale * nw.z;
-                        v.w = v.w * scale * nw.w;
-                        *(float4 *)(&s_x1[i]) = v;
-                    }
-                }
-            } else if (normed) {
-                for (uint32_t i = 4u * threadIdx.x; i < a.cols; i += 4u * 64u * WAVES) {
-                    *(float4 *)(&s_x1[i]) = *(const float4 *)(a.norm_w + i);
-                }
-            }
-            if (sc_staged) { // 16 * blocks * 2 bytes from a 32-byte boundary
-                const uint32_t *src = (const uint32_t *)(a.scales + (uint64_t)r0 * blocks);
-                for (uint32_t i = threadIdx.x; i < 8u * blocks; i += 64u * WAVES) ((uint32_t *)s_sc)[i] = src[i];
-            }
-            __syncthreads();
-            staged = true;
-        }
-#pragma unroll
-        for (int u = 0; u < Q8S_UNROLL; ++u) {
-            const uint32_t b = b0 + u * Q8S_WAVES;
-            if (b < blocks) {
-                if (ONE) {
-                    xa[u] = *(const float4 *)(&s_x1[32u * b + 8u * kg]);
-                    xb[u] = *(const float4 *)(&s_x1[32u * b + 8u * kg + 4u]);
-                }
-                const bf16x8 wb = q8_codes_to_bf16(raw[u]);
-                floatx4 acc;
-                if (XBF16) {
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[u]), wb, zero4, 0, 0, 0);
-                } else {
-                    float xs[8] = {xa[u].x, xa[u].y, xa[u].z, xa[u].w, xb[u].x, xb[u].y, xb[u].z, xb[u].w};
-                    if (!ONE && normed) {
-                        const float sp = s_norm[j];
-                        const float4 wa = *(const float4 *)(&s_x1[32u * b + 8u * kg]);
-                        const float4 wb2 = *(const float4 *)(&s_x1[32u * b + 8u * kg + 4u]);
-                        const float nw[8] = {wa.x, wa.y, wa.z, wa.w, wb2.x, wb2.y, wb2.z, wb2.w};
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) xs[e] = xs[e] * sp * nw[e];
-                    }
-                    bf16x8 hi, lo;
-                    q8_split8(xs, hi, lo);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, wb, zero4, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, wb, acc, 0, 0, 0);
-                }
-                const float sc = f16_bits_to_f32(sc_staged ? s_sc[j * blocks + b] : scale[u]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) y[i] = __builtin_fmaf(sc, acc[i], y[i]);
-            }
-        }
-    }
-    if (stream != 0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s_part[stream - 1][i][lane] = y[i];
-    } else {
-        y0 = y;
-    }
-    }
-    __syncthreads();
-    if (wave != 0) return;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float sum = y0[i];
-#pragma unroll
-        for (int w = 0; w < Q8S_WAVES - 1; ++w) sum += s_part[w][i][lane];
-        const uint32_t p = p0 + 4u * kg + i; // accumulator row = position, column = matrix row
-        if (p < a.n && r0 + j < a.rows) {
-            float *yp = a.y + (uint64_t)p * a.y_stride + r0 + j;
-            if (a.bias) sum = sum + a.bias[r0 + j];
-            if (a.accumulate) sum = *yp + sum; // the residual: h + ((W x) + bias), each sum rounded as the separate dispatches round it
-            *yp = sum;
-        }
-    }
-}
-
-extern "C" __global__ __launch_bounds__(64 * Q8S_WAVES) void lng_q8_stream(lng_k_q8 a) {
-    const uint32_t tile = q8_select_matrix(a);
-    q8_stream_body<false>(a, tile);
-}
-
-extern "C" __global__ __launch_bounds__(64 * Q8S_WAVES) void lng_q8_stream_one(lng_k_q8 a) {
-    const uint32_t tile = q8_select_matrix(a);
-    q8_stream_body<true>(a, tile);
-}
-
-// the same with 8 wavefronts: half the LDS partials and threads, two workgroups per compute unit
-extern "C" __global__ __launch_bounds__(512) void lng_q8_stream_one_w8(lng_k_q8 a) {
-    const uint32_t tile = q8_select_matrix(a);
-    q8_stream_body<true, false, 8>(a, tile);
-}
-
-// positions already in bf16 (the output of a bf16 attention): one matrix instruction per block
-extern "C" __global__ __launch_bounds__(64 * Q8S_WAVES) void lng_q8_stream_bf16(lng_k_q8 a) {
-    const uint32_t tile = q8_select_matrix(a);
-    q8_stream_body<false, true>(a, tile);
 }
 
 // Many positions (bound by the matrix unit): a workgroup of eight wavefronts takes 256 rows x 128
@@ -1946,6 +1736,8 @@ extern "C" __global__ __launch_bounds__(64 * Q8S_WAVES) void lng_q8_stream_bf16(
 #define Q8T_POS 128
 #define Q8T_ROWS 256
 #define Q8T_PLANE (Q8T_POS * 64) // bf16 elements of one plane of one stage
+// Eight signed bytes as eight bf16 values (exact: |code| <= 128 has at most 8 significant bits, so
+// the upper half of its f32 form is the whole number).
 __device__ __forceinline__ bf16x8 q8_codes_to_bf16_perm(uint2 raw) {
     uint32_t w[4];
 #pragma unroll
@@ -2176,6 +1968,7 @@ extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16(lng_k_q8 a) 
 }
 
 #include "lng_q8_mid.h"
+#include "lng_q8_few.h"
 
 // Synthetic data (see LNG_SYNTH_STD in lng_kernel_args.h for the exact integers).
 // A plain streaming read: the XOR of every 16-byte word of a buffer. Consecutive lanes read consecutive 16-byte

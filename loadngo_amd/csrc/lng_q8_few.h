@@ -1,0 +1,355 @@
+// Q8_0 products of fewer than 32 positions (17 to 31 share lng_q8_mid's tiles): lng_q8_norm_frag, lng_q8_few*,
+// lng_q8_one*. (Included by lng_kernels.hip after lng_q8_mid.h; see there for how a product goes through the matrix unit.)
+
+// x[n][x_stride] f32 as the A operands of lng_q8_few and lng_q8_mid, RMS-normalised on the way if norm_w is set
+// (x / sqrt(mean(x^2) + eps) * w): one workgroup per position, lng_q8_frag_x's layout. Rows that pad n to whole groups
+// are not written: what the scratch holds there goes into rows of the products that are not stored.
+extern "C" __global__ __launch_bounds__(512) void lng_q8_norm_frag(lng_k_q8_split a) {
+    __shared__ float s_norm[8];
+    const uint32_t p = blockIdx.x, blocks = a.cols / 32u, chunks = a.cols / 8u;
+    const float *xp = a.x + (uint64_t)p * a.x_stride;
+    float x[8] = {};
+    const uint32_t first = threadIdx.x;
+    auto load = [&](uint32_t chunk) {
+        const float4 u = *(const float4 *)(xp + 8u * chunk), v = *(const float4 *)(xp + 8u * chunk + 4u);
+        x[0] = u.x, x[1] = u.y, x[2] = u.z, x[3] = u.w, x[4] = v.x, x[5] = v.y, x[6] = v.z, x[7] = v.w;
+    };
+    float scale = 0.0f;
+    if (a.norm_w) { // uniform
+        float ss = 0.0f;
+        for (uint32_t c = first + 512u; c < chunks; c += 512u) {
+            load(c);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+        }
+        if (first < chunks) {
+            load(first);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+        if ((threadIdx.x & 63u) == 0) s_norm[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        float total = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) total += s_norm[w];
+        scale = 1.0f / sqrtf(total / (float)a.cols + a.eps);
+    } else if (first < chunks) {
+        load(first);
+    }
+    for (uint32_t c = first; c < chunks; c += 512u) {
+        if (c != first) load(c);
+        if (a.norm_w) {
+            const float4 u = *(const float4 *)(a.norm_w + 8u * c), v = *(const float4 *)(a.norm_w + 8u * c + 4u);
+            const float w[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = x[e] * scale * w[e];
+        }
+        bf16x8 hi, lo;
+        q8_split8(x, hi, lo);
+        const uint32_t lane = 16u * q8_mid_chunk(c & 3u) + (p & 15u); // (q8_mid_chunk is its own inverse)
+        uint4 *to = (uint4 *)a.hi + ((uint64_t)(p >> 4) * blocks + (c >> 2)) * 128u + lane;
+        to[0] = __builtin_bit_cast(uint4, hi);
+        to[64] = __builtin_bit_cast(uint4, lo);
+    }
+}
+
+// The matrix, in the workgroup's run of 16 rows: wavefront w of NW takes a contiguous run of block pairs; a lane loads 16
+// bytes of a row at once, which one swap of register halves makes the B operands of both blocks (lng_q8_mid).
+// The rows' scales wait in LDS, both of a pair in one word, rows an odd number of words apart (no two of the sixteen in
+// one bank); rows of more than 512 blocks read theirs from memory.
+#define Q8F_SC_BLOCKS 512u
+__device__ __forceinline__ uint32_t q8_few_sc_words(uint32_t blocks) { return ((blocks + 1u) / 2u) | 1u; }
+
+template <int NW> struct Q8Few {
+    static constexpr int U = 8; // block pairs in flight: 4,096 columns in one turn of eight wavefronts
+    const int8_t *w_src;
+    const uint16_t *sc_rows;   // the tile's first row of scales
+    uint32_t *s_sc;
+    uint32_t blocks, pairs, from, to, lane, wave, j, kg, rows_here, words;
+    bool staged;
+    uint32_t sc_now[16 / NW];
+    uint4 w[U];
+
+    __device__ __forceinline__ Q8Few(const lng_k_q8 &a, uint32_t tile, uint32_t *lds) : s_sc(lds) {
+        lane = threadIdx.x & 63u;
+        wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        j = lane & 15u;
+        kg = lane >> 4;
+        blocks = a.cols / 32u;
+        pairs = (blocks + 1u) / 2u;
+        from = wave * pairs / NW;
+        to = (wave + 1u) * pairs / NW;
+        const uint32_t r0 = tile * 16u;
+        rows_here = a.rows - r0 < 16u ? a.rows - r0 : 16u;
+        const uint32_t row = j < rows_here ? j : rows_here - 1u;
+        w_src = a.codes + (uint64_t)(r0 + row) * a.cols + 16u * kg;
+        sc_rows = a.scales + (uint64_t)r0 * blocks;
+        staged = blocks <= Q8F_SC_BLOCKS;
+        words = q8_few_sc_words(blocks);
+    }
+    __device__ __forceinline__ uint32_t load_sc(uint32_t row, uint32_t word) const { // scales 2 word and 2 word + 1 of a row
+        const uint16_t *src = sc_rows + row * blocks + 2u * word;
+        if (((blocks & 1u) | ((uintptr_t)sc_rows & 3u)) == 0) return *(const uint32_t *)src; // uniform
+        const uint32_t lo = src[0], hi = 2u * word + 1u < blocks ? src[1] : 0u;
+        return lo | (hi << 16);
+    }
+    __device__ __forceinline__ uint32_t sc_row(int i) const {
+        const uint32_t row = wave * (16 / NW) + i;
+        return row < rows_here ? row : rows_here - 1u;
+    }
+    __device__ __forceinline__ void ask_scales() { // the first 64 words of the wavefront's rows, into registers
+        if (!staged) return;
+#pragma unroll
+        for (int i = 0; i < 16 / NW; ++i) sc_now[i] = lane < pairs ? load_sc(sc_row(i), lane) : 0u;
+    }
+    __device__ __forceinline__ void stage_scales() { // and all of them to LDS
+        if (!staged) return;
+#pragma unroll
+        for (int i = 0; i < 16 / NW; ++i) {
+            uint32_t *to_row = s_sc + (wave * (16 / NW) + i) * words;
+            if (lane < pairs) to_row[lane] = sc_now[i];
+            for (uint32_t at = lane + 64u; at < pairs; at += 64u) to_row[at] = load_sc(sc_row(i), at);
+        }
+    }
+    __device__ __forceinline__ void ask_codes(uint32_t base) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t pair = base + u;
+            w[u] = make_uint4(0, 0, 0, 0);
+            if (pair < to) { // uniform; a last pair of one block: its upper lanes load the block again
+                const int32_t col = (int32_t)(64u * pair) - (2u * pair + 1u == blocks && kg >= 2u ? 32 : 0);
+                w[u] = *(const uint4 *)(w_src + col);
+            }
+        }
+    }
+    // the B operands and the scales of both blocks of a pair
+    __device__ __forceinline__ void operands(int u, uint32_t pair, bf16x8 (&b)[2], float (&sc)[2]) const {
+        const auto s0 = __builtin_amdgcn_permlane32_swap(w[u].x, w[u].z, false, false);
+        const auto s1 = __builtin_amdgcn_permlane32_swap(w[u].y, w[u].w, false, false);
+        b[0] = q8_codes_to_bf16_perm(make_uint2(s0[0], s1[0]));
+        b[1] = q8_codes_to_bf16_perm(make_uint2(s0[1], s1[1]));
+        const uint32_t both = staged ? s_sc[j * words + pair] : load_sc(j < rows_here ? j : rows_here - 1u, pair);
+        sc[0] = f16_bits_to_f32((uint16_t)both);
+        sc[1] = f16_bits_to_f32((uint16_t)(both >> 16)); // zero past an odd number of blocks
+    }
+};
+
+// Bound by latencies - a start, one round trip to memory, the partial sums' way through LDS - before the reading of the
+// matrix: 5,120 x 2,880 (q, k and v, 15.7 MB) with the norm, in a batch of 16 such: 1 position 8.3 us (11.1 when every
+// wavefront asked for half of its blocks at a time and split x for each), 2 to 16: 12 us with the planes' dispatch (20-27
+// when each workgroup normalised and split all positions itself), 31: 14 us (38); 2,880 x 4,096 with bias and residual from
+// bf16 1, 16, 31 positions: 6.9, 8.2, 11 us (9.1, 13, 23), from f32 7.2, 11, 17 (11, 19, 35).
+// Eight wavefronts to 16 rows: two workgroups fit a compute unit, so up to 512 tiles are all in flight at once.
+
+// 2 to 16 positions (more: 16 per blockIdx.y). Every load of a turn is asked for before its first product, the matrix's
+// first: a product is one round trip to memory, not one per block.
+// PLANES 2: x as lng_q8_norm_frag left it; 1: bf16 positions, turned into operand order through LDS that only this
+// wavefront uses (lng_q8_mid).
+template <int PLANES, int NW> __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, char *s_mem) {
+    constexpr int U = Q8Few<NW>::U, D = PLANES == 2 ? 3 : U; // pairs of x in flight
+    constexpr uint32_t STRIDE = 80;
+    __shared__ float s_red[NW][4][64];
+    Q8Few<NW> m(a, tile, (uint32_t *)(s_mem + (PLANES == 1 ? NW * 2u * 16u * STRIDE : 0u)));
+    const uint32_t lane = m.lane, j = m.j, kg = m.kg, p0 = blockIdx.y * 16u, r0 = tile * 16u;
+    char *s_x = s_mem + m.wave * 2u * 16u * STRIDE;
+    const uint32_t put = (lane >> 2) * STRIDE + 16u * (lane & 3u), get = j * STRIDE + 16u * q8_mid_chunk(kg);
+    const uint4 *x_frag = (const uint4 *)a.x_hi + (uint64_t)blockIdx.y * m.blocks * 128u + lane;
+    const uint32_t at_p = p0 + (lane >> 2) < a.n ? p0 + (lane >> 2) : a.n - 1u;
+    const uint16_t *x_row = a.x_hi + (uint64_t)at_p * a.plane_stride + 8u * (lane & 3u);
+    uint4 x[D][2][PLANES];
+    auto ask_x = [&](uint32_t pair, uint4 (&to)[2][PLANES]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t b = 2u * pair + h < m.blocks ? 2u * pair + h : 2u * pair;
+            if constexpr (PLANES == 1) {
+                to[h][0] = *(const uint4 *)(x_row + 32u * b);
+            } else {
+                to[h][0] = x_frag[b * 128u];
+                to[h][1] = x_frag[b * 128u + 64u];
+            }
+        }
+    };
+    // this thread's output, and what is added to it
+    const uint32_t out_p = p0 + 4u * kg + m.wave, out_row = r0 + j; // wavefronts 0-3: accumulator register = wavefront
+    const bool mine = m.wave < 4u && out_p < a.n && j < m.rows_here;
+    float *yp = a.y + (uint64_t)out_p * a.y_stride + out_row;
+    float bias = 0.0f, held = 0.0f;
+    if (mine && a.bias) bias = a.bias[out_row];
+    if (mine && a.accumulate) held = *yp;
+
+    floatx4 y = {0.0f, 0.0f, 0.0f, 0.0f};
+    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto ask = [&](uint32_t base) {
+        m.ask_codes(base);
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+            if (base + u < m.to) ask_x(base + u, x[u]);
+        }
+    };
+    m.ask_scales();
+    __builtin_amdgcn_sched_barrier(0);
+    ask(m.from);
+    __builtin_amdgcn_sched_barrier(0);
+    m.stage_scales();
+    __syncthreads();
+    for (uint32_t base = m.from; base < m.to; base += U) {
+        if (base != m.from) ask(base);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (base + u < m.to) {
+                bf16x8 b[2];
+                float sc[2];
+                m.operands(u, base + u, b, sc);
+                if constexpr (PLANES == 1) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) *(uint4 *)(s_x + h * 16 * STRIDE + put) = x[u % D][h][0];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) x[u % D][h][0] = *(const uint4 *)(s_x + h * 16 * STRIDE + get);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    floatx4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x[u % D][h][0]), b[h], zero4, 0, 0, 0);
+                    if constexpr (PLANES == 2) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x[u % D][h][1]), b[h], acc, 0, 0, 0);
+                    if (h == 0 || 2u * (base + u) + 1u < m.blocks) { // uniform
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) y[i] = __builtin_fmaf(sc[h], acc[i], y[i]);
+                    }
+                }
+                if constexpr (D < U) {
+                    if (u + D < U && base + u + D < m.to) ask_x(base + u + D, x[u % D]);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_red[m.wave][i][lane] = y[i];
+    __syncthreads();
+    if (!mine) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) sum += s_red[w][m.wave][lane];
+    if (a.bias) sum = sum + bias;
+    if (a.accumulate) sum = held + sum; // h + ((W x) + bias), each sum rounded as the separate dispatches round it
+    *yp = sum;
+}
+
+// One position. Its operand planes are made once per workgroup (normalised, split: a thread takes eight columns) and wait
+// in LDS. f32: even rows of the A operand are the hi plane, odd ones the lo plane, and one matrix instruction multiplies
+// a block by both; all rows of bf16 are the position.
+template <bool BF16, int NW> __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem) {
+    constexpr int U = Q8Few<NW>::U, T = 64 * NW;
+    __shared__ float s_red[NW][16];
+    __shared__ float s_norm[NW];
+    Q8Few<NW> m(a, tile, (uint32_t *)(s_mem + (uint64_t)a.cols * (BF16 ? 2u : 4u)));
+    const uint32_t chunks = a.cols / 8u, mine = threadIdx.x, out_row = tile * 16u + mine;
+    const bool writes = mine < m.rows_here;
+    uint4 *s_x = (uint4 *)s_mem; // [plane][chunk of eight columns]
+    float x[8] = {}, nw[8] = {};
+    uint4 x16 = make_uint4(0, 0, 0, 0);
+    auto load = [&](uint32_t chunk, const float *src, float (&to)[8]) {
+        const float4 u = *(const float4 *)(src + 8u * chunk), v = *(const float4 *)(src + 8u * chunk + 4u);
+        to[0] = u.x, to[1] = u.y, to[2] = u.z, to[3] = u.w, to[4] = v.x, to[5] = v.y, to[6] = v.z, to[7] = v.w;
+    };
+    const bool normed = !BF16 && a.norm_w != nullptr; // uniform
+    if (mine < chunks) {
+        if constexpr (BF16) {
+            x16 = *(const uint4 *)(a.x_hi + 8u * mine);
+        } else {
+            load(mine, a.x, x);
+            if (normed) load(mine, a.norm_w, nw);
+        }
+    }
+    m.ask_scales();
+    float bias = 0.0f, held = 0.0f;
+    if (writes && a.bias) bias = a.bias[out_row];
+    if (writes && a.accumulate) held = a.y[out_row];
+    __builtin_amdgcn_sched_barrier(0);
+    m.ask_codes(m.from); // after what is waited for first: loads come back in order
+    __builtin_amdgcn_sched_barrier(0);
+    m.stage_scales();
+    if constexpr (BF16) {
+        if (mine < chunks) s_x[mine] = x16;
+        for (uint32_t c = mine + T; c < chunks; c += T) s_x[c] = *(const uint4 *)(a.x_hi + 8u * c);
+    } else {
+        float scale = 0.0f;
+        if (normed) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x[e] * x[e]; // zeros past the last chunk
+            for (uint32_t c = mine + T; c < chunks; c += T) {
+                float more[8];
+                load(c, a.x, more);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss += more[e] * more[e];
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+            if (m.lane == 0) s_norm[m.wave] = ss;
+            __syncthreads();
+            float total = 0.0f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) total += s_norm[w];
+            scale = 1.0f / sqrtf(total / (float)a.cols + a.eps);
+        }
+        for (uint32_t c = mine; c < chunks; c += T) {
+            if (c != mine) {
+                load(c, a.x, x);
+                if (normed) load(c, a.norm_w, nw);
+            }
+            if (normed) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = x[e] * scale * nw[e];
+            }
+            bf16x8 hi, lo;
+            q8_split8(x, hi, lo);
+            s_x[c] = __builtin_bit_cast(uint4, hi);
+            s_x[chunks + c] = __builtin_bit_cast(uint4, lo);
+        }
+    }
+    __syncthreads();
+    const uint4 *x_at = s_x + q8_mid_chunk(m.kg) + (!BF16 && (m.j & 1u) ? chunks : 0u);
+    float y[2] = {0.0f, 0.0f};
+    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t base = m.from; base < m.to; base += U) {
+        if (base != m.from) m.ask_codes(base);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (base + u < m.to) {
+                bf16x8 b[2];
+                float sc[2];
+                m.operands(u, base + u, b, sc);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t block = 2u * (base + u) + h;
+                    if (h == 0 || block < m.blocks) { // uniform
+                        const floatx4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x_at[4u * block]), b[h], zero4, 0, 0, 0);
+                        y[0] = __builtin_fmaf(sc[h], acc[0], y[0]);
+                        if constexpr (!BF16) y[1] = __builtin_fmaf(sc[h], acc[1], y[1]);
+                    }
+                }
+            }
+        }
+    }
+    if (m.lane < 16u) s_red[m.wave][m.lane] = y[0] + y[1];
+    __syncthreads();
+    if (!writes) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) sum += s_red[w][mine];
+    if (a.bias) sum = sum + bias;
+    if (a.accumulate) sum = held + sum;
+    a.y[out_row] = sum;
+}
+
+#define Q8_FEW(name, body, what, nw) \
+    extern "C" __global__ __launch_bounds__(64 * nw, nw / 2) void name(lng_k_q8 a) { \
+        extern __shared__ __attribute__((aligned(16))) char s_mem[]; /* as many bytes as q8_record_few works out */ \
+        const uint32_t tile = q8_select_matrix(a); \
+        body<what, nw>(a, tile, s_mem); \
+    }
+Q8_FEW(lng_q8_few, q8_few_body, 2, 8)
+Q8_FEW(lng_q8_few_bf16, q8_few_body, 1, 8)
+Q8_FEW(lng_q8_one, q8_one_body, false, 8)
+Q8_FEW(lng_q8_one_bf16, q8_one_body, true, 8)

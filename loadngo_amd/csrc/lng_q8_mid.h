@@ -202,7 +202,12 @@ __device__ __forceinline__ void q8_mid_body(const lng_k_q8 &a, uint32_t row_tile
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t p = p0 + 16u * (at % MT) + 4u * kg + i; // accumulator row = position, column = matrix row
-            if (p < a.n && row < rows_here) a.y[(uint64_t)p * a.y_stride + r0 + row] = sum[i];
+            if (p < a.n && row < rows_here) {
+                float *yp = a.y + (uint64_t)p * a.y_stride + r0 + row;
+                if (a.bias) sum[i] = sum[i] + a.bias[r0 + row];
+                if (a.accumulate) sum[i] = *yp + sum[i]; // the residual: h + ((W x) + bias), rounded as the separate dispatches round it
+                *yp = sum[i];
+            }
         }
     }
 }

@@ -427,3 +427,39 @@ def test_products_whose_wavefronts_share_the_columns(gpu, rows, cols, n, bf16):
         assert not np.isnan(out[:, :rows]).any() and np.isnan(out[:-1, rows:]).all()
         assert np.abs(out[:, :rows] - want).max() / np.abs(want).max() < 1e-5
     assert np.abs(outs[0][:, :rows] - outs[1][:, :rows]).max() / np.abs(want).max() < 2e-5
+
+
+@pytest.mark.parametrize("rows,cols,n,bf16", [
+    (1, 32, 1, False), (17, 64, 1, False), (48, 96, 2, False), (33, 224, 15, False), (16, 4128, 16, False), (31, 12288, 1, False),
+    (20, 12320, 1, False), (20, 16384, 3, False), (20, 16416, 16, False), (20, 16416, 17, False), (37, 160, 17, False), (300, 2880, 31, False),
+    (1, 32, 1, True), (17, 96, 2, True), (33, 224, 16, True), (16, 4128, 1, True), (20, 24576, 1, True), (20, 24608, 1, True),
+    (20, 16416, 5, True), (20, 16416, 31, True), (37, 160, 17, True)])
+def test_products_of_few_positions(gpu, rows, cols, n, bf16):
+    """Fewer than 32 positions: the tiles' edges in rows and positions, one block, an odd number of blocks, fewer pairs of
+    blocks than wavefronts, several turns of a wavefront, the widest rows whose x or scales LDS holds and wider ones; scales
+    on and off a 4-byte boundary; strided x and y, gaps of y untouched. The reference's bound (glue.rs:171)."""
+    from tests.helpers import from_bf16_bits, to_bf16_bits
+    codes, bits, elements = q8_test_matrix(rows, cols, 90 + rows)
+    x = np.full((n, cols + 8), np.nan, np.float32)
+    x[:, :cols] = xorshift_values(29, n * cols).reshape(n, cols)
+    xin = to_bf16_bits(x) if bf16 else x
+    want = (from_bf16_bits(xin) if bf16 else x)[:, :cols].astype(np.float64) @ elements.T
+    y_stride = rows + 4
+    y_len = ((n - 1) * y_stride + rows) * 4
+    for shift in (0, 2):
+        bufs = [gpu.upload(codes), gpu.upload(np.concatenate([np.full(shift // 2, 0x7E00, np.uint16), bits])), gpu.upload(xin), gpu.buffer(y_len)]
+        bufs[3].fill(0xFF)
+        batch = gpu.batch(bufs)
+        m = (C.Slice(0, 0, codes.nbytes), C.Slice(1, shift, bits.nbytes))
+        xs = C.Slice(2, 0, ((n - 1) * (cols + 8) + cols) * (2 if bf16 else 4))
+        (batch.gemm_q8_0_bf16 if bf16 else batch.gemm_q8_0)(m, xs, C.Slice(3, 0, y_len), rows, cols, n, (cols + 8, y_stride))
+        done = batch.run()
+        assert not isinstance(done.gpu_time, Exception), done.gpu_time
+        out = np.full(n * y_stride, np.nan, np.float32)
+        out[:y_len // 4] = bufs[3].read(np.float32)
+        batch.drop()
+        for b in bufs:
+            b.free()
+        out = out.reshape(n, y_stride)
+        assert not np.isnan(out[:, :rows]).any() and np.isnan(out[:-1, rows:]).all()
+        assert np.abs(out[:, :rows] - want).max() / np.abs(want).max() < 1e-5
