@@ -31,6 +31,41 @@ def test_struct_layouts_match_the_header():
     assert ctypes.sizeof(C._Completed) == 24
 
 
+@pytest.mark.parametrize("value", [0, 1, 2**63, 2**64 - 1, np.uint64(2**64 - 1), np.int32(7), 2**64, -1, np.int64(-1), True, 1.0, None])
+def test_conversions_take_the_same_values_at_every_place(value):
+    """Slices, shapes and matrices convert plain ints at once and anything else value by value: each place accepts
+    0 .. 2**64 - 1 of any integer type and refuses the rest, whatever stands beside it."""
+    good = isinstance(value, (int, np.integer)) and not isinstance(value, bool) and 0 <= int(value) < 2**64
+    for at in range(3):
+        fields = [3, 2**64 - 1, 5]
+        fields[at] = value
+        s = C.Slice(*fields)
+        for convert in (s._c, lambda: C._q8_matrices([((C.Slice(1, 2, 3), s), C.Slice(4, 5, 6), 7)])[0].scales):
+            if good:
+                got = convert()
+                assert [got.buffer, got.offset, got.len] == [int(f) for f in fields]
+            else:
+                with pytest.raises(ValueError):
+                    convert()
+    for at in range(7):
+        fields = [3, 5, 64, 8, 64, 2**64 - 1, 9]
+        fields[at] = value
+        if good:
+            got = C.GroupedShape(*fields, 0.5)._c()
+            assert [getattr(got, n) for n in ("t", "start", "heads", "kv_heads", "dim", "window", "slots")] == [int(f) for f in fields]
+            assert got.scale == 0.5
+        else:
+            with pytest.raises(ValueError):
+                C.GroupedShape(*fields, 0.5)._c()
+
+
+def test_matrix_tables_hold_what_the_structures_hold():
+    m = C._q8_matrices([((C.Slice(1, 2, 3), C.Slice(4, 5, 6)), C.Slice(7, 8, 9), 10), ((C.Slice(2**64 - 1, 0, 1), C.Slice(11, 12, 13)), C.Slice(14, 15, 16), 17)])
+    assert ctypes.sizeof(C._Q8Matrix) == 80
+    flat = lambda q: [getattr(s, f) for s in (q.codes, q.scales, q.y) for f in ("buffer", "offset", "len")] + [q.rows]  # noqa: E731
+    assert flat(m[0]) == list(range(1, 11)) and flat(m[1]) == [2**64 - 1, 0, 1] + list(range(11, 18))
+
+
 def test_shape_rules_match_the_reference_lists():
     for case in REF_REJECTED:
         with pytest.raises(C.Dispatch):
