@@ -113,6 +113,7 @@ int lng_hip_device_name(lng_gpu *gpu, char *name, size_t cap);
  *   LNG_PREFILL_UPFRONT 0    narrow windows on the tile-by-tile kernel
  *   LNG_PREFILL_SPLITS n     workgroups per (query tile, kv head) of a prompt pass with fewer workgroups than compute units
  *   LNG_Q8_MID 0|1           never / whenever possible the Q8_0 kernel whose wavefronts share the columns of a tile (32 positions or more)
+ *   LNG_NO_FUSING            a batch runs every dispatch as kernels of its own (as one that is timed dispatch by dispatch does)
  *   LNG_CHECKSUM_WGS n       workgroups per compute unit of lng_hip_checksum's streaming read (default 2)
  *   LNG_TABLE_IN_PLACE n     row tables of n bytes or more stay in pinned host memory, where the kernels read them,
  *                            instead of being copied to the device ahead of the batch (default 8192; 0: always copied)
@@ -176,7 +177,8 @@ int lng_hip_batch_wait(lng_batch *batch, double *gpu_seconds);
  * gpt-oss/src/gpu.rs:247-317 (Profile / PhaseTime). With timing on (set before commit) an
  * event is recorded after every kernel of the batch; after the batch has finished,
  * lng_hip_batch_kernel_seconds sums the time and counts the launches of the kernel named
- * `kernel` (e.g. "lng_decode_bf16_d64"). */
+ * `kernel` (e.g. "lng_decode_bf16_d64"). Without timing, row copies, RMS norms, additions and the splits before Q8_0
+ * products that stand beside each other may run as one kernel, with the same results. */
 int lng_hip_batch_set_timing(lng_batch *batch, int enabled);
 int lng_hip_batch_kernel_seconds(lng_batch *batch, const char *kernel, double *seconds, size_t *launches);
 /* Drop of Batch: an uncommitted batch runs nothing (apple.rs:553-561); a committed one is

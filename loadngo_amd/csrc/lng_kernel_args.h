@@ -76,6 +76,7 @@ typedef struct lng_k_copy {
     uint64_t dst_stride;
     uint32_t src_dtype;
     uint32_t dst_dtype;
+    uint64_t words; /* width and strides count 16-byte words (one dtype) */
 } lng_k_copy;
 
 typedef struct lng_k_fill {
@@ -105,16 +106,27 @@ typedef struct lng_k_add {
     uint64_t rows;
     uint64_t width;
     uint64_t src_stride;
+    uint64_t by4; /* four i a thread */
 } lng_k_add;
 
-/* In place: the first d floats of each row (stride floats apart) times w / sqrt(mean of squares + eps). */
+/* v = the first d floats of each row of src (rows `stride` / `src_stride` floats apart; src == v: in place) times
+ * w / sqrt(mean of squares + eps). lng_rmsnorm_row8 alone reads src and the planes: */
+#define LNG_PLANES_NONE 0u
+#define LNG_PLANES_ROWS 1u    /* as lng_q8_split_x leaves them: [n_pad][d] each */
+#define LNG_PLANES_OPERAND 2u /* as lng_q8_frag_x leaves them, both behind hi */
 typedef struct lng_k_rmsnorm {
     float *v;
     const float *w;
+    const float *src;
+    uint16_t *hi, *lo;        /* the two bf16 planes of the result, rows up to n_pad zero */
     uint32_t rows;
     uint32_t d;
     uint32_t stride;
+    uint32_t src_stride;
+    uint32_t n_pad;           /* workgroups: rows, or those of the planes */
+    uint32_t planes;
     float eps;
+    uint32_t pad_;
 } lng_k_rmsnorm;
 
 /* In-place rotation by halves of x[rows][heads][dim], f32. */
@@ -181,9 +193,11 @@ typedef struct lng_k_q8 {
     uint32_t n_more;         /* 0..LNG_Q8_MORE */
     float eps;               /* of the RMS norm, when norm_w is set */
     /* Few positions only. norm_w (one position): x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
-     * (cols <= 12288). bias: y gets bias[row] added. accumulate: the result is added to what y holds (a residual). */
+     * (cols <= 12288). bias: y gets bias[row] added. accumulate: the result is added to what y holds. (These two and
+     * residual: all kernels of one matrix.) */
     const float *norm_w;
     const float *bias;
+    float *residual;         /* [n][rows], not y: gets the result added as well, or NULL */
     uint32_t accumulate;
     uint32_t tiles;          /* row tiles of all matrices of the dispatch (lng_q8_mid*) */
     struct lng_k_q8_more {

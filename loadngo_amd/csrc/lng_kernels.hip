@@ -1425,9 +1425,17 @@ extern "C" __global__ __launch_bounds__(256) void lng_decode_merge_few(lng_k_att
 
 // =============================================================================================
 // Row copy with optional conversion (Batch::copy_rows, apple.rs:1762; kernels.metal:1127-1138):
-// how new K and V rows enter a cache. One thread per element.
+// how new K and V rows enter a cache. One thread per element or word.
 // =============================================================================================
+// a.words: between rows of one type in words of 16 bytes, which width and strides then count (rows x stride fits 32 bits).
+// 8,192 x 2,880 f32: 28 us a copy (45-50 one element a thread).
 extern "C" __global__ __launch_bounds__(256) void lng_copy_rows(lng_k_copy a) {
+    if (a.words) { // uniform
+        const uint32_t gid = blockIdx.x * 256u + threadIdx.x, width = (uint32_t)a.width;
+        const uint32_t r = gid / width, i = gid - r * width;
+        if (r < (uint32_t)a.rows) ((uint4 *)a.dst)[(uint64_t)r * a.dst_stride + i] = ((const uint4 *)a.src)[(uint64_t)r * a.src_stride + i];
+        return;
+    }
     const uint64_t gid = (uint64_t)blockIdx.x * 256u + threadIdx.x;
     if (gid >= a.rows * a.width) return;
     const uint64_t r = gid / a.width;
@@ -1510,8 +1518,19 @@ extern "C" __global__ __launch_bounds__(256) void lng_rmsnorm_row_wg(lng_k_rmsno
     }
 }
 
-// Batch::add_rows (apple.rs:1886-1911; kernels.metal:1648-1660). One thread per element.
+// Batch::add_rows (apple.rs:1886-1911; kernels.metal:1648-1660). One thread per element, or (a.by4) per four of them:
+// width, source stride and both addresses multiples of 16 bytes (rows x width fits 32 bits). 8,192 x 2,880: 28 us the bias, 42 other rows (42, 65).
 extern "C" __global__ __launch_bounds__(256) void lng_add_rows(lng_k_add a) {
+    if (a.by4) { // uniform
+        const uint32_t gid = blockIdx.x * 256u + threadIdx.x, width = (uint32_t)a.width / 4u;
+        const uint32_t r = gid / width, i = gid - r * width;
+        if (r >= (uint32_t)a.rows) return;
+        const float4 s = *(const float4 *)(a.src + (uint64_t)r * a.src_stride + 4u * i);
+        float4 *to = (float4 *)a.dst + gid;
+        const float4 d = *to;
+        *to = make_float4(d.x + s.x, d.y + s.y, d.z + s.z, d.w + s.w);
+        return;
+    }
     const uint64_t gid = (uint64_t)blockIdx.x * 256u + threadIdx.x;
     if (gid >= a.rows * a.width) return;
     const uint64_t r = gid / a.width;
@@ -1944,15 +1963,44 @@ template <int WAVES, int PLANES = 2> __device__ __forceinline__ void q8_tiled_bo
         __syncthreads();
     }
     if (!rows_here) return;
+    // All of the residual's rows are asked for before the first is added to: read and written one after another they cost
+    // 164 us of 8,192 positions x 2,880 rows.
+    const bool whole = r0 + rw + 64u <= a.rows && p0 + pw + 16u * MT <= a.n; // uniform: every output exists
+    float held[4][MT][4] = {};
+    if (a.residual && whole) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            const float *from = a.residual + (uint64_t)(p0 + pw + 4u * kg) * a.rows + r0 + rw + 16u * nt + j;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) held[nt][mt][i] = from[(uint64_t)(16u * mt + i) * a.rows];
+            }
+        }
+    }
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
         const uint32_t r = r0 + rw + 16u * nt + j;
+        if (a.bias && r < a.rows) {
+            const float bias = a.bias[r];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[nt][mt][i] = y[nt][mt][i] + bias;
+            }
+        }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t p = p0 + pw + 16u * mt + 4u * kg + i;
-                if (p < a.n && r < a.rows) a.y[(uint64_t)p * a.y_stride + r] = y[nt][mt][i];
+                if (whole || (p < a.n && r < a.rows)) {
+                    a.y[(uint64_t)p * a.y_stride + r] = y[nt][mt][i];
+                    if (a.residual) {
+                        float *to = a.residual + (uint64_t)p * a.rows + r;
+                        *to = (whole ? held[nt][mt][i] : *to) + y[nt][mt][i];
+                    }
+                }
             }
         }
     }
@@ -1969,6 +2017,73 @@ extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16(lng_k_q8 a) 
 
 #include "lng_q8_mid.h"
 #include "lng_q8_few.h"
+
+// Batch::rmsnorm_rows in words of 16 bytes, and with it what stands around it in a block (gpt-oss/src/gpu.rs:712-732): the
+// copy of the hidden rows before it (src), the split of the result for the Q8_0 products after it (hi, lo). A workgroup per
+// row of up to 4,096 floats, d % 8 == 0, every row from a 16-byte boundary; a thread holds up to two runs of eight.
+// Bound by memory: 8,192 x 2,880 with copy and planes 54 us (28 + 32 + 28 as three kernels, 45 + 28 + 28 before), 512 rows 8.6 (14.5).
+extern "C" __global__ __launch_bounds__(256) void lng_rmsnorm_row8(lng_k_rmsnorm a) {
+#pragma clang fp contract(off)
+    __shared__ float s_part[4];
+    const uint32_t row = blockIdx.x, chunks = a.d / 8u;
+    float x[2][8] = {}, w[2][8] = {};
+    auto load = [&](const float *from, float (&to)[8]) {
+        const float4 u = *(const float4 *)from, v = *(const float4 *)(from + 4);
+        to[0] = u.x, to[1] = u.y, to[2] = u.z, to[3] = u.w, to[4] = v.x, to[5] = v.y, to[6] = v.z, to[7] = v.w;
+    };
+    if (row < a.rows) { // uniform; the rows after them only pad the planes with zeros
+        const float *src = a.src + (uint64_t)row * a.src_stride;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const uint32_t c = threadIdx.x + 256u * u;
+            if (c < chunks) {
+                load(src + 8u * c, x[u]);
+                load(a.w + 8u * c, w[u]);
+            }
+        }
+        float ss = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x[u][e] * x[u][e];
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+        if ((threadIdx.x & 63u) == 0) s_part[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+        const float scale = 1.0f / sqrtf(ss / (float)a.d + a.eps);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const uint32_t c = threadIdx.x + 256u * u;
+            if (c < chunks) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[u][e] = x[u][e] * scale * w[u][e];
+                float *to = a.v + (uint64_t)row * a.stride + 8u * c;
+                *(float4 *)to = make_float4(x[u][0], x[u][1], x[u][2], x[u][3]);
+                *(float4 *)(to + 4) = make_float4(x[u][4], x[u][5], x[u][6], x[u][7]);
+            }
+        }
+    }
+    if (a.planes == LNG_PLANES_NONE) return;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const uint32_t c = threadIdx.x + 256u * u;
+        if (c < chunks) {
+            bf16x8 hi, lo;
+            q8_split8(x[u], hi, lo);
+            if (a.planes == LNG_PLANES_ROWS) {
+                const uint64_t at = (uint64_t)row * a.d + 8u * c;
+                *(bf16x8 *)(a.hi + at) = hi;
+                *(bf16x8 *)(a.lo + at) = lo;
+            } else {
+                uint4 *to = (uint4 *)a.hi + ((uint64_t)(row >> 4) * (a.d / 32u) + (c >> 2)) * 128u + 16u * q8_mid_chunk(c & 3u) + (row & 15u);
+                to[0] = __builtin_bit_cast(uint4, hi);
+                to[64] = __builtin_bit_cast(uint4, lo);
+            }
+        }
+    }
+}
 
 // Synthetic data (see LNG_SYNTH_STD in lng_kernel_args.h for the exact integers).
 // A plain streaming read: the XOR of every 16-byte word of a buffer. Consecutive lanes read consecutive 16-byte

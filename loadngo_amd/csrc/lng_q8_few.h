@@ -178,6 +178,8 @@ template <int PLANES, int NW> __device__ __forceinline__ void q8_few_body(const 
     float bias = 0.0f, held = 0.0f;
     if (mine && a.bias) bias = a.bias[out_row];
     if (mine && a.accumulate) held = *yp;
+    float *to = a.residual + (uint64_t)out_p * a.rows + out_row; // (never with accumulate)
+    if (mine && a.residual) held = *to;
 
     floatx4 y = {0.0f, 0.0f, 0.0f, 0.0f};
     const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -233,6 +235,7 @@ template <int PLANES, int NW> __device__ __forceinline__ void q8_few_body(const 
     if (a.bias) sum = sum + bias;
     if (a.accumulate) sum = held + sum; // h + ((W x) + bias), each sum rounded as the separate dispatches round it
     *yp = sum;
+    if (a.residual) *to = held + sum;
 }
 
 // One position. Its operand planes are made once per workgroup (normalised, split: a thread takes eight columns) and wait
@@ -265,6 +268,7 @@ template <bool BF16, int NW> __device__ __forceinline__ void q8_one_body(const l
     float bias = 0.0f, held = 0.0f;
     if (writes && a.bias) bias = a.bias[out_row];
     if (writes && a.accumulate) held = a.y[out_row];
+    if (writes && a.residual) held = a.residual[out_row]; // (never with accumulate)
     __builtin_amdgcn_sched_barrier(0);
     m.ask_codes(m.from); // after what is waited for first: loads come back in order
     __builtin_amdgcn_sched_barrier(0);
@@ -341,6 +345,7 @@ template <bool BF16, int NW> __device__ __forceinline__ void q8_one_body(const l
     if (a.bias) sum = sum + bias;
     if (a.accumulate) sum = held + sum;
     a.y[out_row] = sum;
+    if (a.residual) a.residual[out_row] = held + sum;
 }
 
 #define Q8_FEW(name, body, what, nw) \

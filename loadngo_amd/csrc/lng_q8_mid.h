@@ -190,8 +190,25 @@ __device__ __forceinline__ void q8_mid_body(const lng_k_q8 &a, uint32_t row_tile
             s_red[(wave * NT * MT + nt * MT + mt) * 64u + lane] = make_float4(y[nt][mt][0], y[nt][mt][1], y[nt][mt][2], y[nt][mt][3]);
         }
     }
+    constexpr int MINE = (NT * MT + NW - 1) / NW; // of the tile's 16 x 16 parts
+    float bias[MINE] = {}, held[MINE][4] = {};    // what is added, asked for while the partial results meet
+#pragma unroll
+    for (int m = 0; m < MINE; ++m) {
+        const uint32_t at = wave + NW * m, row = 16u * (at / MT) + j, first = p0 + 16u * (at % MT) + 4u * kg;
+        if (at < NT * MT && row < rows_here) {
+            if (a.bias) bias[m] = a.bias[r0 + row];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (first + i < a.n && a.accumulate) held[m][i] = a.y[(uint64_t)(first + i) * a.y_stride + r0 + row];
+                if (first + i < a.n && a.residual) held[m][i] = a.residual[(uint64_t)(first + i) * a.rows + r0 + row]; // never both
+            }
+        }
+    }
     __syncthreads();
-    for (uint32_t at = wave; at < NT * MT; at += NW) {
+#pragma unroll
+    for (int m = 0; m < MINE; ++m) {
+        const uint32_t at = wave + NW * m;
+        if (at >= NT * MT) break;
         float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
@@ -203,10 +220,10 @@ __device__ __forceinline__ void q8_mid_body(const lng_k_q8 &a, uint32_t row_tile
         for (int i = 0; i < 4; ++i) {
             const uint32_t p = p0 + 16u * (at % MT) + 4u * kg + i; // accumulator row = position, column = matrix row
             if (p < a.n && row < rows_here) {
-                float *yp = a.y + (uint64_t)p * a.y_stride + r0 + row;
-                if (a.bias) sum[i] = sum[i] + a.bias[r0 + row];
-                if (a.accumulate) sum[i] = *yp + sum[i]; // the residual: h + ((W x) + bias), rounded as the separate dispatches round it
-                *yp = sum[i];
+                if (a.bias) sum[i] = sum[i] + bias[m];
+                if (a.accumulate) sum[i] = held[m][i] + sum[i]; // the residual: h + ((W x) + bias), rounded as the separate dispatches round it
+                a.y[(uint64_t)p * a.y_stride + r0 + row] = sum[i];
+                if (a.residual) a.residual[(uint64_t)p * a.rows + r0 + row] = held[m][i] + sum[i];
             }
         }
     }

@@ -1,0 +1,121 @@
+"""Sequences of a block's dispatches that run as fewer kernels (copy + RMS norm + the split before Q8_0 products; product +
+bias + residual): every buffer holds bit for bit what it holds when each dispatch is a kernel of its own."""
+import numpy as np
+import pytest
+
+from loadngo_amd import compute as C
+from tests.gpu_common import gpu  # noqa: F401
+from tests.helpers import q8_test_matrix, to_bf16_bits, xorshift_values
+
+pytestmark = pytest.mark.gpu
+
+
+def both_ways(gpu, arrays, record):
+    """Every buffer after `record` ran on fresh copies of the arrays, fused and not."""
+    out = []
+    try:
+        for fusing in (True, False):
+            gpu.debug_set("LNG_NO_FUSING", None if fusing else "1")
+            bufs = [gpu.upload(a) for a in arrays]
+            batch = gpu.batch(bufs)
+            record(batch)
+            done = batch.run()
+            assert not isinstance(done.gpu_time, Exception), done.gpu_time
+            batch.drop()
+            out.append([b.read(np.uint8) for b in bufs])
+            for b in bufs:
+                b.free()
+    finally:
+        gpu.debug_set("LNG_NO_FUSING", None)
+    return out
+
+
+@pytest.mark.parametrize("n,cols,src_stride,x_stride,offset", [
+    (1, 2880, 2880, 2880, 0), (31, 2880, 2880, 2880, 0), (33, 2880, 2880, 2880, 0), (77, 288, 292, 288, 0), (64, 4096, 4096, 4100, 0),
+    (64, 4128, 4128, 4128, 0), (64, 256, 256, 256, 0), (100, 288, 288, 288, 4), (1281, 288, 288, 288, 0), (1300, 320, 320, 324, 0)])
+def test_copy_norm_and_split_in_one_kernel(gpu, n, cols, src_stride, x_stride, offset):
+    """Positions up to and past both ways of splitting, row widths at the edges of the norm kernels, strides, hidden rows
+    off a 16-byte boundary; one product and three, a product of other rows in between, the norm alone."""
+    eps, rows = 1e-5, 80
+    mats = [q8_test_matrix(rows, cols, 30 + i)[:2] for i in range(3)]
+    h = 3 * xorshift_values(71 + n, n * src_stride + 1)
+    x = xorshift_values(72, n * x_stride)
+    arrays = [h, x, 1 + 0.2 * xorshift_values(73, cols), np.zeros(6 * n * rows, np.float32)]
+    for codes, bits in mats:
+        arrays += [codes, bits]
+    hs = C.Slice(0, offset, ((n - 1) * src_stride + cols) * 4)
+    xs, ws = C.Slice(1, 0, ((n - 1) * x_stride + cols) * 4), C.Slice(2, 0, cols * 4)
+    matrix = lambda i: (C.Slice(4 + 2 * i, 0, rows * cols), C.Slice(5 + 2 * i, 0, rows * cols // 16))  # noqa: E731
+    y = lambda i: C.Slice(3, i * n * rows * 4, n * rows * 4)  # noqa: E731
+
+    def record(batch):
+        batch.copy_rows((hs, src_stride), (xs, x_stride), n, cols)
+        batch.rmsnorm_rows((xs, ws), n, (cols, x_stride), eps)
+        batch.gemm_q8_0_many([(matrix(i), y(i), rows) for i in range(3)], xs, cols, n, x_stride)
+        batch.rmsnorm_rows((xs, ws), n, (cols, x_stride), eps)                           # without a copy
+        batch.gemm_q8_0(matrix(0), xs, y(3), rows, cols, n, (x_stride, rows))
+        batch.copy_rows((hs, src_stride), (xs, x_stride), n, cols)                       # without a norm
+        batch.gemm_q8_0(matrix(1), xs, y(4), rows, cols, n, (x_stride, rows))
+        if n > 1:                                                                        # the norm of fewer rows than are copied
+            batch.copy_rows((hs, src_stride), (xs, x_stride), n, cols)
+            batch.rmsnorm_rows((C.Slice(1, 0, ((n - 2) * x_stride + cols) * 4), ws), n - 1, (cols, x_stride), eps)
+            batch.gemm_q8_0(matrix(2), xs, y(5), rows, cols, n, (x_stride, rows))
+
+    fused, apart = both_ways(gpu, arrays, record)
+    for i, (a, b) in enumerate(zip(fused, apart)):
+        assert np.array_equal(a, b), "buffer %d" % i
+    got = fused[3].view(np.float32)
+    assert not np.isnan(got).any() and np.abs(got[:5 * n * rows]).min() >= 0 and np.abs(got).max() > 0
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("n,rows,cols", [(1, 48, 96), (7, 33, 64), (17, 48, 96), (32, 64, 96), (77, 100, 64), (200, 192, 96), (1290, 260, 64)])
+def test_bias_and_residual_in_the_product(gpu, n, rows, cols, bf16):
+    """Each kind of product with bias and residual, bias or residual alone, and the sequences that only look alike: hidden
+    rows over the positions, over the codes or over the bias, a residual of another width, the bias added twice, y with gaps,
+    a second residual."""
+    codes, bits, _ = q8_test_matrix(rows, cols, 51)
+    x = xorshift_values(52 + n, n * cols)
+    x = to_bf16_bits(x) if bf16 else x
+    room = np.zeros(max(n * rows * 4, 4096) // 4 * 4, np.uint8)
+    x_held, codes_held = np.concatenate([x.view(np.uint8), room]), np.concatenate([codes.view(np.uint8), room])
+    bias_held = xorshift_values(53, n * rows)  # the bias is its first row
+    arrays = [x_held, codes_held, bits, bias_held, xorshift_values(54, n * rows), np.zeros(8 * n * rows, np.float32), np.zeros(n * (rows + 4), np.float32)]
+    es = 2 if bf16 else 4
+    xs, m = C.Slice(0, 0, n * cols * es), (C.Slice(1, 0, rows * cols), C.Slice(2, 0, rows * cols // 16))
+    bs, hs, size = C.Slice(3, 0, rows * 4), C.Slice(4, 0, n * rows * 4), n * rows * 4
+
+    def product(batch, y, stride=rows):
+        (batch.gemm_q8_0_bf16 if bf16 else batch.gemm_q8_0)(m, xs, y, rows, cols, n, (cols, stride))
+
+    def record(batch):
+        y = [C.Slice(5, i * size, size) for i in range(8)]
+        product(batch, y[0])
+        batch.add_rows(y[0], (bs, 0), n, rows)
+        batch.add_rows(hs, (y[0], rows), n, rows)
+        product(batch, y[1])
+        batch.add_rows(y[1], (bs, 0), n, rows)                                   # the bias alone, then twice
+        batch.add_rows(y[1], (bs, 0), n, rows)
+        product(batch, y[2])
+        batch.add_rows(hs, (y[2], rows), n, rows)                                # the residual alone, then twice, then the bias
+        batch.add_rows(hs, (y[2], rows), n, rows)
+        batch.add_rows(y[2], (bs, 0), n, rows)
+        product(batch, y[3])
+        batch.add_rows(y[3], (C.Slice(3, 0, size), rows), n, rows)               # another row for every position
+        batch.add_rows(y[4], (y[3], rows), n, rows)                              # and a residual that is no hidden state
+        strided = C.Slice(6, 0, ((n - 1) * (rows + 4) + rows) * 4)
+        product(batch, strided, rows + 4)
+        batch.add_rows(hs, (strided, rows + 4), n, rows)                         # y with gaps
+        product(batch, y[5])
+        batch.add_rows(y[5], (bs, 0), n, rows)
+        batch.add_rows(C.Slice(3, 0, size), (y[5], rows), n, rows)               # over the bias
+        product(batch, y[6])
+        batch.add_rows(C.Slice(1, 0, size), (y[6], rows), n, rows)               # over the codes
+        product(batch, y[7])
+        batch.add_rows(C.Slice(0, 0, size), (y[7], rows), n, rows)               # over the positions
+        product(batch, y[7])
+
+    fused, apart = both_ways(gpu, arrays, record)
+    for i, (a, b) in enumerate(zip(fused, apart)):
+        assert np.array_equal(a, b), "buffer %d" % i
+    assert not np.isnan(fused[5].view(np.float32)[:6 * n * rows]).any()
