@@ -836,6 +836,18 @@ int attention(lng_batch *b, lng_slice q, lng_slice k, lng_slice v, lng_slice out
             // (under a dozen key tiles the partial rows and the merge cost what two splits save: the first 512 rows of a
             // prompt 24.5 us unsplit, 30.8 us in two)
             if (key_tiles < 12) want = 1;
+            // f32: a tile of 64 keys is 8.3 us of matrix work, so a few tiles are worth splitting, down to one each, and
+            // where half of the units would have a workgroup more splits than units even out the unequal runs of a causal
+            // pass. Splits cost 4 us and 7 ns per row and split (64 heads). Whole calls, unsplit / split: 512 rows 75 / 52 us,
+            // 512 after 4,096 341 / 314, 256 rows 42 / 31, 128 25 / 22; through a 128-position window 48 rows 30 / 21, 128
+            // 35 / 25, 256 35 / 31; 512 there stay whole (31 against 39).
+            if (f32) {
+                const bool windowed = p.window != LNG_WINDOW_FULL && p.window < end;
+                want = (plain_wgs * 4 > g->cus && !windowed ? 2 : 1) * g->cus / plain_wgs;
+                want = std::min<uint64_t>(std::min<uint64_t>(want, key_tiles + windowed), 64); // (a window's run starts within a tile)
+                const double tiles = windowed ? (double)visible / 64.0 : (double)key_tiles;
+                if (tiles * 8.3 * (1.0 - 1.0 / (double)want) < 4.0 + 0.007 / 64.0 * (double)(s.t * s.heads * want)) want = 1;
+            }
             if (g->knobs.prefill_splits > 0) want = std::min<uint64_t>(g->knobs.prefill_splits, 64);
             if (want > 1) p.splits = (uint32_t)want;
         }

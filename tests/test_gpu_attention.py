@@ -762,6 +762,20 @@ def test_prefill_f32_matches_the_cpu_reference(gpu, t, start, window, slots, hea
     assert rel_error(generic, want) <= F32_RTOL
 
 
+@pytest.mark.parametrize("t,start,window,slots,heads,kv_heads", [
+    (128, 0, FULL, 128, 64, 8), (97, 30, FULL, 128, 64, 8), (500, 0, FULL, 512, 64, 8), (512, 100, FULL, 640, 64, 8),
+    (48, 2000, 128, 192, 64, 8), (130, 2001, 128, 320, 64, 8), (256, 1000, 100, 1280, 64, 8), (512, 0, FULL, 512, 16, 2)])
+def test_f32_passes_of_few_tiles_split_their_keys(gpu, t, start, window, slots, heads, kv_heads):
+    """Short f32 passes whose keys are split by the planner's own choice, down to one tile of keys each and to splits that
+    have none for the first rows of a causal pass: within 1e-5 (relative to 1 + |x|) of the CPU reference."""
+    q, k, v, sinks = normal_inputs(t + start, t, start + t, heads, kv_heads, 64, scale=0.5)
+    kr, vr = ring_layout(k, t, start, slots, True), ring_layout(v, t, start, slots, True)
+    shape = C.GroupedShape(t, start, heads, kv_heads, 64, window, slots, 0.125)
+    want = oracle.attention_f32(q, k, v, sinks, start, window=window, slots=None, scale=0.125, threads=THREADS)
+    got = run_attention(gpu, q, kr, vr, sinks, shape, True, C.F32, expect_kernel="lng_prefill_merge")
+    assert rel_error(got, want) <= F32_RTOL
+
+
 @pytest.mark.parametrize("t,start,window,slots", [(8, 5000, FULL, 5008), (31, 3000, 2000, 2031), (16, 2100, FULL, 2116),
                                                   (5, 7000, 6999, 7004)])
 def test_several_f32_rows_through_the_row_by_row_operator_over_long_caches(gpu, t, start, window, slots, knobs):
