@@ -626,6 +626,7 @@ struct RowsLaunches {
         const char *name;
         unsigned grid;
         lng_k_attn args;
+        unsigned grid_y = 1;
     } l[2];
 };
 
@@ -675,7 +676,7 @@ int rows_launches(lng_gpu *g, lng_k_attn a, const RowsPlan &p, const lng_k_row *
     }
     if (a.n_chunks > 1 && !a.fused) {
         if (a.n_chunks <= 32 && !g->knobs.merge_wide) { // a wavefront per (row, kv head, query head), four to a workgroup (LNG_MERGE_FEW)
-            out->l[out->n++] = {g->decode_merge_few, "lng_decode_merge_few", (unsigned)(p.pairs * ((group + 3) / 4)), a};
+            out->l[out->n++] = {g->decode_merge_few, "lng_decode_merge_few", (unsigned)(p.pairs * ((group + 3) / 4)), a, a.dim / 64}; // (64 dimensions each)
         } else {                                            // a workgroup per (row, kv head, query head)
             out->l[out->n++] = {g->decode_merge, "lng_decode_merge", (unsigned)(p.pairs * group), a};
         }
@@ -711,6 +712,7 @@ int record_rows(lng_batch *b, lng_k_attn a, const lng_k_row *host_rows, size_t n
         c.fn = launches.l[i].fn;
         c.name = launches.l[i].name;
         c.grid[0] = launches.l[i].grid;
+        c.grid[1] = launches.l[i].grid_y;
         c.block = 256;
         set_args(c, launches.l[i].args);
         b->cmds.push_back(std::move(c));
@@ -1606,7 +1608,7 @@ extern "C" int lng_hip_attention_grouped_static(lng_gpu *g, void *stream, const 
         size_t size = sizeof(lng_k_attn);
         void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, &launches.l[i].args, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
                           HIP_LAUNCH_PARAM_END};
-        const hipError_t e = hipModuleLaunchKernel(launches.l[i].fn, launches.l[i].grid, 1, 1, 256, 1, 1, 0, (hipStream_t)stream, nullptr, config);
+        const hipError_t e = hipModuleLaunchKernel(launches.l[i].fn, launches.l[i].grid, launches.l[i].grid_y, 1, 256, 1, 1, 0, (hipStream_t)stream, nullptr, config);
         if (e != hipSuccess) rc = fail(LNG_ERR_GPU, "%s did not launch: %s", launches.l[i].name, hip_text(e));
     }
     if (before != g->device) hipSetDevice(before);

@@ -1357,10 +1357,13 @@ extern "C" __global__ __launch_bounds__(256) void lng_decode_merge(lng_k_attn a)
 }
 
 // The same merge when no row has more than LNG_MERGE_FEW chunks (many rows in the dispatch: a table of sequences): a
-// wavefront per (row, kv head, query head), four to a workgroup, no LDS and no barrier - the lanes hold the
-// chunks' (max, sum), a lane per dimension adds the partial outputs, asked for eight at a time before the weights
-// are known. A quarter of the workgroups of lng_decode_merge, which at thousands of rows costs more to launch than
-// to run (128 sequences, up to eight chunks: 5.5 us against 17 us).
+// wavefront per (row, kv head, query head, 64 dimensions), four query heads to a workgroup, no LDS and no barrier - the
+// lanes hold the chunks' (max, sum), a lane per dimension adds the partial outputs. A quarter of the workgroups of
+// lng_decode_merge, which at thousands of rows costs more to launch than to run (128 sequences, up to eight chunks: 5.5 us
+// against 17 us).
+// Bound by latencies: the row of the table, then the partials, then the merge's own chain. Sixteen partials are asked for
+// at once, and the slices of a wide head are wavefronts of their own.
+// Wide heads (32 query heads of width 256, nine chunks) 7.6 -> 4.0 us, tables of 16 and 32 sequences 6.0 -> 5.2 and 6.2 -> 4.7.
 #define LNG_MERGE_FEW 32u
 extern "C" __global__ __launch_bounds__(256) void lng_decode_merge_few(lng_k_attn a) {
     const uint32_t group = a.heads / a.kv_heads;
@@ -1371,27 +1374,30 @@ extern "C" __global__ __launch_bounds__(256) void lng_decode_merge_few(lng_k_att
     if (h >= group) return;
     const uint32_t row = pair / a.kv_heads;
     const uint32_t g = pair % a.kv_heads;
-    const lng_k_row it = row_of(a, row);
-    const uint64_t last = it.start;
-    const uint64_t base = first_visible(last, it.window) & ~(uint64_t)31;
-    const uint32_t row_chunks = (uint32_t)((last + 1 - base + a.chunk - 1) / a.chunk); // <= n_chunks <= LNG_MERGE_FEW
-    if (row_chunks == 1) return; // the decode kernel already wrote this row
+    const uint32_t head = g * group + h, db = blockIdx.y * 64u;
     const uint64_t step = (uint64_t)group * a.dim;
-    const uint32_t head = g * group + h;
     const uint64_t slot0 = ((uint64_t)pair * a.n_chunks) * group + h;
-    const float *po = a.partial_o + slot0 * a.dim + lane;
-    float x[8]; // the first 64 dimensions' partial outputs of the first eight chunks, asked for before the weights are known
+    const float *po = a.partial_o + slot0 * a.dim + db + lane;
+    const uint32_t c = lane & (LNG_MERGE_FEW - 1u); // both halves of the wavefront hold the same chunks
+    const float *pml = a.partial_ml + slot0 * 2u;
+    const lng_k_row it = row_of(a, row);
+    const uint64_t base = first_visible(it.start, it.window) & ~(uint64_t)31;
+    const uint32_t row_chunks = (uint32_t)((it.start + 1 - base + a.chunk - 1) / a.chunk); // <= n_chunks <= LNG_MERGE_FEW
+    if (row_chunks == 1) return; // the decode kernel already wrote this row
+    // Chunks past the row's last read the last one again and are replaced: loads behind branches are waited for one by one.
+    float x[16];
+    auto ask = [&](uint32_t c0) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = (uint32_t)u < row_chunks ? po[(uint64_t)u * step] : 0.0f;
+        for (int u = 0; u < 16; ++u) {
+            const uint32_t at = c0 + (uint32_t)u < row_chunks ? c0 + (uint32_t)u : row_chunks - 1u;
+            x[u] = po[(uint64_t)at * step];
+        }
+    };
+    ask(0);
+    const float2 ml = *(const float2 *)(pml + (c < row_chunks ? c : row_chunks - 1u) * group * 2u);
     const float sink2 = it.sinks_offset != LNG_NO_SINKS ? ((const float *)(a.sinks + it.sinks_offset))[head] * LNG_LOG2E
                                                          : LNG_NEG_INF;
-    const uint32_t c = lane & (LNG_MERGE_FEW - 1u); // both halves of the wavefront hold the same chunks
-    float mc = LNG_NEG_INF, lc = 0.0f;
-    if (c < row_chunks) {
-        const float2 ml = *(const float2 *)(a.partial_ml + (slot0 + (uint64_t)c * group) * 2u);
-        mc = ml.x;
-        lc = ml.y;
-    }
+    const float mc = c < row_chunks ? ml.x : LNG_NEG_INF, lc = c < row_chunks ? ml.y : 0.0f;
     float top = fmaxf(mc, sink2);
 #pragma unroll
     for (int s = 16; s >= 1; s >>= 1) top = fmaxf(top, __shfl_xor(top, s, 64));
@@ -1400,26 +1406,23 @@ extern "C" __global__ __launch_bounds__(256) void lng_decode_merge_few(lng_k_att
 #pragma unroll
     for (int s = 16; s >= 1; s >>= 1) z += __shfl_xor(z, s, 64);
     z += sink2 == LNG_NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(sink2 - top);
-    for (uint32_t db = 0; db < a.dim; db += 64u) {
-        float o0 = 0.0f, o1 = 0.0f;
-        for (uint32_t c0 = 0; c0 < row_chunks; c0 += 8u) { // uniform: one turn up to eight chunks
-            if (db || c0) {
+    float o0 = 0.0f, o1 = 0.0f;
+    for (uint32_t c0 = 0; c0 < row_chunks; c0 += 16u) { // uniform: one turn up to sixteen chunks
+        if (c0) ask(c0);
 #pragma unroll
-                for (int u = 0; u < 8; ++u) x[u] = c0 + (uint32_t)u < row_chunks ? po[db + (uint64_t)(c0 + u) * step] : 0.0f;
-            }
+        for (int u = 0; u < 16; ++u) x[u] = c0 + (uint32_t)u < row_chunks ? x[u] : 0.0f;
 #pragma unroll
-            for (int u = 0; u < 8; u += 2) {
-                o0 += x[u] * __shfl(wt, (int)(c0 + u), 64);
-                o1 += x[u + 1] * __shfl(wt, (int)(c0 + u + 1), 64);
-            }
+        for (int u = 0; u < 16; u += 2) { // (the chunk is the same for every lane: its weight comes from a lane's register)
+            o0 += x[u] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wt), (int)(c0 + u)));
+            o1 += x[u + 1] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wt), (int)(c0 + u + 1)));
         }
-        const float res = (o0 + o1) / z;
-        const uint64_t at = (uint64_t)head * a.dim + db + lane;
-        if (a.dtype == LNG_F32) {
-            ((float *)(a.out + it.out_offset))[at] = res;
-        } else {
-            ((uint16_t *)(a.out + it.out_offset))[at] = f32_to_bf16_bits(res);
-        }
+    }
+    const float res = (o0 + o1) / z;
+    const uint64_t at = (uint64_t)head * a.dim + db + lane;
+    if (a.dtype == LNG_F32) {
+        ((float *)(a.out + it.out_offset))[at] = res;
+    } else {
+        ((uint16_t *)(a.out + it.out_offset))[at] = f32_to_bf16_bits(res);
     }
 }
 

@@ -776,6 +776,25 @@ def test_f32_passes_of_few_tiles_split_their_keys(gpu, t, start, window, slots, 
     assert rel_error(got, want) <= F32_RTOL
 
 
+@pytest.mark.parametrize("start", [600, 2040, 2100, 4090])
+@pytest.mark.parametrize("dtype,dim", [(C.F32, 128), (C.F32, 256), (C.BF16, 256), (C.BF16, 64)])
+def test_merges_of_up_to_32_chunks(gpu, dtype, dim, start, knobs):
+    """One row over a run of 5, 16, 17 and 32 chunks merged by lng_decode_merge_few (one turn of sixteen partials, a turn and
+    one more, two), a wavefront per 64 dimensions of the head."""
+    knobs.setenv("LNG_FUSE_WGS", "0")
+    q, k, v, sinks = normal_inputs(start, 1, start + 1, 32, 16, dim, scale=0.5)
+    shape = C.GroupedShape(1, start, 32, 16, dim, FULL, start + 1, 1.0 / np.sqrt(dim))
+    if dtype == C.F32:
+        want = oracle.attention_f32(q, k, v, sinks, start, window=FULL, slots=None, scale=1.0 / np.sqrt(dim), threads=THREADS)
+        got = run_attention(gpu, q, k, v, sinks, shape, False, dtype, expect_kernel="lng_decode_merge_few")
+        assert rel_error(got, want) <= F32_RTOL
+    else:
+        qb, kb, vb = (to_bf16_bits(x) for x in (q, k, v))
+        want = from_bf16_bits(oracle.attention_bf16(qb, kb, vb, sinks, start, window=FULL, scale=1.0 / np.sqrt(dim), threads=THREADS))
+        got = from_bf16_bits(run_attention(gpu, qb, kb, vb, sinks, shape, False, dtype, expect_kernel="lng_decode_merge_few"))
+        assert np.abs(got - want).max() <= BF16_TOL
+
+
 @pytest.mark.parametrize("t,start,window,slots", [(8, 5000, FULL, 5008), (31, 3000, 2000, 2031), (16, 2100, FULL, 2116),
                                                   (5, 7000, 6999, 7004)])
 def test_several_f32_rows_through_the_row_by_row_operator_over_long_caches(gpu, t, start, window, slots, knobs):
