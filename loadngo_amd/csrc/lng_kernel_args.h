@@ -212,6 +212,13 @@ typedef struct lng_k_q8 {
 } lng_k_q8;
 #define LNG_Q8_MORE 3
 
+/* The q, k and v projections of few positions and the preparation of attention from them, in one dispatch: matrices 0, 1
+ * and 2 are q, k and v, position p is item p of the table or row p of the one item; heads of 64, all of it rotated. */
+typedef struct lng_k_q8_prepare {
+    lng_k_q8 q8;
+    lng_k_prepare prepare;
+} lng_k_q8_prepare;
+
 /* Synthetic element i: z = splitmix64 finaliser of (i' + seed * 0x9E3779B97F4A7C15) with
  * i' = period ? i % period : i; s = sum of the four 16-bit fields of z; value =
  * (float)(s - 131070) * factor, one f32 multiply, then narrowed if the dtype is bf16.

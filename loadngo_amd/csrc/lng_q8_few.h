@@ -62,7 +62,12 @@ extern "C" __global__ __launch_bounds__(512) void lng_q8_norm_frag(lng_k_q8_spli
 #define Q8F_SC_BLOCKS 512u
 __device__ __forceinline__ uint32_t q8_few_sc_words(uint32_t blocks) { return ((blocks + 1u) / 2u) | 1u; }
 
-template <int NW> struct Q8Few {
+// HEADS: the tile's sixteen rows are 8 q .. 8 q + 7 and 32 + 8 q .. of a head of 64 (tile = 4 head + q): what rotation by
+// halves pairs is in one tile.
+template <bool HEADS> __device__ __forceinline__ uint32_t q8_tile_row(uint32_t tile) { return HEADS ? (tile >> 2) * 64u + (tile & 3u) * 8u : tile * 16u; }
+template <bool HEADS> __device__ __forceinline__ uint32_t q8_row_in(uint32_t j) { return HEADS ? (j & 7u) + (j >> 3) * 32u : j; }
+
+template <int NW, bool HEADS = false> struct Q8Few {
     static constexpr int U = 8; // block pairs in flight: 4,096 columns in one turn of eight wavefronts
     const int8_t *w_src;
     const uint16_t *sc_rows;   // the tile's first row of scales
@@ -81,9 +86,9 @@ template <int NW> struct Q8Few {
         pairs = (blocks + 1u) / 2u;
         from = wave * pairs / NW;
         to = (wave + 1u) * pairs / NW;
-        const uint32_t r0 = tile * 16u;
-        rows_here = a.rows - r0 < 16u ? a.rows - r0 : 16u;
-        const uint32_t row = j < rows_here ? j : rows_here - 1u;
+        const uint32_t r0 = q8_tile_row<HEADS>(tile);
+        rows_here = HEADS || a.rows - r0 >= 16u ? 16u : a.rows - r0;
+        const uint32_t row = q8_row_in<HEADS>(j < rows_here ? j : rows_here - 1u);
         w_src = a.codes + (uint64_t)(r0 + row) * a.cols + 16u * kg;
         sc_rows = a.scales + (uint64_t)r0 * blocks;
         staged = blocks <= Q8F_SC_BLOCKS;
@@ -97,7 +102,7 @@ template <int NW> struct Q8Few {
     }
     __device__ __forceinline__ uint32_t sc_row(int i) const {
         const uint32_t row = wave * (16 / NW) + i;
-        return row < rows_here ? row : rows_here - 1u;
+        return q8_row_in<HEADS>(row < rows_here ? row : rows_here - 1u);
     }
     __device__ __forceinline__ void ask_scales() { // the first 64 words of the wavefront's rows, into registers
         if (!staged) return;
@@ -130,9 +135,48 @@ template <int NW> struct Q8Few {
         const auto s1 = __builtin_amdgcn_permlane32_swap(w[u].y, w[u].w, false, false);
         b[0] = q8_codes_to_bf16_perm(make_uint2(s0[0], s1[0]));
         b[1] = q8_codes_to_bf16_perm(make_uint2(s0[1], s1[1]));
-        const uint32_t both = staged ? s_sc[j * words + pair] : load_sc(j < rows_here ? j : rows_here - 1u, pair);
+        const uint32_t both = staged ? s_sc[j * words + pair] : load_sc(q8_row_in<HEADS>(j < rows_here ? j : rows_here - 1u), pair);
         sc[0] = f16_bits_to_f32((uint16_t)both);
         sc[1] = f16_bits_to_f32((uint16_t)(both >> 16)); // zero past an odd number of blocks
+    }
+};
+
+// lng_prepare's step for one output of the q, k or v projection (which = 0, 1, 2; heads of 64, all of it rotated): bias,
+// rotation with the value 32 rows away, narrowing, to the prepared queries or the cache. What it needs besides the two values
+// is asked for before the product.
+struct Q8Prepared {
+    float bias, bias_there, c, s;
+    char *to;
+    __device__ __forceinline__ void ask(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row) {
+        const lng_prepare_item it = p.items ? p.items[position] : p.first;
+        const uint32_t r = p.items ? 0u : position; // a table's items are of one position each
+        const float *b = which == 0 ? p.q_bias : which == 1 ? p.k_bias : p.v_bias;
+        bias = b ? b[row] : 0.0f;
+        bias_there = b && which < 2u ? b[row ^ 32u] : 0.0f;
+        c = 0.0f, s = 0.0f;
+        if (which < 2u) {
+            const float2 t = *(const float2 *)(p.table + it.table_offset + ((uint64_t)r * 32u + (row & 31u)) * 8u);
+            c = t.x, s = t.y;
+        }
+        const uint32_t es = p.out_dtype == LNG_BF16 ? 2u : 4u;
+        if (which == 0) {
+            to = p.q_out + it.q_out_offset + ((uint64_t)r * p.heads * 64u + row) * es;
+        } else {
+            const uint64_t at = ((it.start + r) % it.slots * p.kv_heads * 64u + row) * es;
+            to = which == 1 ? p.k_cache + it.k_cache_offset + at : p.v_cache + it.v_cache_offset + at;
+        }
+    }
+    __device__ __forceinline__ void store(const lng_k_prepare &p, uint32_t which, uint32_t row, float here, float there) const {
+#pragma clang fp contract(off)
+        const float *b = which == 0 ? p.q_bias : which == 1 ? p.k_bias : p.v_bias;
+        float x = here, y = there;
+        if (b) {
+            x = x + bias;
+            y = y + bias_there;
+        }
+        if (which < 2u) x = (row & 32u) ? x * c + y * s : x * c - y * s;
+        if (p.out_dtype == LNG_BF16) *(uint16_t *)to = f32_to_bf16_bits(x);
+        else *(float *)to = x;
     }
 };
 
@@ -147,12 +191,13 @@ template <int NW> struct Q8Few {
 // first: a product is one round trip to memory, not one per block.
 // PLANES 2: x as lng_q8_norm_frag left it; 1: bf16 positions, turned into operand order through LDS that only this
 // wavefront uses (lng_q8_mid).
-template <int PLANES, int NW> __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, char *s_mem) {
+template <int PLANES, int NW, bool PREPARE = false>
+__device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
     constexpr int U = Q8Few<NW>::U, D = PLANES == 2 ? 3 : U; // pairs of x in flight
     constexpr uint32_t STRIDE = 80;
     __shared__ float s_red[NW][4][64];
-    Q8Few<NW> m(a, tile, (uint32_t *)(s_mem + (PLANES == 1 ? NW * 2u * 16u * STRIDE : 0u)));
-    const uint32_t lane = m.lane, j = m.j, kg = m.kg, p0 = blockIdx.y * 16u, r0 = tile * 16u;
+    Q8Few<NW, PREPARE> m(a, tile, (uint32_t *)(s_mem + (PLANES == 1 ? NW * 2u * 16u * STRIDE : 0u)));
+    const uint32_t lane = m.lane, j = m.j, kg = m.kg, p0 = blockIdx.y * 16u, r0 = q8_tile_row<PREPARE>(tile);
     char *s_x = s_mem + m.wave * 2u * 16u * STRIDE;
     const uint32_t put = (lane >> 2) * STRIDE + 16u * (lane & 3u), get = j * STRIDE + 16u * q8_mid_chunk(kg);
     const uint4 *x_frag = (const uint4 *)a.x_hi + (uint64_t)blockIdx.y * m.blocks * 128u + lane;
@@ -172,7 +217,7 @@ template <int PLANES, int NW> __device__ __forceinline__ void q8_few_body(const 
         }
     };
     // this thread's output, and what is added to it
-    const uint32_t out_p = p0 + 4u * kg + m.wave, out_row = r0 + j; // wavefronts 0-3: accumulator register = wavefront
+    const uint32_t out_p = p0 + 4u * kg + m.wave, out_row = r0 + q8_row_in<PREPARE>(j); // wavefronts 0-3: accumulator register = wavefront
     const bool mine = m.wave < 4u && out_p < a.n && j < m.rows_here;
     float *yp = a.y + (uint64_t)out_p * a.y_stride + out_row;
     float bias = 0.0f, held = 0.0f;
@@ -180,6 +225,10 @@ template <int PLANES, int NW> __device__ __forceinline__ void q8_few_body(const 
     if (mine && a.accumulate) held = *yp;
     float *to = a.residual + (uint64_t)out_p * a.rows + out_row; // (never with accumulate)
     if (mine && a.residual) held = *to;
+    Q8Prepared ready;
+    if constexpr (PREPARE) {
+        if (mine) ready.ask(*prepare, which, out_p, out_row);
+    }
 
     floatx4 y = {0.0f, 0.0f, 0.0f, 0.0f};
     const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -236,17 +285,19 @@ template <int PLANES, int NW> __device__ __forceinline__ void q8_few_body(const 
     if (a.accumulate) sum = held + sum; // h + ((W x) + bias), each sum rounded as the separate dispatches round it
     *yp = sum;
     if (a.residual) *to = held + sum;
+    if constexpr (PREPARE) ready.store(*prepare, which, out_row, sum, __shfl_xor(sum, 8, 64)); // (all rows of a position are mine or none)
 }
 
 // One position. Its operand planes are made once per workgroup (normalised, split: a thread takes eight columns) and wait
 // in LDS. f32: even rows of the A operand are the hi plane, odd ones the lo plane, and one matrix instruction multiplies
 // a block by both; all rows of bf16 are the position.
-template <bool BF16, int NW> __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem) {
+template <bool BF16, int NW, bool PREPARE = false>
+__device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
     constexpr int U = Q8Few<NW>::U, T = 64 * NW;
     __shared__ float s_red[NW][16];
     __shared__ float s_norm[NW];
-    Q8Few<NW> m(a, tile, (uint32_t *)(s_mem + (uint64_t)a.cols * (BF16 ? 2u : 4u)));
-    const uint32_t chunks = a.cols / 8u, mine = threadIdx.x, out_row = tile * 16u + mine;
+    Q8Few<NW, PREPARE> m(a, tile, (uint32_t *)(s_mem + (uint64_t)a.cols * (BF16 ? 2u : 4u)));
+    const uint32_t chunks = a.cols / 8u, mine = threadIdx.x, out_row = q8_tile_row<PREPARE>(tile) + q8_row_in<PREPARE>(mine & 15u);
     const bool writes = mine < m.rows_here;
     uint4 *s_x = (uint4 *)s_mem; // [plane][chunk of eight columns]
     float x[8] = {}, nw[8] = {};
@@ -269,6 +320,10 @@ template <bool BF16, int NW> __device__ __forceinline__ void q8_one_body(const l
     if (writes && a.bias) bias = a.bias[out_row];
     if (writes && a.accumulate) held = a.y[out_row];
     if (writes && a.residual) held = a.residual[out_row]; // (never with accumulate)
+    Q8Prepared ready;
+    if constexpr (PREPARE) {
+        if (writes) ready.ask(*prepare, which, 0, out_row);
+    }
     __builtin_amdgcn_sched_barrier(0);
     m.ask_codes(m.from); // after what is waited for first: loads come back in order
     __builtin_amdgcn_sched_barrier(0);
@@ -346,6 +401,7 @@ template <bool BF16, int NW> __device__ __forceinline__ void q8_one_body(const l
     if (a.accumulate) sum = held + sum;
     a.y[out_row] = sum;
     if (a.residual) a.residual[out_row] = held + sum;
+    if constexpr (PREPARE) ready.store(*prepare, which, out_row, sum, __shfl_xor(sum, 8, 64));
 }
 
 #define Q8_FEW(name, body, what, nw) \
@@ -358,3 +414,15 @@ Q8_FEW(lng_q8_few, q8_few_body, 2, 8)
 Q8_FEW(lng_q8_few_bf16, q8_few_body, 1, 8)
 Q8_FEW(lng_q8_one, q8_one_body, false, 8)
 Q8_FEW(lng_q8_one_bf16, q8_one_body, true, 8)
+
+// q, k and v with the preparation of attention after them.
+#define Q8_FEW_PREPARE(name, body, what, nw) \
+    extern "C" __global__ __launch_bounds__(64 * nw, nw / 2) void name(lng_k_q8_prepare both) { \
+        extern __shared__ __attribute__((aligned(16))) char s_mem[]; \
+        lng_k_q8 a = both.q8; \
+        const uint32_t which = blockIdx.x >= a.more[1].first_tile ? 2u : blockIdx.x >= a.more[0].first_tile ? 1u : 0u; \
+        const uint32_t tile = q8_select_matrix(a); \
+        body<what, nw, true>(a, tile, s_mem, &both.prepare, which); \
+    }
+Q8_FEW_PREPARE(lng_q8_few_prepare, q8_few_body, 2, 8)
+Q8_FEW_PREPARE(lng_q8_one_prepare, q8_one_body, false, 8)

@@ -119,3 +119,46 @@ def test_bias_and_residual_in_the_product(gpu, n, rows, cols, bf16):
     for i, (a, b) in enumerate(zip(fused, apart)):
         assert np.array_equal(a, b), "buffer %d" % i
     assert not np.isnan(fused[5].view(np.float32)[:6 * n * rows]).any()
+
+
+@pytest.mark.parametrize("dtype", [C.F32, C.BF16])
+@pytest.mark.parametrize("n,one_item,dim,rotary,bias,normed,kind", [
+    (1, True, 64, 64, True, True, ""), (1, True, 64, 64, False, False, ""), (2, False, 64, 64, True, True, ""), (16, False, 64, 64, True, True, ""),
+    (3, True, 64, 64, True, False, ""), (16, True, 64, 64, False, True, ""), (17, False, 64, 64, True, True, ""), (5, False, 64, 32, True, True, ""),
+    (2, False, 128, 128, True, True, ""), (4, False, 64, 64, True, True, "backwards"), (4, False, 64, 64, True, True, "swapped"),
+    (4, False, 64, 64, True, True, "table over q"), (4, False, 64, 64, True, True, "queries over x")])
+def test_projections_and_preparation_in_one_kernel(gpu, n, one_item, dim, rotary, bias, normed, kind, dtype):
+    """q, k and v of up to 16 positions with the preparation after them: tables of items and one item, rings that wrap, with
+    and without biases and norm; and what stays apart: more positions, other widths, items in another order than the rows, k
+    and v the other way round, a rotation table in rows that q is written to, prepared queries where x is."""
+    heads, kv_heads, cols, slots, eps = 6, 2, 96, 24, 1e-5
+    qw, kw, es = heads * dim, kv_heads * dim, 4 if dtype == C.F32 else 2
+    mats = [q8_test_matrix(rows, cols, 60 + i)[:2] for i, rows in enumerate((qw, kw, kw))]
+    arrays = [3 * xorshift_values(81 + n, n * max(cols, qw)), 1 + 0.2 * xorshift_values(82, cols), xorshift_values(83, n * qw),
+              np.zeros(2 * n * kw, np.float32), xorshift_values(84, n * rotary), np.zeros(n * qw * es, np.uint8),
+              np.zeros(2 * n * slots * kw * es, np.uint8), xorshift_values(85, qw + 2 * kw)]
+    for codes, bits in mats:
+        arrays += [codes, bits]
+    table, q_out = (2 if kind == "table over q" else 4), (0 if kind == "queries over x" else 5)
+    k_at, v_at = (n * kw * 4, 0) if kind == "swapped" else (0, n * kw * 4)
+    order = list(range(n))[::-1] if kind == "backwards" else list(range(n))
+    item = lambda i, j, rows, start: C.PrepareItem(  # noqa: E731
+        q_offset=j * qw * 4, k_offset=j * kw * 4, v_offset=n * kw * 4 + j * kw * 4, table_offset=j * rotary * 4, q_out_offset=j * qw * es,
+        k_cache_offset=i * slots * kw * es, v_cache_offset=(n + i) * slots * kw * es, n=rows, start=start, slots=slots)
+    items = C.prepare_items([item(0, 0, n, slots - 1)] if one_item else [item(i, j, 1, 5 + 13 * i) for i, j in enumerate(order)])
+    biases = [C.Slice(7, 0, qw * 4), C.Slice(7, qw * 4, kw * 4), C.Slice(7, (qw + kw) * 4, kw * 4)] if bias else [None] * 3
+
+    def record(batch):
+        many = [((C.Slice(8 + 2 * i, 0, rows * cols), C.Slice(9 + 2 * i, 0, rows * cols // 16)), y, rows)
+                for i, (rows, y) in enumerate(((qw, C.Slice(2, 0, n * qw * 4)), (kw, C.Slice(3, k_at, n * kw * 4)), (kw, C.Slice(3, v_at, n * kw * 4))))]
+        xs = C.Slice(0, 0, n * cols * 4)
+        if normed:
+            batch.gemm_q8_0_many_normed(many, xs, (C.Slice(1, 0, cols * 4), eps), cols, n, cols)
+        else:
+            batch.gemm_q8_0_many(many, xs, cols, n, cols)
+        batch.prepare_attention(dict(q=2, k=3, v=3, table=table, q_out=q_out, k_cache=6, v_cache=6), items, heads, kv_heads, dim, rotary, dtype, *biases)
+
+    fused, apart = both_ways(gpu, arrays, record)
+    for i, (a, b) in enumerate(zip(fused, apart)):
+        assert np.array_equal(a, b), "buffer %d" % i
+    assert fused[5 if q_out == 5 else 0].any() and fused[6].any()
