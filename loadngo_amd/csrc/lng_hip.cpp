@@ -2134,7 +2134,7 @@ int q8_mid_tile(const lng_gpu *g, uint64_t n, uint64_t cols, bool x_bf16) {
 // Fewer than 32: a workgroup per position, with the RMS norm if a.norm_w is set.
 int q8_record_frag(lng_batch *b, lng_k_q8 *a, uint64_t n_pad) {
     const uint64_t cols = a->cols;
-    if (!fits_u32(n_pad * cols)) return fail(LNG_ERR_DISPATCH, "too large");
+    if (a->n >= 32 && !fits_u32(n_pad * cols)) return fail(LNG_ERR_DISPATCH, "too large");
     char *planes = nullptr;
     if (int rc = reserve_x(b->gpu, 2 * n_pad * cols * 2, &planes)) return rc;
     lng_k_q8_split sp{};

@@ -124,7 +124,7 @@ template <int NW, bool HEADS = false> struct Q8Few {
             const uint32_t pair = base + u;
             w[u] = make_uint4(0, 0, 0, 0);
             if (pair < to) { // uniform; a last pair of one block: its upper lanes load the block again
-                const int32_t col = (int32_t)(64u * pair) - (2u * pair + 1u == blocks && kg >= 2u ? 32 : 0);
+                const int64_t col = (int64_t)(64ull * pair) - (2u * pair + 1u == blocks && kg >= 2u ? 32 : 0);
                 w[u] = *(const uint4 *)(w_src + col);
             }
         }
@@ -211,8 +211,8 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
             if constexpr (PLANES == 1) {
                 to[h][0] = *(const uint4 *)(x_row + 32u * b);
             } else {
-                to[h][0] = x_frag[b * 128u];
-                to[h][1] = x_frag[b * 128u + 64u];
+                to[h][0] = x_frag[(uint64_t)b * 128u];
+                to[h][1] = x_frag[(uint64_t)b * 128u + 64u];
             }
         }
     };
