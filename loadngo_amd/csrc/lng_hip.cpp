@@ -2116,18 +2116,47 @@ const Q8MidTile q8_mid_tiles[4] = {{16, 32, 8, {nullptr, "lng_q8_mid_bf16_r16p32
                                    {32, 64, 4, {nullptr, "lng_q8_mid_bf16_r32p64"}},
                                    {64, 64, 4, {"lng_q8_mid_r64p64", "lng_q8_mid_bf16_r64p64"}}};
 
-// The tile of lng_q8_mid* a product takes; -1: lng_q8_few (fewer than 32 positions) or lng_q8_tiled. It depends on nothing that differs between a
-// product alone and among several matrices, so that its sums keep their order.
+// What a product of 32 positions or more takes on either kernel, us on 256 compute units, fitted to 2,400 products of 64 to
+// 201,088 rows, 32 to 12,288 columns and 32 to 1,280 positions (`wide`: the columns, in units of 2,880).
+// lng_q8_tiled: rounds of its 256 x 128 tiles on the device's units (from eight tiles of positions on each XCD keeps to its
+// own, and some may have none: fewer units, a little faster each), and what a full device loses in clock.
+double q8_tiled_us(const lng_gpu *g, uint64_t n, uint64_t rows, uint64_t cols, bool x_bf16) {
+    const uint64_t row_tiles = (rows + 255) / 256, pos_tiles = (n + 127) / 128, per_xcd = (pos_tiles + 7) / 8;
+    const uint64_t tiles = pos_tiles < 8 ? row_tiles * pos_tiles : 8 * per_xcd * ((row_tiles + 7) / 8 * 8);
+    const bool idle = pos_tiles >= 8 && per_xcd * 8 != pos_tiles;
+    const double rounds = (double)((tiles + g->cus - 1) / g->cus), wide = (double)cols / 2880.0;
+    const double work = (double)rows * (double)n / (256.0 * 256.0 * 128.0);
+    if (x_bf16) return rounds * (6.8 + 58.0 * wide * (idle ? 0.92 : 1.0)) + 15.5 * work * wide;
+    return 3.7 + rounds * (5.8 + 82.0 * wide * (idle ? 0.95 : 1.0)) + 18.0 * work * wide;
+}
+// lng_q8_mid*: its tiles, and the codes' way from memory; positions that the L2 caches no longer hold come from further away.
+double q8_mid_us(uint64_t n, uint64_t rows, uint64_t cols, bool x_bf16, int tile) {
+    const Q8MidTile &t = q8_mid_tiles[tile];
+    const double tiles = (double)((rows + t.rows - 1) / t.rows) * (double)((n + t.pos - 1) / t.pos);
+    const double wide = (double)cols / 2880.0, codes = (double)rows / 65536.0 * wide;
+    double us;
+    if (!x_bf16) us = tile == 1 ? 5.0 + tiles * (0.0039 + 0.0235 * wide) + 24.0 * codes : 8.0 + 8.0 * wide + tiles * (0.0069 + 0.058 * wide);
+    else if (tile == 0) us = 3.0 + tiles * 0.002 + codes * (20.0 + 2.6 * (double)n);
+    else if (tile == 2) us = 4.0 + 3.0 * wide + tiles * 0.0023 + codes * ((n > 64 ? 66.0 : 33.0) + 0.45 * (double)n);
+    else us = 5.5 + 7.0 * wide + tiles * (0.0073 + 0.0456 * wide);
+    return n * cols > 8u << 20 ? 1.2 * us : us;
+}
+
+// The tile of lng_q8_mid* a product takes; -1: lng_q8_few (fewer than 32 positions) or lng_q8_tiled. From 32 positions on it
+// depends on nothing that differs between a product alone and among several matrices, so that its sums keep their order.
 // Measured (2,880 x 4,096 bf16 / the 5,120 x 2,880 of q, k and v), us: tiles 16 x 32, 32 x 32, 32 x 64, 64 x 64 at 32
 // positions 8.7, 11, 15, 22 / 14, 12, 16, 22; at 77 20, 19, 16, 24 / 24, 19, 26, 25; at 192 33, 28, 27, 25 / 44, 33, 29, 28.
 // Against lng_q8_tiled: 1,280 positions 82 / 135 against 91 / 297, 1,536 99 / 169 against 92 / 305 (one matrix of 4,096
-// rows 133 against 113): x no longer stays in the L2 caches between the row tiles.
-int q8_mid_tile(const lng_gpu *g, uint64_t n, uint64_t cols, bool x_bf16) {
+// rows 133 against 113): x no longer stays in the L2 caches between the row tiles. Matrices of many rows fill the device
+// with lng_q8_tiled's own tiles, which read every operand less often (65,536 x 2,880 at 128 positions 112 us against 196,
+// bf16 78 against 138; 16,384 x 2,880 at 512 114 against 139, 76 against 107): where the estimates are close, lng_q8_tiled.
+int q8_mid_tile(const lng_gpu *g, uint64_t n, uint64_t rows, uint64_t cols, bool x_bf16) {
     if (n <= 16) return -1; // q8_record_few (17 to 31 as two groups of 16 would read the codes twice)
     if (cols > 32 * 512) return -1; // a tile's scales are held in LDS: at most 64 KB of them
-    if (n >= 32 && (g->knobs.q8_mid == 0 || (g->knobs.q8_mid < 0 && n > 1280))) return -1;
-    if (x_bf16) return n <= 48 ? 0 : n <= 128 ? 2 : 3;
-    return n <= 128 ? 1 : 3;
+    const int tile = x_bf16 ? (n <= 48 ? 0 : n <= 128 ? 2 : 3) : n <= 128 ? 1 : 3;
+    if (n < 32 || g->knobs.q8_mid == 1) return tile;
+    if (g->knobs.q8_mid == 0 || n > 1280) return -1;
+    return 0.95 * q8_tiled_us(g, n, rows, cols, x_bf16) < q8_mid_us(n, rows, cols, x_bf16, tile) ? -1 : tile;
 }
 
 // f32 positions into operand order (a.x_hi): all at once for lng_q8_few, lng_q8_mid and every matrix of the dispatch.
@@ -2262,7 +2291,7 @@ int q8_record_tiled(lng_batch *b, lng_k_q8 a, bool x_bf16, const uint16_t *plane
 
 // A product of one matrix.
 int q8_record(lng_batch *b, lng_k_q8 a, bool x_bf16) {
-    const int tile = q8_mid_tile(b->gpu, a.n, a.cols, x_bf16);
+    const int tile = q8_mid_tile(b->gpu, a.n, a.rows, a.cols, x_bf16);
     if (tile < 0 && a.n >= 32) return q8_record_tiled(b, a, x_bf16);
     const uint64_t tile_rows = tile < 0 ? 16 : q8_mid_tiles[tile].rows;
     a.tiles = (uint32_t)((a.rows + tile_rows - 1) / tile_rows);
@@ -2370,41 +2399,52 @@ int q8_many(lng_batch *b, const lng_q8_matrix *matrices, size_t n_matrices, lng_
             if (overlaps(q[i].y, onw)) return fail(LNG_ERR_DISPATCH, "output overlaps an input");
         }
     }
-    const int tile = q8_mid_tile(b->gpu, n, cols, false);
-    if (n >= 32 && tile < 0) { // the matrix unit is the bound there, not the launches: one product after the other
-        const size_t cmds = b->cmds.size(), dispatches = b->dispatches;
-        const uint16_t *planes = nullptr;
-        for (size_t i = 0; i < n_matrices; ++i) {
-            if (int rc = q8_record_tiled(b, q[i].a, false, planes, &planes)) {
-                b->cmds.resize(cmds); // a refused dispatch leaves nothing behind
-                b->dispatches = dispatches;
-                return rc;
-            }
+    // One dispatch; but from 32 positions on matrices that lng_q8_tiled takes come after it one by one, where the matrix unit
+    // is the bound and not the launches.
+    const size_t cmds = b->cmds.size(), dispatches = b->dispatches;
+    auto refused = [&](int rc) { // a refused dispatch leaves nothing behind
+        b->cmds.resize(cmds);
+        b->dispatches = dispatches;
+        return rc;
+    };
+    bool alone[1 + LNG_Q8_MORE] = {};
+    lng_k_q8 a{};
+    uint64_t tiles = 0, together = 0;
+    int tile = -1; // (of all that share the dispatch: the positions and columns decide it)
+    for (size_t i = 0; i < n_matrices; ++i) {
+        const int own = q8_mid_tile(b->gpu, n, q[i].a.rows, cols, false);
+        alone[i] = n >= 32 && own < 0;
+        if (alone[i]) continue;
+        tile = own;
+        const uint64_t tile_rows = tile < 0 ? 16 : q8_mid_tiles[tile].rows;
+        if (together++ == 0) {
+            a = q[i].a;
+        } else {
+            auto &m = a.more[a.n_more++];
+            m.codes = q[i].a.codes;
+            m.scales = q[i].a.scales;
+            m.y = q[i].a.y;
+            m.rows = q[i].a.rows;
+            m.y_stride = q[i].a.y_stride;
+            m.first_tile = (uint32_t)tiles;
         }
-        return LNG_OK;
-    }
-    const uint64_t tile_rows = tile < 0 ? 16 : q8_mid_tiles[tile].rows;
-    lng_k_q8 a = q[0].a;
-    uint64_t tiles = (a.rows + tile_rows - 1) / tile_rows;
-    a.n_more = (uint32_t)(n_matrices - 1);
-    for (size_t i = 1; i < n_matrices; ++i) {
-        auto &m = a.more[i - 1];
-        m.codes = q[i].a.codes;
-        m.scales = q[i].a.scales;
-        m.y = q[i].a.y;
-        m.rows = q[i].a.rows;
-        m.y_stride = q[i].a.y_stride;
-        m.first_tile = (uint32_t)tiles;
         tiles += (q[i].a.rows + tile_rows - 1) / tile_rows;
     }
-    if (!fits_u32(tiles) || tiles > 0x7fffffffull) return fail(LNG_ERR_DISPATCH, "too large");
+    if (tiles > 0x7fffffffull) return fail(LNG_ERR_DISPATCH, "too large");
     a.tiles = (uint32_t)tiles;
     if (norm_w) {
         a.norm_w = (const float *)((const char *)onw.buf->ptr + norm_w->offset);
         a.eps = eps;
     }
-    if (int rc = tile < 0 ? q8_record_few(b, a, tiles, false) : q8_record_mid(b, a, false, tile)) return rc;
-    b->dispatches += n < 32 ? 1 : n_matrices; // from 32 positions on counted as the products it stands for
+    if (together) {
+        if (int rc = tile < 0 ? q8_record_few(b, a, tiles, false) : q8_record_mid(b, a, false, tile)) return refused(rc);
+        b->dispatches += n < 32 ? 1 : together; // from 32 positions on counted as the products it stands for
+    }
+    const uint16_t *planes = nullptr;
+    for (size_t i = 0; i < n_matrices; ++i) {
+        if (!alone[i]) continue;
+        if (int rc = q8_record_tiled(b, q[i].a, false, planes, &planes)) return refused(rc);
+    }
     return LNG_OK;
 }
 } // namespace

@@ -5,6 +5,7 @@
 //    wrong length, outside their buffer or off their element size (apple.rs:860-887), outputs in resident memory or
 //    over an input (apple.rs:889-906), buffers that belong to a batch in flight, and the refusals of copy_rows,
 //    prepare_attention and the Q8_0 products; a refused call records nothing.
+//  - the kernels that Q8_0 products are recorded as.
 //  - the development switches (environment at open, lng_hip_debug_set afterwards) and lng_hip_checksum: refusals and
 //    what is recorded.
 //  - ownership: batches hand their buffers back; close with buffers alive; the last buffer freed on one thread while
@@ -195,6 +196,56 @@ static void refusals() {
     CHECK(lng_hip_upload(f.bufs[0], MB - 2, word, 4) == LNG_ERR_DISPATCH);
     f.rebatch();
     CHECK(lng_hip_buffer_free(res) == LNG_OK);
+    lng_null_clear();
+}
+
+static std::vector<std::string> launched() { // the kernels launched since the last clear, in order
+    std::vector<std::string> names;
+    for (size_t i = 0; i < lng_null_launch_count(); ++i) {
+        const char *name = nullptr;
+        CHECK(lng_null_launch(i, &name, nullptr, nullptr, nullptr, nullptr) == 0);
+        names.push_back(name);
+    }
+    return names;
+}
+
+// Products of 32 positions or more: lng_q8_mid* where the tiles of lng_q8_tiled would leave units idle, lng_q8_tiled where
+// they fill the device, whichever number of positions; a matrix takes the same kernel alone and among others.
+static void products_and_their_kernels() {
+    Fixture f(4, 66ull << 20);
+    const uint64_t cols = 512;
+    auto run = [&]() {
+        CHECK(lng_hip_batch_commit(f.batch, nullptr, nullptr) == LNG_OK);
+        CHECK(lng_hip_batch_wait(f.batch, nullptr) == LNG_OK);
+        const std::vector<std::string> names = launched();
+        lng_null_clear();
+        f.rebatch();
+        return names;
+    };
+    auto product = [&](uint64_t rows, uint64_t n, bool bf16) {
+        const lng_slice codes{0, 0, rows * cols}, scales{1, 0, rows * cols / 16}, x{2, 0, n * cols * (bf16 ? 2u : 4u)}, y{3, 0, n * rows * 4};
+        CHECK((bf16 ? lng_hip_gemm_q8_0_bf16 : lng_hip_gemm_q8_0)(f.batch, codes, scales, x, y, rows, cols, n, cols, rows) == LNG_OK);
+        return run().back();
+    };
+    const struct { uint64_t rows, n; bool bf16; const char *kernel; } wanted[] = {
+        {2880, 32, false, "lng_q8_mid_r32p32"}, {2880, 129, false, "lng_q8_mid_r64p64"}, {2880, 512, false, "lng_q8_mid_r64p64"}, {2880, 1281, false, "lng_q8_tiled"},
+        {65536, 128, false, "lng_q8_tiled"}, {32768, 512, false, "lng_q8_tiled"}, {16384, 512, false, "lng_q8_tiled"}, {16384, 32, false, "lng_q8_mid_r32p32"},
+        {65536, 31, false, "lng_q8_mid_r32p32"},
+        {2880, 32, true, "lng_q8_mid_bf16_r16p32"}, {2880, 77, true, "lng_q8_mid_bf16_r32p64"}, {2880, 512, true, "lng_q8_mid_bf16_r64p64"}, {2880, 1281, true, "lng_q8_tiled_bf16"},
+        {65536, 128, true, "lng_q8_tiled_bf16"}, {16384, 512, true, "lng_q8_tiled_bf16"}, {65536, 17, true, "lng_q8_mid_bf16_r16p32"}};
+    for (const auto &w : wanted) {
+        const std::string kernel = product(w.rows, w.n, w.bf16);
+        if (kernel != w.kernel) fprintf(stderr, "%llu rows, %llu positions, bf16 %d: %s\n", (unsigned long long)w.rows, (unsigned long long)w.n, w.bf16, kernel.c_str());
+        CHECK(kernel == w.kernel);
+    }
+    // several matrices: those of many rows after the dispatch that the others share, each with the kernel it takes alone
+    const uint64_t n = 128, rows[3] = {512, 62464, 2560}, at[3] = {0, 512, 62976};
+    lng_q8_matrix m[3];
+    for (int i = 0; i < 3; ++i) m[i] = {{0, at[i] * cols, rows[i] * cols}, {1, at[i] * cols / 16, rows[i] * cols / 16}, {3, at[i] * n * 4, rows[i] * n * 4}, rows[i]};
+    CHECK(lng_hip_gemm_q8_0_many(f.batch, m, 3, lng_slice{2, 0, n * cols * 4}, cols, n, cols) == LNG_OK);
+    CHECK(lng_hip_batch_dispatches(f.batch) == 3);
+    const std::vector<std::string> names = run();
+    CHECK((names == std::vector<std::string>{"lng_q8_frag_x", "lng_q8_mid_r32p32", "lng_q8_split_x", "lng_q8_tiled"}));
     lng_null_clear();
 }
 
@@ -614,6 +665,7 @@ static void planner_fuzz(size_t dispatches) {
 int main(int argc, char **argv) {
     const size_t dispatches = argc > 1 ? (size_t)strtoull(argv[1], nullptr, 10) : 100000;
     refusals();
+    products_and_their_kernels();
     switches_and_checksum();
     lifetimes();
     allocation_failures();

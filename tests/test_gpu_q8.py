@@ -463,3 +463,40 @@ def test_products_of_few_positions(gpu, rows, cols, n, bf16):
         out = out.reshape(n, y_stride)
         assert not np.isnan(out[:, :rows]).any() and np.isnan(out[:-1, rows:]).all()
         assert np.abs(out[:, :rows] - want).max() / np.abs(want).max() < 1e-5
+
+
+@pytest.mark.parametrize("n", [33, 128, 200, 700])
+def test_matrices_of_many_rows_among_others(gpu, n):
+    """32 positions or more: a matrix whose tiles of 256 x 128 fill the device and two that leave it mostly idle, in one call
+    and each alone: the same bits, within the reference's bound (glue.rs:171) of float64."""
+    cols = 64
+    shapes = [(96, 7), (20000, 8), (513, 9)]
+    x = xorshift_values(41, n * cols).reshape(n, cols)
+    mats = [q8_test_matrix(rows, cols, seed) for rows, seed in shapes]
+    y_lens = [n * rows * 4 for rows, _ in shapes]
+    bufs = [gpu.upload(x)]
+    for codes, bits, _ in mats:
+        bufs += [gpu.upload(codes), gpu.upload(bits)]
+    bufs += [gpu.buffer(2 * sum(y_lens))]
+    bufs[-1].fill(0xFF)
+    batch = gpu.batch(bufs)
+    xs, many, offset = C.Slice(0, 0, x.nbytes), [], 0
+    for i, ((rows, _), (codes, bits, _)) in enumerate(zip(shapes, mats)):
+        m = (C.Slice(1 + 2 * i, 0, codes.nbytes), C.Slice(2 + 2 * i, 0, bits.nbytes))
+        many.append((m, C.Slice(7, offset, y_lens[i]), rows))
+        batch.gemm_q8_0(m, xs, C.Slice(7, sum(y_lens) + offset, y_lens[i]), rows, cols, n, (cols, rows))
+        offset += y_lens[i]
+    batch.gemm_q8_0_many(many, xs, cols, n, cols)
+    done = batch.run()
+    assert not isinstance(done.gpu_time, Exception), done.gpu_time
+    raw = bufs[-1].read(np.float32)
+    batch.drop()
+    for b in bufs:
+        b.free()
+    together, alone = raw[:raw.size // 2], raw[raw.size // 2:]
+    assert not np.isnan(together).any() and np.array_equal(together, alone)
+    offset = 0
+    for (rows, _), (_, _, elements) in zip(shapes, mats):
+        want = x.astype(np.float64) @ elements.T
+        assert np.abs(alone[offset:offset + n * rows].reshape(n, rows) - want).max() / np.abs(want).max() < 1e-5
+        offset += n * rows
