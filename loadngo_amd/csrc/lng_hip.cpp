@@ -134,6 +134,7 @@ struct lng_gpu {
     hipFunction_t prepare_v4 = nullptr, prepare_v1 = nullptr;
     hipFunction_t q8_split_x = nullptr, q8_tiled = nullptr,
                   q8_tiled_bf16 = nullptr, q8_frag_x = nullptr;
+    hipFunction_t q8_tiled_add = nullptr, q8_tiled_bf16_add = nullptr;
     hipFunction_t q8_norm_frag = nullptr, q8_few[2] = {}, q8_one[2] = {}; // [bf16 positions]
     hipFunction_t q8_few_prepare = nullptr, q8_one_prepare = nullptr;
     hipFunction_t q8_mid[2][4] = {}; // [bf16 positions][tile, see q8_mid_tile]
@@ -1049,7 +1050,7 @@ bool fuse_split(const lng_gpu *g, Cmd &c, const Cmd &after) {
 // `c` (a product of one matrix) with the addition `after` it, of a bias into the product or of the product into other rows.
 bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
     if (after.fn != g->add_rows) return false;
-    bool product = c.fn == g->q8_tiled || c.fn == g->q8_tiled_bf16;
+    bool product = c.fn == g->q8_tiled || c.fn == g->q8_tiled_bf16 || c.fn == g->q8_tiled_add || c.fn == g->q8_tiled_bf16_add;
     for (int i = 0; i < 2; ++i) {
         product = product || c.fn == g->q8_few[i] || c.fn == g->q8_one[i];
         for (hipFunction_t fn : g->q8_mid[i]) product = product || (fn && c.fn == fn);
@@ -1070,6 +1071,8 @@ bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
     } else {
         return false;
     }
+    if (c.fn == g->q8_tiled) c.fn = g->q8_tiled_add, c.name = "lng_q8_tiled_add";
+    if (c.fn == g->q8_tiled_bf16) c.fn = g->q8_tiled_bf16_add, c.name = "lng_q8_tiled_bf16_add";
     set_args(c, a);
     return true;
 }
@@ -1201,6 +1204,8 @@ extern "C" int lng_hip_open(int device, lng_gpu **out) {
         {"lng_q8_split_x", &g->q8_split_x, true},
         {"lng_q8_tiled", &g->q8_tiled, true},
         {"lng_q8_tiled_bf16", &g->q8_tiled_bf16, true},
+        {"lng_q8_tiled_add", &g->q8_tiled_add, true},
+        {"lng_q8_tiled_bf16_add", &g->q8_tiled_bf16_add, true},
         {"lng_q8_frag_x", &g->q8_frag_x, true},
         {"lng_q8_norm_frag", &g->q8_norm_frag, true},
         {"lng_q8_few", &g->q8_few[0], true},

@@ -1776,7 +1776,9 @@ __device__ __forceinline__ bf16x8 q8_codes_to_bf16_perm(uint2 raw) {
 // 32 positions each, four per SIMD with half the registers) measures the same and is not instantiated.
 // PLANES: 2 for f32 positions split into hi and lo bf16 planes; 1 when the positions are bf16 already
 // (x_hi is then x itself, its rows plane_stride apart and only n of them: rows past n repeat the last).
-template <int WAVES, int PLANES = 2> __device__ __forceinline__ void q8_tiled_body(const lng_k_q8 &a) {
+// ADD: with a bias or a residual after the product, in kernels of their own: in the plain one the longer end costs 2-5 %
+// (the 2,880 rows of 512 columns at 2,048 positions 28.8 -> 30.1 us) through the registers that the loop gets.
+template <int WAVES, int PLANES = 2, bool ADD = false> __device__ __forceinline__ void q8_tiled_body(const lng_k_q8 &a) {
     constexpr int MT = WAVES == 8 ? 4 : 2;       // groups of 16 positions per wavefront
     constexpr int XQ = 16 * PLANES / WAVES;      // x loads per wavefront and stage (PLANES x 16 groups of 8 positions in all)
     constexpr int WQ = 16 / WAVES;               // code loads (16 in all: groups of 16 rows)
@@ -1966,57 +1968,53 @@ template <int WAVES, int PLANES = 2> __device__ __forceinline__ void q8_tiled_bo
         __syncthreads();
     }
     if (!rows_here) return;
-    // All of the residual's rows are asked for before the first is added to: read and written one after another they cost
-    // 164 us of 8,192 positions x 2,880 rows.
-    const bool whole = r0 + rw + 64u <= a.rows && p0 + pw + 16u * MT <= a.n; // uniform: every output exists
-    float held[4][MT][4] = {};
-    if (a.residual && whole) {
+    auto each = [&](auto f) {
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
-            const float *from = a.residual + (uint64_t)(p0 + pw + 4u * kg) * a.rows + r0 + rw + 16u * nt + j;
+            const uint32_t r = r0 + rw + 16u * nt + j;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) held[nt][mt][i] = from[(uint64_t)(16u * mt + i) * a.rows];
+                for (int i = 0; i < 4; ++i) f(nt, mt, i, p0 + pw + 16u * mt + 4u * kg + i, r);
             }
+        }
+    };
+    if constexpr (ADD) {
+        if (a.bias) {
+            float bias[4];
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) bias[nt] = r0 + rw + 16u * nt + j < a.rows ? a.bias[r0 + rw + 16u * nt + j] : 0.0f;
+            each([&](int nt, int mt, int i, uint32_t, uint32_t) { y[nt][mt][i] = y[nt][mt][i] + bias[nt]; });
+        }
+        // All of the residual's rows are asked for before the first is added to: read and written one after another they cost
+        // 164 us of 8,192 positions x 2,880 rows. (With the rows that exist told apart once and not at every store: 510 -> 487
+        // us there with 4,096 columns, 334 -> 320 from bf16.)
+        if (a.residual && r0 + rw + 64u <= a.rows && p0 + pw + 16u * MT <= a.n) { // uniform: every output exists
+            float held[4][MT][4];
+            each([&](int nt, int mt, int i, uint32_t p, uint32_t r) { held[nt][mt][i] = a.residual[(uint64_t)p * a.rows + r]; });
+            each([&](int nt, int mt, int i, uint32_t p, uint32_t r) {
+                a.y[(uint64_t)p * a.y_stride + r] = y[nt][mt][i];
+                a.residual[(uint64_t)p * a.rows + r] = held[nt][mt][i] + y[nt][mt][i];
+            });
+            return;
         }
     }
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        const uint32_t r = r0 + rw + 16u * nt + j;
-        if (a.bias && r < a.rows) {
-            const float bias = a.bias[r];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) y[nt][mt][i] = y[nt][mt][i] + bias;
+    each([&](int nt, int mt, int i, uint32_t p, uint32_t r) {
+        if (p < a.n && r < a.rows) {
+            a.y[(uint64_t)p * a.y_stride + r] = y[nt][mt][i];
+            if constexpr (ADD) {
+                if (a.residual) a.residual[(uint64_t)p * a.rows + r] += y[nt][mt][i];
             }
         }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t p = p0 + pw + 16u * mt + 4u * kg + i;
-                if (whole || (p < a.n && r < a.rows)) {
-                    a.y[(uint64_t)p * a.y_stride + r] = y[nt][mt][i];
-                    if (a.residual) {
-                        float *to = a.residual + (uint64_t)p * a.rows + r;
-                        *to = (whole ? held[nt][mt][i] : *to) + y[nt][mt][i];
-                    }
-                }
-            }
-        }
-    }
+    });
 }
 
-extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled(lng_k_q8 a) {
-    q8_tiled_body<8>(a);
-}
+extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled(lng_k_q8 a) { q8_tiled_body<8>(a); }
+extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_add(lng_k_q8 a) { q8_tiled_body<8, 2, true>(a); }
 
-// positions already in bf16: one plane, half the matrix instructions, no split kernel before it
-extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16(lng_k_q8 a) {
-    q8_tiled_body<8, 1>(a);
-}
+// positions already in bf16: one plane, half the matrix instructions
+extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16(lng_k_q8 a) { q8_tiled_body<8, 1>(a); }
+extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16_add(lng_k_q8 a) { q8_tiled_body<8, 1, true>(a); }
 
 #include "lng_q8_mid.h"
 #include "lng_q8_few.h"
