@@ -73,8 +73,8 @@ template <int NW, bool HEADS = false> struct Q8Few {
     const uint16_t *sc_rows;   // the tile's first row of scales
     uint32_t *s_sc;
     uint32_t blocks, pairs, from, to, lane, wave, j, kg, rows_here, words;
-    bool staged;
-    uint32_t sc_now[16 / NW];
+    bool staged, words_aligned;
+    uint32_t sc_now[16 / NW], sc_then[16 / NW];
     uint4 w[U];
 
     __device__ __forceinline__ Q8Few(const lng_k_q8 &a, uint32_t tile, uint32_t *lds) : s_sc(lds) {
@@ -92,13 +92,27 @@ template <int NW, bool HEADS = false> struct Q8Few {
         w_src = a.codes + (uint64_t)(r0 + row) * a.cols + 16u * kg;
         sc_rows = a.scales + (uint64_t)r0 * blocks;
         staged = blocks <= Q8F_SC_BLOCKS;
+        words_aligned = ((blocks & 1u) | ((uintptr_t)sc_rows & 3u)) == 0;
         words = q8_few_sc_words(blocks);
     }
-    __device__ __forceinline__ uint32_t load_sc(uint32_t row, uint32_t word) const { // scales 2 word and 2 word + 1 of a row
+    // Scales 2 word and 2 word + 1 of a row: one load, or (off a 4-byte boundary) two, which are put together where they are
+    // used: nothing waits here for what it asks for.
+    __device__ __forceinline__ void ask_sc(uint32_t row, uint32_t word, uint32_t &first, uint32_t &second) const {
         const uint16_t *src = sc_rows + row * blocks + 2u * word;
-        if (((blocks & 1u) | ((uintptr_t)sc_rows & 3u)) == 0) return *(const uint32_t *)src; // uniform
-        const uint32_t lo = src[0], hi = 2u * word + 1u < blocks ? src[1] : 0u;
-        return lo | (hi << 16);
+        if (words_aligned) { // uniform
+            first = *(const uint32_t *)src;
+        } else {
+            first = src[0];
+            if (2u * word + 1u < blocks) second = src[1];
+        }
+    }
+    __device__ __forceinline__ uint32_t both_sc(uint32_t word, uint32_t first, uint32_t second) const { // zero past the last block
+        return words_aligned || 2u * word + 1u >= blocks ? first : first | (second << 16);
+    }
+    __device__ __forceinline__ uint32_t load_sc(uint32_t row, uint32_t word) const {
+        uint32_t first, second;
+        ask_sc(row, word, first, second);
+        return both_sc(word, first, second);
     }
     __device__ __forceinline__ uint32_t sc_row(int i) const {
         const uint32_t row = wave * (16 / NW) + i;
@@ -107,23 +121,26 @@ template <int NW, bool HEADS = false> struct Q8Few {
     __device__ __forceinline__ void ask_scales() { // the first 64 words of the wavefront's rows, into registers
         if (!staged) return;
 #pragma unroll
-        for (int i = 0; i < 16 / NW; ++i) sc_now[i] = lane < pairs ? load_sc(sc_row(i), lane) : 0u;
+        for (int i = 0; i < 16 / NW; ++i) {
+            if (lane < pairs) ask_sc(sc_row(i), lane, sc_now[i], sc_then[i]);
+        }
     }
     __device__ __forceinline__ void stage_scales() { // and all of them to LDS
         if (!staged) return;
 #pragma unroll
         for (int i = 0; i < 16 / NW; ++i) {
             uint32_t *to_row = s_sc + (wave * (16 / NW) + i) * words;
-            if (lane < pairs) to_row[lane] = sc_now[i];
+            if (lane < pairs) to_row[lane] = both_sc(lane, sc_now[i], sc_then[i]);
             for (uint32_t at = lane + 64u; at < pairs; at += 64u) to_row[at] = load_sc(sc_row(i), at);
         }
     }
+    // (Nothing is put in place of what is not loaded - the products skip it too - and the first load is asked for in any case:
+    // a value merged with another after a branch is copied, and the copy waits for the load.)
     __device__ __forceinline__ void ask_codes(uint32_t base) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint32_t pair = base + u;
-            w[u] = make_uint4(0, 0, 0, 0);
-            if (pair < to) { // uniform; a last pair of one block: its upper lanes load the block again
+            const uint32_t pair = u || base < to ? base + u : pairs - 1u;
+            if (u == 0 || pair < to) { // uniform; a last pair of one block: its upper lanes load the block again
                 const int64_t col = (int64_t)(64ull * pair) - (2u * pair + 1u == blocks && kg >= 2u ? 32 : 0);
                 w[u] = *(const uint4 *)(w_src + col);
             }
@@ -185,6 +202,8 @@ struct Q8Prepared {
 // wavefront asked for half of its blocks at a time and split x for each), 2 to 16: 12 us with the planes' dispatch (20-27
 // when each workgroup normalised and split all positions itself), 31: 14 us (38); 2,880 x 4,096 with bias and residual from
 // bf16 1, 16, 31 positions: 6.9, 8.2, 11 us (9.1, 13, 23), from f32 7.2, 11, 17 (11, 19, 35).
+// One position with every load of a turn really on its way before the first is waited for: 16,384 x 2,880 14.9 -> 11.7 us
+// (bf16 14.3 -> 11.3), 2,048 rows 6.0 -> 5.1 (5.8 -> 4.7).
 // Eight wavefronts to 16 rows: two workgroups fit a compute unit, so up to 512 tiles are all in flight at once.
 
 // 2 to 16 positions (more: 16 per blockIdx.y). Every load of a turn is asked for before its first product, the matrix's
@@ -193,7 +212,7 @@ struct Q8Prepared {
 // wavefront uses (lng_q8_mid).
 template <int PLANES, int NW, bool PREPARE = false>
 __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
-    constexpr int U = Q8Few<NW>::U, D = PLANES == 2 ? 3 : U; // pairs of x in flight
+    constexpr int U = Q8Few<NW>::U, D = PLANES == 2 ? 3 : 6; // pairs of x in flight (what the registers hold)
     constexpr uint32_t STRIDE = 80;
     __shared__ float s_red[NW][4][64];
     Q8Few<NW, PREPARE> m(a, tile, (uint32_t *)(s_mem + (PLANES == 1 ? NW * 2u * 16u * STRIDE : 0u)));
