@@ -136,7 +136,8 @@ struct lng_gpu {
                   q8_tiled_bf16 = nullptr, q8_frag_x = nullptr;
     hipFunction_t q8_tiled_add = nullptr, q8_tiled_bf16_add = nullptr;
     hipFunction_t q8_norm_frag = nullptr, q8_few[2] = {}, q8_one[2] = {}; // [bf16 positions]
-    hipFunction_t q8_few_prepare = nullptr, q8_one_prepare = nullptr;
+    hipFunction_t q8_few_f32 = nullptr;
+    hipFunction_t q8_few_prepare = nullptr, q8_few_f32_prepare = nullptr, q8_one_prepare = nullptr;
     hipFunction_t q8_mid[2][4] = {}; // [bf16 positions][tile, see q8_mid_tile]
     std::string name;
     unsigned cus = 256;
@@ -1051,6 +1052,7 @@ bool fuse_split(const lng_gpu *g, Cmd &c, const Cmd &after) {
 bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
     if (after.fn != g->add_rows) return false;
     bool product = c.fn == g->q8_tiled || c.fn == g->q8_tiled_bf16 || c.fn == g->q8_tiled_add || c.fn == g->q8_tiled_bf16_add;
+    product = product || c.fn == g->q8_few_f32;
     for (int i = 0; i < 2; ++i) {
         product = product || c.fn == g->q8_few[i] || c.fn == g->q8_one[i];
         for (hipFunction_t fn : g->q8_mid[i]) product = product || (fn && c.fn == fn);
@@ -1080,7 +1082,7 @@ bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
 // `c` (the q, k and v projections of up to 16 positions) with the preparation of attention `after` it.
 // (A token through 24 blocks: f32 1,082 -> 1,023 us, bf16 1,027 -> 977, 16 sequences 1,615 -> 1,536.)
 bool fuse_prepare(const lng_gpu *g, Cmd &c, const Cmd &after) {
-    if ((after.fn != g->prepare_v4 && after.fn != g->prepare_v1) || (c.fn != g->q8_few[0] && c.fn != g->q8_one[0])) return false;
+    if ((after.fn != g->prepare_v4 && after.fn != g->prepare_v1) || (c.fn != g->q8_few[0] && c.fn != g->q8_few_f32 && c.fn != g->q8_one[0])) return false;
     lng_k_q8_prepare both{};
     both.q8 = args_of<lng_k_q8>(c);
     both.prepare = args_of<lng_k_prepare>(after);
@@ -1110,8 +1112,9 @@ bool fuse_prepare(const lng_gpu *g, Cmd &c, const Cmd &after) {
     for (const auto &out : made.outs) {
         if (!apart(out.at, out.len, a.x, ((uint64_t)(a.n - 1) * a.x_stride + a.cols) * 4) || (a.norm_w && !apart(out.at, out.len, a.norm_w, (uint64_t)a.cols * 4))) return false;
     }
-    c.name = c.fn == g->q8_one[0] ? "lng_q8_one_prepare" : "lng_q8_few_prepare";
-    c.fn = c.fn == g->q8_one[0] ? g->q8_one_prepare : g->q8_few_prepare;
+    const bool one = c.fn == g->q8_one[0], direct = c.fn == g->q8_few_f32;
+    c.name = one ? "lng_q8_one_prepare" : direct ? "lng_q8_few_f32_prepare" : "lng_q8_few_prepare";
+    c.fn = one ? g->q8_one_prepare : direct ? g->q8_few_f32_prepare : g->q8_few_prepare;
     set_args(c, both);
     return true;
 }
@@ -1210,8 +1213,10 @@ extern "C" int lng_hip_open(int device, lng_gpu **out) {
         {"lng_q8_norm_frag", &g->q8_norm_frag, true},
         {"lng_q8_few", &g->q8_few[0], true},
         {"lng_q8_few_bf16", &g->q8_few[1], true},
+        {"lng_q8_few_f32", &g->q8_few_f32, true},
         {"lng_q8_one", &g->q8_one[0], true},
         {"lng_q8_few_prepare", &g->q8_few_prepare, true},
+        {"lng_q8_few_f32_prepare", &g->q8_few_f32_prepare, true},
         {"lng_q8_one_prepare", &g->q8_one_prepare, true},
         {"lng_q8_one_bf16", &g->q8_one[1], true},
         {"lng_q8_mid_r32p32", &g->q8_mid[0][1], true},
@@ -2147,8 +2152,9 @@ double q8_mid_us(uint64_t n, uint64_t rows, uint64_t cols, bool x_bf16, int tile
     return n * cols > 8u << 20 ? 1.2 * us : us;
 }
 
-// The tile of lng_q8_mid* a product takes; -1: lng_q8_few (fewer than 32 positions) or lng_q8_tiled. From 32 positions on it
-// depends on nothing that differs between a product alone and among several matrices, so that its sums keep their order.
+// The tile of lng_q8_mid* a product takes; -1: lng_q8_few (fewer than 32 positions) or lng_q8_tiled. `rows`: of the matrix, or
+// (fewer than 32 positions) of all matrices of the dispatch. From 32 positions on it depends on nothing that differs between
+// a product alone and among several matrices, so that its sums keep their order.
 // Measured (2,880 x 4,096 bf16 / the 5,120 x 2,880 of q, k and v), us: tiles 16 x 32, 32 x 32, 32 x 64, 64 x 64 at 32
 // positions 8.7, 11, 15, 22 / 14, 12, 16, 22; at 77 20, 19, 16, 24 / 24, 19, 26, 25; at 192 33, 28, 27, 25 / 44, 33, 29, 28.
 // Against lng_q8_tiled: 1,280 positions 82 / 135 against 91 / 297, 1,536 99 / 169 against 92 / 305 (one matrix of 4,096
@@ -2156,8 +2162,12 @@ double q8_mid_us(uint64_t n, uint64_t rows, uint64_t cols, bool x_bf16, int tile
 // with lng_q8_tiled's own tiles, which read every operand less often (65,536 x 2,880 at 128 positions 112 us against 196,
 // bf16 78 against 138; 16,384 x 2,880 at 512 114 against 139, 76 against 107): where the estimates are close, lng_q8_tiled.
 int q8_mid_tile(const lng_gpu *g, uint64_t n, uint64_t rows, uint64_t cols, bool x_bf16) {
-    if (n <= 16) return -1; // q8_record_few (17 to 31 as two groups of 16 would read the codes twice)
+    if (n <= 16) return -1; // q8_record_few
     if (cols > 32 * 512) return -1; // a tile's scales are held in LDS: at most 64 KB of them
+    // 17 to 31 positions as two groups of 16 read the codes twice, but with so few rows a tile of 16 has a unit to itself in either
+    // form: 2,880 columns, 1,280 rows 9.3 us against 12.8 (bf16 5.9 against 7.3), 2,880 rows 12.2 against 12.9 (8.7, 7.5),
+    // 4,096 rows 15.9 against 13.1. Both forms add up in the same order.
+    if (n < 32 && (rows + 15) / 16 * 2 <= (x_bf16 ? g->cus : g->cus * 3 / 2)) return -1;
     const int tile = x_bf16 ? (n <= 48 ? 0 : n <= 128 ? 2 : 3) : n <= 128 ? 1 : 3;
     if (n < 32 || g->knobs.q8_mid == 1) return tile;
     if (g->knobs.q8_mid == 0 || n > 1280) return -1;
@@ -2215,23 +2225,39 @@ int q8_record_mid(lng_batch *b, lng_k_q8 a, bool x_bf16, int tile) {
     return LNG_OK;
 }
 
+// Whether 2 to 31 f32 positions are split (and normalised) by every workgroup of the product, or once, by a dispatch before
+// it. That dispatch and its gap cost 2 us; splitting in the product costs by the columns, the positions (of a group of 16) and
+// the rounds of workgroups. us, in the product / before it: 512 columns, up to 4,096 rows, 2 and 16 positions 3.9 and 4.6 /
+// 5.7 and 5.8, 16,384 rows 7.9 and 10 / 9.7 and 9.8; 2,880 columns, 2,880 rows 2, 8, 16 positions 8.3, 9.3, 11 / 9.2, 9.3, 9.5,
+// 5,120 rows 2, 4 positions 11.6, 12.6 / 11.6, 11.7. With the norm 512 columns 4.6 and 5.4 / 6.1 and 6.3, 1,024 columns 2, 8,
+// 16 positions 5.8, 6.6, 7.3 / 6.8, 6.9, 7.0, 2,880 columns 2 positions 10 / 9.4.
+bool q8_few_direct(const lng_gpu *g, const lng_k_q8 &a, uint64_t wgs) {
+    const uint64_t n = std::min<uint64_t>(a.n, 16), cols = a.cols, rounds = (wgs + g->cus - 1) / g->cus;
+    if (a.norm_w) return cols * rounds <= 2048 && n * cols * rounds <= 8192;
+    return n * cols * rounds <= 18432;
+}
+
 // Fewer than 32 positions: bound by reading the matrix, in tiles of 16 rows. One position splits (and normalises) x in
-// the kernel, whose LDS holds up to 48 KB of it; more go through the planes of q8_record_frag.
+// the kernel, whose LDS holds up to 48 KB of it; more go through the planes of q8_record_frag or are split by every workgroup.
 // `a` may name further matrices of the same dispatch (first_tile in tiles of 16 rows).
 int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
     const uint64_t blocks = a.cols / 32, groups = (a.n + 15) / 16;
     const bool one = a.n == 1 && a.cols <= (x_bf16 ? 24576u : 12288u);
-    if (!one && !x_bf16) {
-        if (int rc = q8_record_frag(b, &a, groups * 16)) return rc;
+    bool direct = !one && !x_bf16 && q8_few_direct(b->gpu, a, row_tiles * groups);
+    if (!one && !x_bf16 && !direct) {
+        const int rc = q8_record_frag(b, &a, groups * 16);
+        if (rc == LNG_ERR_ALLOC) direct = true; // no memory for the planes
+        else if (rc) return rc;
     }
     Cmd c;
-    c.fn = one ? b->gpu->q8_one[x_bf16] : b->gpu->q8_few[x_bf16];
-    c.name = one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
+    c.fn = one ? b->gpu->q8_one[x_bf16] : direct ? b->gpu->q8_few_f32 : b->gpu->q8_few[x_bf16];
+    c.name = one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : direct ? "lng_q8_few_f32" : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
     c.grid[0] = (unsigned)row_tiles;
     c.grid[1] = (unsigned)groups;
     c.block = 512;
     const uint64_t scales = blocks <= 512 ? 16 * (((blocks + 1) / 2) | 1) * 4 : 0; // both of a pair of blocks in a word
-    c.lds = (unsigned)(scales + (one ? a.cols * (x_bf16 ? 2u : 4u) : x_bf16 ? 8 * 2 * 16 * 80 : 0)); // x's planes, or the turning buffers
+    // x's planes, the weights of its norm, or the turning buffers
+    c.lds = (unsigned)(scales + (one ? a.cols * (x_bf16 ? 2u : 4u) : direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
     set_args(c, a);
     b->cmds.push_back(std::move(c));
     return LNG_OK;
@@ -2294,9 +2320,16 @@ int q8_record_tiled(lng_batch *b, lng_k_q8 a, bool x_bf16, const uint16_t *plane
     return LNG_OK;
 }
 
+// q8_mid_tile, but lng_q8_few*, which can do without them, for 17 to 31 f32 positions that there is no memory for the planes of.
+int q8_tile(lng_batch *b, uint64_t n, uint64_t rows, uint64_t cols, bool x_bf16) {
+    const int tile = q8_mid_tile(b->gpu, n, rows, cols, x_bf16);
+    char *planes = nullptr;
+    return tile >= 0 && n < 32 && !x_bf16 && reserve_x(b->gpu, 2 * 32 * cols * 2, &planes) ? -1 : tile;
+}
+
 // A product of one matrix.
 int q8_record(lng_batch *b, lng_k_q8 a, bool x_bf16) {
-    const int tile = q8_mid_tile(b->gpu, a.n, a.rows, a.cols, x_bf16);
+    const int tile = q8_tile(b, a.n, a.rows, a.cols, x_bf16);
     if (tile < 0 && a.n >= 32) return q8_record_tiled(b, a, x_bf16);
     const uint64_t tile_rows = tile < 0 ? 16 : q8_mid_tiles[tile].rows;
     a.tiles = (uint32_t)((a.rows + tile_rows - 1) / tile_rows);
@@ -2413,14 +2446,18 @@ int q8_many(lng_batch *b, const lng_q8_matrix *matrices, size_t n_matrices, lng_
         return rc;
     };
     bool alone[1 + LNG_Q8_MORE] = {};
+    uint64_t all_rows = 0;
+    for (size_t i = 0; i < n_matrices; ++i) all_rows += q[i].a.rows;
     lng_k_q8 a{};
     uint64_t tiles = 0, together = 0;
-    int tile = -1; // (of all that share the dispatch: the positions and columns decide it)
+    int tile = n < 32 ? q8_tile(b, n, all_rows, cols, false) : -1; // of all that share the dispatch (from 32 positions on they and the columns decide it)
     for (size_t i = 0; i < n_matrices; ++i) {
-        const int own = q8_mid_tile(b->gpu, n, q[i].a.rows, cols, false);
-        alone[i] = n >= 32 && own < 0;
-        if (alone[i]) continue;
-        tile = own;
+        if (n >= 32) {
+            const int own = q8_tile(b, n, q[i].a.rows, cols, false);
+            alone[i] = own < 0;
+            if (alone[i]) continue;
+            tile = own;
+        }
         const uint64_t tile_rows = tile < 0 ? 16 : q8_mid_tiles[tile].rows;
         if (together++ == 0) {
             a = q[i].a;

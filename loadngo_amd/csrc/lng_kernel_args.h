@@ -177,7 +177,7 @@ typedef struct lng_k_q8_split {
 typedef struct lng_k_q8 {
     const int8_t *codes;     /* [rows][cols] */
     const uint16_t *scales;  /* [rows][cols/32] binary16 */
-    const float *x;          /* [n][x_stride] (one position: split by the kernel) */
+    const float *x;          /* [n][x_stride] (lng_q8_one, lng_q8_few_f32*: split by the kernel) */
     const uint16_t *x_hi;    /* [n_pad][cols] bf16 (the planes lng_q8_split_x, lng_q8_frag_x or lng_q8_norm_frag wrote) */
     const uint16_t *x_lo;
     float *y;                /* [n][y_stride] */
@@ -192,7 +192,7 @@ typedef struct lng_k_q8 {
      * Workgroups from `first_tile` (in units of 16 rows) on belong to matrix more[i]; first_tile ascends. */
     uint32_t n_more;         /* 0..LNG_Q8_MORE */
     float eps;               /* of the RMS norm, when norm_w is set */
-    /* Few positions only. norm_w (one position): x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
+    /* Few positions only. norm_w (lng_q8_one*, lng_q8_few_f32*): x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
      * (cols <= 12288). bias: y gets bias[row] added. accumulate: the result is added to what y holds. (These two and
      * residual: all kernels of one matrix.) */
     const float *norm_w;

@@ -1,5 +1,5 @@
-// Q8_0 products of fewer than 32 positions (17 to 31 share lng_q8_mid's tiles): lng_q8_norm_frag, lng_q8_few*,
-// lng_q8_one*. (Included by lng_kernels.hip after lng_q8_mid.h; see there for how a product goes through the matrix unit.)
+// Q8_0 products of fewer than 32 positions (17 to 31 of matrices of many rows share lng_q8_mid's tiles): lng_q8_norm_frag,
+// lng_q8_few*, lng_q8_one*. (Included by lng_kernels.hip after lng_q8_mid.h; see there for how a product goes through the matrix unit.)
 
 // x[n][x_stride] f32 as the A operands of lng_q8_few and lng_q8_mid, RMS-normalised on the way if norm_w is set
 // (x / sqrt(mean(x^2) + eps) * w): one workgroup per position, lng_q8_frag_x's layout. Rows that pad n to whole groups
@@ -208,13 +208,16 @@ struct Q8Prepared {
 
 // 2 to 16 positions (more: 16 per blockIdx.y). Every load of a turn is asked for before its first product, the matrix's
 // first: a product is one round trip to memory, not one per block.
-// PLANES 2: x as lng_q8_norm_frag left it; 1: bf16 positions, turned into operand order through LDS that only this
-// wavefront uses (lng_q8_mid).
-template <int PLANES, int NW, bool PREPARE = false>
+#define Q8F_PLANES 0 // x as lng_q8_norm_frag left it
+#define Q8F_BF16 1   // bf16 positions, turned into operand order through LDS that only this wavefront uses (lng_q8_mid)
+#define Q8F_F32 2    // f32 positions, split (and normalised, if a.norm_w is set) by every workgroup for itself: see q8_few_direct
+template <int X, int NW, bool PREPARE = false>
 __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
-    constexpr int U = Q8Few<NW>::U, D = PLANES == 2 ? 3 : 6; // pairs of x in flight (what the registers hold)
+    constexpr int PLANES = X == Q8F_BF16 ? 1 : 2;
+    constexpr int U = Q8Few<NW>::U, D = PLANES == 2 ? (X == Q8F_F32 && PREPARE ? 2 : 3) : 6; // pairs of x in flight (what the registers hold)
     constexpr uint32_t STRIDE = 80;
     __shared__ float s_red[NW][4][64];
+    __shared__ float s_norm[X == Q8F_F32 ? 16 : 1];
     Q8Few<NW, PREPARE> m(a, tile, (uint32_t *)(s_mem + (PLANES == 1 ? NW * 2u * 16u * STRIDE : 0u)));
     const uint32_t lane = m.lane, j = m.j, kg = m.kg, p0 = blockIdx.y * 16u, r0 = q8_tile_row<PREPARE>(tile);
     char *s_x = s_mem + m.wave * 2u * 16u * STRIDE;
@@ -222,13 +225,17 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
     const uint4 *x_frag = (const uint4 *)a.x_hi + (uint64_t)blockIdx.y * m.blocks * 128u + lane;
     const uint32_t at_p = p0 + (lane >> 2) < a.n ? p0 + (lane >> 2) : a.n - 1u;
     const uint16_t *x_row = a.x_hi + (uint64_t)at_p * a.plane_stride + 8u * (lane & 3u);
-    uint4 x[D][2][PLANES];
+    const float *x_f32 = a.x + (uint64_t)(p0 + j < a.n ? p0 + j : a.n - 1u) * a.x_stride + 8u * q8_mid_chunk(kg);
+    uint4 x[D][2][PLANES]; // (Q8F_F32: eight floats until they are split)
     auto ask_x = [&](uint32_t pair, uint4 (&to)[2][PLANES]) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const uint32_t b = 2u * pair + h < m.blocks ? 2u * pair + h : 2u * pair;
-            if constexpr (PLANES == 1) {
+            if constexpr (X == Q8F_BF16) {
                 to[h][0] = *(const uint4 *)(x_row + 32u * b);
+            } else if constexpr (X == Q8F_F32) {
+                to[h][0] = *(const uint4 *)(x_f32 + 32ull * b);
+                to[h][1] = *(const uint4 *)(x_f32 + 32ull * b + 4u);
             } else {
                 to[h][0] = x_frag[(uint64_t)b * 128u];
                 to[h][1] = x_frag[(uint64_t)b * 128u + 64u];
@@ -263,7 +270,37 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
     ask(m.from);
     __builtin_amdgcn_sched_barrier(0);
     m.stage_scales();
+    float *s_nw = (float *)(s_mem + (m.staged ? 64u * m.words : 0u));
+    const bool normed = X == Q8F_F32 && a.norm_w != nullptr; // uniform
+    if constexpr (X == Q8F_F32) {
+        if (normed) {
+            for (uint32_t c = 4u * threadIdx.x; c < a.cols; c += 4u * 64u * NW) *(float4 *)(s_nw + c) = *(const float4 *)(a.norm_w + c);
+            static_assert(NW == 8, "a wavefront takes positions w and w + 8 of the sixteen");
+            if (p0 + m.wave < a.n) { // uniform
+                const float *x0 = a.x + (uint64_t)(p0 + m.wave) * a.x_stride;
+                const bool two = p0 + m.wave + 8u < a.n; // (else the first position again)
+                const float *x1 = two ? x0 + 8ull * a.x_stride : x0;
+                float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll 2
+                for (uint32_t c = 4u * lane; c < a.cols; c += 256u) {
+                    const float4 v = *(const float4 *)(x0 + c), w = *(const float4 *)(x1 + c);
+                    s0 += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+                    s1 += w.x * w.x + w.y * w.y + w.z * w.z + w.w * w.w;
+                }
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) {
+                    s0 += __shfl_xor(s0, off, 64);
+                    s1 += __shfl_xor(s1, off, 64);
+                }
+                if (lane == 0) {
+                    s_norm[m.wave] = 1.0f / sqrtf(s0 / (float)a.cols + a.eps);
+                    if (two) s_norm[m.wave + 8u] = 1.0f / sqrtf(s1 / (float)a.cols + a.eps);
+                }
+            }
+        }
+    }
     __syncthreads();
+    const float scale = normed ? s_norm[p0 + j < a.n ? j : a.n - 1u - p0] : 1.0f;
     for (uint32_t base = m.from; base < m.to; base += U) {
         if (base != m.from) ask(base);
 #pragma unroll
@@ -277,6 +314,23 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
                     for (int h = 0; h < 2; ++h) *(uint4 *)(s_x + h * 16 * STRIDE + put) = x[u % D][h][0];
 #pragma unroll
                     for (int h = 0; h < 2; ++h) x[u % D][h][0] = *(const uint4 *)(s_x + h * 16 * STRIDE + get);
+                }
+                if constexpr (X == Q8F_F32) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const uint4 u0 = x[u % D][h][0], u1 = x[u % D][h][1];
+                        float v[8] = {__uint_as_float(u0.x), __uint_as_float(u0.y), __uint_as_float(u0.z), __uint_as_float(u0.w),
+                                      __uint_as_float(u1.x), __uint_as_float(u1.y), __uint_as_float(u1.z), __uint_as_float(u1.w)};
+                        if (normed) {
+                            const float *w = s_nw + 32u * (2u * (base + u) + h < m.blocks ? 2u * (base + u) + h : 2u * (base + u)) + 8u * q8_mid_chunk(kg);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) v[e] = v[e] * scale * w[e];
+                        }
+                        bf16x8 hi, lo;
+                        q8_split8(v, hi, lo);
+                        x[u % D][h][0] = __builtin_bit_cast(uint4, hi);
+                        x[u % D][h][1] = __builtin_bit_cast(uint4, lo);
+                    }
                 }
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -429,8 +483,9 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
         const uint32_t tile = q8_select_matrix(a); \
         body<what, nw>(a, tile, s_mem); \
     }
-Q8_FEW(lng_q8_few, q8_few_body, 2, 8)
-Q8_FEW(lng_q8_few_bf16, q8_few_body, 1, 8)
+Q8_FEW(lng_q8_few, q8_few_body, Q8F_PLANES, 8)
+Q8_FEW(lng_q8_few_bf16, q8_few_body, Q8F_BF16, 8)
+Q8_FEW(lng_q8_few_f32, q8_few_body, Q8F_F32, 8)
 Q8_FEW(lng_q8_one, q8_one_body, false, 8)
 Q8_FEW(lng_q8_one_bf16, q8_one_body, true, 8)
 
@@ -443,5 +498,6 @@ Q8_FEW(lng_q8_one_bf16, q8_one_body, true, 8)
         const uint32_t tile = q8_select_matrix(a); \
         body<what, nw, true>(a, tile, s_mem, &both.prepare, which); \
     }
-Q8_FEW_PREPARE(lng_q8_few_prepare, q8_few_body, 2, 8)
+Q8_FEW_PREPARE(lng_q8_few_prepare, q8_few_body, Q8F_PLANES, 8)
+Q8_FEW_PREPARE(lng_q8_few_f32_prepare, q8_few_body, Q8F_F32, 8)
 Q8_FEW_PREPARE(lng_q8_one_prepare, q8_one_body, false, 8)

@@ -131,8 +131,10 @@ __device__ __forceinline__ void q8_mid_body(const lng_k_q8 &a, uint32_t row_tile
     };
 
     uint4 w_next[NT], xa[MT][PLANES], xb[MT][PLANES];
-    const uint32_t full = blocks / 2u; // whole pairs; a block left over is a turn of its own after them
-    const uint32_t from = wave * full / NW, to = (wave + 1u) * full / NW;
+    // whole pairs; a block left over is the last wavefront's, a turn of its own after them (the runs of lng_q8_few*: the same
+    // sums in the same order)
+    const uint32_t full = blocks / 2u, pairs = (blocks + 1u) / 2u;
+    const uint32_t from = wave * pairs / NW, to = wave == NW - 1u ? full : (wave + 1u) * pairs / NW;
     if (from < to) {
         load_w(from, w_next);
         load_x(2u * from, xa);
@@ -168,7 +170,7 @@ __device__ __forceinline__ void q8_mid_body(const lng_k_q8 &a, uint32_t row_tile
         turn_x(xb);
         multiply(2u * pair + 1u, w1, xb);
     }
-    if ((blocks & 1u) && wave == 0) {
+    if ((blocks & 1u) && wave == NW - 1u) {
         load_w(full, w_next);
         load_x(2u * full, xa);
         uint2 w0[NT];

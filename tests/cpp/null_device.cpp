@@ -209,7 +209,8 @@ static std::vector<std::string> launched() { // the kernels launched since the l
     return names;
 }
 
-// Products of 32 positions or more: lng_q8_mid* where the tiles of lng_q8_tiled would leave units idle, lng_q8_tiled where
+// Which kernels Q8_0 products run as.
+// 32 positions or more: lng_q8_mid* where the tiles of lng_q8_tiled would leave units idle, lng_q8_tiled where
 // they fill the device, whichever number of positions; a matrix takes the same kernel alone and among others.
 static void products_and_their_kernels() {
     Fixture f(4, 66ull << 20);
@@ -246,6 +247,23 @@ static void products_and_their_kernels() {
     CHECK(lng_hip_batch_dispatches(f.batch) == 3);
     const std::vector<std::string> names = run();
     CHECK((names == std::vector<std::string>{"lng_q8_frag_x", "lng_q8_mid_r32p32", "lng_q8_split_x", "lng_q8_tiled"}));
+    // 2 to 31 positions: f32 ones are split by the product itself where that is less than a dispatch before it
+    typedef std::vector<std::string> Names;
+    auto few = [&](uint64_t rows, uint64_t cols, uint64_t n, bool normed) {
+        const lng_slice x{2, 0, n * cols * 4}, norm{2, x.len, cols * 4};
+        const lng_q8_matrix m{{0, 0, rows * cols}, {1, 0, rows * cols / 16}, {3, 0, n * rows * 4}, rows};
+        if (normed) CHECK(lng_hip_gemm_q8_0_many_normed(f.batch, &m, 1, x, norm, 1e-5f, cols, n, cols) == LNG_OK);
+        else CHECK(lng_hip_gemm_q8_0(f.batch, m.codes, m.scales, x, m.y, rows, cols, n, cols, rows) == LNG_OK);
+        return run();
+    };
+    for (const bool normed : {false, true}) {
+        CHECK(few(2880, 512, 2, normed) == Names{"lng_q8_few_f32"});
+        CHECK(few(4096, 512, 16, normed) == Names{"lng_q8_few_f32"});
+        CHECK((few(2880, 2880, 16, normed) == Names{"lng_q8_norm_frag", "lng_q8_few"}));
+        CHECK(few(2048, 512, 31, normed) == Names{"lng_q8_few_f32"});
+        CHECK((few(2880, 2880, 31, normed) == Names{"lng_q8_norm_frag", "lng_q8_few"}));
+        CHECK((few(4096, 2880, 31, normed) == Names{"lng_q8_norm_frag", "lng_q8_mid_r32p32"}));
+    }
     lng_null_clear();
 }
 
@@ -429,6 +447,22 @@ static void allocation_failures() {
     }
     CHECK(lng_hip_attention_grouped(batch, q, k, v, o, nullptr, &s, LNG_BF16) == LNG_OK);
     CHECK(lng_hip_batch_dispatches(batch) == 1);
+    // Q8_0 products of few positions do without the planes of their positions when there is no memory for them (17 to 31, which
+    // prefer lng_q8_mid, ask a second time, which succeeds here)
+    for (const uint64_t n : {16, 31}) {
+        for (const bool normed : {false, true}) {
+            Fixture f(4, 9 << 20);
+            const uint64_t rows = 4096, cols = 2048;
+            const lng_slice codes{0, 0, rows * cols}, scales{1, 0, rows * cols / 16}, x{2, 0, n * cols * 4}, y{3, 0, n * rows * 4}, norm{2, x.len, cols * 4};
+            const lng_q8_matrix m{codes, scales, y, rows};
+            lng_null_clear();
+            lng_null_fail_malloc_after(1);
+            CHECK((normed ? lng_hip_gemm_q8_0_many_normed(f.batch, &m, 1, x, norm, 1e-5f, cols, n, cols) : lng_hip_gemm_q8_0(f.batch, codes, scales, x, y, rows, cols, n, cols, rows)) == LNG_OK);
+            lng_null_fail_malloc_after(0);
+            CHECK(lng_hip_batch_commit(f.batch, nullptr, nullptr) == LNG_OK && lng_hip_batch_wait(f.batch, nullptr) == LNG_OK);
+            CHECK(launched() == (n == 16 ? std::vector<std::string>{"lng_q8_few_f32"} : std::vector<std::string>{"lng_q8_norm_frag", "lng_q8_few"}));
+        }
+    }
     lng_hip_batch_drop(batch);
     for (lng_buffer *b : bufs) CHECK(lng_hip_buffer_free(b) == LNG_OK);
     lng_hip_close(gpu);

@@ -500,3 +500,50 @@ def test_matrices_of_many_rows_among_others(gpu, n):
         want = x.astype(np.float64) @ elements.T
         assert np.abs(alone[offset:offset + n * rows].reshape(n, rows) - want).max() / np.abs(want).max() < 1e-5
         offset += n * rows
+
+
+def _product(gpu, codes, bits, xin, rows, cols, n, norm=None):
+    """y[n][rows] of the first `rows` rows of a matrix."""
+    bufs = [gpu.upload(codes), gpu.upload(bits), gpu.upload(xin), gpu.buffer(n * rows * 4)] + ([gpu.upload(norm)] if norm is not None else [])
+    bufs[3].fill(0xFF)
+    batch = gpu.batch(bufs)
+    m, xs, ys = (C.Slice(0, 0, rows * cols), C.Slice(1, 0, rows * cols // 16)), C.Slice(2, 0, xin.nbytes), C.Slice(3, 0, n * rows * 4)
+    if norm is not None:
+        batch.gemm_q8_0_many_normed([(m, ys, rows)], xs, (C.Slice(4, 0, cols * 4), 1e-5), cols, n, cols)
+    else:
+        (batch.gemm_q8_0_bf16 if xin.dtype == np.uint16 else batch.gemm_q8_0)(m, xs, ys, rows, cols, n, (cols, rows))
+    done = batch.run()
+    assert not isinstance(done.gpu_time, Exception), done.gpu_time
+    y = bufs[3].read(np.float32).reshape(n, rows)
+    batch.drop()
+    for b in bufs:
+        b.free()
+    return y
+
+
+@pytest.mark.parametrize("cols,n,bf16", [(32, 2, False), (96, 16, False), (224, 17, False), (512, 31, False), (1152, 16, False),
+                                         (96, 17, True), (512, 31, True)])
+def test_few_positions_give_the_same_bits_in_every_kernel(gpu, cols, n, bf16):
+    """A few rows and all rows of one matrix: split by the product itself and before it, in tiles of 16 rows and of 32 x 32
+    (16 x 32 from bf16), with whole pairs of blocks and a block left over; within the reference's bound (glue.rs:171) of float64."""
+    from tests.helpers import from_bf16_bits, to_bf16_bits
+    rows, few = 9000, 40
+    codes, bits, elements = q8_test_matrix(rows, cols, 30 + cols)
+    x = xorshift_values(43, n * cols).reshape(n, cols)
+    xin = to_bf16_bits(x) if bf16 else x
+    want = (from_bf16_bits(xin) if bf16 else x).astype(np.float64) @ elements.T
+    whole, part = _product(gpu, codes, bits, xin, rows, cols, n), _product(gpu, codes, bits, xin, few, cols, n)
+    assert np.array_equal(whole[:, :few], part)
+    assert np.abs(whole - want).max() / np.abs(want).max() < 1e-5
+
+
+@pytest.mark.parametrize("rows,cols,n", [(40, 32, 2), (100, 512, 8), (37, 512, 9), (16, 512, 16), (2100, 96, 17), (300, 256, 31), (33, 2048, 4), (5000, 512, 8)])
+def test_positions_normalised_by_the_product_itself(gpu, rows, cols, n):
+    """Narrow matrices of up to 31 positions: one wavefront and both take a position's sum of squares, groups of 16 positions;
+    within the reference's bound (glue.rs:171) of float64."""
+    codes, bits, elements = q8_test_matrix(rows, cols, 50 + cols)
+    x, w = 3 * xorshift_values(44, n * cols).reshape(n, cols), 1 + 0.2 * xorshift_values(45, cols)
+    xd = x.astype(np.float64)
+    want = (xd / np.sqrt((xd * xd).mean(axis=1, keepdims=True) + 1e-5) * w) @ elements.T
+    got = _product(gpu, codes, bits, x, rows, cols, n, w)
+    assert np.abs(got - want).max() / np.abs(want).max() < 1e-5
