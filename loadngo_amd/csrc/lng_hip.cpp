@@ -8,6 +8,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <cmath>
 #include <atomic>
 #include <condition_variable>
 #include <cstdarg>
@@ -849,17 +850,32 @@ int attention(lng_batch *b, lng_slice q, lng_slice k, lng_slice v, lng_slice out
             // (under a dozen key tiles the partial rows and the merge cost what two splits save: the first 512 rows of a
             // prompt 24.5 us unsplit, 30.8 us in two)
             if (key_tiles < 12) want = 1;
-            // f32: a tile of 64 keys is 8.3 us of matrix work, so a few tiles are worth splitting, down to one each, and
-            // where half of the units would have a workgroup more splits than units even out the unequal runs of a causal
-            // pass. Splits cost 4 us and 7 ns per row and split (64 heads). Whole calls, unsplit / split: 512 rows 75 / 52 us,
-            // 512 after 4,096 341 / 314, 256 rows 42 / 31, 128 25 / 22; through a 128-position window 48 rows 30 / 21, 128
-            // 35 / 25, 256 35 / 31; 512 there stay whole (31 against 39).
+            // f32: a tile of 64 keys is 8 us of matrix work (4.3 for up to four heads a kv head, where a SIMD has one wavefront), so
+            // a few tiles are worth splitting, down to one each, and twice as many workgroups as units even out the unequal
+            // runs of a causal pass. The candidates are compared by their time: the longest share and 9 us around it, more
+            // with every further round of workgroups (the more, the more alike the runs are: late in a context), 3 us for the
+            // merge (4.5 through a window, whose shares seldom come out even) and 7 ns per row and split (64 heads). Fitted to 540 calls of 33-1,000 rows (64/8, 32/8, 16/8, 8/8, 8/1,
+            // 64/64 heads, after 0-4,096 positions, with windows of 128 and 1,024): 1 % from the best candidate, none more than 6 %
+            // slower than the splits for one round. Whole calls, us, whole / split: 512 rows 77 / 52, 512 after 4,096
+            // 357 / 318, 256 rows 42 / 30, 128 25 / 22; through a 128-position window 48 rows 30 / 21, 128 35 / 25, 256 35 / 31;
+            // more rows there stay whole (340: 32 against 36).
             if (f32) {
                 const bool windowed = p.window != LNG_WINDOW_FULL && p.window < end;
-                want = (plain_wgs * 4 > g->cus && !windowed ? 2 : 1) * g->cus / plain_wgs;
-                want = std::min<uint64_t>(std::min<uint64_t>(want, key_tiles + windowed), 64); // (a window's run starts within a tile)
-                const double tiles = windowed ? (double)visible / 64.0 : (double)key_tiles;
-                if (tiles * 8.3 * (1.0 - 1.0 / (double)want) < 4.0 + 0.007 / 64.0 * (double)(s.t * s.heads * want)) want = 1;
+                const bool halves = s.heads / s.kv_heads > 4; // two wavefronts on every SIMD
+                const double run = (double)visible / 64.0 + (windowed ? 0.5 : 0.0); // (a window's run starts within a tile)
+                const double repeat = 0.25 + 0.6 * (double)s.start / (double)end + (halves ? 0.0 : 0.2);
+                auto us = [&](uint64_t n) {
+                    const double share = n == 1 ? std::max(run, 1.0) : std::ceil(run / (double)n);
+                    const double rounds = std::max((double)(plain_wgs * n) / (double)g->cus, 1.0);
+                    return ((halves ? 8.0 : 4.3) * share + 9.0) * (1.0 + repeat * (rounds - 1.0)) +
+                           (n > 1 ? (windowed ? 4.5 : 3.0) + 0.007 / 64.0 * (double)(s.t * s.heads * n) : 0.0);
+                };
+                const uint64_t one_round = want, most = std::min<uint64_t>(key_tiles + windowed, 64);
+                want = 1;
+                for (const uint64_t n : {one_round, std::min<uint64_t>(g->cus / plain_wgs, most),
+                                         plain_wgs * 4 > g->cus && !windowed ? std::min<uint64_t>(2 * g->cus / plain_wgs, most) : 1}) {
+                    if (n > 1 && us(n) < us(want)) want = n;
+                }
             }
             if (g->knobs.prefill_splits > 0) want = std::min<uint64_t>(g->knobs.prefill_splits, 64);
             if (want > 1) p.splits = (uint32_t)want;
@@ -867,7 +883,10 @@ int attention(lng_batch *b, lng_slice q, lng_slice k, lng_slice v, lng_slice out
         if (p.splits > 1) {
             const size_t slots = (size_t)s.t * s.heads * p.splits;
             Scratch sc;
-            if (int rc = reserve_scratch(g, slots * 64, slots * 2, 0, &sc)) return rc;
+            if (int rc = reserve_scratch(g, slots * 64, slots * 2, 0, &sc)) {
+                if (!f32 || rc != LNG_ERR_ALLOC) return rc;
+                p.splits = 1; // no memory for partial rows: whole
+            }
             p.partial_o = sc.o;
             p.partial_ml = sc.ml;
         }

@@ -335,6 +335,37 @@ static void switches_and_checksum() {
         CHECK(lng_hip_debug_set(big.gpu, "LNG_PREFILL_PAIR", nullptr) == LNG_OK);
         lng_null_clear();
     }
+    // f32 passes: the keys are split where the time of the longest share and of every further round of workgroups is less
+    {
+        Fixture big(4, 24 * MB);
+        auto splits = [&](uint64_t t, uint64_t start, uint64_t heads, uint64_t window, bool fails = false) {
+            const uint64_t rows = (t + 31) / 32 * 32, kv = (start + t + 31) / 32 * 32;
+            const lng_grouped_shape s = shape(t, start, heads, 8, 64, window, start + t, 0.125f);
+            const lng_slice q{0, 0, rows * heads * 256}, k{1, 0, kv * 2048}, v{2, 0, kv * 2048}, o{3, 0, rows * heads * 256};
+            lng_null_clear();
+            lng_null_fail_malloc_after(fails ? 1 : 0);
+            CHECK(lng_hip_attention_grouped_tiled(big.batch, q, k, v, o, nullptr, &s, LNG_F32) == LNG_OK);
+            lng_null_fail_malloc_after(0);
+            CHECK(lng_hip_batch_commit(big.batch, nullptr, nullptr) == LNG_OK && lng_hip_batch_wait(big.batch, nullptr) == LNG_OK);
+            const void *args = nullptr;
+            size_t args_size = 0;
+            CHECK(lng_null_launch(0, nullptr, nullptr, nullptr, &args, &args_size) == 0 && args_size == sizeof(lng_k_prefill));
+            lng_k_prefill p{};
+            memcpy(&p, args, sizeof p);
+            CHECK(lng_null_launch_count() == (p.splits > 1 ? 2 : 1));
+            if (p.splits > 1) CHECK(lng_null_bytes_from(p.partial_o) >= t * heads * p.splits * 256);
+            big.rebatch();
+            return p.splits;
+        };
+        CHECK(splits(512, 0, 64, LNG_WINDOW_FULL, true) == 1); // no memory for partial rows
+        CHECK(splits(512, 0, 64, LNG_WINDOW_FULL) == 4 && splits(256, 0, 64, LNG_WINDOW_FULL) == 4 && splits(64, 0, 64, LNG_WINDOW_FULL) == 1);
+        CHECK(splits(48, 2000, 64, 128) > 1 && splits(256, 2000, 64, 128) == 4);
+        CHECK(splits(673, 1000, 64, LNG_WINDOW_FULL) == 2 && splits(992, 4096, 64, LNG_WINDOW_FULL) == 2 && splits(1024, 0, 64, LNG_WINDOW_FULL) == 1);
+        CHECK(splits(384, 0, 64, 128) == 1 && splits(450, 1000, 64, 128) == 1 && splits(512, 4096, 32, 128) == 1); // two tiles of keys: not worth a second round
+        CHECK(splits(72, 0, 64, LNG_WINDOW_FULL) == 1 && splits(72, 0, 32, LNG_WINDOW_FULL) == 1);                 // nor the eight keys of a second
+        CHECK(splits(300, 1000, 64, LNG_WINDOW_FULL) == 3 && splits(320, 1000, 32, LNG_WINDOW_FULL) == 3);         // one round of shares of seven against two of four
+        lng_null_clear();
+    }
     CHECK(refused(lng_hip_debug_set(f.gpu, "LNG_NO_SUCH_SWITCH", "1"), "no development switch"));
     CHECK(refused(lng_hip_debug_set(f.gpu, nullptr, "1"), "no name"));
     CHECK(lng_hip_debug_set(nullptr, "LNG_PREFILL_SPLITS", "1") != LNG_OK);
