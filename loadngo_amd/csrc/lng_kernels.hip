@@ -2021,32 +2021,34 @@ extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16_add(lng_k_q8
 
 // Batch::rmsnorm_rows in words of 16 bytes, and with it what stands around it in a block (gpt-oss/src/gpu.rs:712-732): the
 // copy of the hidden rows before it (src), the split of the result for the Q8_0 products after it (hi, lo). A workgroup per
-// row of up to 4,096 floats, d % 8 == 0, every row from a 16-byte boundary; a thread holds up to two runs of eight.
-// Bound by memory: 8,192 x 2,880 with copy and planes 54 us (28 + 32 + 28 as three kernels, 45 + 28 + 28 before), 512 rows 8.6 (14.5).
+// row of up to 4,096 floats, d % 8 == 0, every row from a 16-byte boundary; a thread holds up to four words of the row.
+// Bound by memory: 8,192 x 2,880 with copy and planes 54 us (28 + 32 + 28 as three kernels, 45 + 28 + 28 before), 512 rows 8.6
+// (14.5). Neighbouring threads hold neighbouring words: with runs of eight floats a thread the norm alone was slower than
+// lng_rmsnorm_row_wg from some 500 rows on (2,048 x 2,880 8.7 us against 6.7).
 extern "C" __global__ __launch_bounds__(256) void lng_rmsnorm_row8(lng_k_rmsnorm a) {
 #pragma clang fp contract(off)
     __shared__ float s_part[4];
-    const uint32_t row = blockIdx.x, chunks = a.d / 8u;
-    float x[2][8] = {}, w[2][8] = {};
-    auto load = [&](const float *from, float (&to)[8]) {
-        const float4 u = *(const float4 *)from, v = *(const float4 *)(from + 4);
-        to[0] = u.x, to[1] = u.y, to[2] = u.z, to[3] = u.w, to[4] = v.x, to[5] = v.y, to[6] = v.z, to[7] = v.w;
+    const uint32_t row = blockIdx.x, words = a.d / 4u;
+    float x[4][4] = {}, w[4][4] = {};
+    auto load = [&](const float *from, float (&to)[4]) {
+        const float4 u = *(const float4 *)from;
+        to[0] = u.x, to[1] = u.y, to[2] = u.z, to[3] = u.w;
     };
     if (row < a.rows) { // uniform; the rows after them only pad the planes with zeros
         const float *src = a.src + (uint64_t)row * a.src_stride;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < 4; ++u) {
             const uint32_t c = threadIdx.x + 256u * u;
-            if (c < chunks) {
-                load(src + 8u * c, x[u]);
-                load(a.w + 8u * c, w[u]);
+            if (c < words) {
+                load(src + 4u * c, x[u]);
+                load(a.w + 4u * c, w[u]);
             }
         }
         float ss = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < 4; ++u) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss += x[u][e] * x[u][e];
+            for (int e = 0; e < 4; ++e) ss += x[u][e] * x[u][e];
         }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
@@ -2055,33 +2057,37 @@ extern "C" __global__ __launch_bounds__(256) void lng_rmsnorm_row8(lng_k_rmsnorm
         ss = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
         const float scale = 1.0f / sqrtf(ss / (float)a.d + a.eps);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < 4; ++u) {
             const uint32_t c = threadIdx.x + 256u * u;
-            if (c < chunks) {
+            if (c < words) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[u][e] = x[u][e] * scale * w[u][e];
-                float *to = a.v + (uint64_t)row * a.stride + 8u * c;
-                *(float4 *)to = make_float4(x[u][0], x[u][1], x[u][2], x[u][3]);
-                *(float4 *)(to + 4) = make_float4(x[u][4], x[u][5], x[u][6], x[u][7]);
+                for (int e = 0; e < 4; ++e) x[u][e] = x[u][e] * scale * w[u][e];
+                *(float4 *)(a.v + (uint64_t)row * a.stride + 4u * c) = make_float4(x[u][0], x[u][1], x[u][2], x[u][3]);
             }
         }
     }
     if (a.planes == LNG_PLANES_NONE) return;
+    // Eight columns of a plane are two threads' (d % 8 == 0: both are here): the even one stores hi of both, the odd one lo.
+    const uint32_t odd = threadIdx.x & 1u;
+    auto pick = [&](uint32_t if_odd, uint32_t if_even) { return (if_odd & (0u - odd)) | (if_even & (odd - 1u)); }; // (a branch would cut the store in two)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < 4; ++u) {
         const uint32_t c = threadIdx.x + 256u * u;
-        if (c < chunks) {
-            bf16x8 hi, lo;
-            q8_split8(x[u], hi, lo);
-            if (a.planes == LNG_PLANES_ROWS) {
-                const uint64_t at = (uint64_t)row * a.d + 8u * c;
-                *(bf16x8 *)(a.hi + at) = hi;
-                *(bf16x8 *)(a.lo + at) = lo;
-            } else {
-                uint4 *to = (uint4 *)a.hi + ((uint64_t)(row >> 4) * (a.d / 32u) + (c >> 2)) * 128u + 16u * q8_mid_chunk(c & 3u) + (row & 15u);
-                to[0] = __builtin_bit_cast(uint4, hi);
-                to[64] = __builtin_bit_cast(uint4, lo);
+        if (c < words) {
+            uint32_t hi[2], lo[2], got[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const __bf16 h0 = (__bf16)x[u][2 * i], h1 = (__bf16)x[u][2 * i + 1];
+                const __bf16 l0 = (__bf16)(x[u][2 * i] - (float)h0), l1 = (__bf16)(x[u][2 * i + 1] - (float)h1);
+                hi[i] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | (uint32_t)__builtin_bit_cast(uint16_t, h1) << 16;
+                lo[i] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | (uint32_t)__builtin_bit_cast(uint16_t, l1) << 16;
+                got[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)pick(hi[i], lo[i]), 0xB1, 0xf, 0xf, true); // the neighbour's
             }
+            const uint4 eight = make_uint4(pick(got[0], hi[0]), pick(got[1], hi[1]), pick(lo[0], got[0]), pick(lo[1], got[1]));
+            const uint32_t chunk = c >> 1;
+            uint4 *rows_at = (uint4 *)((odd ? a.lo : a.hi) + (uint64_t)row * a.d) + chunk;
+            uint4 *operand_at = (uint4 *)a.hi + ((uint64_t)(row >> 4) * (a.d / 32u) + (chunk >> 2)) * 128u + 16u * q8_mid_chunk(chunk & 3u) + (row & 15u) + 64u * odd;
+            *(a.planes == LNG_PLANES_ROWS ? rows_at : operand_at) = eight;
         }
     }
 }

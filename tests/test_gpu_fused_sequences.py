@@ -68,6 +68,27 @@ def test_copy_norm_and_split_in_one_kernel(gpu, n, cols, src_stride, x_stride, o
     assert not np.isnan(got).any() and np.abs(got[:5 * n * rows]).min() >= 0 and np.abs(got).max() > 0
 
 
+@pytest.mark.parametrize("d,stride", [(264, 264), (1024, 1028), (1032, 1032), (4088, 4092), (4096, 4096)])
+def test_norm_at_the_edges_of_its_words(gpu, d, stride):
+    """Rows that end within a thread's share of words, and gaps between rows that stay as they are."""
+    rows, eps = 5, 1e-5
+    x, w = 3 * xorshift_values(91, (rows - 1) * stride + d), 1 + 0.2 * xorshift_values(92, d)
+    bufs = [gpu.upload(x), gpu.upload(w)]
+    batch = gpu.batch(bufs)
+    batch.rmsnorm_rows((C.Slice(0, 0, x.nbytes), C.Slice(1, 0, w.nbytes)), rows, (d, stride), eps)
+    done = batch.run()
+    assert not isinstance(done.gpu_time, Exception), done.gpu_time
+    got = bufs[0].read(np.float32)
+    batch.drop()
+    for b in bufs:
+        b.free()
+    for r in range(rows):
+        row = x[r * stride:r * stride + d].astype(np.float64)
+        want = row / np.sqrt((row * row).mean() + eps) * w
+        assert np.abs(got[r * stride:r * stride + d] - want).max() <= 1e-6 * np.abs(want).max()  # (a sum of 4,096 squares and three roundings in f32)
+        assert np.array_equal(got[r * stride + d:(r + 1) * stride], x[r * stride + d:(r + 1) * stride])
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("n,rows,cols", [(1, 48, 96), (7, 33, 64), (17, 48, 96), (32, 64, 96), (77, 100, 64), (200, 192, 96), (1290, 260, 64)])
 def test_bias_and_residual_in_the_product(gpu, n, rows, cols, bf16):
