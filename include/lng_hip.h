@@ -113,6 +113,7 @@ int lng_hip_device_name(lng_gpu *gpu, char *name, size_t cap);
  *   LNG_PREFILL_UPFRONT 0    narrow windows on the tile-by-tile kernel
  *   LNG_PREFILL_SPLITS n     workgroups per (query tile, kv head) of a prompt pass with fewer workgroups than compute units
  *   LNG_Q8_MID 0|1           never / whenever possible the Q8_0 kernel whose wavefronts share the columns of a tile (32 positions or more)
+ *   LNG_Q8_W16               without effect (the kernel it chose is gone; accepted for programs that still set it)
  *   LNG_NO_FUSING            a batch runs every dispatch as kernels of its own (as one that is timed dispatch by dispatch does)
  *   LNG_CHECKSUM_WGS n       workgroups per compute unit of lng_hip_checksum's streaming read (default 2)
  *   LNG_TABLE_IN_PLACE n     row tables of n bytes or more stay in pinned host memory, where the kernels read them,

@@ -306,6 +306,7 @@ bool set_knob(lng_gpu *g, const char *name, const char *value) {
     if (!strcmp(name, "LNG_PREFILL_PAIR")) return choice(k.prefill_pair, defaults.prefill_pair);
     if (!strcmp(name, "LNG_PREFILL_UPFRONT")) return choice(k.prefill_upfront, defaults.prefill_upfront);
     if (!strcmp(name, "LNG_NO_FUSING")) return flag(k.no_fusing);
+    if (!strcmp(name, "LNG_Q8_W16")) return true; // the kernel it chose is gone
     if (!strcmp(name, "LNG_Q8_MID")) return choice(k.q8_mid, defaults.q8_mid);
     if (!strcmp(name, "LNG_CHECKSUM_WGS")) return choice(k.checksum_wgs, defaults.checksum_wgs);
     if (!strcmp(name, "LNG_TABLE_IN_PLACE")) {

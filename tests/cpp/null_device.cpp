@@ -367,6 +367,7 @@ static void switches_and_checksum() {
         lng_null_clear();
     }
     CHECK(refused(lng_hip_debug_set(f.gpu, "LNG_NO_SUCH_SWITCH", "1"), "no development switch"));
+    CHECK(lng_hip_debug_set(f.gpu, "LNG_Q8_W16", "1") == LNG_OK && lng_hip_debug_set(f.gpu, "LNG_Q8_W16", nullptr) == LNG_OK); // of a kernel that is gone
     CHECK(refused(lng_hip_debug_set(f.gpu, nullptr, "1"), "no name"));
     CHECK(lng_hip_debug_set(nullptr, "LNG_PREFILL_SPLITS", "1") != LNG_OK);
     uint64_t n = 99;
