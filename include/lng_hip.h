@@ -178,8 +178,11 @@ int lng_hip_batch_wait(lng_batch *batch, double *gpu_seconds);
  * gpt-oss/src/gpu.rs:247-317 (Profile / PhaseTime). With timing on (set before commit) an
  * event is recorded after every kernel of the batch; after the batch has finished,
  * lng_hip_batch_kernel_seconds sums the time and counts the launches of the kernel named
- * `kernel` (e.g. "lng_decode_bf16_d64"). Without timing, row copies, RMS norms, additions and the splits before Q8_0
- * products that stand beside each other may run as one kernel, with the same results. */
+ * `kernel` (e.g. "lng_decode_bf16_d64"). Without timing, sequences of a block's dispatches may run as one kernel, with the
+ * same results: a row copy, the RMS norm after it and the split of its rows for the Q8_0 products after that; a product and
+ * the additions of its bias and of the product to other rows; the q, k and v projections of up to 16 positions and the
+ * preparation of attention. A timed batch runs each as kernels of its own, whose names and times are those of an untimed
+ * batch only where no such sequence stands. */
 int lng_hip_batch_set_timing(lng_batch *batch, int enabled);
 int lng_hip_batch_kernel_seconds(lng_batch *batch, const char *kernel, double *seconds, size_t *launches);
 /* Drop of Batch: an uncommitted batch runs nothing (apple.rs:553-561); a committed one is

@@ -2288,6 +2288,7 @@ int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
 // planes.
 int q8_record_tiled(lng_batch *b, lng_k_q8 a, bool x_bf16, const uint16_t *planes_of = nullptr, const uint16_t **planes_out = nullptr) {
     const uint64_t n = a.n, cols = a.cols, rows = a.rows;
+    if (a.accumulate) return fail(LNG_ERR_DISPATCH, "%u positions: the product of many positions does not add to its output", a.n);
     const uint64_t n_pad = (n + 127) / 128 * 128;
     if (n_pad / 128 > 65535) return fail(LNG_ERR_DISPATCH, "too large");
     // one-dimensional grid; the kernel maps ids to tiles (XCD-aware from eight position tiles on,

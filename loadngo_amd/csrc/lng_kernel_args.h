@@ -188,13 +188,14 @@ typedef struct lng_k_q8 {
     uint32_t y_stride;
     uint32_t plane_stride;   /* elements between positions of x_hi / x_lo: cols for the split planes; x's own stride
                                 when the positions are bf16 already (x_hi = x, no x_lo, n rows only) */
-    /* Few positions only: further matrices of the same dispatch, multiplied by the same x (same cols, n).
-     * Workgroups from `first_tile` (in units of 16 rows) on belong to matrix more[i]; first_tile ascends. */
+    /* Not lng_q8_tiled*: further matrices of the same dispatch, multiplied by the same x (same cols, n). Row tiles from
+     * `first_tile` on (of the kernel's own height: lng_q8_few* and lng_q8_one* 16 rows, lng_q8_mid* 16, 32 or 64) belong to
+     * matrix more[i]; first_tile ascends. */
     uint32_t n_more;         /* 0..LNG_Q8_MORE */
     float eps;               /* of the RMS norm, when norm_w is set */
     /* Few positions only. norm_w (lng_q8_one*, lng_q8_few_f32*): x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
-     * (cols <= 12288). bias: y gets bias[row] added. accumulate: the result is added to what y holds. (These two and
-     * residual: all kernels of one matrix.) */
+     * (cols <= 12288). Of one matrix: bias: y gets bias[row] added (lng_q8_few*, lng_q8_one*, lng_q8_mid*, lng_q8_tiled*_add; so
+     * with residual). accumulate: the result is added to what y holds (these, but not lng_q8_tiled*_add). */
     const float *norm_w;
     const float *bias;
     float *residual;         /* [n][rows], not y: gets the result added as well, or NULL */
