@@ -5,7 +5,8 @@
 //    wrong length, outside their buffer or off their element size (apple.rs:860-887), outputs in resident memory or
 //    over an input (apple.rs:889-906), buffers that belong to a batch in flight, and the refusals of copy_rows,
 //    prepare_attention and the Q8_0 products; a refused call records nothing.
-//  - the kernels that Q8_0 products are recorded as.
+//  - the kernels that Q8_0 products are recorded as, and the sequences that a commit makes one kernel of: which do, with
+//    which arguments, and which only look alike.
 //  - the development switches (environment at open, lng_hip_debug_set afterwards) and lng_hip_checksum: refusals and
 //    what is recorded.
 //  - ownership: batches hand their buffers back; close with buffers alive; the last buffer freed on one thread while
@@ -265,6 +266,180 @@ static void products_and_their_kernels() {
         CHECK((few(4096, 2880, 31, normed) == Names{"lng_q8_norm_frag", "lng_q8_mid_r32p32"}));
     }
     lng_null_clear();
+}
+
+// One recorded launch by its name's beginning: its arguments, or NULL.
+template <typename A> static bool launch_args(size_t i, const char *prefix, A *a, unsigned *grid0 = nullptr) {
+    const char *name = nullptr;
+    const void *args = nullptr;
+    size_t size = 0;
+    unsigned grid[3];
+    if (lng_null_launch(i, &name, grid, nullptr, &args, &size) != 0 || strncmp(name, prefix, strlen(prefix)) != 0 || size < sizeof(A)) return false;
+    memcpy(a, args, sizeof(A));
+    if (grid0) *grid0 = grid[0];
+    return true;
+}
+
+// Sequences of a block's dispatches that a commit makes one kernel of, and sequences that only look alike.
+static void fused_sequences() {
+    typedef std::vector<std::string> Names;
+    Fixture f(9, 6 << 20);
+    auto run = [&]() {
+        CHECK(lng_hip_batch_commit(f.batch, nullptr, nullptr) == LNG_OK && lng_hip_batch_wait(f.batch, nullptr) == LNG_OK);
+        return launched();
+    };
+    auto again = [&]() {
+        lng_null_clear();
+        f.rebatch();
+    };
+
+    // ---- copy + RMS norm + split before Q8_0 products ----
+    {
+        const uint64_t cols = 288, rows = 64;
+        auto block = [&](uint64_t n, uint64_t copied, uint64_t normed, uint64_t x_stride) { // n positions of hidden rows (buffer 0), x in buffer 1
+            const lng_slice h{0, 0, copied * cols * 4}, x{1, 0, ((copied - 1) * x_stride + cols) * 4}, v{1, 0, ((normed - 1) * x_stride + cols) * 4};
+            CHECK(lng_hip_copy_rows(f.batch, h, cols, LNG_F32, x, x_stride, LNG_F32, copied, cols) == LNG_OK);
+            CHECK(lng_hip_rmsnorm_rows(f.batch, v, lng_slice{2, 0, cols * 4}, normed, cols, x_stride, 1e-5f) == LNG_OK);
+            CHECK(lng_hip_gemm_q8_0(f.batch, lng_slice{3, 0, rows * cols}, lng_slice{4, 0, rows * cols / 16}, lng_slice{1, 0, ((n - 1) * x_stride + cols) * 4},
+                                    lng_slice{5, 0, n * rows * 4}, rows, cols, n, x_stride, rows) == LNG_OK);
+        };
+        lng_k_rmsnorm norm{};
+        lng_k_q8 product{};
+        unsigned grid = 0;
+        block(77, 77, 77, cols);
+        CHECK((run() == Names{"lng_rmsnorm_row8", "lng_q8_mid_r32p32"}));
+        CHECK(launch_args(0, "lng_rmsnorm_row8", &norm, &grid) && launch_args(1, "lng_q8_mid", &product));
+        CHECK(norm.planes == LNG_PLANES_OPERAND && norm.hi == product.x_hi && grid == 96 && norm.n_pad == 96 && norm.rows == 77 && norm.src != norm.v && norm.v == product.x);
+        again();
+        block(1300, 1300, 1300, cols);
+        CHECK((run() == Names{"lng_rmsnorm_row8", "lng_q8_tiled"}));
+        CHECK(launch_args(0, "lng_rmsnorm_row8", &norm, &grid) && launch_args(1, "lng_q8_tiled", &product));
+        CHECK(norm.planes == LNG_PLANES_ROWS && norm.hi == product.x_hi && norm.lo == product.x_lo && grid == 1408 && norm.src != norm.v);
+        again();
+        block(77, 77, 76, cols); // the norm of fewer rows than are copied, the product of more than are normalised
+        CHECK((run() == Names{"lng_copy_rows", "lng_rmsnorm_row8", "lng_q8_frag_x", "lng_q8_mid_r32p32"}));
+        CHECK(launch_args(1, "lng_rmsnorm_row8", &norm) && norm.src == norm.v && norm.planes == LNG_PLANES_NONE);
+        again();
+        block(16, 16, 16, cols); // few positions: the copy is part of the norm, the product splits by itself
+        CHECK((run() == Names{"lng_rmsnorm_row8", "lng_q8_few_f32"}));
+        again();
+        for (int how = 0; how < 2; ++how) { // timed, or switched off: every dispatch as its own kernels
+            if (how) CHECK(lng_hip_debug_set(f.gpu, "LNG_NO_FUSING", "1") == LNG_OK);
+            else CHECK(lng_hip_batch_set_timing(f.batch, 1) == LNG_OK);
+            block(77, 77, 77, cols);
+            CHECK((run() == Names{"lng_copy_rows", "lng_rmsnorm_row8", "lng_q8_frag_x", "lng_q8_mid_r32p32"}));
+            again();
+        }
+        CHECK(lng_hip_debug_set(f.gpu, "LNG_NO_FUSING", nullptr) == LNG_OK);
+        // a copy to other rows, a norm of other rows than the product's
+        CHECK(lng_hip_copy_rows(f.batch, lng_slice{0, 0, 40 * cols * 4}, cols, LNG_F32, lng_slice{6, 0, 40 * cols * 4}, cols, LNG_F32, 40, cols) == LNG_OK);
+        CHECK(lng_hip_rmsnorm_rows(f.batch, lng_slice{1, 0, 40 * cols * 4}, lng_slice{2, 0, cols * 4}, 40, cols, cols, 1e-5f) == LNG_OK);
+        CHECK(lng_hip_gemm_q8_0(f.batch, lng_slice{3, 0, rows * cols}, lng_slice{4, 0, rows * cols / 16}, lng_slice{6, 0, 40 * cols * 4}, lng_slice{5, 0, 40 * rows * 4}, rows, cols, 40, cols, rows) == LNG_OK);
+        CHECK((run() == Names{"lng_copy_rows", "lng_rmsnorm_row8", "lng_q8_frag_x", "lng_q8_mid_r32p32"}));
+        again();
+    }
+
+    // ---- product + bias + residual ----
+    const struct { uint64_t n; bool bf16; const char *kernel, *folded; } products[] = {
+        {1, false, "lng_q8_one", "lng_q8_one"}, {7, false, "lng_q8_few_f32", "lng_q8_few_f32"}, {33, false, "lng_q8_mid_r32p32", "lng_q8_mid_r32p32"},
+        {1290, false, "lng_q8_tiled", "lng_q8_tiled_add"}, {1, true, "lng_q8_one_bf16", "lng_q8_one_bf16"}, {16, true, "lng_q8_few_bf16", "lng_q8_few_bf16"},
+        {129, true, "lng_q8_mid_bf16_r64p64", "lng_q8_mid_bf16_r64p64"}, {1290, true, "lng_q8_tiled_bf16", "lng_q8_tiled_bf16_add"}};
+    for (const auto &w : products) {
+        const uint64_t rows = 64, cols = 96, n = w.n, len = n * rows * 4;
+        const lng_slice x{0, 0, n * cols * (w.bf16 ? 2u : 4u)}, codes{3, 0, rows * cols}, scales{4, 0, rows * cols / 16}, y{5, 0, len}, bias{2, 0, rows * 4}, h{6, 0, len};
+        auto product = [&](uint64_t y_stride = 64) {
+            const lng_slice out{5, 0, ((n - 1) * y_stride + rows) * 4};
+            CHECK((w.bf16 ? lng_hip_gemm_q8_0_bf16 : lng_hip_gemm_q8_0)(f.batch, codes, scales, x, out, rows, cols, n, cols, y_stride) == LNG_OK);
+        };
+        auto add = [&](lng_slice dst, lng_slice src, uint64_t stride) { CHECK(lng_hip_add_rows(f.batch, dst, src, stride, n, rows) == LNG_OK); };
+        auto last = [&](const char *kernel, size_t adds) { // the product (and what splits before it), then so many additions
+            const Names names = run();
+            const size_t at = names.size() - 1 - adds;
+            CHECK(names.size() > adds && names[at] == kernel);
+            for (size_t i = at + 1; i < names.size(); ++i) CHECK(names[i] == "lng_add_rows");
+            return at;
+        };
+        lng_k_q8 a{};
+        product(), add(y, bias, 0), add(h, y, rows);
+        CHECK(launch_args(last(w.folded, 0), "lng_q8", &a) && a.bias && a.residual && a.residual != a.y && !a.accumulate);
+        again();
+        product(), add(h, y, rows), add(h, y, rows), add(y, bias, 0); // the residual, and what comes after it
+        CHECK(launch_args(last(w.folded, 2), "lng_q8", &a) && !a.bias && a.residual);
+        again();
+        product(), add(y, bias, 0), add(y, bias, 0);
+        CHECK(launch_args(last(w.folded, 1), "lng_q8", &a) && a.bias && !a.residual);
+        again();
+        if (n > 1) {
+            product(68); // y with gaps
+            CHECK(lng_hip_add_rows(f.batch, h, lng_slice{5, 0, ((n - 1) * 68 + rows) * 4}, 68, n, rows) == LNG_OK);
+            CHECK(launch_args(last(w.kernel, 1), "lng_q8", &a) && !a.residual);
+            again();
+        }
+        for (const lng_slice over : {lng_slice{0, 0, len}, lng_slice{3, 0, len}, lng_slice{4, 0, len}}) { // other workgroups still read what it is added to
+            product(), add(over, y, rows);
+            CHECK(launch_args(last(w.kernel, 1), "lng_q8", &a) && !a.residual);
+            again();
+        }
+        product(), add(y, bias, 0), add(lng_slice{2, 0, len}, y, rows); // over the bias
+        CHECK(launch_args(last(w.folded, 1), "lng_q8", &a) && a.bias && !a.residual);
+        again();
+    }
+
+    // ---- the q, k and v projections + the preparation of attention ----
+    struct Case { uint64_t n, cols, rotary; bool normed, one_item; const char *kind; Names names; };
+    const Case cases[] = {
+        {1, 96, 64, true, true, "", {"lng_q8_one_prepare"}},
+        {4, 96, 64, true, false, "", {"lng_q8_few_f32_prepare"}},
+        {16, 96, 64, false, true, "", {"lng_q8_few_f32_prepare"}},
+        {4, 2880, 64, true, false, "", {"lng_q8_norm_frag", "lng_q8_few_prepare"}},
+        {17, 96, 64, true, false, "", {"lng_q8_few_f32", "lng_prepare"}},
+        {4, 96, 32, true, false, "", {"lng_q8_few_f32", "lng_prepare"}},
+        {4, 96, 64, true, false, "backwards", {"lng_q8_few_f32", "lng_prepare"}},
+        {4, 96, 64, true, false, "swapped", {"lng_q8_few_f32", "lng_prepare"}},
+        {4, 96, 64, true, false, "table over q", {"lng_q8_few_f32", "lng_prepare"}},
+        {4, 96, 64, true, false, "queries over x", {"lng_q8_few_f32", "lng_prepare"}},
+        {4, 96, 64, true, false, "biases over v", {"lng_q8_few_f32", "lng_prepare"}},
+    };
+    for (const Case &c : cases) {
+        const uint64_t heads = 6, kv = 2, qw = heads * 64, kw = kv * 64, n = c.n, slots = 24;
+        const std::string kind = c.kind;
+        const uint64_t k_at = kind == "swapped" ? n * kw * 4 : 0, v_at = kind == "swapped" ? 0 : n * kw * 4;
+        const lng_slice x{0, 0, n * c.cols * 4}, norm{2, 0, c.cols * 4};
+        const uint64_t widths[3] = {qw, kw, kw};
+        const lng_slice ys[3] = {{5, 0, n * qw * 4}, {6, k_at, n * kw * 4}, {6, v_at, n * kw * 4}};
+        lng_q8_matrix m[3];
+        uint64_t at = 0;
+        for (int i = 0; i < 3; ++i) {
+            m[i] = {{3, at * c.cols, widths[i] * c.cols}, {4, at * c.cols / 16, widths[i] * c.cols / 16}, ys[i], widths[i]};
+            at += widths[i];
+        }
+        if (c.normed) CHECK(lng_hip_gemm_q8_0_many_normed(f.batch, m, 3, x, norm, 1e-5f, c.cols, n, c.cols) == LNG_OK);
+        else CHECK(lng_hip_gemm_q8_0_many(f.batch, m, 3, x, c.cols, n, c.cols) == LNG_OK);
+        const uint64_t biases_in = kind == "biases over v" ? 6 : 1, bias_at = kind == "biases over v" ? v_at : 0; // (read by the preparation only)
+        const lng_slice qb{1, 0, qw * 4}, kb{biases_in, bias_at, kw * 4}, vb{1, 8192, kw * 4};
+        const lng_prepare_buffers pb{5, 6, 6, (uint64_t)(kind == "table over q" ? 5 : 7), (uint64_t)(kind == "queries over x" ? 0 : 8), 7, 7, &qb, &kb, &vb};
+        std::vector<lng_prepare_item> items;
+        for (uint64_t i = 0; i < (c.one_item ? 1 : n); ++i) {
+            const uint64_t j = kind == "backwards" ? n - 1 - i : i;
+            lng_prepare_item it{};
+            it.q_offset = j * qw * 4, it.k_offset = j * kw * 4, it.v_offset = n * kw * 4 + j * kw * 4, it.table_offset = (pb.table == 7 ? 3 << 20 : 0) + j * c.rotary * 4;
+            it.q_out_offset = j * qw * 2, it.k_cache_offset = i * slots * kw * 2, it.v_cache_offset = (n + i) * slots * kw * 2;
+            it.n = c.one_item ? n : 1, it.start = 5 + i, it.slots = slots;
+            items.push_back(it);
+        }
+        CHECK(lng_hip_prepare_attention(f.batch, &pb, items.data(), items.size(), heads, kv, 64, c.rotary, LNG_BF16) == LNG_OK);
+        const Names names = run();
+        bool same = names.size() == c.names.size();
+        for (size_t i = 0; same && i < names.size(); ++i) same = names[i].rfind(c.names[i], 0) == 0 && (c.names[i] == "lng_prepare" || names[i] == c.names[i]);
+        if (!same) fprintf(stderr, "%llu positions, %llu columns, %llu rotated, %s: %zu launches, first %s\n", (unsigned long long)n, (unsigned long long)c.cols, (unsigned long long)c.rotary, c.kind, names.size(), names[0].c_str());
+        CHECK(same);
+        if (names.back().find("_prepare") != std::string::npos && names.back().rfind("lng_q8", 0) == 0) {
+            lng_k_q8_prepare both{};
+            CHECK(launch_args(names.size() - 1, "lng_q8", &both) && both.q8.n == n && both.q8.n_more == 2 && both.prepare.heads == heads && both.prepare.kv_heads == kv);
+            CHECK((both.prepare.items == nullptr) == (items.size() == 1) && both.prepare.q_bias && both.prepare.k_bias && both.prepare.v_bias);
+        }
+        again();
+    }
 }
 
 // The development switches (read from the environment once, at open; afterwards only lng_hip_debug_set) and the
@@ -732,6 +907,7 @@ int main(int argc, char **argv) {
     const size_t dispatches = argc > 1 ? (size_t)strtoull(argv[1], nullptr, 10) : 100000;
     refusals();
     products_and_their_kernels();
+    fused_sequences();
     switches_and_checksum();
     lifetimes();
     allocation_failures();

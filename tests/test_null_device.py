@@ -6,7 +6,7 @@ tests/cpp/null_device.cpp then drives the C ABI: the refusals of metal-compute/s
 1243-1277 (the reference's rejected shapes, slices of the wrong length, outside their buffer or off their
 element size, outputs in resident memory or over an input, buffers of a batch in flight), the refusals of
 copy_rows, prepare_attention and the Q8_0 products, the kernels that Q8_0 products are recorded as, the
-development switches (environment at open,
+sequences that a commit makes one kernel of and those that only look alike, the development switches (environment at open,
 lng_hip_debug_set afterwards) and lng_hip_checksum, ownership and lifetimes (close racing the last free on two
 threads), allocation failures while recording, and 100,000 random dispatches through the decode planner with
 every grid, work table, chunk and scratch size checked on the host. Any sanitizer report fails the run."""
