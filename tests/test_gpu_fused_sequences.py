@@ -1,13 +1,16 @@
 """Sequences of a block's dispatches that run as fewer kernels (copy + RMS norm + the split before Q8_0 products; product +
 bias + residual): every buffer holds bit for bit what it holds when each dispatch is a kernel of its own."""
+import functools
+
 import numpy as np
 import pytest
 
 from loadngo_amd import compute as C
 from tests.gpu_common import gpu  # noqa: F401
-from tests.helpers import q8_test_matrix, to_bf16_bits, xorshift_values
+from tests.helpers import from_bf16_bits, q8_test_matrix, to_bf16_bits, xorshift_values
 
 pytestmark = pytest.mark.gpu
+_matrix = functools.lru_cache(maxsize=None)(q8_test_matrix)
 
 
 def both_ways(gpu, arrays, record):
@@ -37,11 +40,12 @@ def test_copy_norm_and_split_in_one_kernel(gpu, n, cols, src_stride, x_stride, o
     """Positions up to and past both ways of splitting, row widths at the edges of the norm kernels, strides, hidden rows
     off a 16-byte boundary; one product and three, a product of other rows in between, the norm alone."""
     eps, rows = 1e-5, 80
-    mats = [q8_test_matrix(rows, cols, 30 + i)[:2] for i in range(3)]
+    mats = [q8_test_matrix(rows, cols, 30 + i) for i in range(3)]
     h = 3 * xorshift_values(71 + n, n * src_stride + 1)
     x = xorshift_values(72, n * x_stride)
-    arrays = [h, x, 1 + 0.2 * xorshift_values(73, cols), np.zeros(6 * n * rows, np.float32)]
-    for codes, bits in mats:
+    weights = 1 + 0.2 * xorshift_values(73, cols)
+    arrays = [h, x, weights, np.zeros(6 * n * rows, np.float32)]
+    for codes, bits, _ in mats:
         arrays += [codes, bits]
     hs = C.Slice(0, offset, ((n - 1) * src_stride + cols) * 4)
     xs, ws = C.Slice(1, 0, ((n - 1) * x_stride + cols) * 4), C.Slice(2, 0, cols * 4)
@@ -64,8 +68,13 @@ def test_copy_norm_and_split_in_one_kernel(gpu, n, cols, src_stride, x_stride, o
     fused, apart = both_ways(gpu, arrays, record)
     for i, (a, b) in enumerate(zip(fused, apart)):
         assert np.array_equal(a, b), "buffer %d" % i
-    got = fused[3].view(np.float32)
-    assert not np.isnan(got).any() and np.abs(got[:5 * n * rows]).min() >= 0 and np.abs(got).max() > 0
+    got = fused[3].view(np.float32).reshape(6, n, rows)
+    hidden = np.stack([h[offset // 4 + p * src_stride:][:cols] for p in range(n)]).astype(np.float64)
+    once = hidden / np.sqrt((hidden * hidden).mean(axis=1, keepdims=True) + eps) * weights
+    twice = once / np.sqrt((once * once).mean(axis=1, keepdims=True) + eps) * weights
+    for y_i, positions, i in ((0, once, 0), (1, once, 1), (2, once, 2), (3, twice, 0), (4, hidden, 1)):
+        want = positions @ mats[i][2].T
+        assert np.abs(got[y_i] - want).max() / np.abs(want).max() < 1e-5, y_i  # the reference's bound (glue.rs:171)
 
 
 @pytest.mark.parametrize("d,stride", [(264, 264), (1024, 1028), (1032, 1032), (4088, 4092), (4096, 4096)])
@@ -143,18 +152,30 @@ def test_bias_and_residual_in_the_product(gpu, n, rows, cols, bf16):
 
 
 @pytest.mark.parametrize("dtype", [C.F32, C.BF16])
-@pytest.mark.parametrize("n,one_item,dim,rotary,bias,normed,kind", [
+@pytest.mark.parametrize("n,one_item,dim,rotary,bias,normed,kind,cols,heads,kv_heads", [(*c, 96, 6, 2) for c in (
     (1, True, 64, 64, True, True, ""), (1, True, 64, 64, False, False, ""), (2, False, 64, 64, True, True, ""), (16, False, 64, 64, True, True, ""),
     (3, True, 64, 64, True, False, ""), (16, True, 64, 64, False, True, ""), (17, False, 64, 64, True, True, ""), (5, False, 64, 32, True, True, ""),
     (2, False, 128, 128, True, True, ""), (4, False, 64, 64, True, True, "backwards"), (4, False, 64, 64, True, True, "swapped"),
-    (4, False, 64, 64, True, True, "table over q"), (4, False, 64, 64, True, True, "queries over x")])
-def test_projections_and_preparation_in_one_kernel(gpu, n, one_item, dim, rotary, bias, normed, kind, dtype):
+    (4, False, 64, 64, True, True, "table over q"), (4, False, 64, 64, True, True, "queries over x"))] + [
+    (1, True, 64, 64, True, True, "", 2880, 6, 2), (16, False, 64, 64, True, True, "", 2880, 6, 2), (5, False, 64, 64, True, False, "", 2880, 6, 2),
+    (1, True, 64, 64, True, True, "", 352, 64, 8), (16, True, 64, 64, False, False, "", 352, 64, 8), (1, True, 64, 64, False, False, "", 4160, 2, 1),
+    (7, False, 64, 64, True, False, "", 4160, 2, 1), (1, True, 64, 64, True, True, "", 12288, 2, 1), (3, False, 64, 64, True, True, "", 12288, 2, 1),
+    (6, False, 64, 64, True, False, "", 16416, 2, 1), (9, False, 64, 64, True, True, "", 512, 6, 2), (16, False, 64, 64, True, False, "", 544, 6, 2)])
+def test_projections_and_preparation_in_one_kernel(gpu, n, one_item, dim, rotary, bias, normed, kind, cols, heads, kv_heads, dtype):
     """q, k and v of up to 16 positions with the preparation after them: tables of items and one item, rings that wrap, with
     and without biases and norm; and what stays apart: more positions, other widths, items in another order than the rows, k
-    and v the other way round, a rotation table in rows that q is written to, prepared queries where x is."""
-    heads, kv_heads, cols, slots, eps = 6, 2, 96, 24, 1e-5
+    and v the other way round, a rotation table in rows that q is written to, prepared queries where x is. Columns: fewer
+    pairs of blocks than wavefronts, several pairs a wavefront, more than one turn of 4,096, a block left over, scales that
+    wait in LDS in more than 64 words a row or do not fit there; positions split by the product itself and before it. The
+    products and the prepared rows against float64, too."""
+    slots, eps = 24, 1e-5
     qw, kw, es = heads * dim, kv_heads * dim, 4 if dtype == C.F32 else 2
-    mats = [q8_test_matrix(rows, cols, 60 + i)[:2] for i, rows in enumerate((qw, kw, kw))]
+    elements = []
+    mats = []
+    for i, rows in enumerate((qw, kw, kw)):
+        codes, bits, e = _matrix(rows, cols, 60 + i)
+        mats.append((codes, bits))
+        elements.append(e)
     arrays = [3 * xorshift_values(81 + n, n * max(cols, qw)), 1 + 0.2 * xorshift_values(82, cols), xorshift_values(83, n * qw),
               np.zeros(2 * n * kw, np.float32), xorshift_values(84, n * rotary), np.zeros(n * qw * es, np.uint8),
               np.zeros(2 * n * slots * kw * es, np.uint8), xorshift_values(85, qw + 2 * kw)]
@@ -183,3 +204,29 @@ def test_projections_and_preparation_in_one_kernel(gpu, n, one_item, dim, rotary
     for i, (a, b) in enumerate(zip(fused, apart)):
         assert np.array_equal(a, b), "buffer %d" % i
     assert fused[5 if q_out == 5 else 0].any() and fused[6].any()
+    if kind or rotary != 64 or dim != 64:
+        return
+    x = arrays[0][:n * cols].reshape(n, cols).astype(np.float64)
+    if normed:
+        x = x / np.sqrt((x * x).mean(axis=1, keepdims=True) + eps) * arrays[1]
+    want = [x @ e.T for e in elements]
+    tol = [1e-5 * np.abs(w).max() for w in want]  # the reference's bound of the products (glue.rs:171)
+    got_kv = fused[3].view(np.float32).reshape(2, n, kw)
+    for got, w, t in zip((fused[2].view(np.float32)[:n * qw].reshape(n, qw), got_kv[0], got_kv[1]), want, tol):
+        assert np.abs(got - w).max() <= t
+    if bias:
+        want = [w + b for w, b in zip(want, np.split(arrays[7].astype(np.float64), [qw, qw + kw]))]
+    angles = arrays[4][:n * 64].reshape(n, 1, 32, 2).astype(np.float64)  # cosine and sine of every pair
+
+    def rotate(rows):
+        r = rows.reshape(n, -1, 2, 32)
+        low, high = r[:, :, 0], r[:, :, 1]
+        return np.stack([low * angles[..., 0] - high * angles[..., 1], high * angles[..., 0] + low * angles[..., 1]], axis=2).reshape(n, -1)
+
+    want = [rotate(want[0]), rotate(want[1]), want[2]]
+    values = (lambda raw: raw.view(np.float32)) if dtype == C.F32 else (lambda raw: from_bf16_bits(raw.view(np.uint16)))
+    caches = values(fused[6]).reshape(2, n, slots, kw)
+    at = [(0, (slots - 1 + p) % slots) if one_item else (p, (5 + 13 * p) % slots) for p in range(n)]
+    got = [values(fused[5]).reshape(n, qw), np.stack([caches[0][c, s] for c, s in at]), np.stack([caches[1][c, s] for c, s in at])]
+    for g, w, t in zip(got, want, tol):  # a rotated value is two products of values that far off, each times at most 1.2; narrowing: half of 2^-8
+        assert (np.abs(g - w) <= 3 * t + 1e-6 + (0 if dtype == C.F32 else 2.0 ** -8) * np.abs(w)).all()
