@@ -107,7 +107,8 @@ template <int NW, bool HEADS = false> struct Q8Few {
         }
     }
     __device__ __forceinline__ uint32_t both_sc(uint32_t word, uint32_t first, uint32_t second) const { // zero past the last block
-        return words_aligned || 2u * word + 1u >= blocks ? first : first | (second << 16);
+        // (low halves of both; a shift of the second alone would be moved to its load, and wait there)
+        return words_aligned || 2u * word + 1u >= blocks ? first : __builtin_amdgcn_perm(second, first, 0x05040100u);
     }
     __device__ __forceinline__ uint32_t load_sc(uint32_t row, uint32_t word) const {
         uint32_t first, second;

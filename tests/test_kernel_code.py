@@ -39,4 +39,7 @@ def test_products_of_few_positions_ask_for_all_before_they_wait(kernels):
         # (the last load of a turn may stand right before the wait)
         waited = [i for i in loads if re.match(r"s_waitcnt vmcnt\(0\)", code[name][i + 1])]
         assert len(loads) >= 8 and len(waited) <= 1, "%s waits for %d of its %d loads of 16 bytes one by one" % (name, len(waited), len(loads))
+        # (the preparation of attention looks its item up in a table first)
+        early = [] if "prepare" in name else [line for line in code[name][:loads[7]] if re.match(r"s_waitcnt.*vmcnt", line)]
+        assert not early, "%s waits for memory before it has asked for its first eight loads of 16 bytes" % name
         assert scratch[name] == 0, "%s keeps %d bytes a lane in memory" % (name, scratch[name])
