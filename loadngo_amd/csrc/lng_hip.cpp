@@ -1133,6 +1133,7 @@ bool fuse_prepare(const lng_gpu *g, Cmd &c, const Cmd &after) {
         if (!apart(out.at, out.len, a.x, ((uint64_t)(a.n - 1) * a.x_stride + a.cols) * 4) || (a.norm_w && !apart(out.at, out.len, a.norm_w, (uint64_t)a.cols * 4))) return false;
     }
     const bool one = c.fn == g->q8_one[0], direct = c.fn == g->q8_few_f32;
+    if (one) both.prepare.first.start %= both.prepare.first.slots; // lng_q8_one_prepare: the row itself (one position is one item, not a table)
     c.name = one ? "lng_q8_one_prepare" : direct ? "lng_q8_few_f32_prepare" : "lng_q8_few_prepare";
     c.fn = one ? g->q8_one_prepare : direct ? g->q8_few_f32_prepare : g->q8_few_prepare;
     set_args(c, both);
@@ -2257,6 +2258,22 @@ bool q8_few_direct(const lng_gpu *g, const lng_k_q8 &a, uint64_t wgs) {
     return n * cols * rounds <= 18432;
 }
 
+// Rows of a workgroup of lng_q8_one: of all that a compute unit can hold at once it should get as many as the next, and no
+// unit be without: 2,880 rows as 240 tiles of 12 take 5.5 us (4,096 columns), as 180 of 16 5.9; 5,120 as 428 of 12 7.6, as 320 of
+// 16 7.8 (the second workgroup of a unit waits for the first one's loads: those with two finish last).
+unsigned q8_one_rows(const lng_gpu *g, const lng_k_q8 &a) {
+    unsigned best = 16;
+    uint64_t best_load = UINT64_MAX;
+    for (unsigned t = 16; t >= 8; t -= 2) { // (even: lng_q8_one_prepare takes pairs of rows)
+        uint64_t wgs = (a.rows + t - 1) / t;
+        for (uint32_t i = 0; i < a.n_more; ++i) wgs += (a.more[i].rows + t - 1) / t;
+        if (wgs > 2ull * g->cus) break;
+        const uint64_t load = (wgs + g->cus - 1) / g->cus * t;
+        if (load < best_load) best = t, best_load = load;
+    }
+    return best;
+}
+
 // Fewer than 32 positions: bound by reading the matrix, in tiles of 16 rows. One position splits (and normalises) x in
 // the kernel, whose LDS holds up to 48 KB of it; more go through the planes of q8_record_frag or are split by every workgroup.
 // `a` may name further matrices of the same dispatch (first_tile in tiles of 16 rows).
@@ -2269,15 +2286,23 @@ int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
         if (rc == LNG_ERR_ALLOC) direct = true; // no memory for the planes
         else if (rc) return rc;
     }
+    if (one) {
+        a.one_rows = q8_one_rows(b->gpu, a);
+        row_tiles = (a.rows + a.one_rows - 1) / a.one_rows;
+        for (uint32_t i = 0; i < a.n_more; ++i) {
+            a.more[i].first_tile = (uint32_t)row_tiles;
+            row_tiles += (a.more[i].rows + a.one_rows - 1) / a.one_rows;
+        }
+    }
     Cmd c;
     c.fn = one ? b->gpu->q8_one[x_bf16] : direct ? b->gpu->q8_few_f32 : b->gpu->q8_few[x_bf16];
     c.name = one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : direct ? "lng_q8_few_f32" : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
     c.grid[0] = (unsigned)row_tiles;
     c.grid[1] = (unsigned)groups;
     c.block = 512;
-    const uint64_t scales = blocks <= 512 ? 16 * (((blocks + 1) / 2) | 1) * 4 : 0; // both of a pair of blocks in a word
-    // x's planes, the weights of its norm, or the turning buffers
-    c.lds = (unsigned)(scales + (one ? a.cols * (x_bf16 ? 2u : 4u) : direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
+    const uint64_t pairs = (blocks + 1) / 2, scales = blocks <= 512 ? 16 * (pairs | 1) * 4 : 0; // both of a pair of blocks in a word
+    // one: x's planes and units (Q8ONE_PAIR), of one pair more; else the scales and the weights of x's norm or the turning buffers
+    c.lds = (unsigned)(one ? (pairs + 1) * (256 + 8) : scales + (direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
     set_args(c, a);
     b->cmds.push_back(std::move(c));
     return LNG_OK;

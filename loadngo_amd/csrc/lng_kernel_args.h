@@ -189,7 +189,7 @@ typedef struct lng_k_q8 {
     uint32_t plane_stride;   /* elements between positions of x_hi / x_lo: cols for the split planes; x's own stride
                                 when the positions are bf16 already (x_hi = x, no x_lo, n rows only) */
     /* Not lng_q8_tiled*: further matrices of the same dispatch, multiplied by the same x (same cols, n). Row tiles from
-     * `first_tile` on (of the kernel's own height: lng_q8_few* and lng_q8_one* 16 rows, lng_q8_mid* 16, 32 or 64) belong to
+     * `first_tile` on (of the kernel's own height: lng_q8_few* 16 rows, lng_q8_one* one_rows, lng_q8_mid* 16, 32 or 64) belong to
      * matrix more[i]; first_tile ascends. */
     uint32_t n_more;         /* 0..LNG_Q8_MORE */
     float eps;               /* of the RMS norm, when norm_w is set */
@@ -201,6 +201,8 @@ typedef struct lng_k_q8 {
     float *residual;         /* [n][rows], not y: gets the result added as well, or NULL */
     uint32_t accumulate;
     uint32_t tiles;          /* row tiles of all matrices of the dispatch (lng_q8_mid*) */
+    uint32_t one_rows;       /* lng_q8_one*: rows of a tile, even, at most 16 */
+    uint32_t pad_;
     struct lng_k_q8_more {
         const int8_t *codes;
         const uint16_t *scales;

@@ -165,22 +165,30 @@ template <int NW, bool HEADS = false> struct Q8Few {
 struct Q8Prepared {
     float bias, bias_there, c, s;
     char *to;
-    __device__ __forceinline__ void ask(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row) {
-        const lng_prepare_item it = p.items ? p.items[position] : p.first;
-        const uint32_t r = p.items ? 0u : position; // a table's items are of one position each
+    // (Loads of what is absent read `any` instead: a load behind a branch would be waited for before the branch ends.)
+    // ONE position is the one item, whose `start` is the row of the caches already (q8's fuse_prepare).
+    template <bool ONE> static __device__ __forceinline__ lng_prepare_item item_of(const lng_k_prepare &p, uint32_t position, uint32_t &r) {
+        r = ONE || p.items ? 0u : position; // a table's items are of one position each
+        if constexpr (ONE) return p.first;
+        else return p.items ? p.items[position] : p.first;
+    }
+    template <bool ONE> __device__ __forceinline__ void ask(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row, const float *any) {
+        uint32_t r;
+        const lng_prepare_item it = item_of<ONE>(p, position, r);
         const float *b = which == 0 ? p.q_bias : which == 1 ? p.k_bias : p.v_bias;
-        bias = b ? b[row] : 0.0f;
-        bias_there = b && which < 2u ? b[row ^ 32u] : 0.0f;
-        c = 0.0f, s = 0.0f;
-        if (which < 2u) {
-            const float2 t = *(const float2 *)(p.table + it.table_offset + ((uint64_t)r * 32u + (row & 31u)) * 8u);
-            c = t.x, s = t.y;
-        }
+        bias = *(b ? b + row : any);
+        bias_there = *(b && which < 2u ? b + (row ^ 32u) : any);
+        const float2 t = *(const float2 *)(which < 2u ? p.table + it.table_offset + ((uint64_t)r * 32u + (row & 31u)) * 8u : (const char *)any);
+        c = t.x, s = t.y;
+    }
+    template <bool ONE> __device__ __forceinline__ void place(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row) {
+        uint32_t r;
+        const lng_prepare_item it = item_of<ONE>(p, position, r);
         const uint32_t es = p.out_dtype == LNG_BF16 ? 2u : 4u;
         if (which == 0) {
             to = p.q_out + it.q_out_offset + ((uint64_t)r * p.heads * 64u + row) * es;
         } else {
-            const uint64_t at = ((it.start + r) % it.slots * p.kv_heads * 64u + row) * es;
+            const uint64_t at = ((ONE ? it.start : (it.start + r) % it.slots) * p.kv_heads * 64u + row) * es;
             to = which == 1 ? p.k_cache + it.k_cache_offset + at : p.v_cache + it.v_cache_offset + at;
         }
     }
@@ -199,12 +207,9 @@ struct Q8Prepared {
 };
 
 // Bound by latencies - a start, one round trip to memory, the partial sums' way through LDS - before the reading of the
-// matrix: 5,120 x 2,880 (q, k and v, 15.7 MB) with the norm, in a batch of 16 such: 1 position 7.8 us (11.1 when every
-// wavefront asked for half of its blocks at a time and split x for each), 2 to 16: 12 us with the planes' dispatch (20-27
+// matrix: 5,120 x 2,880 (q, k and v, 15.7 MB) with the norm, in a batch of 16 such: 2 to 16 positions 12 us with the planes' dispatch (20-27
 // when each workgroup normalised and split all positions itself), 31: 14 us (38); 2,880 x 4,096 with bias and residual from
-// bf16 1, 16, 31 positions: 6.7, 8.1, 10 us (9.1, 13, 23), from f32 6.9, 11, 16 (11, 19, 35).
-// One position with every load of a turn really on its way before the first is waited for: 16,384 x 2,880 14.9 -> 11.7 us
-// (bf16 14.3 -> 11.3), 2,048 rows 6.0 -> 5.1 (5.8 -> 4.7).
+// bf16 16, 31 positions: 8.1, 10 us (13, 23), from f32 11, 16 (19, 35). One position: see q8_one_body.
 // Eight wavefronts to 16 rows: two workgroups fit a compute unit, so up to 512 tiles are all in flight at once.
 
 // 2 to 16 positions (more: 16 per blockIdx.y). Every load of a turn is asked for before its first product, the matrix's
@@ -254,7 +259,10 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
     if (mine && a.residual) held = *to;
     Q8Prepared ready;
     if constexpr (PREPARE) {
-        if (mine) ready.ask(*prepare, which, out_p, out_row);
+        if (mine) {
+            ready.ask<false>(*prepare, which, out_p, out_row, (const float *)a.codes);
+            ready.place<false>(*prepare, which, out_p, out_row);
+        }
     }
 
     floatx4 y = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -362,71 +370,161 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
     if constexpr (PREPARE) ready.store(*prepare, which, out_row, sum, __shfl_xor(sum, 8, 64)); // (all rows of a position are mine or none)
 }
 
-// One position. Its operand planes are made once per workgroup (normalised, split: a thread takes eight columns) and wait
-// in LDS. f32: even rows of the A operand are the hi plane, odd ones the lo plane, and one matrix instruction multiplies
-// a block by both; all rows of bf16 are the position.
+// One position, on the integer matrix unit, which takes the codes as they are: widening them for the other one was most of
+// the vector unit's work here. x goes in as whole numbers too: of each block of 32 columns the largest |x| sets a power of
+// two, every x of the block becomes a 30-bit number of that unit (exact where it is within 2^-6 of the largest, else rounded
+// at 2^-30 of it: nowhere worse than the products' f32 sums, and better than two bf16 values), and its four signed bytes lie in
+// four planes in LDS. One matrix instruction multiplies 16 rows by 64 columns, two blocks: rows 0-3 of the other operand are
+// the first block's planes (zero in the second's columns), rows 4-7 the second's; the next pair's go into rows 8-15 and the
+// same accumulators. So lane group kg ends with the four planes' exact sums of block kg of four, and puts them together.
+// A block with an x that is not finite gives NaN, as the split into two bf16 values does.
+// Bound by memory and by what lies before and after it: 1 us until all loads are on their way, a round trip, the matrix at the
+// rate of the whole device (15.7 MB: 2.6 us), 0.8 us of sums and their way through LDS, a dispatch's start and end. In a token
+// through 24 blocks (kernel trace): 5,120 x 2,880 with norm and preparation 9.1 us -> 7.6, 2,880 x 4,096 with bias and residual
+// 7.2 -> 5.5 from bf16, 7.3 -> 5.2 from f32; of which the whole numbers 9.1 -> 7.8 and 7.2 -> 5.9 (the sums of 4,096 columns took
+// a wavefront 1.55 us, now 0.5), tiles of 10 to 14 rows and x before the codes the rest.
+struct Q8Whole { // eight columns, a quarter of a block; the other three are in the neighbouring lanes
+    uint2 plane[4];
+    float unit;
+    __device__ __forceinline__ void make(const float (&x)[8]) {
+        uint32_t top = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t magnitude = __float_as_uint(x[e]) & 0x7fffffffu;
+            top = top > magnitude ? top : magnitude;
+        }
+        const uint32_t one = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0xB1, 0xf, 0xf, true); // quad_perm [1,0,3,2]
+        top = top > one ? top : one;
+        const uint32_t two = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x4E, 0xf, 0xf, true); // quad_perm [2,3,0,1]
+        top = top > two ? top : two;
+        const int32_t exponent = (int32_t)(top >> 23) > 7 ? (int32_t)(top >> 23) - 127 : -120; // the unit of smaller blocks: 2^-149
+        unit = top >= 0x7f800000u ? __uint_as_float(0x7fc00000u) : __builtin_amdgcn_ldexpf(1.0f, exponent - 29);
+        uint32_t q[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e] = ((uint32_t)(int32_t)__builtin_rintf(__builtin_amdgcn_ldexpf(x[e], 29 - exponent)) + 0x00808080u) ^ 0x00808080u; // signed bytes
+        uint32_t word[4][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t a = __builtin_amdgcn_perm(q[4 * h + 1], q[4 * h], 0x05010400u), b = __builtin_amdgcn_perm(q[4 * h + 1], q[4 * h], 0x07030602u);
+            const uint32_t c = __builtin_amdgcn_perm(q[4 * h + 3], q[4 * h + 2], 0x05010400u), d = __builtin_amdgcn_perm(q[4 * h + 3], q[4 * h + 2], 0x07030602u);
+            word[0][h] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+            word[1][h] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+            word[2][h] = __builtin_amdgcn_perm(d, b, 0x05040100u);
+            word[3][h] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) plane[k] = make_uint2(word[k][0], word[k][1]);
+    }
+};
+
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+// LDS of q8_one_body: the planes of each pair of blocks (and of one more, that the last turn may read and not use), the units.
+#define Q8ONE_PAIR 256u // bytes
 template <bool BF16, int NW, bool PREPARE = false>
 __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
-    constexpr int U = Q8Few<NW>::U, T = 64 * NW;
-    __shared__ float s_red[NW][16];
+    constexpr int U = 4, T = 64 * NW; // U: twos of pairs in flight, 4,096 columns in one turn of eight wavefronts
+    __shared__ float s_red[NW][64];
     __shared__ float s_norm[NW];
-    Q8Few<NW, PREPARE> m(a, tile, (uint32_t *)(s_mem + (uint64_t)a.cols * (BF16 ? 2u : 4u)));
-    const uint32_t chunks = a.cols / 8u, mine = threadIdx.x, out_row = q8_tile_row<PREPARE>(tile) + q8_row_in<PREPARE>(mine & 15u);
-    const bool writes = mine < m.rows_here;
-    uint4 *s_x = (uint4 *)s_mem; // [plane][chunk of eight columns]
-    float x[8] = {}, nw[8] = {};
-    uint4 x16 = make_uint4(0, 0, 0, 0);
-    auto load = [&](uint32_t chunk, const float *src, float (&to)[8]) {
+    __shared__ __attribute__((aligned(16))) uint32_t s_zero[512]; // what lanes read that hold rows of the other block or pair
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15u, kg = lane >> 4;
+    const uint32_t blocks = a.cols / 32u, pairs = (blocks + 1u) / 2u, chunks = a.cols / 8u, mine = threadIdx.x;
+    const uint32_t from = wave * pairs / NW, to = (wave + 1u) * pairs / NW;
+    // The tile's rows, the instruction's columns: a.one_rows of them, one after another or (PREPARE: what rotation by halves pairs
+    // belongs to one tile) half as many pairs of rows 32 apart, in lanes j and j + 8. The columns past them repeat the last.
+    uint32_t row;      // of the matrix
+    bool row_mine;
+    if constexpr (PREPARE) {
+        const uint32_t half = a.one_rows / 2u, first = tile * half, last = (a.rows / 2u - first < half ? a.rows / 2u - first : half) - 1u;
+        const uint32_t pair = first + ((j & 7u) < last ? j & 7u : last);
+        row = (pair >> 5) * 64u + (pair & 31u) + (j & 8u) * 4u;
+        row_mine = (j & 7u) <= last;
+    } else {
+        const uint32_t first = tile * a.one_rows, last = (a.rows - first < a.one_rows ? a.rows - first : a.one_rows) - 1u;
+        row = first + (j < last ? j : last);
+        row_mine = j <= last;
+    }
+    // (a uniform base and 32-bit offsets: a row of the tile is at most 127 x 24,576 bytes on)
+    const uint32_t r0 = __builtin_amdgcn_readfirstlane(row), row_on = row - r0, out_row = row;
+    const int8_t *w_src = a.codes + (uint64_t)r0 * a.cols;
+    const uint16_t *sc_src = a.scales + (uint64_t)r0 * blocks;
+    const uint32_t w_row = row_on * a.cols + 16u * kg, w_row_odd = w_row - ((blocks & 1u) && kg >= 2u ? 32u : 0u), sc_row = row_on * blocks;
+    float *s_unit = (float *)(s_mem + (pairs + 1u) * Q8ONE_PAIR);
+
+    // A compute unit's loads come back in the order in which its wavefronts ask for them. x (and the weights of its norm) is
+    // waited for first, so every wavefront asks for its part before any asks for codes; then the scales, the codes, what is
+    // added and prepared at the end. Nothing is waited for before all of it is asked for.
+    float x[8], nw[8];
+    uint4 x16;
+    auto load = [&](uint32_t chunk, const float *src, float (&into)[8]) {
         const float4 u = *(const float4 *)(src + 8u * chunk), v = *(const float4 *)(src + 8u * chunk + 4u);
-        to[0] = u.x, to[1] = u.y, to[2] = u.z, to[3] = u.w, to[4] = v.x, to[5] = v.y, to[6] = v.z, to[7] = v.w;
+        into[0] = u.x, into[1] = u.y, into[2] = u.z, into[3] = u.w, into[4] = v.x, into[5] = v.y, into[6] = v.z, into[7] = v.w;
     };
     const bool normed = !BF16 && a.norm_w != nullptr; // uniform
-    if (mine < chunks) {
-        if constexpr (BF16) {
-            x16 = *(const uint4 *)(a.x_hi + 8u * mine);
-        } else {
-            load(mine, a.x, x);
-            if (normed) load(mine, a.norm_w, nw);
-        }
-    }
-    m.ask_scales();
-    float bias = 0.0f, held = 0.0f;
-    if (writes && a.bias) bias = a.bias[out_row];
-    if (writes && a.accumulate) held = a.y[out_row];
-    if (writes && a.residual) held = a.residual[out_row]; // (never with accumulate)
-    Q8Prepared ready;
-    if constexpr (PREPARE) {
-        if (writes) ready.ask(*prepare, which, 0, out_row);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    m.ask_codes(m.from); // after what is waited for first: loads come back in order
-    __builtin_amdgcn_sched_barrier(0);
-    m.stage_scales();
+    const uint32_t own = mine < chunks ? mine : chunks - 1u;
     if constexpr (BF16) {
-        if (mine < chunks) s_x[mine] = x16;
-        for (uint32_t c = mine + T; c < chunks; c += T) s_x[c] = *(const uint4 *)(a.x_hi + 8u * c);
+        x16 = *(const uint4 *)(a.x_hi + 8u * own);
     } else {
-        float scale = 0.0f;
-        if (normed) {
-            float ss = 0.0f;
+        load(own, a.x, x);
+        load(own, normed ? a.norm_w : a.x, nw);
+    }
+    uint16_t sc[U];
+    uint4 w[2 * U];
+    auto ask = [&](uint32_t base) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss += x[e] * x[e]; // zeros past the last chunk
-            for (uint32_t c = mine + T; c < chunks; c += T) {
-                float more[8];
-                load(c, a.x, more);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ss += more[e] * more[e];
-            }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-            if (m.lane == 0) s_norm[m.wave] = ss;
-            __syncthreads();
-            float total = 0.0f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) total += s_norm[w];
-            scale = 1.0f / sqrtf(total / (float)a.cols + a.eps);
+        for (int u = 0; u < U; ++u) {
+            const uint32_t block = 2u * base + 4u * u + kg;
+            sc[u] = sc_src[sc_row + (block < blocks ? block : blocks - 1u)];
         }
-        for (uint32_t c = mine; c < chunks; c += T) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u == 0 || base + 2u * u < to) { // uniform; (nothing is put in place of what is not loaded: a value merged after a branch is copied, and waits)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) { // a pair past the run: its last again, with a scale of zero
+                    const uint32_t at = base + 2u * u + h, pair = at < to ? at : to ? to - 1u : 0u;
+                    w[2 * u + h] = *(const uint4 *)(w_src + ((pair == pairs - 1u ? w_row_odd : w_row) + 64u * pair)); // a last pair of one block: the block again
+                }
+            }
+        }
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier(); // (waits for no memory)
+    __builtin_amdgcn_sched_barrier(0);
+    ask(from);
+    const float *any = (const float *)a.codes;
+    const float bias = *(a.bias ? a.bias + out_row : any);
+    const float held = *(a.accumulate ? a.y + out_row : a.residual ? a.residual + out_row : any); // (never both)
+    Q8Prepared ready;
+    if constexpr (PREPARE) ready.ask<true>(*prepare, which, 0, out_row, any);
+    __builtin_amdgcn_sched_barrier(0);
+
+    for (uint32_t i = mine; i < 512u; i += T) s_zero[i] = 0u;
+    float scale = 1.0f;
+    if (normed) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+        if (mine >= chunks) ss = 0.0f;
+        for (uint32_t c = mine + T; c < chunks; c += T) {
+            float more[8];
+            load(c, a.x, more);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += more[e] * more[e];
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) s_norm[wave] = ss;
+        __syncthreads();
+        float total = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) total += s_norm[i];
+        scale = 1.0f / sqrtf(total / (float)a.cols + a.eps);
+    }
+    for (uint32_t c = mine; c < chunks; c += T) { // (four chunks to a block, T and the chunks multiples of four: quads of lanes stay together)
+        if constexpr (BF16) {
+            if (c != mine) x16 = *(const uint4 *)(a.x_hi + 8u * c);
+            const uint32_t half[4] = {x16.x, x16.y, x16.z, x16.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[2 * e] = __uint_as_float(half[e] << 16), x[2 * e + 1] = __uint_as_float(half[e] & 0xffff0000u);
+        } else {
             if (c != mine) {
                 load(c, a.x, x);
                 if (normed) load(c, a.norm_w, nw);
@@ -435,47 +533,68 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
 #pragma unroll
                 for (int e = 0; e < 8; ++e) x[e] = x[e] * scale * nw[e];
             }
-            bf16x8 hi, lo;
-            q8_split8(x, hi, lo);
-            s_x[c] = __builtin_bit_cast(uint4, hi);
-            s_x[chunks + c] = __builtin_bit_cast(uint4, lo);
         }
+        Q8Whole whole;
+        whole.make(x);
+        char *put = s_mem + (c >> 3) * Q8ONE_PAIR + (c & 7u) * 8u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) *(uint2 *)(put + 64u * k) = whole.plane[k];
+        if ((c & 3u) == 0) s_unit[c >> 2] = whole.unit;
     }
+    if constexpr (PREPARE) ready.place<true>(*prepare, which, 0, out_row);
     __syncthreads();
-    const uint4 *x_at = s_x + q8_mid_chunk(m.kg) + (!BF16 && (m.j & 1u) ? chunks : 0u);
-    float y[2] = {0.0f, 0.0f};
-    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t base = m.from; base < m.to; base += U) {
-        if (base != m.from) m.ask_codes(base);
+
+    float y = 0.0f;
+    const i32x4 zero = {0, 0, 0, 0};
+    const bool block_mine = ((j >> 2) & 1u) == (kg >> 1);
+    for (uint32_t base = from; base < to; base += 2u * U) {
+        if (base != from) ask(base);
+        const char *planes = s_mem + base * Q8ONE_PAIR + (j & 3u) * 64u + 16u * kg;
+        const char *first = block_mine && j < 8u ? planes : (const char *)s_zero;
+        const char *second = block_mine && j >= 8u ? planes + Q8ONE_PAIR : (const char *)s_zero;
+        i32x4 p[2 * U];
+        float unit[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (base + u < m.to) {
-                bf16x8 b[2];
-                float sc[2];
-                m.operands(u, base + u, b, sc);
+            if (u == 0 || base + 2u * u < to) {
+                p[2 * u] = *(const i32x4 *)(first + 2u * u * Q8ONE_PAIR);
+                p[2 * u + 1] = *(const i32x4 *)(second + 2u * u * Q8ONE_PAIR);
+                unit[u] = s_unit[2u * base + 4u * u + kg];
+            }
+        }
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const uint32_t block = 2u * (base + u) + h;
-                    if (h == 0 || block < m.blocks) { // uniform
-                        const floatx4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(x_at[4u * block]), b[h], zero4, 0, 0, 0);
-                        y[0] = __builtin_fmaf(sc[h], acc[0], y[0]);
-                        if constexpr (!BF16) y[1] = __builtin_fmaf(sc[h], acc[1], y[1]);
-                    }
-                }
+        for (int u = 0; u < U; ++u) {
+            if (u == 0 || base + 2u * u < to) {
+                i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(p[2 * u], __builtin_bit_cast(i32x4, w[2 * u]), zero, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(p[2 * u + 1], __builtin_bit_cast(i32x4, w[2 * u + 1]), acc, 0, 0, 0);
+                float sum = __builtin_fmaf((float)acc[3], 256.0f, (float)acc[2]);
+                sum = __builtin_fmaf(sum, 256.0f, (float)acc[1]);
+                sum = __builtin_fmaf(sum, 256.0f, (float)acc[0]);
+                const uint32_t block = 2u * base + 4u * u + kg;
+                const float next = __builtin_fmaf(sum * f16_bits_to_f32(sc[u]), unit[u], y);
+                y = block < 2u * to && block < blocks ? next : y;
             }
         }
     }
-    if (m.lane < 16u) s_red[m.wave][m.lane] = y[0] + y[1];
+    s_red[wave][lane] = y;
     __syncthreads();
-    if (!writes) return;
+    if (wave != 0) return;
     float sum = 0.0f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) sum += s_red[w][mine];
+    for (int i = 0; i < NW; ++i) sum += s_red[i][lane];
+    const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+    sum = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
+    const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+    sum = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
     if (a.bias) sum = sum + bias;
     if (a.accumulate) sum = held + sum;
+    if (lane >= 16u || !row_mine) return;
     a.y[out_row] = sum;
     if (a.residual) a.residual[out_row] = held + sum;
-    if constexpr (PREPARE) ready.store(*prepare, which, out_row, sum, __shfl_xor(sum, 8, 64));
+    if constexpr (PREPARE) {
+        const float there = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sum), 0x128, 0xf, 0xf, true)); // row_ror:8, 32 rows away
+        ready.store(*prepare, which, out_row, sum, there);
+    }
 }
 
 #define Q8_FEW(name, body, what, nw) \

@@ -547,3 +547,31 @@ def test_positions_normalised_by_the_product_itself(gpu, rows, cols, n):
     want = (xd / np.sqrt((xd * xd).mean(axis=1, keepdims=True) + 1e-5) * w) @ elements.T
     got = _product(gpu, codes, bits, x, rows, cols, n, w)
     assert np.abs(got - want).max() / np.abs(want).max() < 1e-5
+
+
+@pytest.mark.parametrize("rows,cols,bf16", [(1, 32, False), (37, 96, False), (130, 4128, False), (2880, 4096, False), (5120, 2880, False), (8200, 64, False),
+                                            (33, 12288, False), (9, 32, True), (2880, 4096, True), (3600, 160, True), (40, 24576, True)])
+def test_one_position_in_whole_numbers(gpu, rows, cols, bf16):
+    """lng_q8_one takes a block of x as 30-bit whole numbers of a unit of its own: tiles of 8 to 16 rows and their remainders,
+    one block, an odd number of blocks, several turns, values of a block far apart, blocks from the smallest normal numbers to
+    2^60. Every sum is exact within a block; per output at most 6 roundings of a block's value, blocks / 32 + 1 of a lane's sum and
+    10 of the lanes' and wavefronts', each 2^-24 of the terms, and 2^-30 of a block's largest x for each x. A value that is not
+    finite makes its block, and the outputs, NaN."""
+    from tests.helpers import from_bf16_bits, to_bf16_bits
+    codes, bits, elements = q8_test_matrix(rows, cols, 90 + rows)
+    blocks = cols // 32
+    rng = np.random.default_rng(rows + cols)
+    for spread, units in ((0, np.zeros(blocks)), (24, rng.integers(-126, 60, blocks))):
+        x = xorshift_values(31, cols).reshape(blocks, 32) * np.exp2(-rng.integers(0, spread + 1, (blocks, 32))) * np.exp2(units)[:, None]
+        xin = to_bf16_bits(x.astype(np.float32).reshape(1, cols)) if bf16 else x.astype(np.float32).reshape(1, cols)
+        exact = (from_bf16_bits(xin) if bf16 else xin).astype(np.float64)
+        outs = [_product(gpu, codes, bits, xin, rows, cols, 1)]
+        want = exact @ elements.T
+        terms = np.abs(exact) @ np.abs(elements).T
+        largest = np.abs(exact).reshape(blocks, 32).max(1) @ np.abs(elements).reshape(rows, blocks, 32).sum(2).T
+        bound = (17 + blocks / 32) * 2.0**-24 * terms[0] + 2.0**-30 * largest + (blocks + 32) * 2.0**-140  # (the last: f32's own end)
+        assert (np.abs(outs[0][0] - want[0]) <= bound).all()
+    for bad in (np.inf, np.nan):
+        x = xorshift_values(32, cols).astype(np.float32).reshape(1, cols)
+        x[0, cols - 5] = bad
+        assert np.isnan(_product(gpu, codes, bits, to_bf16_bits(x) if bf16 else x, rows, cols, 1)).all()
