@@ -126,7 +126,7 @@ struct lng_gpu {
     hipModule_t module = nullptr;
     // kernels of the embedded code object
     hipFunction_t generic_f32 = nullptr, generic_bf16 = nullptr;
-    hipFunction_t decode_bf16_d64 = nullptr, decode_bf16_d64_o4 = nullptr, decode_bf16_d64_w8 = nullptr, decode_f32_d64 = nullptr, decode_f32_d64_w8 = nullptr, decode_merge = nullptr, decode_merge_few = nullptr;
+    hipFunction_t decode_bf16_d64 = nullptr, decode_bf16_d64_o4 = nullptr, decode_f32_d64 = nullptr, decode_merge = nullptr, decode_merge_few = nullptr;
     hipFunction_t decode_bf16_wide[3] = {}, decode_f32_wide[3] = {}; // head widths 128, 256, 512
     hipFunction_t prefill_bf16_d64 = nullptr, prefill_bf16_d64_h1 = nullptr, prefill_bf16_d64_h1w = nullptr, prefill_bf16_d64_stream = nullptr, prefill_bf16_d64_pair = nullptr, prefill_f32_d64 = nullptr, prefill_f32_d64_w4 = nullptr, prefill_merge = nullptr;
     hipFunction_t prefill_bf16_wide[3] = {}, prefill_f32_wide[3] = {}; // head widths 128, 256, 512
@@ -596,38 +596,11 @@ DecodePlan plan_decode(lng_gpu *g, const lng_k_row *rows, size_t n, uint64_t t_u
 struct RowsPlan {
     enum Kind { Generic, Bf16, F32 } kind = Generic;
     int wide = -1;               // -1: head width 64; 0, 1, 2: the kernels for widths 128, 256, 512
-    unsigned waves = 4;          // wavefronts of a workgroup, each with a tile of 32 positions at a time
     DecodePlan chunks;
     bool fused = false;          // split-K merged inside the decode kernel (tickets) instead of by lng_decode_merge
     size_t partial_slots = 0;    // (row, kv head, chunk, query head of the group) slots of split-K partials; 0: none
     size_t pairs = 0;            // rows x kv heads
 };
-
-// Rows that see up to 512 positions, no more (row, kv head) pairs than compute units: a workgroup of eight wavefronts takes such a
-// row whole, twice the tiles at a time (bf16, us: 160 positions 1, 16, 30 sequences 5.3, 6.7, 7.2 -> 4.7, 6.0, 6.5; 300 6.7, 8.4,
-// 10.2 -> 6.2, 7.4, 9.0; 500 8.1, 11.6, 13.1 -> 7.5, 10.7, 12.3; sixteen wavefronts up to 1,024 gain nothing over chunks). f32, whose
-// tiles take twice the bytes and eight times the matrix instructions: 160 positions 7.3, 9.0, 10.9 -> 6.7, 8.0, 9.8; past 256 a
-// few rows are better off in chunks of 128 with a merge (300 and 500 positions, 1 sequence 10.1, 13.9 -> 9.0, 9.1, whole on eight
-// wavefronts 9.3, 11.8; 16 sequences 13.0, 17.0 whole, 14.1, 16.0 in chunks; 30 14.4, 19.4 and 21, 25).
-void short_rows(const lng_gpu *g, const lng_k_row *rows, size_t n, uint64_t t_uniform, RowsPlan *p) {
-    if (p->pairs > g->cus) return;
-    uint64_t longest = 0;
-    for (size_t i = 0; i < n && !t_uniform; ++i) longest = std::max(longest, visible_from_tile(rows[i]));
-    for (uint64_t i = 0; i < t_uniform; ++i) { // (no more than pairs)
-        lng_k_row r = rows[0];
-        r.start += i;
-        longest = std::max(longest, visible_from_tile(r));
-    }
-    if (longest > 512) return;
-    if (p->kind == RowsPlan::F32 && longest > 256 && 4 * p->pairs <= g->cus) {
-        p->chunks.chunk = 128;
-        p->chunks.n_chunks = (uint32_t)((longest + 127) / 128);
-    } else {
-        p->waves = 8;
-        p->chunks.chunk = (uint32_t)((longest + 127) / 128 * 128);
-        p->chunks.n_chunks = 1;
-    }
-}
 
 RowsPlan plan_rows(lng_gpu *g, const lng_k_attn &a, const lng_k_row *host_rows, size_t n_rows, uint64_t t_uniform,
                    bool aligned16) {
@@ -649,7 +622,6 @@ RowsPlan plan_rows(lng_gpu *g, const lng_k_attn &a, const lng_k_row *host_rows, 
     p.kind = fast ? RowsPlan::Bf16 : RowsPlan::F32;
     p.wide = wide;
     p.chunks = plan_decode(g, host_rows, n_rows, t_uniform, a.kv_heads, fast ? 1u : 2u, a.dim / 64);
-    if (wide < 0) short_rows(g, host_rows, n_rows, t_uniform, &p);
     if (p.chunks.n_chunks > 1) {
         p.partial_slots = p.pairs * (size_t)p.chunks.n_chunks * group;
         // Small grids merge inside the kernel; large ones with a second dispatch (the f32 and wide-head kernels always).
@@ -668,7 +640,6 @@ struct RowsLaunches {
         unsigned grid;
         lng_k_attn args;
         unsigned grid_y = 1;
-        unsigned block = 256;
     } l[2];
 };
 
@@ -712,13 +683,9 @@ int rows_launches(lng_gpu *g, lng_k_attn a, const RowsPlan &p, const lng_k_row *
                             p.kind == RowsPlan::Bf16 ? wide_bf16[p.wide] : wide_f32[p.wide], (unsigned)wgs, a};
     } else {
         // (many workgroups of short chunks - a table of sequences: the build of the bf16 kernel with four wavefronts per SIMD)
-        const bool o4 = p.waves == 4 && a.chunk < 2048u && wgs > 3ull * g->cus && !g->knobs.decode_o3;
-        RowsLaunches::One &one = out->l[out->n++];
-        if (p.kind == RowsPlan::F32) one = p.waves == 8 ? RowsLaunches::One{g->decode_f32_d64_w8, "lng_decode_f32_d64_w8", (unsigned)wgs, a} : RowsLaunches::One{g->decode_f32_d64, "lng_decode_f32_d64", (unsigned)wgs, a};
-        else if (p.waves == 8) one = {g->decode_bf16_d64_w8, "lng_decode_bf16_d64_w8", (unsigned)wgs, a};
-        else if (o4) one = {g->decode_bf16_d64_o4, "lng_decode_bf16_d64_o4", (unsigned)wgs, a};
-        else one = {g->decode_bf16_d64, "lng_decode_bf16_d64", (unsigned)wgs, a};
-        one.block = 64 * p.waves;
+        const bool o4 = p.kind == RowsPlan::Bf16 && a.chunk < 2048u && wgs > 3ull * g->cus && !g->knobs.decode_o3;
+        out->l[out->n++] = {p.kind == RowsPlan::Bf16 ? (o4 ? g->decode_bf16_d64_o4 : g->decode_bf16_d64) : g->decode_f32_d64,
+                            p.kind == RowsPlan::Bf16 ? (o4 ? "lng_decode_bf16_d64_o4" : "lng_decode_bf16_d64") : "lng_decode_f32_d64", (unsigned)wgs, a};
     }
     if (a.n_chunks > 1 && !a.fused) {
         if (a.n_chunks <= 32 && !g->knobs.merge_wide) { // a wavefront per (row, kv head, query head), four to a workgroup (LNG_MERGE_FEW)
@@ -759,7 +726,7 @@ int record_rows(lng_batch *b, lng_k_attn a, const lng_k_row *host_rows, size_t n
         c.name = launches.l[i].name;
         c.grid[0] = launches.l[i].grid;
         c.grid[1] = launches.l[i].grid_y;
-        c.block = launches.l[i].block;
+        c.block = 256;
         set_args(c, launches.l[i].args);
         b->cmds.push_back(std::move(c));
     }
@@ -1227,11 +1194,9 @@ extern "C" int lng_hip_open(int device, lng_gpu **out) {
         {"lng_attn_generic_bf16", &g->generic_bf16, true},
         {"lng_decode_bf16_d64", &g->decode_bf16_d64, true},
         {"lng_decode_bf16_d64_o4", &g->decode_bf16_d64_o4, true},
-        {"lng_decode_bf16_d64_w8", &g->decode_bf16_d64_w8, true},
         {"lng_decode_merge", &g->decode_merge, true},
         {"lng_decode_merge_few", &g->decode_merge_few, true},
         {"lng_decode_f32_d64", &g->decode_f32_d64, true},
-        {"lng_decode_f32_d64_w8", &g->decode_f32_d64_w8, true},
         {"lng_decode_bf16_w128", &g->decode_bf16_wide[0], true},
         {"lng_decode_bf16_w256", &g->decode_bf16_wide[1], true},
         {"lng_decode_bf16_w512", &g->decode_bf16_wide[2], true},
@@ -1724,7 +1689,7 @@ extern "C" int lng_hip_attention_grouped_static(lng_gpu *g, void *stream, const 
         size_t size = sizeof(lng_k_attn);
         void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, &launches.l[i].args, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
                           HIP_LAUNCH_PARAM_END};
-        const hipError_t e = hipModuleLaunchKernel(launches.l[i].fn, launches.l[i].grid, launches.l[i].grid_y, 1, launches.l[i].block, 1, 1, 0, (hipStream_t)stream, nullptr, config);
+        const hipError_t e = hipModuleLaunchKernel(launches.l[i].fn, launches.l[i].grid, launches.l[i].grid_y, 1, 256, 1, 1, 0, (hipStream_t)stream, nullptr, config);
         if (e != hipSuccess) rc = fail(LNG_ERR_GPU, "%s did not launch: %s", launches.l[i].name, hip_text(e));
     }
     if (before != g->device) hipSetDevice(before);

@@ -258,9 +258,9 @@ extern "C" __global__ __launch_bounds__(256) void lng_attn_generic_bf16(lng_k_at
 // Decode kernel, bf16, head width 64, up to 16 query heads per kv head.
 //
 // Grid: one workgroup per (row, kv head, chunk), see work_of; a row of v visible positions has
-// ceil(v / a.chunk) chunks, and chunk c of n is the groups of 128 positions (32 a wavefront) c, c + n, c + 2n, ... of the
+// ceil(v / a.chunk) chunks, and chunk c of n is the groups of 128 positions c, c + n, c + 2n, ... of the
 // row. A workgroup serves ALL query heads of its kv head at once, so each cached K and V row is read
-// from HBM once per group instead of once per query head. Its four (or eight) wavefronts take a tile of 32
+// from HBM once per group instead of once per query head. Its four wavefronts take a tile of 32
 // positions of each group. Everything is lane-local between the three MFMA stages:
 //
 //   S^T[tok][head] = K[tok][:] . Q[head][:]        2x2 v_mfma_f32_16x16x32_bf16 per tile
@@ -309,7 +309,7 @@ template <bool COHERENT> __device__ __forceinline__ float load_partial(const flo
     return *p;
 }
 
-template <bool COHERENT, uint32_t THREADS = 256u>
+template <bool COHERENT>
 __device__ __forceinline__ void merge_chunks(const lng_k_attn &a, const lng_k_row &it, uint32_t pair, uint32_t g,
                                              uint32_t group, uint32_t row_chunks) {
     __shared__ float s_w[16][LNG_MAX_CHUNKS];
@@ -344,7 +344,7 @@ __device__ __forceinline__ void merge_chunks(const lng_k_attn &a, const lng_k_ro
         }
     }
     __syncthreads();
-    for (uint32_t idx = threadIdx.x; idx < group * 64u; idx += THREADS) {
+    for (uint32_t idx = threadIdx.x; idx < group * 64u; idx += 256u) {
         const uint32_t h = idx >> 6;
         const uint32_t d = idx & 63u;
         const float *po = a.partial_o + (((uint64_t)pair * a.n_chunks) * group + h) * 64u + d;
@@ -390,10 +390,10 @@ struct kv_tile {
     uint4 v[2][2];
 };
 
-template <uint32_t NW> __device__ __forceinline__ void decode_bf16_d64_body(const lng_k_attn a) {
-    __shared__ float s_m[NW][16];
-    __shared__ float s_l[NW][16];
-    __shared__ float s_o[NW][16][65];
+__device__ __forceinline__ void decode_bf16_d64_body(const lng_k_attn a) {
+    __shared__ float s_m[4][16];
+    __shared__ float s_l[4][16];
+    __shared__ float s_o[4][16][65];
 
     const work_item wi = work_of(a);
     const uint32_t row = wi.pair / a.kv_heads;
@@ -407,9 +407,9 @@ template <uint32_t NW> __device__ __forceinline__ void decode_bf16_d64_body(cons
     // The row's workgroups take interleaved groups of 128 positions (workgroup c: groups c, c + chunks, ...), not
     // a run of a.chunk positions each: together they sweep one window of the row, and every workgroup of a row
     // has the same number of groups to within one, however the row's length divides.
-    const uint64_t c0 = base + (uint64_t)wi.chunk * (32u * NW);
+    const uint64_t c0 = base + (uint64_t)wi.chunk * 128u;
     const uint64_t c1 = last + 1;
-    const uint64_t tile_stride = 32ull * NW * row_chunks;
+    const uint64_t tile_stride = 128ull * row_chunks;
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
@@ -519,7 +519,7 @@ template <uint32_t NW> __device__ __forceinline__ void decode_bf16_d64_body(cons
         cur = nxt;
     }
 
-    // ---- merge the wavefronts ---------------------------------------------------------
+    // ---- merge the four wavefronts ---------------------------------------------------------
     {
         float lt = l + __shfl_xor(l, 16, 64);
         lt += __shfl_xor(lt, 32, 64);
@@ -534,15 +534,15 @@ template <uint32_t NW> __device__ __forceinline__ void decode_bf16_d64_body(cons
         }
     }
     __syncthreads();
-    for (uint32_t idx = threadIdx.x; idx < group * 64u; idx += 64u * NW) {
+    for (uint32_t idx = threadIdx.x; idx < group * 64u; idx += 256u) {
         const uint32_t h = idx >> 6;
         const uint32_t d = idx & 63u;
         float top = LNG_NEG_INF;
 #pragma unroll
-        for (uint32_t w = 0; w < NW; ++w) top = fmaxf(top, s_m[w][h]);
+        for (int w = 0; w < 4; ++w) top = fmaxf(top, s_m[w][h]);
         float sum = 0.0f, o = 0.0f;
 #pragma unroll
-        for (uint32_t w = 0; w < NW; ++w) {
+        for (int w = 0; w < 4; ++w) {
             const float wt = s_m[w][h] == LNG_NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][h] - top);
             sum += s_l[w][h] * wt;
             o += s_o[w][h][d] * wt;
@@ -599,17 +599,15 @@ template <uint32_t NW> __device__ __forceinline__ void decode_bf16_d64_body(cons
     asm volatile("" ::: "memory");
     if (threadIdx.x == 0) __hip_atomic_store(&a.tickets[wi.pair], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-    merge_chunks<true, 64u * NW>(a, it, wi.pair, g, group, row_chunks);
+    merge_chunks<true>(a, it, wi.pair, g, group, row_chunks);
 }
 
-// Three builds of the same body: 130 registers and three wavefronts per SIMD for long chunks (what a long context
+// Two builds of the same body: 130 registers and three wavefronts per SIMD for long chunks (what a long context
 // streams best with), 125 registers and four for dispatches of many workgroups with chunks under 2,048 positions
 // (a table of sequences), where workgroups are short-lived and a fourth one per compute unit hides more of their
-// start-up (32 sequences 65 -> 62 us, 128 sequences 243 -> 236 us; on 4,096-position chunks it is 1.7 % slower). _w8: eight
-// wavefronts for rows taken whole (the host's short_rows says what it gives).
-extern "C" __global__ __launch_bounds__(256, 2) void lng_decode_bf16_d64(lng_k_attn a) { decode_bf16_d64_body<4>(a); }
-extern "C" __global__ __launch_bounds__(256, 4) void lng_decode_bf16_d64_o4(lng_k_attn a) { decode_bf16_d64_body<4>(a); }
-extern "C" __global__ __launch_bounds__(512, 4) void lng_decode_bf16_d64_w8(lng_k_attn a) { decode_bf16_d64_body<8>(a); }
+// start-up (32 sequences 65 -> 62 us, 128 sequences 243 -> 236 us; on 4,096-position chunks it is 1.7 % slower).
+extern "C" __global__ __launch_bounds__(256, 2) void lng_decode_bf16_d64(lng_k_attn a) { decode_bf16_d64_body(a); }
+extern "C" __global__ __launch_bounds__(256, 4) void lng_decode_bf16_d64_o4(lng_k_attn a) { decode_bf16_d64_body(a); }
 
 // =============================================================================================
 // Decode kernel, f32 (the reference's own element type), head width 64, up to 16 query heads per
@@ -633,10 +631,10 @@ struct kv_tile_f32 {
     float v[2][16];  // [position half][4 * i + mm]: position 4j + i, dim 16mm + n
 };
 
-template <uint32_t NW> __device__ __forceinline__ void decode_f32_d64_body(const lng_k_attn a) {
-    __shared__ float s_m[NW][16];
-    __shared__ float s_l[NW][16];
-    __shared__ float s_o[NW][16][65];
+extern "C" __global__ __launch_bounds__(256, 2) void lng_decode_f32_d64(lng_k_attn a) {
+    __shared__ float s_m[4][16];
+    __shared__ float s_l[4][16];
+    __shared__ float s_o[4][16][65];
 
     const work_item wi = work_of(a);
     const uint32_t row = wi.pair / a.kv_heads;
@@ -650,9 +648,9 @@ template <uint32_t NW> __device__ __forceinline__ void decode_f32_d64_body(const
     if (wi.chunk >= row_chunks) return; // this row has fewer chunks than the longest one
     // interleaved groups of 128 positions, as in the bf16 kernel; the host keeps last below 2^32 - 65,536, so
     // neither last + 1 nor a position plus the stride (at most 256 chunks x 128) leaves 32 bits
-    const uint32_t c0 = base + wi.chunk * (32u * NW);
+    const uint32_t c0 = base + wi.chunk * 128u;
     const uint32_t c1 = last + 1u;
-    const uint32_t tile_stride = 32u * NW * row_chunks;
+    const uint32_t tile_stride = 128u * row_chunks;
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -715,16 +713,16 @@ template <uint32_t NW> __device__ __forceinline__ void decode_f32_d64_body(const
     for (; tp < c1; tp += tile_stride) {
         if (c1 - tp > tile_stride) load_tile(tp + tile_stride, nxt);
 
-        floatx4 st[2]; // (two chains of dependent products, in turn)
-        st[0] = st[1] = (floatx4){0.f, 0.f, 0.f, 0.f};
+        floatx4 st[2];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const floatx4 q = {qv[s].x, qv[s].y, qv[s].z, qv[s].w};
-            const floatx4 k[2] = {{cur.k[0][s].x, cur.k[0][s].y, cur.k[0][s].z, cur.k[0][s].w}, {cur.k[1][s].x, cur.k[1][s].y, cur.k[1][s].z, cur.k[1][s].w}};
+        for (int half = 0; half < 2; ++half) {
+            st[half] = (floatx4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-#pragma unroll
-                for (int half = 0; half < 2; ++half) st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[half][e], q[e], st[half], 0, 0, 0);
+            for (int s = 0; s < 4; ++s) {
+                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].x, qv[s].x, st[half], 0, 0, 0);
+                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].y, qv[s].y, st[half], 0, 0, 0);
+                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].z, qv[s].z, st[half], 0, 0, 0);
+                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].w, qv[s].w, st[half], 0, 0, 0);
             }
         }
         float tmax = LNG_NEG_INF;
@@ -758,19 +756,20 @@ template <uint32_t NW> __device__ __forceinline__ void decode_f32_d64_body(const
         l = l * alpha + psum;
         m = m_new;
 #pragma unroll
-        for (int mm = 0; mm < 4; ++mm) ot[mm] = ot[mm] * alpha;
+        for (int mm = 0; mm < 4; ++mm) {
+            ot[mm] = ot[mm] * alpha;
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
+            for (int half = 0; half < 2; ++half) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-#pragma unroll
-                for (int mm = 0; mm < 4; ++mm) ot[mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.v[half][4 * i + mm], st[half][i], ot[mm], 0, 0, 0);
+                for (int i = 0; i < 4; ++i) {
+                    ot[mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.v[half][4 * i + mm], st[half][i], ot[mm], 0, 0, 0);
+                }
             }
         }
         cur = nxt;
     }
 
-    // ---- merge the wavefronts ---------------------------------------------------------
+    // ---- merge the four wavefronts ---------------------------------------------------------
     {
         float lt = l + __shfl_xor(l, 16, 64);
         lt += __shfl_xor(lt, 32, 64);
@@ -785,15 +784,15 @@ template <uint32_t NW> __device__ __forceinline__ void decode_f32_d64_body(const
         }
     }
     __syncthreads();
-    for (uint32_t idx = threadIdx.x; idx < group * 64u; idx += 64u * NW) {
+    for (uint32_t idx = threadIdx.x; idx < group * 64u; idx += 256u) {
         const uint32_t h = idx >> 6;
         const uint32_t d = idx & 63u;
         float top = LNG_NEG_INF;
 #pragma unroll
-        for (uint32_t w = 0; w < NW; ++w) top = fmaxf(top, s_m[w][h]);
+        for (int w = 0; w < 4; ++w) top = fmaxf(top, s_m[w][h]);
         float sum = 0.0f, o = 0.0f;
 #pragma unroll
-        for (uint32_t w = 0; w < NW; ++w) {
+        for (int w = 0; w < 4; ++w) {
             const float wt = s_m[w][h] == LNG_NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][h] - top);
             sum += s_l[w][h] * wt;
             o += s_o[w][h][d] * wt;
@@ -817,9 +816,6 @@ template <uint32_t NW> __device__ __forceinline__ void decode_f32_d64_body(const
         }
     }
 }
-
-extern "C" __global__ __launch_bounds__(256, 2) void lng_decode_f32_d64(lng_k_attn a) { decode_f32_d64_body<4>(a); }
-extern "C" __global__ __launch_bounds__(512, 2) void lng_decode_f32_d64_w8(lng_k_attn a) { decode_f32_d64_body<8>(a); }
 
 // =============================================================================================
 // Decode kernels for head widths 128, 256 and 512 (DS slices of 64 dimensions): the plan of the two

@@ -731,37 +731,6 @@ def test_decode_f32_at_head_width_64(gpu, t, start, window, slots, heads, kv_hea
         assert rel_error(generic, want) <= F32_RTOL
 
 
-@pytest.mark.parametrize("dtype", [C.BF16, C.F32])
-@pytest.mark.parametrize("t,start,window,slots,heads,kv_heads", [
-    (1, 0, FULL, 1, 64, 8), (1, 255, FULL, 256, 64, 8), (1, 256, FULL, 257, 64, 8), (1, 511, FULL, 512, 64, 8), (1, 512, FULL, 513, 64, 8),
-    (1, 5000, 128, 129, 64, 8), (1, 1003, 300, 311, 16, 2), (1, 900, 480, 500, 32, 2), (3, 253, FULL, 256, 12, 4), (31, 224, 200, 231, 5, 1),
-    (7, 490, FULL, 497, 64, 32), (9, 490, FULL, 499, 64, 32)])
-def test_short_rows_are_taken_whole_by_eight_wavefronts(gpu, dtype, t, start, window, slots, heads, kv_heads):
-    """Rows of up to 512 positions at the edges of tiles and of the eight wavefronts' 256 positions, one more than 512, f32 rows
-    past 256 of few sequences (chunks and a merge) and of many (whole), more rows and kv heads than compute units (four wavefronts),
-    rings that wrap; against the CPU reference."""
-    end = start + t
-    rng = np.random.default_rng(start + t)
-    q = (rng.standard_normal((t, heads, 64)) * 0.7).astype(np.float32)
-    k = (rng.standard_normal((end, kv_heads, 64)) * 0.7).astype(np.float32)
-    v = rng.standard_normal((end, kv_heads, 64)).astype(np.float32)
-    sinks = rng.standard_normal(heads).astype(np.float32)
-    if dtype == C.BF16:
-        q, k, v = (from_bf16_bits(to_bf16_bits(x)) for x in (q, k, v))
-    longest = max(i + 1 - ((max(0, i + 1 - window) if window != FULL else 0) & ~31) for i in range(start, end))
-    whole = longest <= 512 and t * kv_heads <= 256 and (dtype == C.BF16 or longest <= 256 or 4 * t * kv_heads > 256)
-    kernel = ("lng_decode_bf16_d64" if dtype == C.BF16 else "lng_decode_f32_d64") + ("_w8" if whole else "")
-    kr, vr = ring_layout(k, t, start, slots, False), ring_layout(v, t, start, slots, False)
-    shape = C.GroupedShape(t, start, heads, kv_heads, 64, window, slots, 0.125)
-    if dtype == C.BF16:
-        want = oracle.attention_bf16(*(to_bf16_bits(x) for x in (q, k, v)), sinks, start, window=window, scale=0.125, threads=THREADS)
-        got = run_attention(gpu, *(to_bf16_bits(x) for x in (q, kr, vr)), sinks, shape, False, dtype, expect_kernel=kernel)
-        assert max_error(from_bf16_bits(got), from_bf16_bits(want)) < BF16_TOL
-    else:
-        want = oracle.attention_f32(q, k, v, sinks, start, window=window, slots=None, scale=0.125, threads=THREADS)
-        assert rel_error(run_attention(gpu, q, kr, vr, sinks, shape, False, dtype, expect_kernel=kernel), want) <= F32_RTOL
-
-
 # ---- prompt passes in f32 (f32 matrix-instruction kernel) -------------------------------------
 @pytest.mark.parametrize("t,start,window,slots,heads,kv_heads,forced", [
     (64, 0, FULL, 64, 64, 8, None), (33, 5, FULL, 64, 64, 8, None), (100, 37, FULL, 160, 16, 2, None), (65, 0, 1, 96, 64, 8, None),
