@@ -420,9 +420,11 @@ struct Q8Whole { // eight columns, a quarter of a block; the other three are in 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 // LDS of q8_one_body: the planes of each pair of blocks (and of one more, that the last turn may read and not use), the units.
 #define Q8ONE_PAIR 256u // bytes
-template <bool BF16, int NW, bool PREPARE = false>
-__device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
-    constexpr int U = 4, T = 64 * NW; // U: twos of pairs in flight, 4,096 columns in one turn of eight wavefronts
+// U: twos of pairs of blocks a wavefront has in flight. 4: 4,096 columns in one turn of eight wavefronts. 1: up to 1,024 columns,
+// where what a workgroup asks for beyond its share costs more than the waits it saves (16,384 x 512 9.7 us with 4, 5.7 with 1).
+template <bool BF16, int NW, bool PREPARE, int U>
+__device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
+    constexpr int T = 64 * NW;
     __shared__ float s_red[NW][64];
     __shared__ float s_norm[NW];
     __shared__ __attribute__((aligned(16))) uint32_t s_zero[512]; // what lanes read that hold rows of the other block or pair
@@ -465,10 +467,13 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
         x16 = *(const uint4 *)(a.x_hi + 8u * own);
     } else {
         load(own, a.x, x);
-        load(own, normed ? a.norm_w : a.x, nw);
+        if (normed) load(own, a.norm_w, nw);
     }
     uint16_t sc[U];
     uint4 w[2 * U];
+    // (Nothing is put in place of what is not loaded: a value merged with another after a branch is copied, and waits. And what
+    // is loaded in every case is what the wait for x can count on being behind it: so the first two pairs, a pair past the run
+    // as the last one again, and all scales.)
     auto ask = [&](uint32_t base) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -477,11 +482,11 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (u == 0 || base + 2u * u < to) { // uniform; (nothing is put in place of what is not loaded: a value merged after a branch is copied, and waits)
+            if (u == 0 || base + 2u * u < to) { // uniform
 #pragma unroll
-                for (int h = 0; h < 2; ++h) { // a pair past the run: its last again, with a scale of zero
+                for (int h = 0; h < 2; ++h) {
                     const uint32_t at = base + 2u * u + h, pair = at < to ? at : to ? to - 1u : 0u;
-                    w[2 * u + h] = *(const uint4 *)(w_src + ((pair == pairs - 1u ? w_row_odd : w_row) + 64u * pair)); // a last pair of one block: the block again
+                    if (U > 1 || h == 0 || at < to) w[2 * u + h] = *(const uint4 *)(w_src + ((pair == pairs - 1u ? w_row_odd : w_row) + 64u * pair)); // a last pair of one block: the block again
                 }
             }
         }
@@ -491,8 +496,15 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
     __builtin_amdgcn_sched_barrier(0);
     ask(from);
     const float *any = (const float *)a.codes;
-    const float bias = *(a.bias ? a.bias + out_row : any);
-    const float held = *(a.accumulate ? a.y + out_row : a.residual ? a.residual + out_row : any); // (never both)
+    float bias, held;
+    if constexpr (U > 1) {
+        bias = *(a.bias ? a.bias + out_row : any);
+        held = *(a.accumulate ? a.y + out_row : a.residual ? a.residual + out_row : any); // (never both)
+    } else {
+        if (a.bias) bias = a.bias[out_row];
+        if (a.accumulate) held = a.y[out_row];
+        if (a.residual) held = a.residual[out_row];
+    }
     Q8Prepared ready;
     if constexpr (PREPARE) ready.ask<true>(*prepare, which, 0, out_row, any);
     __builtin_amdgcn_sched_barrier(0);
@@ -595,6 +607,12 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
         const float there = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sum), 0x128, 0xf, 0xf, true)); // row_ror:8, 32 rows away
         ready.store(*prepare, which, out_row, sum, there);
     }
+}
+
+template <bool BF16, int NW, bool PREPARE = false>
+__device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
+    if (a.cols <= 128u * NW) q8_one_turns<BF16, NW, PREPARE, 1>(a, tile, s_mem, prepare, which);
+    else q8_one_turns<BF16, NW, PREPARE, 4>(a, tile, s_mem, prepare, which);
 }
 
 #define Q8_FEW(name, body, what, nw) \
