@@ -550,7 +550,7 @@ uint64_t visible_from_tile(const lng_k_row &r) { // positions from the tile-alig
 }
 
 DecodePlan plan_decode(lng_gpu *g, const lng_k_row *rows, size_t n, uint64_t t_uniform, uint32_t kv_heads, unsigned wgs_per_cu,
-                       unsigned width = 1 /* head width in units of 64: bytes per position grow with it */) {
+                       unsigned width = 1 /* head width in units of 64: bytes per position grow with it */, bool in_f32 = false /* at head width 64 */) {
     // rows == the table, or one row standing for t_uniform consecutive queries of one cache
     uint64_t total = 0, longest = 0;
     if (t_uniform) {
@@ -586,7 +586,10 @@ DecodePlan plan_decode(lng_gpu *g, const lng_k_row *rows, size_t n, uint64_t t_u
     chunk = std::max<uint64_t>(chunk, ((longest + LNG_MAX_CHUNKS - 1) / LNG_MAX_CHUNKS + 127) / 128 * 128);
     // Short runs (a 128-token window seen from its 32-aligned start is up to 159 positions) stay whole: two
     // chunks would mean partials, arrival counters and a merge for five tiles of work.
-    if (longest <= 512) chunk = std::max<uint64_t>(chunk, (longest + 127) / 128 * 128);
+    // f32, whose tiles take twice the bytes and eight times the matrix instructions, past 256 positions only where the pairs
+    // fill the device: 300 and 500 positions whole and in chunks with a merge, us, 1 sequence 10.1, 13.9 and 9.0, 9.1, 4 sequences
+    // 10.9, 14.4 and 9.5, 9.7, 16 sequences 14.0, 18.8 and 14.1, 16.0, 30 sequences 15.6, 20.8 and 21, 24.5.
+    if (longest <= (in_f32 && 4 * pairs <= g->cus ? 256u : 512u)) chunk = std::max<uint64_t>(chunk, (longest + 127) / 128 * 128);
     p.chunk = (uint32_t)chunk;
     p.n_chunks = (uint32_t)((longest + chunk - 1) / chunk);
     return p;
@@ -621,7 +624,7 @@ RowsPlan plan_rows(lng_gpu *g, const lng_k_attn &a, const lng_k_row *host_rows, 
     if (!fast && !fast_f32) return p;
     p.kind = fast ? RowsPlan::Bf16 : RowsPlan::F32;
     p.wide = wide;
-    p.chunks = plan_decode(g, host_rows, n_rows, t_uniform, a.kv_heads, fast ? 1u : 2u, a.dim / 64);
+    p.chunks = plan_decode(g, host_rows, n_rows, t_uniform, a.kv_heads, fast ? 1u : 2u, a.dim / 64, fast_f32 && wide < 0);
     if (p.chunks.n_chunks > 1) {
         p.partial_slots = p.pairs * (size_t)p.chunks.n_chunks * group;
         // Small grids merge inside the kernel; large ones with a second dispatch (the f32 and wide-head kernels always).
@@ -701,10 +704,15 @@ int rows_launches(lng_gpu *g, lng_k_attn a, const RowsPlan &p, const lng_k_row *
 int record_rows(lng_batch *b, lng_k_attn a, const lng_k_row *host_rows, size_t n_rows, uint64_t t_uniform,
                 bool aligned16) {
     lng_gpu *g = b->gpu;
-    const RowsPlan p = plan_rows(g, a, host_rows, n_rows, t_uniform, aligned16);
+    RowsPlan p = plan_rows(g, a, host_rows, n_rows, t_uniform, aligned16);
     if (p.partial_slots) {
         Scratch sc;
-        if (int rc = reserve_scratch(g, p.partial_slots * a.dim, p.partial_slots * 2, p.pairs, &sc)) return rc;
+        if (int rc = reserve_scratch(g, p.partial_slots * a.dim, p.partial_slots * 2, p.pairs, &sc)) {
+            if (rc != LNG_ERR_ALLOC || p.wide >= 0 || p.chunks.chunk * (uint64_t)p.chunks.n_chunks > 512) return rc;
+            p.chunks = DecodePlan{512, 1}; // no memory for the partials: short rows can do without
+            p.partial_slots = 0;
+            p.fused = false;
+        }
         a.partial_o = sc.o;
         a.partial_ml = sc.ml;
         a.tickets = sc.tickets;

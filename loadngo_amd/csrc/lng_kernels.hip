@@ -713,16 +713,16 @@ extern "C" __global__ __launch_bounds__(256, 2) void lng_decode_f32_d64(lng_k_at
     for (; tp < c1; tp += tile_stride) {
         if (c1 - tp > tile_stride) load_tile(tp + tile_stride, nxt);
 
-        floatx4 st[2];
+        floatx4 st[2]; // (two chains of dependent products, in turn)
+        st[0] = st[1] = (floatx4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            st[half] = (floatx4){0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < 4; ++s) {
+            const floatx4 q = {qv[s].x, qv[s].y, qv[s].z, qv[s].w};
+            const floatx4 k[2] = {{cur.k[0][s].x, cur.k[0][s].y, cur.k[0][s].z, cur.k[0][s].w}, {cur.k[1][s].x, cur.k[1][s].y, cur.k[1][s].z, cur.k[1][s].w}};
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].x, qv[s].x, st[half], 0, 0, 0);
-                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].y, qv[s].y, st[half], 0, 0, 0);
-                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].z, qv[s].z, st[half], 0, 0, 0);
-                st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[half][s].w, qv[s].w, st[half], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int half = 0; half < 2; ++half) st[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[half][e], q[e], st[half], 0, 0, 0);
             }
         }
         float tmax = LNG_NEG_INF;
@@ -756,14 +756,13 @@ extern "C" __global__ __launch_bounds__(256, 2) void lng_decode_f32_d64(lng_k_at
         l = l * alpha + psum;
         m = m_new;
 #pragma unroll
-        for (int mm = 0; mm < 4; ++mm) {
-            ot[mm] = ot[mm] * alpha;
+        for (int mm = 0; mm < 4; ++mm) ot[mm] = ot[mm] * alpha;
 #pragma unroll
-            for (int half = 0; half < 2; ++half) {
+        for (int half = 0; half < 2; ++half) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    ot[mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.v[half][4 * i + mm], st[half][i], ot[mm], 0, 0, 0);
-                }
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int mm = 0; mm < 4; ++mm) ot[mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.v[half][4 * i + mm], st[half][i], ot[mm], 0, 0, 0);
             }
         }
         cur = nxt;

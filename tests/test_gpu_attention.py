@@ -731,6 +731,28 @@ def test_decode_f32_at_head_width_64(gpu, t, start, window, slots, heads, kv_hea
         assert rel_error(generic, want) <= F32_RTOL
 
 
+@pytest.mark.parametrize("t,start,window,slots,heads,kv_heads", [
+    (1, 255, FULL, 256, 64, 8), (1, 256, FULL, 257, 64, 8), (1, 511, FULL, 512, 64, 8), (1, 1003, 300, 311, 16, 2), (3, 253, FULL, 256, 12, 4),
+    (2, 500, FULL, 502, 64, 32), (3, 500, FULL, 503, 64, 32), (8, 280, 270, 288, 64, 8)])
+def test_short_f32_rows_whole_and_in_chunks(gpu, t, start, window, slots, heads, kv_heads):
+    """f32 rows of 256 positions and fewer go whole, longer ones in chunks of 128 with a merge while four times the pairs of rows
+    and kv heads do not exceed the compute units (a quarter of 256 and one row more here), rings that wrap; against the CPU
+    reference."""
+    end = start + t
+    rng = np.random.default_rng(start + t)
+    q = (rng.standard_normal((t, heads, 64)) * 0.7).astype(np.float32)
+    k = (rng.standard_normal((end, kv_heads, 64)) * 0.7).astype(np.float32)
+    v = rng.standard_normal((end, kv_heads, 64)).astype(np.float32)
+    sinks = rng.standard_normal(heads).astype(np.float32)
+    longest = max(i + 1 - ((max(0, i + 1 - window) if window != FULL else 0) & ~31) for i in range(start, end))
+    chunks = longest > 256 and 4 * t * kv_heads <= 256
+    kr, vr = ring_layout(k, t, start, slots, False), ring_layout(v, t, start, slots, False)
+    shape = C.GroupedShape(t, start, heads, kv_heads, 64, window, slots, 0.125)
+    want = oracle.attention_f32(q, k, v, sinks, start, window=window, slots=None, scale=0.125, threads=THREADS)
+    got = run_attention(gpu, q, kr, vr, sinks, shape, False, C.F32, expect_kernel="lng_decode_merge_few" if chunks else "lng_decode_f32_d64")
+    assert rel_error(got, want) <= F32_RTOL
+
+
 # ---- prompt passes in f32 (f32 matrix-instruction kernel) -------------------------------------
 @pytest.mark.parametrize("t,start,window,slots,heads,kv_heads,forced", [
     (64, 0, FULL, 64, 64, 8, None), (33, 5, FULL, 64, 64, 8, None), (100, 37, FULL, 160, 16, 2, None), (65, 0, 1, 96, 64, 8, None),
