@@ -1,6 +1,7 @@
 """Builds liblng_hip.so in-tree: the gfx950 code object from csrc/lng_kernels.hip
 (``hipcc --genco``), embedded into the host library compiled from csrc/lng_hip.cpp, plus
-csrc/lng_static.hip (the fixed device scratch array and the host code that finds it).
+csrc/lng_static.hip (the fixed device scratch array and the host code that finds it); and the Python extension
+of csrc/lng_record.cpp.
 
     python -m loadngo_amd.build
     python -m loadngo_amd.build --null-device   # the host library alone, against csrc/null_device, with sanitizers
@@ -8,6 +9,7 @@ csrc/lng_static.hip (the fixed device scratch array and the host code that finds
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -52,7 +54,26 @@ def build(verbose=False):
     ])
     if verbose and out:
         print(out)
+    build_record(verbose)
     return LIB
+
+
+RECORD = os.path.join(HERE, "_record.so")
+
+
+def build_record(verbose=False):
+    """csrc/lng_record.cpp, the short way from compute.py into the library; without Python's headers compute.py does
+    without it."""
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        if os.path.exists(RECORD):
+            os.remove(RECORD)  # of an older build: may not fit the library any more
+        return None
+    out = _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-Wextra", "-Wno-cast-function-type", "-I" + include,
+                os.path.join(CSRC, "lng_record.cpp"), "-o", RECORD])
+    if verbose and out:
+        print(out)
+    return RECORD
 
 
 NULL_LIB = os.path.join(HERE, "liblng_hip_null.so")

@@ -16,6 +16,11 @@ import threading
 
 import numpy as np
 
+try:
+    from loadngo_amd import _record  # csrc/lng_record.cpp: the same calls for plain arguments, without ctypes
+except ImportError:  # not built (no Python headers where the library was)
+    _record = None
+
 FULL = 2**64 - 1  # GroupedShape.window = usize::MAX
 NO_SINKS = 2**64 - 1
 F32, BF16 = 0, 1
@@ -92,6 +97,7 @@ class _Completed(ctypes.Structure):
 
 
 _ON_DONE = ctypes.CFUNCTYPE(None, ctypes.POINTER(_Completed), ctypes.c_void_p)
+_NO_CALLBACK = ctypes.cast(None, _ON_DONE)
 
 # Every symbol include/lng_hip.h declares: (restype, argtypes)
 _P = ctypes.c_void_p
@@ -167,11 +173,14 @@ def library():
                 fn = getattr(lib, name)
                 fn.restype = restype
                 fn.argtypes = argtypes
+            if _record is not None:
+                _record.bind({name: ctypes.cast(getattr(lib, name), _P).value for name in SYMBOLS}, Slice, GroupedShape, _Item, _PrepareItem)
             _lib = lib
     return _lib
 
 
 def _check(rc):
+    """A status of the library; raises its error."""
     if rc != 0:
         message = library().lng_hip_last_error().decode("utf-8", "replace")
         raise _ERRORS.get(rc, Error)(message)
@@ -184,10 +193,12 @@ def _u64(name, value):
     return int(value)
 
 
-# Recording a dispatch is mostly the conversion of its slices, so plain ints take the short way through each conversion
-# below: all of them at once are of type int and in 0 .. 2**64 - 1 (the OR of several is, exactly if each is). Anything
-# else (other integer types, values out of range) goes through _u64, one by one, which accepts or refuses it.
-# A token through 24 attention blocks (97 dispatches, 578 slices) is recorded in 300 us, 670 when every value went there.
+# Recording a dispatch is mostly the conversion of its arguments. The methods below hand theirs to _record, which makes the call
+# if all are of the plain kinds it takes (see there) and gives the library's status, else None: then ctypes does it. The
+# conversions for ctypes take plain ints a short way too: all of them at once are of type int and in 0 .. 2**64 - 1 (the OR of
+# several is, exactly if each is). Anything else (other integer types, values out of range) goes through _u64, one by one, which
+# accepts or refuses it.
+# A token through 24 attention blocks (97 dispatches, 578 slices) is recorded in 54 us; 300 through ctypes.
 _TOP = 2**64
 
 
@@ -374,7 +385,7 @@ class Gpu:
         lib = library()
         handle = _P()
         _check(lib.lng_hip_open(device, ctypes.byref(handle)))
-        self._h = handle
+        self._h = handle.value
 
     @classmethod
     def new(cls):
@@ -399,13 +410,13 @@ class Gpu:
     def buffer(self, len):
         h = _P()
         _check(library().lng_hip_buffer(self._h, len, ctypes.byref(h)))
-        return Buffer(self, h, len)
+        return Buffer(self, h.value, len)
 
     def resident(self, data):
         a = np.ascontiguousarray(data)
         h = _P()
         _check(library().lng_hip_resident(self._h, a.ctypes.data_as(_P), a.nbytes, ctypes.byref(h)))
-        return Resident(self, h, a.nbytes)
+        return Resident(self, h.value, a.nbytes)
 
     def upload(self, array):
         """A buffer holding ``array`` (the tests' ``upload`` helper, attention_grouped.rs:37-41)."""
@@ -422,8 +433,10 @@ class Gpu:
         """The plain operator on raw device addresses (``Buffer.device_ptr()`` plus a byte offset), launched at
         once on ``stream`` (a hipStream_t as an integer; None: the default stream) without allocating anything;
         no counterpart in the reference. Returns without waiting."""
-        _check(library().lng_hip_attention_grouped_static(self._h, stream, q, k, v, out, sinks or None,
-                                                          ctypes.byref(shape._c()), dtype))
+        rc = _record and _record.attention_grouped_static(self._h, stream, q, k, v, out, sinks or None, shape, dtype)
+        if rc is None:
+            rc = library().lng_hip_attention_grouped_static(self._h, stream, q, k, v, out, sinks or None, ctypes.byref(shape._c()), dtype)
+        _check(rc)
 
     def close(self):
         if self._h:
@@ -438,9 +451,14 @@ class Batch:
         self._gpu = gpu
         self.buffers = buffers
         self._residents = []
-        arr = (_P * max(len(buffers), 1))(*[b._h for b in buffers])
-        h = _P()
-        _check(library().lng_hip_batch(gpu._h, arr, len(buffers), ctypes.byref(h)))
+        h = _record and _record.batch(gpu._h, [b._h for b in buffers])
+        if h is None:
+            arr = (_P * max(len(buffers), 1))(*[b._h for b in buffers])
+            handle = _P()
+            _check(library().lng_hip_batch(gpu._h, arr, len(buffers), ctypes.byref(handle)))
+            h = handle.value
+        elif h < 0:
+            _check(h)
         self._h = h
         self._callback = None
         self._committed = False
@@ -459,46 +477,65 @@ class Batch:
         _check(library().lng_hip_batch_barrier(self._h))
 
     def attention_grouped(self, q, k, v, out, shape, dtype=F32):
-        _check(library().lng_hip_attention_grouped(self._h, q._c(), k._c(), v._c(), out._c(), None,
-                                                   ctypes.byref(shape._c()), dtype))
+        rc = _record and _record.attention_grouped(self._h, q, k, v, out, None, shape, dtype)
+        if rc is None:
+            rc = library().lng_hip_attention_grouped(self._h, q._c(), k._c(), v._c(), out._c(), None, ctypes.byref(shape._c()), dtype)
+        _check(rc)
 
     def attention_grouped_with_sinks(self, qkv, sinks, out, shape, dtype=F32):
         q, k, v = qkv
-        _check(library().lng_hip_attention_grouped(self._h, q._c(), k._c(), v._c(), out._c(),
-                                                   ctypes.byref(sinks._c()), ctypes.byref(shape._c()), dtype))
+        rc = _record and _record.attention_grouped(self._h, q, k, v, out, sinks or 0, shape, dtype)  # (0: not a slice)
+        if rc is None:
+            rc = library().lng_hip_attention_grouped(self._h, q._c(), k._c(), v._c(), out._c(), ctypes.byref(sinks._c()), ctypes.byref(shape._c()), dtype)
+        _check(rc)
 
     def attention_grouped_tiled(self, q, k, v, out, shape, dtype=F32):
-        _check(library().lng_hip_attention_grouped_tiled(self._h, q._c(), k._c(), v._c(), out._c(), None,
-                                                         ctypes.byref(shape._c()), dtype))
+        rc = _record and _record.attention_grouped_tiled(self._h, q, k, v, out, None, shape, dtype)
+        if rc is None:
+            rc = library().lng_hip_attention_grouped_tiled(self._h, q._c(), k._c(), v._c(), out._c(), None, ctypes.byref(shape._c()), dtype)
+        _check(rc)
 
     def attention_grouped_tiled_with_sinks(self, qkv, sinks, out, shape, dtype=F32):
         q, k, v = qkv
-        _check(library().lng_hip_attention_grouped_tiled(self._h, q._c(), k._c(), v._c(), out._c(),
-                                                         ctypes.byref(sinks._c()), ctypes.byref(shape._c()), dtype))
+        rc = _record and _record.attention_grouped_tiled(self._h, q, k, v, out, sinks or 0, shape, dtype)
+        if rc is None:
+            rc = library().lng_hip_attention_grouped_tiled(self._h, q._c(), k._c(), v._c(), out._c(), ctypes.byref(sinks._c()), ctypes.byref(shape._c()), dtype)
+        _check(rc)
 
     def copy_rows(self, src, dst, rows, width, src_dtype=F32, dst_dtype=None):
         """``copy_rows((src, src_stride), (dst, dst_stride), rows, width)`` (apple.rs:1762)."""
-        (s, s_stride), (d, d_stride) = src, dst
         dst_dtype = src_dtype if dst_dtype is None else dst_dtype
-        _check(library().lng_hip_copy_rows(self._h, s._c(), s_stride, src_dtype, d._c(), d_stride, dst_dtype,
-                                           rows, width))
+        rc = _record and _record.copy_rows(self._h, src, dst, rows, width, src_dtype, dst_dtype)
+        if rc is None:
+            (s, s_stride), (d, d_stride) = src, dst
+            rc = library().lng_hip_copy_rows(self._h, s._c(), s_stride, src_dtype, d._c(), d_stride, dst_dtype, rows, width)
+        _check(rc)
 
     def attention_decode_batched(self, q_buffer, k_buffer, v_buffer, out_buffer, sinks_buffer, items, heads,
                                  kv_heads, dim, scale, dtype=BF16):
-        arr = items if isinstance(items, ctypes.Array) else decode_items(items)
-        _check(library().lng_hip_attention_decode_batched(self._h, q_buffer, k_buffer, v_buffer, out_buffer,
-                                                          sinks_buffer, arr, len(items), heads, kv_heads, dim,
-                                                          scale, dtype))
+        rc = _record and _record.attention_decode_batched(self._h, q_buffer, k_buffer, v_buffer, out_buffer, sinks_buffer, items, heads,
+                                                          kv_heads, dim, scale, dtype)
+        if rc is None:
+            arr = items if isinstance(items, ctypes.Array) else decode_items(items)
+            rc = library().lng_hip_attention_decode_batched(self._h, q_buffer, k_buffer, v_buffer, out_buffer, sinks_buffer, arr,
+                                                            len(items), heads, kv_heads, dim, scale, dtype)
+        _check(rc)
 
     def rmsnorm_rows(self, v_w, rows, d_stride, eps):
         """``rmsnorm_rows((v, w), rows, (d, stride), eps)`` (apple.rs:1733), f32, in place."""
-        (v, w), (d, stride) = v_w, d_stride
-        _check(library().lng_hip_rmsnorm_rows(self._h, v._c(), w._c(), rows, d, stride, eps))
+        rc = _record and _record.rmsnorm_rows(self._h, v_w, rows, d_stride, eps)
+        if rc is None:
+            (v, w), (d, stride) = v_w, d_stride
+            rc = library().lng_hip_rmsnorm_rows(self._h, v._c(), w._c(), rows, d, stride, eps)
+        _check(rc)
 
     def add_rows(self, dst, src, rows, width):
         """``add_rows(dst, (src, src_stride), rows, width)`` (apple.rs:1886), f32."""
-        s, s_stride = src
-        _check(library().lng_hip_add_rows(self._h, dst._c(), s._c(), s_stride, rows, width))
+        rc = _record and _record.add_rows(self._h, dst, src, rows, width)
+        if rc is None:
+            s, s_stride = src
+            rc = library().lng_hip_add_rows(self._h, dst._c(), s._c(), s_stride, rows, width)
+        _check(rc)
 
     def rotate_halves(self, x, table, rows, heads_dim):
         """``rotate_halves(x, table, rows, (heads, dim))`` (apple.rs:1916), f32, in place."""
@@ -515,12 +552,15 @@ class Batch:
         """Biases, rotation, narrowing and cache append of gpt-oss/src/gpu.rs:733-759 in one dispatch.
         ``buffers`` maps q, k, v, table, q_out, k_cache, v_cache to buffer numbers of this batch;
         the biases are slices (or None)."""
+        rotary = dim if rotary is None else rotary
+        rc = _record and _record.prepare_attention(self._h, buffers, items, heads, kv_heads, dim, rotary, out_dtype, q_bias, k_bias, v_bias)
+        if rc is not None:
+            return _check(rc)
         held = [None if b is None else b._c() for b in (q_bias, k_bias, v_bias)]
         pb = _PrepareBuffers(buffers["q"], buffers["k"], buffers["v"], buffers["table"], buffers["q_out"], buffers["k_cache"],
                              buffers["v_cache"], *[None if h is None else _SLICE_POINTER(h) for h in held])
         arr = items if isinstance(items, ctypes.Array) else prepare_items(items)
-        _check(library().lng_hip_prepare_attention(self._h, ctypes.byref(pb), arr, len(arr), heads, kv_heads, dim,
-                                                   dim if rotary is None else rotary, out_dtype))
+        _check(library().lng_hip_prepare_attention(self._h, ctypes.byref(pb), arr, len(arr), heads, kv_heads, dim, rotary, out_dtype))
 
     def gemv_q8_0(self, matrix, x, y, rows, cols):
         """``gemv_q8_0((codes, scales), x, y, rows, cols)`` (apple.rs:1812)."""
@@ -529,39 +569,52 @@ class Batch:
 
     def gemm_q8_0(self, matrix, x, y, rows, cols, n, strides):
         """``gemm_q8_0((codes, scales), x, y, rows, cols, n, (x_stride, y_stride))`` (apple.rs:1833)."""
-        codes, scales = matrix
-        _check(library().lng_hip_gemm_q8_0(self._h, codes._c(), scales._c(), x._c(), y._c(), rows, cols, n,
-                                           strides[0], strides[1]))
+        rc = _record and _record.gemm_q8_0(self._h, matrix, x, y, rows, cols, n, strides)
+        if rc is None:
+            codes, scales = matrix
+            rc = library().lng_hip_gemm_q8_0(self._h, codes._c(), scales._c(), x._c(), y._c(), rows, cols, n, strides[0], strides[1])
+        _check(rc)
 
     def gemm_q8_0_tiled(self, matrix, x, y, rows, cols, n, strides):
         """``gemm_q8_0_tiled(...)`` (apple.rs:1857): needs rows % 64, cols % 32 and n % 32 == 0."""
-        codes, scales = matrix
-        _check(library().lng_hip_gemm_q8_0_tiled(self._h, codes._c(), scales._c(), x._c(), y._c(), rows, cols, n,
-                                                 strides[0], strides[1]))
+        rc = _record and _record.gemm_q8_0_tiled(self._h, matrix, x, y, rows, cols, n, strides)
+        if rc is None:
+            codes, scales = matrix
+            rc = library().lng_hip_gemm_q8_0_tiled(self._h, codes._c(), scales._c(), x._c(), y._c(), rows, cols, n, strides[0], strides[1])
+        _check(rc)
 
     def gemm_q8_0_bf16(self, matrix, x, y, rows, cols, n, strides):
         """The Q8_0 product of bf16 positions (no counterpart in the reference): x is [n][x_stride] bf16, y f32."""
-        codes, scales = matrix
-        _check(library().lng_hip_gemm_q8_0_bf16(self._h, codes._c(), scales._c(), x._c(), y._c(), rows, cols, n,
-                                                strides[0], strides[1]))
+        rc = _record and _record.gemm_q8_0_bf16(self._h, matrix, x, y, rows, cols, n, strides)
+        if rc is None:
+            codes, scales = matrix
+            rc = library().lng_hip_gemm_q8_0_bf16(self._h, codes._c(), scales._c(), x._c(), y._c(), rows, cols, n, strides[0], strides[1])
+        _check(rc)
 
     def gemm_q8_0_many(self, matrices, x, cols, n, x_stride):
         """Up to four Q8_0 products of the same positions (no counterpart in the reference, which records one
         per matrix: gpu.rs:724-732): ``matrices`` is a list of ``((codes, scales), y, rows)``, each y dense
         [n][rows]; one dispatch below 32 positions."""
-        arr = _q8_matrices(matrices)
-        _check(library().lng_hip_gemm_q8_0_many(self._h, arr, len(matrices), x._c(), cols, n, x_stride))
+        rc = _record and _record.gemm_q8_0_many(self._h, matrices, x, cols, n, x_stride)
+        if rc is None:
+            rc = library().lng_hip_gemm_q8_0_many(self._h, _q8_matrices(matrices), len(matrices), x._c(), cols, n, x_stride)
+        _check(rc)
 
     def gemm_q8_0_many_normed(self, matrices, x, norm, cols, n, x_stride):
         """``gemm_q8_0_many`` of the RMS-normalised positions (``norm`` = (weights slice, eps)); x is not changed.
         Replaces copy_rows + rmsnorm_rows + the products of gpu.rs:712-732; fewer than 32 positions."""
-        arr = _q8_matrices(matrices)
-        w, eps = norm
-        _check(library().lng_hip_gemm_q8_0_many_normed(self._h, arr, len(matrices), x._c(), w._c(), eps, cols, n, x_stride))
+        rc = _record and _record.gemm_q8_0_many_normed(self._h, matrices, x, norm, cols, n, x_stride)
+        if rc is None:
+            w, eps = norm
+            rc = library().lng_hip_gemm_q8_0_many_normed(self._h, _q8_matrices(matrices), len(matrices), x._c(), w._c(), eps, cols, n, x_stride)
+        _check(rc)
 
     def gemm_q8_0_residual(self, matrix, x, bias, h, rows, cols, n, strides, x_dtype=F32):
         """h += W x + bias in one dispatch, bit for bit gemm_q8_0 + add_rows(bias) + add_rows(residual) of
         gpu.rs:807-827; x f32 or bf16; fewer than 32 positions. ``strides`` = (x_stride, h_stride)."""
+        rc = _record and _record.gemm_q8_0_residual(self._h, matrix, x, bias, h, rows, cols, n, strides, x_dtype)
+        if rc is not None:
+            return _check(rc)
         codes, scales = matrix
         held = None if bias is None else bias._c()
         _check(library().lng_hip_gemm_q8_0_residual(self._h, codes._c(), scales._c(), x._c(), x_dtype,
@@ -599,14 +652,21 @@ class Batch:
                 on_done(Completed(self.buffers, gpu_time))
             self._callback = _ON_DONE(trampoline)
         else:
-            self._callback = ctypes.cast(None, _ON_DONE)
+            self._callback = _NO_CALLBACK
         self._committed = True
-        _check(library().lng_hip_batch_commit(self._h, self._callback, None))
+        rc = _record and on_done is None and _record.commit(self._h)
+        if rc is None or rc is False:
+            rc = library().lng_hip_batch_commit(self._h, self._callback, None)
+        _check(rc)
 
     def wait(self):
         """Blocks until a committed batch has finished; returns ``Completed``."""
-        seconds = ctypes.c_double()
-        rc = library().lng_hip_batch_wait(self._h, ctypes.byref(seconds))
+        done = _record and _record.wait(self._h)
+        if type(done) is float:
+            return Completed(self.buffers, done)
+        seconds, rc = ctypes.c_double(), done
+        if rc is None:
+            rc = library().lng_hip_batch_wait(self._h, ctypes.byref(seconds))
         if rc == -5:
             return Completed(self.buffers, GpuFailure(library().lng_hip_last_error().decode()))
         _check(rc)
@@ -620,7 +680,8 @@ class Batch:
 
     def drop(self):
         if self._h:
-            library().lng_hip_batch_drop(self._h)
+            if (_record and _record.drop(self._h)) is None:
+                library().lng_hip_batch_drop(self._h)
             self._h = None
 
     def __del__(self):
