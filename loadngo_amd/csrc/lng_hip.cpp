@@ -137,7 +137,7 @@ struct lng_gpu {
                   q8_tiled_bf16 = nullptr, q8_frag_x = nullptr;
     hipFunction_t q8_tiled_add = nullptr, q8_tiled_bf16_add = nullptr;
     hipFunction_t q8_norm_frag = nullptr, q8_few[2] = {}, q8_one[2] = {}; // [bf16 positions]
-    hipFunction_t q8_few_f32 = nullptr;
+    hipFunction_t q8_few_f32 = nullptr, q8_few_split = nullptr, q8_few_split_prepare = nullptr;
     hipFunction_t q8_few_prepare = nullptr, q8_few_f32_prepare = nullptr, q8_one_prepare = nullptr;
     hipFunction_t q8_mid[2][4] = {}; // [bf16 positions][tile, see q8_mid_tile]
     std::string name;
@@ -1080,7 +1080,7 @@ bool fuse_split(const lng_gpu *g, Cmd &c, const Cmd &after) {
 bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
     if (after.fn != g->add_rows) return false;
     bool product = c.fn == g->q8_tiled || c.fn == g->q8_tiled_bf16 || c.fn == g->q8_tiled_add || c.fn == g->q8_tiled_bf16_add;
-    product = product || c.fn == g->q8_few_f32;
+    product = product || c.fn == g->q8_few_f32 || c.fn == g->q8_few_split;
     for (int i = 0; i < 2; ++i) {
         product = product || c.fn == g->q8_few[i] || c.fn == g->q8_one[i];
         for (hipFunction_t fn : g->q8_mid[i]) product = product || (fn && c.fn == fn);
@@ -1110,7 +1110,7 @@ bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
 // `c` (the q, k and v projections of up to 16 positions) with the preparation of attention `after` it.
 // (A token through 24 blocks: f32 1,082 -> 1,023 us, bf16 1,027 -> 977, 16 sequences 1,615 -> 1,536.)
 bool fuse_prepare(const lng_gpu *g, Cmd &c, const Cmd &after) {
-    if ((after.fn != g->prepare_v4 && after.fn != g->prepare_v1) || (c.fn != g->q8_few[0] && c.fn != g->q8_few_f32 && c.fn != g->q8_one[0])) return false;
+    if ((after.fn != g->prepare_v4 && after.fn != g->prepare_v1) || (c.fn != g->q8_few[0] && c.fn != g->q8_few_f32 && c.fn != g->q8_few_split && c.fn != g->q8_one[0])) return false;
     lng_k_q8_prepare both{};
     both.q8 = args_of<lng_k_q8>(c);
     both.prepare = args_of<lng_k_prepare>(after);
@@ -1142,8 +1142,9 @@ bool fuse_prepare(const lng_gpu *g, Cmd &c, const Cmd &after) {
     }
     const bool one = c.fn == g->q8_one[0], direct = c.fn == g->q8_few_f32;
     if (one) both.prepare.first.start %= both.prepare.first.slots; // lng_q8_one_prepare: the row itself (one position is one item, not a table)
-    c.name = one ? "lng_q8_one_prepare" : direct ? "lng_q8_few_f32_prepare" : "lng_q8_few_prepare";
-    c.fn = one ? g->q8_one_prepare : direct ? g->q8_few_f32_prepare : g->q8_few_prepare;
+    const bool split = c.fn == g->q8_few_split;
+    c.name = one ? "lng_q8_one_prepare" : split ? "lng_q8_few_split_prepare" : direct ? "lng_q8_few_f32_prepare" : "lng_q8_few_prepare";
+    c.fn = one ? g->q8_one_prepare : split ? g->q8_few_split_prepare : direct ? g->q8_few_f32_prepare : g->q8_few_prepare;
     set_args(c, both);
     return true;
 }
@@ -1243,6 +1244,8 @@ extern "C" int lng_hip_open(int device, lng_gpu **out) {
         {"lng_q8_few", &g->q8_few[0], true},
         {"lng_q8_few_bf16", &g->q8_few[1], true},
         {"lng_q8_few_f32", &g->q8_few_f32, true},
+        {"lng_q8_few_split", &g->q8_few_split, true},
+        {"lng_q8_few_split_prepare", &g->q8_few_split_prepare, true},
         {"lng_q8_one", &g->q8_one[0], true},
         {"lng_q8_few_prepare", &g->q8_few_prepare, true},
         {"lng_q8_few_f32_prepare", &g->q8_few_f32_prepare, true},
@@ -2282,20 +2285,33 @@ unsigned q8_one_rows(const lng_gpu *g, const lng_k_q8 &a) {
     return best;
 }
 
+// Rows of a workgroup of lng_q8_few_split; 0: not for it. It is for matrices whose tiles of 16 rows would leave some compute units
+// with two workgroups, each reading all of x: as many rows, dealt out evenly, as make it one (only one fits).
+unsigned q8_few_split_rows(const lng_gpu *g, const lng_k_q8 &a) {
+    if (a.n < 2 || a.n > 16 || a.cols < 2048 || a.cols > 4096) return 0;
+    for (unsigned t = 16; t <= 32; t += 2) { // (even: lng_q8_few_split_prepare takes pairs of rows)
+        uint64_t wgs = (a.rows + t - 1) / t;
+        for (uint32_t i = 0; i < a.n_more; ++i) wgs += (a.more[i].rows + t - 1) / t;
+        if (wgs <= g->cus) return t > 16 && (t <= 28 || a.n >= 4 || a.norm_w) ? t : 0; // (2 and 3 without a norm: planes are as quick)
+    }
+    return 0;
+}
+
 // Fewer than 32 positions: bound by reading the matrix, in tiles of 16 rows. One position splits (and normalises) x in
 // the kernel, whose LDS holds up to 48 KB of it; more go through the planes of q8_record_frag or are split by every workgroup.
 // `a` may name further matrices of the same dispatch (first_tile in tiles of 16 rows).
 int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
     const uint64_t blocks = a.cols / 32, groups = (a.n + 15) / 16;
     const bool one = a.n == 1 && a.cols <= (x_bf16 ? 24576u : 12288u);
-    bool direct = !one && !x_bf16 && q8_few_direct(b->gpu, a, row_tiles * groups);
-    if (!one && !x_bf16 && !direct) {
+    const unsigned split = one || x_bf16 ? 0 : q8_few_split_rows(b->gpu, a); // rows of a workgroup
+    bool direct = !one && !x_bf16 && !split && q8_few_direct(b->gpu, a, row_tiles * groups);
+    if (!one && !x_bf16 && !split && !direct) {
         const int rc = q8_record_frag(b, &a, groups * 16);
         if (rc == LNG_ERR_ALLOC) direct = true; // no memory for the planes
         else if (rc) return rc;
     }
-    if (one) {
-        a.one_rows = q8_one_rows(b->gpu, a);
+    if (one || split) {
+        a.one_rows = one ? q8_one_rows(b->gpu, a) : split;
         row_tiles = (a.rows + a.one_rows - 1) / a.one_rows;
         for (uint32_t i = 0; i < a.n_more; ++i) {
             a.more[i].first_tile = (uint32_t)row_tiles;
@@ -2303,14 +2319,14 @@ int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
         }
     }
     Cmd c;
-    c.fn = one ? b->gpu->q8_one[x_bf16] : direct ? b->gpu->q8_few_f32 : b->gpu->q8_few[x_bf16];
-    c.name = one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : direct ? "lng_q8_few_f32" : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
+    c.fn = one ? b->gpu->q8_one[x_bf16] : split ? b->gpu->q8_few_split : direct ? b->gpu->q8_few_f32 : b->gpu->q8_few[x_bf16];
+    c.name = one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : split ? "lng_q8_few_split" : direct ? "lng_q8_few_f32" : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
     c.grid[0] = (unsigned)row_tiles;
     c.grid[1] = (unsigned)groups;
     c.block = 512;
     const uint64_t pairs = (blocks + 1) / 2, scales = blocks <= 512 ? 16 * (pairs | 1) * 4 : 0; // both of a pair of blocks in a word
     // one: x's planes and units (Q8ONE_PAIR), of one pair more; else the scales and the weights of x's norm or the turning buffers
-    c.lds = (unsigned)(one ? (pairs + 1) * (256 + 8) : scales + (direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
+    c.lds = (unsigned)(one ? (pairs + 1) * (256 + 8) : split ? 8 * 4 * 16 * 80 + 32 * (pairs | 1) * 4 : scales + (direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
     set_args(c, a);
     b->cmds.push_back(std::move(c));
     return LNG_OK;

@@ -201,7 +201,7 @@ typedef struct lng_k_q8 {
     float *residual;         /* [n][rows], not y: gets the result added as well, or NULL */
     uint32_t accumulate;
     uint32_t tiles;          /* row tiles of all matrices of the dispatch (lng_q8_mid*) */
-    uint32_t one_rows;       /* lng_q8_one*: rows of a tile, even, at most 16 */
+    uint32_t one_rows;       /* lng_q8_one*, lng_q8_few_split*: rows of a tile, even, at most 16 or 32 */
     uint32_t pad_;
     struct lng_k_q8_more {
         const int8_t *codes;

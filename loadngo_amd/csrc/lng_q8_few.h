@@ -172,25 +172,32 @@ struct Q8Prepared {
         if constexpr (ONE) return p.first;
         else return p.items ? p.items[position] : p.first;
     }
-    template <bool ONE> __device__ __forceinline__ void ask(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row, const float *any) {
-        uint32_t r;
-        const lng_prepare_item it = item_of<ONE>(p, position, r);
+    __device__ __forceinline__ void ask_of(const lng_k_prepare &p, uint32_t which, const lng_prepare_item &it, uint32_t r, uint32_t row, const float *any) {
         const float *b = which == 0 ? p.q_bias : which == 1 ? p.k_bias : p.v_bias;
         bias = *(b ? b + row : any);
         bias_there = *(b && which < 2u ? b + (row ^ 32u) : any);
         const float2 t = *(const float2 *)(which < 2u ? p.table + it.table_offset + ((uint64_t)r * 32u + (row & 31u)) * 8u : (const char *)any);
         c = t.x, s = t.y;
     }
-    template <bool ONE> __device__ __forceinline__ void place(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row) {
-        uint32_t r;
-        const lng_prepare_item it = item_of<ONE>(p, position, r);
+    // ROW: it.start is the row of the caches already.
+    template <bool ROW = false> __device__ __forceinline__ void place_of(const lng_k_prepare &p, uint32_t which, const lng_prepare_item &it, uint32_t r, uint32_t row) {
         const uint32_t es = p.out_dtype == LNG_BF16 ? 2u : 4u;
         if (which == 0) {
             to = p.q_out + it.q_out_offset + ((uint64_t)r * p.heads * 64u + row) * es;
         } else {
-            const uint64_t at = ((ONE ? it.start : (it.start + r) % it.slots) * p.kv_heads * 64u + row) * es;
+            const uint64_t at = ((ROW ? it.start : (it.start + r) % it.slots) * p.kv_heads * 64u + row) * es;
             to = which == 1 ? p.k_cache + it.k_cache_offset + at : p.v_cache + it.v_cache_offset + at;
         }
+    }
+    template <bool ONE> __device__ __forceinline__ void ask(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row, const float *any) {
+        uint32_t r;
+        const lng_prepare_item it = item_of<ONE>(p, position, r);
+        ask_of(p, which, it, r, row, any);
+    }
+    template <bool ONE> __device__ __forceinline__ void place(const lng_k_prepare &p, uint32_t which, uint32_t position, uint32_t row) {
+        uint32_t r;
+        const lng_prepare_item it = item_of<ONE>(p, position, r);
+        place_of<ONE>(p, which, it, r, row);
     }
     __device__ __forceinline__ void store(const lng_k_prepare &p, uint32_t which, uint32_t row, float here, float there) const {
 #pragma clang fp contract(off)
@@ -615,6 +622,219 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
     else q8_one_turns<BF16, NW, PREPARE, 4>(a, tile, s_mem, prepare, which);
 }
 
+// 2 to 16 f32 positions of 2,048 to 4,096 columns in one dispatch, with the RMS norm if norm_w is set: x goes through the matrix
+// unit as it is (times the norm's weights), its squares are added up on the way and each position's scale multiplies the result.
+// So there is no dispatch of planes before it and x is read once: eight lanes to a position's 128 bytes of a block, split, and
+// turned into operand order through LDS that only this wavefront uses. x is most of what a workgroup reads (16 positions of 2,880
+// columns: 184 KB beside 46 KB of codes for 16 rows), so a workgroup takes up to 32 rows, NT runs of 16, and has a compute unit
+// to itself: all its loads of a turn but the last pairs' x are on their way at once.
+// With planes made by a dispatch before it and tiles of 16 rows / so, us, 16 positions: 5,120 x 2,880 12.4 / 10.9 with the norm,
+// 11.9 / 11.1 without, 4,112 x 4,096 15.7 / 13.1 and 15.1 / 13.4, 8,192 x 2,048 11.3 / 10.6 and 10.7 / 10.4; in a decoding step of
+// sixteen sequences (kernel trace, preparation included) 4.7 + 11.3 / 13.2. As many rows as have a unit each with one workgroup
+// of 16 gain nothing (2,880 x 4,096 10.9 / 10.8).
+// U: pairs of blocks of a wavefront (2,880 columns: five or six of 6; up to 4,096: 8).
+template <int U, bool PREPARE>
+__device__ __forceinline__ void q8_few_split_turn(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
+    constexpr int NW = 8, NT = 2, D = 3; // D: pairs of x in flight
+    constexpr uint32_t STRIDE = 80, PLANE = 16 * STRIDE;
+    __shared__ float s_red[NW][NT * 4][64];
+    __shared__ float s_ss[NW][16];
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15u, kg = lane >> 4;
+    const uint32_t blocks = a.cols / 32u, pairs = (blocks + 1u) / 2u, from = wave * pairs / NW, to = (wave + 1u) * pairs / NW, words = pairs | 1u;
+    char *s_x = s_mem + wave * 4u * PLANE; // [block of a pair][plane][position]
+    uint32_t *s_sc = (uint32_t *)(s_mem + NW * 4u * PLANE);
+    // the tile's row k of 16 NT (see q8_one_turns), those past its last the last again
+    const uint32_t first = tile * (PREPARE ? a.one_rows / 2u : a.one_rows), rows = PREPARE ? a.rows / 2u : a.rows;
+    const uint32_t last = (rows - first < (PREPARE ? a.one_rows / 2u : a.one_rows) ? rows - first : (PREPARE ? a.one_rows / 2u : a.one_rows)) - 1u;
+    auto row_of = [&](uint32_t k) {
+        if constexpr (PREPARE) {
+            const uint32_t at = (k >> 4) * 8u + (k & 7u), pair = first + (at < last ? at : last);
+            return (pair >> 5) * 64u + (pair & 31u) + (k & 8u) * 4u;
+        } else {
+            return first + (k < last ? k : last);
+        }
+    };
+    auto has_row = [&](uint32_t k) { return (PREPARE ? (k >> 4) * 8u + (k & 7u) : k) <= last; };
+    const uint32_t r0 = row_of(0);
+    const int8_t *w_src = a.codes + (uint64_t)r0 * a.cols; // (uniform bases and 32-bit offsets, as in q8_one_turns)
+    const uint16_t *sc_src = a.scales + (uint64_t)r0 * blocks;
+    uint32_t w_row[NT], w_row_odd[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        w_row[nt] = (row_of(16u * nt + j) - r0) * a.cols + 16u * kg;
+        w_row_odd[nt] = w_row[nt] - ((blocks & 1u) && kg >= 2u ? 32u : 0u);
+    }
+    // this thread's output: accumulator register wave % 4 of run wave / 4
+    const uint32_t out_p = 4u * kg + (wave & 3u), out_k = 16u * (wave >> 2) + j, out_row = row_of(out_k);
+    const bool mine = wave < 4u * NT && out_p < a.n && has_row(out_k);
+    const uint32_t some_p = out_p < a.n ? out_p : a.n - 1u;
+
+    // What is asked for first comes first. The preparation's items (their table's rows are asked for once x is here), the scales,
+    // x, the codes.
+    lng_prepare_item it;
+    if constexpr (PREPARE) {
+        if (prepare->items) it = prepare->items[some_p];
+    }
+    const bool whole_words = (((uintptr_t)sc_src & 3u) | (blocks & 1u)) == 0; // uniform
+    uint32_t sc_now[2 * NT], sc_then[2 * NT];
+    auto sc_row = [&](int i) { return (row_of(wave * 2u * NT + i) - r0) * blocks; }; // (scalar)
+    {
+        const uint32_t at = lane < pairs ? lane : pairs - 1u; // (at most 64 pairs)
+#pragma unroll
+        for (int i = 0; i < 2 * NT; ++i) {
+            const uint16_t *src = sc_src + sc_row(i) + 2u * at;
+            if (whole_words) {
+                sc_now[i] = *(const uint32_t *)src;
+            } else {
+                sc_now[i] = src[0];
+                sc_then[i] = src[2u * at + 1u < blocks ? 1 : 0];
+            }
+        }
+    }
+    const float *x_src[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t p = 8u * h + (lane >> 3);
+        x_src[h] = a.x + (uint64_t)(p < a.n ? p : a.n - 1u) * a.x_stride + 4u * (lane & 7u);
+    }
+    const bool normed = a.norm_w != nullptr; // uniform
+    const float *nw_src = (normed ? a.norm_w : a.x) + 4u * (lane & 7u);
+    float4 x[D][2][2], nw[D][2]; // [pair][block][positions 0-7, 8-15]
+    // (A pair past the run loads its first again and is not used: nothing is loaded behind a branch, so every wait knows what is
+    // behind what it waits for.)
+    auto pair_of = [&](uint32_t u) { return from + u < to ? from + u : from; };
+    auto ask_x = [&](uint32_t pair, float4 (&into)[2][2], float4 (&weights)[2]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t b = 2u * pair + h < blocks ? 2u * pair + h : blocks - 1u;
+            into[h][0] = *(const float4 *)(x_src[0] + 32u * b);
+            into[h][1] = *(const float4 *)(x_src[1] + 32u * b);
+            weights[h] = *(const float4 *)(nw_src + 32u * b);
+        }
+    };
+    uint4 w[U][NT];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) ask_x(pair_of(d), x[d], nw[d]);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier(); // every wavefront's x before any one's codes; waits for no memory
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t pair = pair_of(u);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) w[u][nt] = *(const uint4 *)(w_src + ((pair == pairs - 1u ? w_row_odd[nt] : w_row[nt]) + 64u * pair));
+    }
+    const float *any = (const float *)a.codes;
+    const float bias = *(a.bias ? a.bias + out_row : any);
+    float *yp = a.y + (uint64_t)some_p * a.y_stride + out_row, *res = a.residual + (uint64_t)some_p * a.rows + out_row;
+    const float held = *(a.accumulate ? yp : a.residual ? res : any); // (never both)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) {
+        uint32_t *to_row = s_sc + (wave * 2u * NT + i) * words;
+        const uint32_t both = whole_words ? sc_now[i] : __builtin_amdgcn_perm(sc_then[i], sc_now[i], 0x05040100u);
+        if (lane < pairs) to_row[lane] = both;
+    }
+    __syncthreads();
+    Q8Prepared ready;
+    if constexpr (PREPARE) {
+        lng_prepare_item one = prepare->first;
+        if (prepare->items) one = it;
+        ready.ask_of(*prepare, which, one, prepare->items ? 0u : some_p, out_row, any);
+        ready.place_of(*prepare, which, one, prepare->items ? 0u : some_p, out_row);
+    }
+
+    floatx4 y[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) y[nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    float ss[2] = {0.0f, 0.0f};
+    const uint32_t put = (lane >> 3) * STRIDE + 8u * (lane & 7u), get = j * STRIDE + 16u * q8_mid_chunk(kg);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t pair = from + u;
+        if (pair < to) { // uniform
+            const bool second = 2u * pair + 1u < blocks; // uniform
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const float4 v = x[u % D][h][g], n = nw[u % D][h];
+                    float e[4] = {v.x, v.y, v.z, v.w};
+                    if (h == 0 || second) ss[g] += e[0] * e[0] + e[1] * e[1] + e[2] * e[2] + e[3] * e[3];
+                    if (normed) e[0] *= n.x, e[1] *= n.y, e[2] *= n.z, e[3] *= n.w;
+                    bf16x4 hi, lo;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const __bf16 top = (__bf16)e[i];
+                        hi[i] = top;
+                        lo[i] = (__bf16)(e[i] - (float)top);
+                    }
+                    *(bf16x4 *)(s_x + (2 * h) * PLANE + 8 * g * STRIDE + put) = hi;
+                    *(bf16x4 *)(s_x + (2 * h + 1) * PLANE + 8 * g * STRIDE + put) = lo;
+                }
+            }
+            bf16x8 op[2][2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                op[h][0] = as_bf16x8(*(const uint4 *)(s_x + (2 * h) * PLANE + get));
+                op[h][1] = as_bf16x8(*(const uint4 *)(s_x + (2 * h + 1) * PLANE + get));
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const auto s0 = __builtin_amdgcn_permlane32_swap(w[u][nt].x, w[u][nt].z, false, false);
+                const auto s1 = __builtin_amdgcn_permlane32_swap(w[u][nt].y, w[u][nt].w, false, false);
+                const bf16x8 b0 = q8_codes_to_bf16_perm(make_uint2(s0[0], s1[0])), b1 = q8_codes_to_bf16_perm(make_uint2(s0[1], s1[1]));
+                const uint32_t both = s_sc[(16u * nt + j) * words + pair];
+                const float c0 = f16_bits_to_f32((uint16_t)both), c1 = f16_bits_to_f32((uint16_t)(both >> 16));
+                floatx4 p0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[0][0], b0, zero4, 0, 0, 0);
+                floatx4 p1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[1][0], b1, zero4, 0, 0, 0);
+                p0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[0][1], b0, p0, 0, 0, 0);
+                p1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[1][1], b1, p1, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[nt][i] = __builtin_fmaf(c0, p0[i], y[nt][i]);
+                if (second) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) y[nt][i] = __builtin_fmaf(c1, p1[i], y[nt][i]);
+                }
+            }
+        }
+        if (u + D < U) {
+            __builtin_amdgcn_sched_barrier(0);
+            ask_x(pair_of(u + D), x[u % D], nw[u % D]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) { // over the eight lanes of a position
+        auto across = [&](auto ctrl) { ss[g] += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(ss[g]), decltype(ctrl)::value, 0xf, 0xf, true)); };
+        across(std::integral_constant<int, 0xB1>{});  // quad_perm [1,0,3,2]
+        across(std::integral_constant<int, 0x4E>{});  // quad_perm [2,3,0,1]
+        across(std::integral_constant<int, 0x141>{}); // row_half_mirror
+        if ((lane & 7u) == 0) s_ss[wave][8u * g + (lane >> 3)] = ss[g];
+    }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s_red[wave][4 * nt + i][lane] = y[nt][i];
+    }
+    __syncthreads();
+    if (wave >= 4u * NT) return;
+    float sum = 0.0f, squares = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) sum += s_red[i][wave][lane], squares += s_ss[i][out_p];
+    if (normed) sum = sum * (1.0f / sqrtf(squares / (float)a.cols + a.eps));
+    if (a.bias) sum = sum + bias;
+    if (a.accumulate) sum = held + sum;
+    float there = 0.0f;
+    if constexpr (PREPARE) there = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sum), 0x128, 0xf, 0xf, true)); // row_ror:8, 32 rows away
+    if (!mine) return;
+    *yp = sum;
+    if (a.residual) *res = held + sum;
+    if constexpr (PREPARE) ready.store(*prepare, which, out_row, sum, there);
+}
+
 #define Q8_FEW(name, body, what, nw) \
     extern "C" __global__ __launch_bounds__(64 * nw, nw / 2) void name(lng_k_q8 a) { \
         extern __shared__ __attribute__((aligned(16))) char s_mem[]; /* as many bytes as q8_record_few works out */ \
@@ -639,3 +859,22 @@ Q8_FEW(lng_q8_one_bf16, q8_one_body, true, 8)
 Q8_FEW_PREPARE(lng_q8_few_prepare, q8_few_body, Q8F_PLANES, 8)
 Q8_FEW_PREPARE(lng_q8_few_f32_prepare, q8_few_body, Q8F_F32, 8)
 Q8_FEW_PREPARE(lng_q8_one_prepare, q8_one_body, false, 8)
+
+template <bool PREPARE = false>
+__device__ __forceinline__ void q8_few_split_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
+    if (a.cols <= 3072u) q8_few_split_turn<6, PREPARE>(a, tile, s_mem, prepare, which);
+    else q8_few_split_turn<8, PREPARE>(a, tile, s_mem, prepare, which);
+}
+
+extern "C" __global__ __launch_bounds__(512, 2) void lng_q8_few_split(lng_k_q8 a) {
+    extern __shared__ __attribute__((aligned(16))) char s_mem[];
+    const uint32_t tile = q8_select_matrix(a);
+    q8_few_split_body(a, tile, s_mem);
+}
+extern "C" __global__ __launch_bounds__(512, 2) void lng_q8_few_split_prepare(lng_k_q8_prepare both) {
+    extern __shared__ __attribute__((aligned(16))) char s_mem[];
+    lng_k_q8 a = both.q8;
+    const uint32_t which = blockIdx.x >= a.more[1].first_tile ? 2u : blockIdx.x >= a.more[0].first_tile ? 1u : 0u;
+    const uint32_t tile = q8_select_matrix(a);
+    q8_few_split_body<true>(a, tile, s_mem, &both.prepare, which);
+}

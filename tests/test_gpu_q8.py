@@ -575,3 +575,32 @@ def test_one_position_in_whole_numbers(gpu, rows, cols, bf16):
         x = xorshift_values(32, cols).astype(np.float32).reshape(1, cols)
         x[0, cols - 5] = bad
         assert np.isnan(_product(gpu, codes, bits, to_bf16_bits(x) if bf16 else x, rows, cols, 1)).all()
+
+
+@pytest.mark.parametrize("rows,cols,n", [(4098, 2048, 2), (4100, 2080, 16), (5120, 2880, 9), (5121, 3104, 3), (8192, 4096, 16), (8150, 4064, 15), (7000, 2048, 3)])
+def test_positions_split_by_the_product_itself(gpu, rows, cols, n):
+    """2 to 16 f32 positions of more rows than compute units have 16 for, one dispatch with and without the RMS norm: workgroups of 18
+    to 32 rows and their remainders, an odd number of blocks, wavefronts with a pair fewer than others, one column size either side
+    of the two numbers of pairs a wavefront holds; positions of very different sizes; scales off a 4-byte boundary. Within the
+    reference's bound (glue.rs:171) of float64 at each position."""
+    codes, bits, elements = q8_test_matrix(rows, cols, 33 + rows)
+    x = (xorshift_values(34 + n, n * cols).reshape(n, cols) * (10.0 ** np.arange(-8, 8))[:n, None]).astype(np.float32)
+    w = xorshift_values(35, cols).astype(np.float32) + 1.0
+    normed = x.astype(np.float64) / np.sqrt((x.astype(np.float64) ** 2).mean(1, keepdims=True) + 1e-5) * w
+    bufs = [gpu.upload(codes), gpu.upload(np.concatenate([np.array([0x7E00], np.uint16), bits])), gpu.upload(x), gpu.upload(w), gpu.buffer(n * rows * 4), gpu.buffer(n * rows * 4)]
+    for b in bufs[4:]:
+        b.fill(0xFF)
+    batch = gpu.batch(bufs)
+    batch.set_timing(True)
+    m, xs = (C.Slice(0, 0, codes.nbytes), C.Slice(1, 2, bits.nbytes)), C.Slice(2, 0, x.nbytes)
+    batch.gemm_q8_0(m, xs, C.Slice(4, 0, n * rows * 4), rows, cols, n, (cols, rows))
+    batch.gemm_q8_0_many_normed([(m, C.Slice(5, 0, n * rows * 4), rows)], xs, (C.Slice(3, 0, w.nbytes), 1e-5), cols, n, cols)
+    done = batch.run()
+    assert not isinstance(done.gpu_time, Exception), done.gpu_time
+    assert batch.kernel_seconds("lng_q8_few_split")[1] == 2 and batch.dispatches() == 2
+    batch.drop()
+    for buf, values in ((bufs[4], x.astype(np.float64)), (bufs[5], normed)):
+        want, got = values @ elements.T, buf.read(np.float32).reshape(n, rows)
+        assert (np.abs(got - want).max(1) < 1e-5 * np.abs(want).max(1)).all()
+    for b in bufs:
+        b.free()
