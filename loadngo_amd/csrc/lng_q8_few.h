@@ -630,12 +630,12 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
 // to itself: all its loads of a turn but the last pairs' x are on their way at once.
 // With planes made by a dispatch before it and tiles of 16 rows / so, us, 16 positions: 5,120 x 2,880 12.4 / 10.9 with the norm,
 // 11.9 / 11.1 without, 4,112 x 4,096 15.7 / 13.1 and 15.1 / 13.4, 8,192 x 2,048 11.3 / 10.6 and 10.7 / 10.4; in a decoding step of
-// sixteen sequences (kernel trace, preparation included) 4.7 + 11.3 / 13.2. As many rows as have a unit each with one workgroup
+// sixteen sequences (kernel trace, preparation included) 4.7 + 11.3 / 12.9. As many rows as have a unit each with one workgroup
 // of 16 gain nothing (2,880 x 4,096 10.9 / 10.8).
 // U: pairs of blocks of a wavefront (2,880 columns: five or six of 6; up to 4,096: 8).
 template <int U, bool PREPARE>
 __device__ __forceinline__ void q8_few_split_turn(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
-    constexpr int NW = 8, NT = 2, D = 3; // D: pairs of x in flight
+    constexpr int NW = 8, NT = 2, D = 2; // D: pairs of x in flight (3: 2 % slower, 6: 8 %)
     constexpr uint32_t STRIDE = 80, PLANE = 16 * STRIDE;
     __shared__ float s_red[NW][NT * 4][64];
     __shared__ float s_ss[NW][16];
