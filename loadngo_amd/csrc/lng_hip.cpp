@@ -2325,8 +2325,9 @@ int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
     c.grid[1] = (unsigned)groups;
     c.block = 512;
     const uint64_t pairs = (blocks + 1) / 2, scales = blocks <= 512 ? 16 * (pairs | 1) * 4 : 0; // both of a pair of blocks in a word
-    // one: x's planes and units (Q8ONE_PAIR), of one pair more; else the scales and the weights of x's norm or the turning buffers
-    c.lds = (unsigned)(one ? (pairs + 1) * (256 + 8) : split ? 8 * 4 * 16 * 80 + 32 * (pairs | 1) * 4 : scales + (direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
+    // one: x's planes and units (Q8ONE_PAIR), of one pair more, (f32) the planes of its rest; else the scales and the weights of x's
+    // norm or the turning buffers
+    c.lds = (unsigned)(one ? ((pairs + 1) * (256 + 8) + 15) / 16 * 16 + (x_bf16 ? 0 : (pairs + 1) * 128) : split ? 8 * 4 * 16 * 80 + 32 * (pairs | 1) * 4 : scales + (direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
     set_args(c, a);
     b->cmds.push_back(std::move(c));
     return LNG_OK;

@@ -380,35 +380,59 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
 // One position, on the integer matrix unit, which takes the codes as they are: widening them for the other one was most of
 // the vector unit's work here. x goes in as whole numbers too: of each block of 32 columns the largest |x| sets a power of
 // two, every x of the block becomes a 30-bit number of that unit (exact where it is within 2^-6 of the largest, else rounded
-// at 2^-30 of it: nowhere worse than the products' f32 sums, and better than two bf16 values), and its four signed bytes lie in
-// four planes in LDS. One matrix instruction multiplies 16 rows by 64 columns, two blocks: rows 0-3 of the other operand are
+// at 2^-30 of it), and its four signed bytes lie in four planes in LDS. One matrix instruction multiplies 16 rows by 64 columns, two blocks: rows 0-3 of the other operand are
 // the first block's planes (zero in the second's columns), rows 4-7 the second's; the next pair's go into rows 8-15 and the
 // same accumulators. So lane group kg ends with the four planes' exact sums of block kg of four, and puts them together.
+// The other products hold 2^-18 of each x, however small (two bf16 values; from bf16 all of it). The planes hold that much of x from
+// 2^-12 of the block's largest on (bf16: 2^-22). One block in eighty of normally distributed f32 has a smaller one: what rounding
+// left of such a block, as whole numbers of 2^-15 of its unit, lies in two planes more, enough for x down to 2^-26; what is still
+// missing, in blocks of any spread, q8_one_rest adds. Looking for such blocks and, in most calls, adding some costs 0.3 us (without:
+// 5,120 x 2,880 5.5, with: 5.8; 2,880 x 4,096 5.3 and 5.6; from bf16, where they are rare, 5.2 and 5.3).
 // A block with an x that is not finite gives NaN, as the split into two bf16 values does.
 // Bound by memory and by what lies before and after it: 1 us until all loads are on their way, a round trip, the matrix at the
 // rate of the whole device (15.7 MB: 2.6 us), 0.8 us of sums and their way through LDS, a dispatch's start and end. In a token
 // through 24 blocks (kernel trace): 5,120 x 2,880 with norm and preparation 9.1 us -> 7.6, 2,880 x 4,096 with bias and residual
 // 7.2 -> 5.5 from bf16, 7.3 -> 5.2 from f32; of which the whole numbers 9.1 -> 7.8 and 7.2 -> 5.9 (the sums of 4,096 columns took
 // a wavefront 1.55 us, now 0.5), tiles of 10 to 14 rows and x before the codes the rest.
+#define Q8WHOLE_REST 15
 struct Q8Whole { // eight columns, a quarter of a block; the other three are in the neighbouring lanes
     uint2 plane[4];
-    float unit;
-    __device__ __forceinline__ void make(const float (&x)[8]) {
-        uint32_t top = 0;
+    float unit;    // 2^-shift; negative: the block has an x of which the planes hold less than BITS
+    int32_t shift;
+    uint32_t top, low; // the block's largest, and its smallest but zero, less one
+    static __device__ __forceinline__ float whole(float v, int32_t shift) { return __builtin_amdgcn_ldexpf(v, shift); }
+    // what rounding leaves, in units of 2^-Q8WHOLE_REST (exact: it has no more digits than x)
+    static __device__ __forceinline__ float rest(float v, int32_t shift) {
+        const float w = whole(v, shift);
+        return (w - __builtin_rintf(w)) * (float)(1 << Q8WHOLE_REST);
+    }
+    __device__ __forceinline__ bool below(uint32_t exponent) const { // whether an x is not zero and below 2^-exponent of the largest's power of two
+        const uint32_t of_top = top >> 23; // (all of them below 2^-127 + exponent: what is not held is nothing in f32)
+        return of_top > exponent && low < ((of_top - exponent) << 23) - 1u;
+    }
+    template <int BITS> __device__ __forceinline__ void make(const float (&x)[8]) {
+        top = 0, low = ~0u;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const uint32_t magnitude = __float_as_uint(x[e]) & 0x7fffffffu;
             top = top > magnitude ? top : magnitude;
+            low = low < magnitude - 1u ? low : magnitude - 1u;
         }
         const uint32_t one = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0xB1, 0xf, 0xf, true); // quad_perm [1,0,3,2]
         top = top > one ? top : one;
         const uint32_t two = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x4E, 0xf, 0xf, true); // quad_perm [2,3,0,1]
         top = top > two ? top : two;
+        const uint32_t low_one = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0xB1, 0xf, 0xf, true);
+        low = low < low_one ? low : low_one;
+        const uint32_t low_two = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0x4E, 0xf, 0xf, true);
+        low = low < low_two ? low : low_two;
         const int32_t exponent = (int32_t)(top >> 23) > 7 ? (int32_t)(top >> 23) - 127 : -120; // the unit of smaller blocks: 2^-149
-        unit = top >= 0x7f800000u ? __uint_as_float(0x7fc00000u) : __builtin_amdgcn_ldexpf(1.0f, exponent - 29);
+        shift = 29 - exponent;
+        unit = __builtin_amdgcn_ldexpf(below(30 - BITS) ? -1.0f : 1.0f, -shift);
+        if (top >= 0x7f800000u) unit = __uint_as_float(0x7fc00000u);
         uint32_t q[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) q[e] = ((uint32_t)(int32_t)__builtin_rintf(__builtin_amdgcn_ldexpf(x[e], 29 - exponent)) + 0x00808080u) ^ 0x00808080u; // signed bytes
+        for (int e = 0; e < 8; ++e) q[e] = ((uint32_t)(int32_t)__builtin_rintf(whole(x[e], shift)) + 0x00808080u) ^ 0x00808080u; // signed bytes
         uint32_t word[4][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -422,19 +446,76 @@ struct Q8Whole { // eight columns, a quarter of a block; the other three are in 
 #pragma unroll
         for (int k = 0; k < 4; ++k) plane[k] = make_uint2(word[k][0], word[k][1]);
     }
+    // the rest's two planes: at most 2^14 of its units, cut off
+    __device__ __forceinline__ void make_rest(const float (&x)[8], uint2 (&to)[2]) const {
+        uint32_t q[8], word[2][2];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e] = ((uint32_t)(int32_t)rest(x[e], shift) + 0x80u) ^ 0x80u;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t a = __builtin_amdgcn_perm(q[4 * h + 1], q[4 * h], 0x05010400u), c = __builtin_amdgcn_perm(q[4 * h + 3], q[4 * h + 2], 0x05010400u);
+            word[0][h] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+            word[1][h] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) to[k] = make_uint2(word[k][0], word[k][1]);
+    }
 };
 
+// What a block's planes and (f32) those of its rest do not hold, as two bf16 values of each x (one, exactly, where the positions are
+// bf16), times the row's codes and scale; every lane group returns the same. x is read and normalised once more.
+template <bool BF16>
+__device__ __forceinline__ float q8_one_rest(const lng_k_q8 &a, uint32_t block, bool normed, float scale, float unit, const int8_t *codes, float sc) {
+    const uint32_t lane = threadIdx.x & 63u, j = lane & 15u, at = block * 32u + (lane >> 4) * 8u; // this lane's columns
+    float x[8];
+    if constexpr (BF16) {
+        const uint4 x16 = *(const uint4 *)(a.x_hi + at);
+        const uint32_t half[4] = {x16.x, x16.y, x16.z, x16.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[2 * e] = __uint_as_float(half[e] << 16), x[2 * e + 1] = __uint_as_float(half[e] & 0xffff0000u);
+    } else {
+        const float4 u = *(const float4 *)(a.x + at), v = *(const float4 *)(a.x + at + 4u);
+        x[0] = u.x, x[1] = u.y, x[2] = u.z, x[3] = u.w, x[4] = v.x, x[5] = v.y, x[6] = v.z, x[7] = v.w;
+        if (normed) {
+            const float4 n = *(const float4 *)(a.norm_w + at), m = *(const float4 *)(a.norm_w + at + 4u);
+            const float nw[8] = {n.x, n.y, n.z, n.w, m.x, m.y, m.z, m.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = x[e] * scale * nw[e];
+        }
+    }
+    const uint2 w = *(const uint2 *)(codes + at);
+    const int32_t shift = 1 - __builtin_amdgcn_frexp_expf(unit);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float rest = Q8Whole::rest(x[e], shift), of_rest = BF16 ? 0.0f : __builtin_truncf(rest);
+        const float less = __builtin_amdgcn_ldexpf(rest - of_rest, -(shift + Q8WHOLE_REST));
+        x[e] = __builtin_fabsf(Q8Whole::whole(x[e], shift)) < 1.0f / (float)(1 << Q8WHOLE_REST) ? x[e] : less; // (all of it, which `whole` may be too small for)
+    }
+    bf16x8 hi, lo;
+    q8_split8(x, hi, lo);
+    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    const floatx4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j & 1u ? lo : hi, q8_codes_to_bf16_perm(w), zero4, 0, 0, 0);
+    return (sum[0] + sum[1]) * sc;
+}
+
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
-// LDS of q8_one_body: the planes of each pair of blocks (and of one more, that the last turn may read and not use), the units.
+// LDS of q8_one_body: the planes of each pair of blocks (and of one more, that the last turn may read and not use), the units, and
+// (f32) the planes of the rest.
 #define Q8ONE_PAIR 256u // bytes
+#define Q8ONE_REST 128u
+template <int NW> struct Q8OneLds { // (one for all numbers of pairs in flight: each would have its own)
+    float red[NW][64], norm[NW];
+    uint32_t finer[NW];
+    __attribute__((aligned(16))) uint32_t zero[512]; // what lanes read that hold rows of the other block or pair
+};
 // U: twos of pairs of blocks a wavefront has in flight. 4: 4,096 columns in one turn of eight wavefronts. 1: up to 1,024 columns,
 // where what a workgroup asks for beyond its share costs more than the waits it saves (16,384 x 512 9.7 us with 4, 5.7 with 1).
 template <bool BF16, int NW, bool PREPARE, int U>
-__device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
+__device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, char *s_mem, Q8OneLds<NW> &lds, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
     constexpr int T = 64 * NW;
-    __shared__ float s_red[NW][64];
-    __shared__ float s_norm[NW];
-    __shared__ __attribute__((aligned(16))) uint32_t s_zero[512]; // what lanes read that hold rows of the other block or pair
+    float (&s_red)[NW][64] = lds.red;
+    float (&s_norm)[NW] = lds.norm;
+    uint32_t (&s_finer)[NW] = lds.finer, (&s_zero)[512] = lds.zero;
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15u, kg = lane >> 4;
     const uint32_t blocks = a.cols / 32u, pairs = (blocks + 1u) / 2u, chunks = a.cols / 8u, mine = threadIdx.x;
     const uint32_t from = wave * pairs / NW, to = (wave + 1u) * pairs / NW;
@@ -458,6 +539,7 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
     const uint16_t *sc_src = a.scales + (uint64_t)r0 * blocks;
     const uint32_t w_row = row_on * a.cols + 16u * kg, w_row_odd = w_row - ((blocks & 1u) && kg >= 2u ? 32u : 0u), sc_row = row_on * blocks;
     float *s_unit = (float *)(s_mem + (pairs + 1u) * Q8ONE_PAIR);
+    char *s_rest = s_mem + ((pairs + 1u) * (Q8ONE_PAIR + 8u) + 15u) / 16u * 16u;
 
     // A compute unit's loads come back in the order in which its wavefronts ask for them. x (and the weights of its norm) is
     // waited for first, so every wavefront asks for its part before any asks for codes; then the scales, the codes, what is
@@ -537,6 +619,7 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
         for (int i = 0; i < NW; ++i) total += s_norm[i];
         scale = 1.0f / sqrtf(total / (float)a.cols + a.eps);
     }
+    bool finer = false;
     for (uint32_t c = mine; c < chunks; c += T) { // (four chunks to a block, T and the chunks multiples of four: quads of lanes stay together)
         if constexpr (BF16) {
             if (c != mine) x16 = *(const uint4 *)(a.x_hi + 8u * c);
@@ -554,16 +637,31 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
             }
         }
         Q8Whole whole;
-        whole.make(x);
+        whole.make<BF16 ? 8 : 18>(x);
         char *put = s_mem + (c >> 3) * Q8ONE_PAIR + (c & 7u) * 8u;
 #pragma unroll
         for (int k = 0; k < 4; ++k) *(uint2 *)(put + 64u * k) = whole.plane[k];
         if ((c & 3u) == 0) s_unit[c >> 2] = whole.unit;
+        if (whole.unit < 0.0f) {
+            if constexpr (BF16) {
+                finer = true;
+            } else {
+                finer |= whole.below(26);
+                uint2 rest[2];
+                whole.make_rest(x, rest);
+                put = s_rest + (c >> 3) * Q8ONE_REST + (c & 7u) * 8u;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) *(uint2 *)(put + 64u * k) = rest[k];
+            }
+        }
     }
+    const bool some_finer = __builtin_amdgcn_ballot_w64(finer) != 0;
+    if (lane == 0) s_finer[wave] = some_finer;
     if constexpr (PREPARE) ready.place<true>(*prepare, which, 0, out_row);
     __syncthreads();
 
     float y = 0.0f;
+    const uint32_t some = s_finer[lane & (NW - 1u)];
     const i32x4 zero = {0, 0, 0, 0};
     const bool block_mine = ((j >> 2) & 1u) == (kg >> 1);
     for (uint32_t base = from; base < to; base += 2u * U) {
@@ -590,8 +688,30 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
                 sum = __builtin_fmaf(sum, 256.0f, (float)acc[1]);
                 sum = __builtin_fmaf(sum, 256.0f, (float)acc[0]);
                 const uint32_t block = 2u * base + 4u * u + kg;
-                const float next = __builtin_fmaf(sum * f16_bits_to_f32(sc[u]), unit[u], y);
-                y = block < 2u * to && block < blocks ? next : y;
+                const bool used = block < 2u * to && block < blocks;
+                if constexpr (!BF16) {
+                    if (__builtin_amdgcn_ballot_w64(used && unit[u] < 0.0f)) {
+                        const char *rest = s_rest + (base + 2u * u) * Q8ONE_REST + (j & 3u) * 64u + 16u * kg;
+                        const i32x4 r0 = *(const i32x4 *)(block_mine && (j & 3u) < 2u && j < 8u ? rest : (const char *)s_zero);
+                        const i32x4 r1 = *(const i32x4 *)(block_mine && (j & 3u) < 2u && j >= 8u ? rest + Q8ONE_REST : (const char *)s_zero);
+                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(r0, __builtin_bit_cast(i32x4, w[2 * u]), zero, 0, 0, 0);
+                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(r1, __builtin_bit_cast(i32x4, w[2 * u + 1]), acc, 0, 0, 0);
+                        const float more = __builtin_fmaf((float)acc[1], 256.0f, (float)acc[0]);
+                        if (unit[u] < 0.0f) sum = __builtin_fmaf(more, 1.0f / (float)(1 << Q8WHOLE_REST), sum);
+                    }
+                }
+                const float next = __builtin_fmaf(sum * f16_bits_to_f32(sc[u]), __builtin_fabsf(unit[u]), y);
+                y = used ? next : y;
+            }
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(some != 0u)) { // uniform in the workgroup
+        for (uint32_t b = 2u * from; b < 2u * to; b += 64u) {
+            const bool more = b + lane < 2u * to && b + lane < blocks && s_unit[b + lane] < 0.0f;
+            for (uint64_t left = __builtin_amdgcn_ballot_w64(more); left; left &= left - 1u) {
+                const uint32_t block = b + (uint32_t)__builtin_ctzll(left);
+                const float rest = q8_one_rest<BF16>(a, block, normed, scale, -s_unit[block], w_src + row_on * a.cols, f16_bits_to_f32(sc_src[sc_row + block]));
+                if (kg == 0) y += rest;
             }
         }
     }
@@ -618,8 +738,9 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
 
 template <bool BF16, int NW, bool PREPARE = false>
 __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
-    if (a.cols <= 128u * NW) q8_one_turns<BF16, NW, PREPARE, 1>(a, tile, s_mem, prepare, which);
-    else q8_one_turns<BF16, NW, PREPARE, 4>(a, tile, s_mem, prepare, which);
+    __shared__ Q8OneLds<NW> lds;
+    if (a.cols <= 128u * NW) q8_one_turns<BF16, NW, PREPARE, 1>(a, tile, s_mem, lds, prepare, which);
+    else q8_one_turns<BF16, NW, PREPARE, 4>(a, tile, s_mem, lds, prepare, which);
 }
 
 // 2 to 16 f32 positions of 2,048 to 4,096 columns in one dispatch, with the RMS norm if norm_w is set: x goes through the matrix

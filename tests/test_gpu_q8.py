@@ -577,6 +577,36 @@ def test_one_position_in_whole_numbers(gpu, rows, cols, bf16):
         assert np.isnan(_product(gpu, codes, bits, to_bf16_bits(x) if bf16 else x, rows, cols, 1)).all()
 
 
+@pytest.mark.parametrize("rows,cols,bf16", [(40, 32, False), (2880, 4096, False), (5120, 2880, False), (130, 4128, False), (70, 160, False), (33, 8192, False), (33, 8224, False), (33, 12288, False),
+                                            (40, 32, True), (2880, 4096, True), (130, 5152, True), (40, 24576, True)])
+@pytest.mark.parametrize("outlier", [2.0**13, 2.0**20, 2.0**31, 2.0**45, 2.0**90])
+def test_one_position_of_values_far_apart(gpu, rows, cols, bf16, outlier):
+    """One x of each block is `outlier` times the others, and every other row has the code 0 there, so that all of its result is of the
+    small ones. An x counts with 2^-18 of itself (two bf16 values; bf16 positions: exactly) whatever else its block holds, a bf16
+    value below 2^-126 perhaps as zero; the sums round at most 64 times within a block and blocks / 32 + 16 times after it. With a
+    norm too, whose own roundings are eight of each x."""
+    from tests.helpers import from_bf16_bits, to_bf16_bits
+    codes, bits, elements = q8_test_matrix(rows, cols, 60 + rows)
+    blocks = cols // 32
+    rng = np.random.default_rng(rows + cols)
+    at = np.arange(blocks) * 32 + rng.integers(0, 32, blocks)
+    codes = codes.reshape(rows, cols).copy()
+    elements = elements.copy()
+    codes[::2, at] = 0
+    elements[::2, at] = 0.0
+    x = xorshift_values(36, cols).astype(np.float32) * 2.0**-20
+    x[at] *= np.float32(outlier)
+    w = np.exp2(np.floor(rng.random(cols) * 3)).astype(np.float32)
+    xin = (to_bf16_bits(x) if bf16 else x).reshape(1, cols)
+    exact = (from_bf16_bits(xin) if bf16 else xin)[0].astype(np.float64)
+    for norm in (None,) if bf16 or outlier > 2.0**60 else (None, w):
+        xs = exact if norm is None else exact / np.sqrt((exact * exact).mean() + 1e-5) * norm
+        got = _product(gpu, codes.reshape(-1), bits, xin, rows, cols, 1, norm)[0]
+        terms = np.abs(elements) @ np.abs(xs)
+        bound = ((0 if bf16 else 2.0**-18) + (80 + blocks / 32 + (0 if norm is None else 8)) * 2.0**-24) * terms + np.abs(elements).sum(1) * 2.0**-126
+        assert (np.abs(got - elements @ xs) <= bound).all(), np.max(np.abs(got - elements @ xs) / bound)
+
+
 @pytest.mark.parametrize("rows,cols,n", [(4098, 2048, 2), (4100, 2080, 16), (5120, 2880, 9), (5121, 3104, 3), (8192, 4096, 16), (8150, 4064, 15), (7000, 2048, 3)])
 def test_positions_split_by_the_product_itself(gpu, rows, cols, n):
     """2 to 16 f32 positions of more rows than compute units have 16 for, one dispatch with and without the RMS norm: workgroups of 18
