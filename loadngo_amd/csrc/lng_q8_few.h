@@ -388,7 +388,8 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
 // left of such a block, as whole numbers of 2^-15 of its unit, lies in two planes more, enough for x down to 2^-26; what is still
 // missing, in blocks of any spread, q8_one_rest adds. Looking for such blocks and, in most calls, adding some costs 0.3 us (without:
 // 5,120 x 2,880 5.5, with: 5.8; 2,880 x 4,096 5.3 and 5.6; from bf16, where they are rare, 5.2 and 5.3).
-// A block with an x that is not finite gives NaN, as the split into two bf16 values does.
+// An x that is not finite goes through q8_one_rest as well: an infinity of f32 gives NaN (its lower bf16 value is one), of bf16
+// infinities, and NaN where the code is 0, as in the other products.
 // Bound by memory and by what lies before and after it: 1 us until all loads are on their way, a round trip, the matrix at the
 // rate of the whole device (15.7 MB: 2.6 us), 0.8 us of sums and their way through LDS, a dispatch's start and end. In a token
 // through 24 blocks (kernel trace): 5,120 x 2,880 with norm and preparation 9.1 us -> 7.6, 2,880 x 4,096 with bias and residual
@@ -399,6 +400,7 @@ struct Q8Whole { // eight columns, a quarter of a block; the other three are in 
     uint2 plane[4];
     float unit;    // 2^-shift; negative: the block has an x of which the planes hold less than BITS
     int32_t shift;
+    bool not_finite;
     uint32_t top, low; // the block's largest, and its smallest but zero, less one
     static __device__ __forceinline__ float whole(float v, int32_t shift) { return __builtin_amdgcn_ldexpf(v, shift); }
     // what rounding leaves, in units of 2^-Q8WHOLE_REST (exact: it has no more digits than x)
@@ -410,7 +412,7 @@ struct Q8Whole { // eight columns, a quarter of a block; the other three are in 
         const uint32_t of_top = top >> 23; // (all of them below 2^-127 + exponent: what is not held is nothing in f32)
         return of_top > exponent && low < ((of_top - exponent) << 23) - 1u;
     }
-    template <int BITS> __device__ __forceinline__ void make(const float (&x)[8]) {
+    __device__ __forceinline__ void measure(const float (&x)[8]) {
         top = 0, low = ~0u;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -426,10 +428,19 @@ struct Q8Whole { // eight columns, a quarter of a block; the other three are in 
         low = low < low_one ? low : low_one;
         const uint32_t low_two = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0x4E, 0xf, 0xf, true);
         low = low < low_two ? low : low_two;
+    }
+    // An x that is not finite is left to q8_one_rest: it becomes zero here.
+    template <int BITS> __device__ __forceinline__ void make(float (&x)[8]) {
+        measure(x);
+        not_finite = top >= 0x7f800000u; // of the whole quad
+        if (not_finite) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = (__float_as_uint(x[e]) & 0x7fffffffu) >= 0x7f800000u ? 0.0f : x[e];
+            measure(x);
+        }
         const int32_t exponent = (int32_t)(top >> 23) > 7 ? (int32_t)(top >> 23) - 127 : -120; // the unit of smaller blocks: 2^-149
         shift = 29 - exponent;
-        unit = __builtin_amdgcn_ldexpf(below(30 - BITS) ? -1.0f : 1.0f, -shift);
-        if (top >= 0x7f800000u) unit = __uint_as_float(0x7fc00000u);
+        unit = __builtin_amdgcn_ldexpf(not_finite || below(30 - BITS) ? -1.0f : 1.0f, -shift);
         uint32_t q[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) q[e] = ((uint32_t)(int32_t)__builtin_rintf(whole(x[e], shift)) + 0x00808080u) ^ 0x00808080u; // signed bytes
@@ -489,13 +500,15 @@ __device__ __forceinline__ float q8_one_rest(const lng_k_q8 &a, uint32_t block, 
     for (int e = 0; e < 8; ++e) {
         const float rest = Q8Whole::rest(x[e], shift), of_rest = BF16 ? 0.0f : __builtin_truncf(rest);
         const float less = __builtin_amdgcn_ldexpf(rest - of_rest, -(shift + Q8WHOLE_REST));
-        x[e] = __builtin_fabsf(Q8Whole::whole(x[e], shift)) < 1.0f / (float)(1 << Q8WHOLE_REST) ? x[e] : less; // (all of it, which `whole` may be too small for)
+        const float whole = __builtin_fabsf(Q8Whole::whole(x[e], shift));
+        // (all of it: what `whole` may be too small for, what is not finite)
+        x[e] = whole >= 1.0f / (float)(1 << Q8WHOLE_REST) && whole <= 0x1p30f ? less : x[e];
     }
     bf16x8 hi, lo;
     q8_split8(x, hi, lo);
     const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    const floatx4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j & 1u ? lo : hi, q8_codes_to_bf16_perm(w), zero4, 0, 0, 0);
-    return (sum[0] + sum[1]) * sc;
+    const floatx4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(!BF16 && (j & 1u) ? lo : hi, q8_codes_to_bf16_perm(w), zero4, 0, 0, 0);
+    return (BF16 ? sum[0] : sum[0] + sum[1]) * sc;
 }
 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
@@ -646,7 +659,7 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
             if constexpr (BF16) {
                 finer = true;
             } else {
-                finer |= whole.below(26);
+                finer |= whole.not_finite || whole.below(26);
                 uint2 rest[2];
                 whole.make_rest(x, rest);
                 put = s_rest + (c >> 3) * Q8ONE_REST + (c & 7u) * 8u;

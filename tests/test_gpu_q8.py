@@ -555,8 +555,9 @@ def test_one_position_in_whole_numbers(gpu, rows, cols, bf16):
     """lng_q8_one takes a block of x as 30-bit whole numbers of a unit of its own: tiles of 8 to 16 rows and their remainders,
     one block, an odd number of blocks, several turns, values of a block far apart, blocks from the smallest normal numbers to
     2^60. Every sum is exact within a block; per output at most 6 roundings of a block's value, blocks / 32 + 1 of a lane's sum and
-    10 of the lanes' and wavefronts', each 2^-24 of the terms, and 2^-30 of a block's largest x for each x. A value that is not
-    finite makes its block, and the outputs, NaN."""
+    10 of the lanes' and wavefronts', each 2^-24 of the terms, and 2^-30 of a block's largest x for each x. NaN makes the outputs
+    NaN, an infinity too from f32 (the lower of its two bf16 values is NaN); from bf16 it gives infinities, and NaN where the code
+    is 0, as two positions of it do."""
     from tests.helpers import from_bf16_bits, to_bf16_bits
     codes, bits, elements = q8_test_matrix(rows, cols, 90 + rows)
     blocks = cols // 32
@@ -574,7 +575,13 @@ def test_one_position_in_whole_numbers(gpu, rows, cols, bf16):
     for bad in (np.inf, np.nan):
         x = xorshift_values(32, cols).astype(np.float32).reshape(1, cols)
         x[0, cols - 5] = bad
-        assert np.isnan(_product(gpu, codes, bits, to_bf16_bits(x) if bf16 else x, rows, cols, 1)).all()
+        got = _product(gpu, codes, bits, to_bf16_bits(x) if bf16 else x, rows, cols, 1)
+        if not bf16 or np.isnan(bad):
+            assert np.isnan(got).all()
+        else:
+            column = elements[:, cols - 5]  # (code times scale, which may be negative)
+            assert np.array_equal(got[0], np.where(column == 0, np.nan, np.copysign(np.inf, column)), equal_nan=True)
+            assert np.array_equal(got.repeat(2, 0), _product(gpu, codes, bits, to_bf16_bits(x.repeat(2, 0)), rows, cols, 2), equal_nan=True)
 
 
 @pytest.mark.parametrize("rows,cols,bf16", [(40, 32, False), (2880, 4096, False), (5120, 2880, False), (130, 4128, False), (70, 160, False), (33, 8192, False), (33, 8224, False), (33, 12288, False),
