@@ -521,8 +521,10 @@ template <int NW> struct Q8OneLds { // (one for all numbers of pairs in flight: 
     uint32_t finer[NW];
     __attribute__((aligned(16))) uint32_t zero[512]; // what lanes read that hold rows of the other block or pair
 };
-// U: twos of pairs of blocks a wavefront has in flight. 4: 4,096 columns in one turn of eight wavefronts. 1: up to 1,024 columns,
-// where what a workgroup asks for beyond its share costs more than the waits it saves (16,384 x 512 9.7 us with 4, 5.7 with 1).
+// U: twos of pairs of blocks a wavefront has in flight, no more than its share: what all wavefronts ask for beyond it costs more
+// than it saves in waits. us, with 4 / the smallest that takes the columns in one turn: 16,384 x 512 9.7 / 5.7, x 1,056 7.2 / 6.4,
+// x 1,536 10.9 / 8.8, x 2,048 11.0 / 10.0, x 2,560 12.9 / 12.0, 2,880 x 2,048 3.9 / 3.6; past 2,560 columns no gain (16,384 x 2,880
+// 11.7 / 11.8), so 4 there: 4,096 columns in one turn of eight wavefronts.
 template <bool BF16, int NW, bool PREPARE, int U>
 __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, char *s_mem, Q8OneLds<NW> &lds, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
     constexpr int T = 64 * NW;
@@ -574,8 +576,8 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
     uint16_t sc[U];
     uint4 w[2 * U];
     // (Nothing is put in place of what is not loaded: a value merged with another after a branch is copied, and waits. And what
-    // is loaded in every case is what the wait for x can count on being behind it: so the first two pairs, a pair past the run
-    // as the last one again, and all scales.)
+    // is loaded in every case is what the wait for x can count on being behind it: so the first two pairs (past the run: the last
+    // one again) and all scales.)
     auto ask = [&](uint32_t base) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -588,7 +590,7 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const uint32_t at = base + 2u * u + h, pair = at < to ? at : to ? to - 1u : 0u;
-                    if (U > 1 || h == 0 || at < to) w[2 * u + h] = *(const uint4 *)(w_src + ((pair == pairs - 1u ? w_row_odd : w_row) + 64u * pair)); // a last pair of one block: the block again
+                    if (h == 0 || (U > 1 && u == 0) || at < to) w[2 * u + h] = *(const uint4 *)(w_src + ((pair == pairs - 1u ? w_row_odd : w_row) + 64u * pair)); // a last pair of one block: the block again
                 }
             }
         }
@@ -753,6 +755,8 @@ template <bool BF16, int NW, bool PREPARE = false>
 __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, char *s_mem, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
     __shared__ Q8OneLds<NW> lds;
     if (a.cols <= 128u * NW) q8_one_turns<BF16, NW, PREPARE, 1>(a, tile, s_mem, lds, prepare, which);
+    else if (a.cols <= 256u * NW) q8_one_turns<BF16, NW, PREPARE, 2>(a, tile, s_mem, lds, prepare, which);
+    else if (a.cols <= 320u * NW) q8_one_turns<BF16, NW, PREPARE, 3>(a, tile, s_mem, lds, prepare, which);
     else q8_one_turns<BF16, NW, PREPARE, 4>(a, tile, s_mem, lds, prepare, which);
 }
 

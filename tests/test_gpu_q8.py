@@ -614,6 +614,21 @@ def test_one_position_of_values_far_apart(gpu, rows, cols, bf16, outlier):
         assert (np.abs(got - elements @ xs) <= bound).all(), np.max(np.abs(got - elements @ xs) / bound)
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("rows,cols", [(40, 1024), (40, 1056), (37, 1536), (300, 1568), (5120, 2048), (33, 2080), (2880, 2560), (33, 2592), (17, 6176)])
+def test_one_position_at_the_edges_of_what_is_in_flight(gpu, rows, cols, bf16):
+    """Columns either side of the numbers of pairs of blocks that a wavefront asks for at once, odd numbers of pairs and of blocks
+    among them; the bound of test_one_position_in_whole_numbers."""
+    from tests.helpers import from_bf16_bits, to_bf16_bits
+    codes, bits, elements = q8_test_matrix(rows, cols, 70 + rows)
+    x = xorshift_values(37, cols).astype(np.float32).reshape(1, cols)
+    xin = to_bf16_bits(x) if bf16 else x
+    exact = (from_bf16_bits(xin) if bf16 else xin)[0].astype(np.float64)
+    got = _product(gpu, codes, bits, xin, rows, cols, 1)[0]
+    largest = np.abs(elements).reshape(rows, cols // 32, 32).sum(2) @ np.abs(exact).reshape(cols // 32, 32).max(1)
+    assert (np.abs(got - elements @ exact) <= (17 + cols / 1024) * 2.0**-24 * (np.abs(elements) @ np.abs(exact)) + 2.0**-30 * largest).all()
+
+
 @pytest.mark.parametrize("rows,cols,n", [(4098, 2048, 2), (4100, 2080, 16), (5120, 2880, 9), (5121, 3104, 3), (8192, 4096, 16), (8150, 4064, 15), (7000, 2048, 3)])
 def test_positions_split_by_the_product_itself(gpu, rows, cols, n):
     """2 to 16 f32 positions of more rows than compute units have 16 for, one dispatch with and without the RMS norm: workgroups of 18
