@@ -136,7 +136,7 @@ struct lng_gpu {
     hipFunction_t q8_split_x = nullptr, q8_tiled = nullptr,
                   q8_tiled_bf16 = nullptr, q8_frag_x = nullptr;
     hipFunction_t q8_tiled_add = nullptr, q8_tiled_bf16_add = nullptr;
-    hipFunction_t q8_norm_frag = nullptr, q8_few[2] = {}, q8_one[2] = {}; // [bf16 positions]
+    hipFunction_t q8_norm_frag = nullptr, q8_few[2] = {}, q8_one[2] = {}, q8_tall[2] = {}; // [bf16 positions]
     hipFunction_t q8_few_f32 = nullptr, q8_few_split = nullptr, q8_few_split_prepare = nullptr;
     hipFunction_t q8_few_prepare = nullptr, q8_few_f32_prepare = nullptr, q8_one_prepare = nullptr;
     hipFunction_t q8_mid[2][4] = {}; // [bf16 positions][tile, see q8_mid_tile]
@@ -1082,7 +1082,7 @@ bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
     bool product = c.fn == g->q8_tiled || c.fn == g->q8_tiled_bf16 || c.fn == g->q8_tiled_add || c.fn == g->q8_tiled_bf16_add;
     product = product || c.fn == g->q8_few_f32 || c.fn == g->q8_few_split;
     for (int i = 0; i < 2; ++i) {
-        product = product || c.fn == g->q8_few[i] || c.fn == g->q8_one[i];
+        product = product || c.fn == g->q8_few[i] || c.fn == g->q8_one[i] || c.fn == g->q8_tall[i];
         for (hipFunction_t fn : g->q8_mid[i]) product = product || (fn && c.fn == fn);
     }
     if (!product) return false;
@@ -1110,7 +1110,7 @@ bool fuse_add(const lng_gpu *g, Cmd &c, const Cmd &after) {
 // `c` (the q, k and v projections of up to 16 positions) with the preparation of attention `after` it.
 // (A token through 24 blocks: f32 1,082 -> 1,023 us, bf16 1,027 -> 977, 16 sequences 1,615 -> 1,536.)
 bool fuse_prepare(const lng_gpu *g, Cmd &c, const Cmd &after) {
-    if ((after.fn != g->prepare_v4 && after.fn != g->prepare_v1) || (c.fn != g->q8_few[0] && c.fn != g->q8_few_f32 && c.fn != g->q8_few_split && c.fn != g->q8_one[0])) return false;
+    if ((after.fn != g->prepare_v4 && after.fn != g->prepare_v1) || (c.fn != g->q8_few[0] && c.fn != g->q8_few_f32 && c.fn != g->q8_few_split && c.fn != g->q8_one[0] && c.fn != g->q8_tall[0])) return false;
     lng_k_q8_prepare both{};
     both.q8 = args_of<lng_k_q8>(c);
     both.prepare = args_of<lng_k_prepare>(after);
@@ -1140,7 +1140,8 @@ bool fuse_prepare(const lng_gpu *g, Cmd &c, const Cmd &after) {
     for (const auto &out : made.outs) {
         if (!apart(out.at, out.len, a.x, ((uint64_t)(a.n - 1) * a.x_stride + a.cols) * 4) || (a.norm_w && !apart(out.at, out.len, a.norm_w, (uint64_t)a.cols * 4))) return false;
     }
-    const bool one = c.fn == g->q8_one[0], direct = c.fn == g->q8_few_f32;
+    const bool one = c.fn == g->q8_one[0] || c.fn == g->q8_tall[0], direct = c.fn == g->q8_few_f32;
+    if (one) c.grid[0] = a.tiles; // a workgroup to each
     if (one) both.prepare.first.start %= both.prepare.first.slots; // lng_q8_one_prepare: the row itself (one position is one item, not a table)
     const bool split = c.fn == g->q8_few_split;
     c.name = one ? "lng_q8_one_prepare" : split ? "lng_q8_few_split_prepare" : direct ? "lng_q8_few_f32_prepare" : "lng_q8_few_prepare";
@@ -1247,6 +1248,8 @@ extern "C" int lng_hip_open(int device, lng_gpu **out) {
         {"lng_q8_few_split", &g->q8_few_split, true},
         {"lng_q8_few_split_prepare", &g->q8_few_split_prepare, true},
         {"lng_q8_one", &g->q8_one[0], true},
+        {"lng_q8_tall", &g->q8_tall[0], true},
+        {"lng_q8_tall_bf16", &g->q8_tall[1], true},
         {"lng_q8_few_prepare", &g->q8_few_prepare, true},
         {"lng_q8_few_f32_prepare", &g->q8_few_f32_prepare, true},
         {"lng_q8_one_prepare", &g->q8_one_prepare, true},
@@ -2269,16 +2272,17 @@ bool q8_few_direct(const lng_gpu *g, const lng_k_q8 &a, uint64_t wgs) {
     return n * cols * rounds <= 18432;
 }
 
-// Rows of a workgroup of lng_q8_one: of all that a compute unit can hold at once it should get as many as the next, and no
+// Rows of a tile of lng_q8_one: of all that a compute unit can hold at once it should get as many as the next, and no
 // unit be without: 2,880 rows as 240 tiles of 12 take 5.5 us (4,096 columns), as 180 of 16 5.9; 5,120 as 428 of 12 7.6, as 320 of
-// 16 7.8 (the second workgroup of a unit waits for the first one's loads: those with two finish last).
-unsigned q8_one_rows(const lng_gpu *g, const lng_k_q8 &a) {
+// 16 7.8 (the second workgroup of a unit waits for the first one's loads: those with two finish last). Of more than `held` tiles
+// (lng_q8_tall) 16: a tile costs a good part of its time whatever its rows (9,000 x 512 as 563 of 16 4.4, as 900 of 10 5.1).
+unsigned q8_one_rows(const lng_gpu *g, const lng_k_q8 &a, uint64_t held) {
     unsigned best = 16;
     uint64_t best_load = UINT64_MAX;
     for (unsigned t = 16; t >= 8; t -= 2) { // (even: lng_q8_one_prepare takes pairs of rows)
         uint64_t wgs = (a.rows + t - 1) / t;
         for (uint32_t i = 0; i < a.n_more; ++i) wgs += (a.more[i].rows + t - 1) / t;
-        if (wgs > 2ull * g->cus) break;
+        if (wgs > held) break;
         const uint64_t load = (wgs + g->cus - 1) / g->cus * t;
         if (load < best_load) best = t, best_load = load;
     }
@@ -2310,24 +2314,32 @@ int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
         if (rc == LNG_ERR_ALLOC) direct = true; // no memory for the planes
         else if (rc) return rc;
     }
+    const uint64_t pairs = (blocks + 1) / 2, scales = blocks <= 512 ? 16 * (pairs | 1) * 4 : 0; // both of a pair of blocks in a word
+    // one: x's planes and units (Q8ONE_PAIR), of one pair more, (f32) the planes of its rest; else the scales and the weights of x's
+    // norm or the turning buffers
+    const uint64_t lds = one ? ((pairs + 1) * (256 + 8) + 15) / 16 * 16 + (x_bf16 ? 0 : (pairs + 1) * 128)
+                       : split ? 8 * 4 * 16 * 80 + 32 * (pairs | 1) * 4
+                               : scales + (direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0);
+    // Workgroups of lng_q8_one that the device holds: two a unit by their registers, one where their LDS is more than half of it
+    // (72 KB and 7 KB more that every one has).
+    const uint64_t held = (lds > 72 * 1024 ? 1ull : 2ull) * b->gpu->cus;
     if (one || split) {
-        a.one_rows = one ? q8_one_rows(b->gpu, a) : split;
+        a.one_rows = one ? q8_one_rows(b->gpu, a, held) : split;
         row_tiles = (a.rows + a.one_rows - 1) / a.one_rows;
         for (uint32_t i = 0; i < a.n_more; ++i) {
             a.more[i].first_tile = (uint32_t)row_tiles;
             row_tiles += (a.more[i].rows + a.one_rows - 1) / a.one_rows;
         }
+        a.tiles = (uint32_t)row_tiles;
     }
+    const bool many = one && row_tiles > held; // each workgroup takes several tiles, for the same planes of x
     Cmd c;
-    c.fn = one ? b->gpu->q8_one[x_bf16] : split ? b->gpu->q8_few_split : direct ? b->gpu->q8_few_f32 : b->gpu->q8_few[x_bf16];
-    c.name = one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : split ? "lng_q8_few_split" : direct ? "lng_q8_few_f32" : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
-    c.grid[0] = (unsigned)row_tiles;
+    c.fn = one ? (many ? b->gpu->q8_tall : b->gpu->q8_one)[x_bf16] : split ? b->gpu->q8_few_split : direct ? b->gpu->q8_few_f32 : b->gpu->q8_few[x_bf16];
+    c.name = many ? (x_bf16 ? "lng_q8_tall_bf16" : "lng_q8_tall") : one ? (x_bf16 ? "lng_q8_one_bf16" : "lng_q8_one") : split ? "lng_q8_few_split" : direct ? "lng_q8_few_f32" : (x_bf16 ? "lng_q8_few_bf16" : "lng_q8_few");
+    c.grid[0] = (unsigned)(many ? held : row_tiles);
     c.grid[1] = (unsigned)groups;
     c.block = 512;
-    const uint64_t pairs = (blocks + 1) / 2, scales = blocks <= 512 ? 16 * (pairs | 1) * 4 : 0; // both of a pair of blocks in a word
-    // one: x's planes and units (Q8ONE_PAIR), of one pair more, (f32) the planes of its rest; else the scales and the weights of x's
-    // norm or the turning buffers
-    c.lds = (unsigned)(one ? ((pairs + 1) * (256 + 8) + 15) / 16 * 16 + (x_bf16 ? 0 : (pairs + 1) * 128) : split ? 8 * 4 * 16 * 80 + 32 * (pairs | 1) * 4 : scales + (direct ? (a.norm_w ? a.cols * 4u : 0u) : x_bf16 ? 8 * 2 * 16 * 80 : 0));
+    c.lds = (unsigned)lds;
     set_args(c, a);
     b->cmds.push_back(std::move(c));
     return LNG_OK;

@@ -177,7 +177,7 @@ typedef struct lng_k_q8_split {
 typedef struct lng_k_q8 {
     const int8_t *codes;     /* [rows][cols] */
     const uint16_t *scales;  /* [rows][cols/32] binary16 */
-    const float *x;          /* [n][x_stride] (lng_q8_one, lng_q8_few_f32*: split by the kernel) */
+    const float *x;          /* [n][x_stride] (lng_q8_one, lng_q8_tall, lng_q8_few_f32*, lng_q8_few_split*: split by the kernel) */
     const uint16_t *x_hi;    /* [n_pad][cols] bf16 (the planes lng_q8_split_x, lng_q8_frag_x or lng_q8_norm_frag wrote) */
     const uint16_t *x_lo;
     float *y;                /* [n][y_stride] */
@@ -189,19 +189,19 @@ typedef struct lng_k_q8 {
     uint32_t plane_stride;   /* elements between positions of x_hi / x_lo: cols for the split planes; x's own stride
                                 when the positions are bf16 already (x_hi = x, no x_lo, n rows only) */
     /* Not lng_q8_tiled*: further matrices of the same dispatch, multiplied by the same x (same cols, n). Row tiles from
-     * `first_tile` on (of the kernel's own height: lng_q8_few* 16 rows, lng_q8_one* one_rows, lng_q8_mid* 16, 32 or 64) belong to
+     * `first_tile` on (of the kernel's own height: lng_q8_few* 16 rows, lng_q8_one*, lng_q8_tall* and lng_q8_few_split* one_rows, lng_q8_mid* 16, 32 or 64) belong to
      * matrix more[i]; first_tile ascends. */
     uint32_t n_more;         /* 0..LNG_Q8_MORE */
     float eps;               /* of the RMS norm, when norm_w is set */
-    /* Few positions only. norm_w (lng_q8_one*, lng_q8_few_f32*): x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
-     * (cols <= 12288). Of one matrix: bias: y gets bias[row] added (lng_q8_few*, lng_q8_one*, lng_q8_mid*, lng_q8_tiled*_add; so
+    /* Few positions only. norm_w (lng_q8_one*, lng_q8_tall, lng_q8_few_f32*, lng_q8_few_split*): x is RMS-normalised on the way in, x'[c] = (x[c] / sqrt(mean(x^2) + eps)) * norm_w[c]
+     * (cols <= 12288). Of one matrix: bias: y gets bias[row] added (lng_q8_few*, lng_q8_one*, lng_q8_tall*, lng_q8_mid*, lng_q8_tiled*_add; so
      * with residual). accumulate: the result is added to what y holds (these, but not lng_q8_tiled*_add). */
     const float *norm_w;
     const float *bias;
     float *residual;         /* [n][rows], not y: gets the result added as well, or NULL */
     uint32_t accumulate;
-    uint32_t tiles;          /* row tiles of all matrices of the dispatch (lng_q8_mid*) */
-    uint32_t one_rows;       /* lng_q8_one*, lng_q8_few_split*: rows of a tile, even, at most 16 or 32 */
+    uint32_t tiles;          /* row tiles of all matrices of the dispatch (lng_q8_mid*, lng_q8_tall*) */
+    uint32_t one_rows;       /* lng_q8_one*, lng_q8_tall*, lng_q8_few_split*: rows of a tile, even, at most 16 or 32 */
     uint32_t pad_;
     struct lng_k_q8_more {
         const int8_t *codes;

@@ -1721,22 +1721,23 @@ __device__ __forceinline__ void q8_split8(const float (&x)[8], bf16x8 &hi, bf16x
     }
 }
 
-// The matrix a workgroup of a several-matrix dispatch works on becomes the one `a` names; returns its row tile.
-__device__ __forceinline__ uint32_t q8_select_matrix(lng_k_q8 &a) {
-    uint32_t tile = blockIdx.x;
+// The matrix of row tile `id` of a several-matrix dispatch becomes the one `a` names; returns the tile within it.
+__device__ __forceinline__ uint32_t q8_select_matrix(lng_k_q8 &a, uint32_t id) {
+    uint32_t tile = id;
 #pragma unroll
     for (int i = 0; i < LNG_Q8_MORE; ++i) {
-        if ((uint32_t)i < a.n_more && blockIdx.x >= a.more[i].first_tile) { // uniform: scalar selects
+        if ((uint32_t)i < a.n_more && id >= a.more[i].first_tile) { // uniform: scalar selects
             a.codes = a.more[i].codes;
             a.scales = a.more[i].scales;
             a.y = a.more[i].y;
             a.rows = a.more[i].rows;
             a.y_stride = a.more[i].y_stride;
-            tile = blockIdx.x - a.more[i].first_tile;
+            tile = id - a.more[i].first_tile;
         }
     }
     return tile;
 }
+__device__ __forceinline__ uint32_t q8_select_matrix(lng_k_q8 &a) { return q8_select_matrix(a, blockIdx.x); }
 
 // Many positions (bound by the matrix unit): a workgroup of eight wavefronts takes 256 rows x 128
 // positions, wavefront (w % 4, w / 4) the 64 x 64 corner of it: four 16-row B operands of codes

@@ -479,13 +479,20 @@ template <bool BF16>
 __device__ __forceinline__ float q8_one_rest(const lng_k_q8 &a, uint32_t block, bool normed, float scale, float unit, const int8_t *codes, float sc) {
     const uint32_t lane = threadIdx.x & 63u, j = lane & 15u, at = block * 32u + (lane >> 4) * 8u; // this lane's columns
     float x[8];
+    uint4 x16;
+    float4 u, v;
     if constexpr (BF16) {
-        const uint4 x16 = *(const uint4 *)(a.x_hi + at);
+        x16 = *(const uint4 *)(a.x_hi + at);
+    } else {
+        u = *(const float4 *)(a.x + at), v = *(const float4 *)(a.x + at + 4u);
+    }
+    const uint2 w = *(const uint2 *)(codes + at);
+    __builtin_amdgcn_sched_barrier(0); // (both on their way before either is waited for)
+    if constexpr (BF16) {
         const uint32_t half[4] = {x16.x, x16.y, x16.z, x16.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[2 * e] = __uint_as_float(half[e] << 16), x[2 * e + 1] = __uint_as_float(half[e] & 0xffff0000u);
     } else {
-        const float4 u = *(const float4 *)(a.x + at), v = *(const float4 *)(a.x + at + 4u);
         x[0] = u.x, x[1] = u.y, x[2] = u.z, x[3] = u.w, x[4] = v.x, x[5] = v.y, x[6] = v.z, x[7] = v.w;
         if (normed) {
             const float4 n = *(const float4 *)(a.norm_w + at), m = *(const float4 *)(a.norm_w + at + 4u);
@@ -494,7 +501,6 @@ __device__ __forceinline__ float q8_one_rest(const lng_k_q8 &a, uint32_t block, 
             for (int e = 0; e < 8; ++e) x[e] = x[e] * scale * nw[e];
         }
     }
-    const uint2 w = *(const uint2 *)(codes + at);
     const int32_t shift = 1 - __builtin_amdgcn_frexp_expf(unit);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -516,8 +522,8 @@ typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 // (f32) the planes of the rest.
 #define Q8ONE_PAIR 256u // bytes
 #define Q8ONE_REST 128u
-template <int NW> struct Q8OneLds { // (one for all numbers of pairs in flight: each would have its own)
-    float red[NW][64], norm[NW];
+template <int NW, int REDS = 1> struct Q8OneLds { // (one for all numbers of pairs in flight: each would have its own)
+    float red[REDS][NW][64], norm[NW];
     uint32_t finer[NW];
     __attribute__((aligned(16))) uint32_t zero[512]; // what lanes read that hold rows of the other block or pair
 };
@@ -525,10 +531,11 @@ template <int NW> struct Q8OneLds { // (one for all numbers of pairs in flight: 
 // than it saves in waits. us, with 4 / the smallest that takes the columns in one turn: 16,384 x 512 9.7 / 5.7, x 1,056 7.2 / 6.4,
 // x 1,536 10.9 / 8.8, x 2,048 11.0 / 10.0, x 2,560 12.9 / 12.0, 2,880 x 2,048 3.9 / 3.6; past 2,560 columns no gain (16,384 x 2,880
 // 11.7 / 11.8), so 4 there: 4,096 columns in one turn of eight wavefronts.
-template <bool BF16, int NW, bool PREPARE, int U>
-__device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, char *s_mem, Q8OneLds<NW> &lds, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
+// MANY: the workgroup takes the row tiles blockIdx.x, blockIdx.x + gridDim.x, .. of a.tiles, of all matrices that `a` names, and asks
+// for the next one's codes before it puts the sums of one together. (Else one tile, of the matrix that `a` has been made to name.)
+template <bool BF16, int NW, bool PREPARE, int U, bool MANY = false>
+__device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, char *s_mem, Q8OneLds<NW, MANY ? 2 : 1> &lds, const lng_k_prepare *prepare = nullptr, uint32_t which = 0) {
     constexpr int T = 64 * NW;
-    float (&s_red)[NW][64] = lds.red;
     float (&s_norm)[NW] = lds.norm;
     uint32_t (&s_finer)[NW] = lds.finer, (&s_zero)[512] = lds.zero;
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15u, kg = lane >> 4;
@@ -536,23 +543,45 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
     const uint32_t from = wave * pairs / NW, to = (wave + 1u) * pairs / NW;
     // The tile's rows, the instruction's columns: a.one_rows of them, one after another or (PREPARE: what rotation by halves pairs
     // belongs to one tile) half as many pairs of rows 32 apart, in lanes j and j + 8. The columns past them repeat the last.
-    uint32_t row;      // of the matrix
-    bool row_mine;
-    if constexpr (PREPARE) {
-        const uint32_t half = a.one_rows / 2u, first = tile * half, last = (a.rows / 2u - first < half ? a.rows / 2u - first : half) - 1u;
-        const uint32_t pair = first + ((j & 7u) < last ? j & 7u : last);
-        row = (pair >> 5) * 64u + (pair & 31u) + (j & 8u) * 4u;
-        row_mine = (j & 7u) <= last;
-    } else {
-        const uint32_t first = tile * a.one_rows, last = (a.rows - first < a.one_rows ? a.rows - first : a.one_rows) - 1u;
-        row = first + (j < last ? j : last);
-        row_mine = j <= last;
-    }
     // (a uniform base and 32-bit offsets: a row of the tile is at most 127 x 24,576 bytes on)
-    const uint32_t r0 = __builtin_amdgcn_readfirstlane(row), row_on = row - r0, out_row = row;
-    const int8_t *w_src = a.codes + (uint64_t)r0 * a.cols;
-    const uint16_t *sc_src = a.scales + (uint64_t)r0 * blocks;
-    const uint32_t w_row = row_on * a.cols + 16u * kg, w_row_odd = w_row - ((blocks & 1u) && kg >= 2u ? 32u : 0u), sc_row = row_on * blocks;
+    bool row_mine;
+    uint32_t row_on, out_row, w_row, w_row_odd, sc_row; // out_row: of the matrix
+    const int8_t *w_src;
+    const uint16_t *sc_src;
+    float *y_dst;
+    auto aim = [&](const int8_t *codes, const uint16_t *scales, float *to, uint32_t rows, uint32_t at) {
+        if constexpr (PREPARE) {
+            const uint32_t half = a.one_rows / 2u, first = at * half, last = (rows / 2u - first < half ? rows / 2u - first : half) - 1u;
+            const uint32_t pair = first + ((j & 7u) < last ? j & 7u : last);
+            out_row = (pair >> 5) * 64u + (pair & 31u) + (j & 8u) * 4u;
+            row_mine = (j & 7u) <= last;
+        } else {
+            const uint32_t first = at * a.one_rows, last = (rows - first < a.one_rows ? rows - first : a.one_rows) - 1u;
+            out_row = first + (j < last ? j : last);
+            row_mine = j <= last;
+        }
+        const uint32_t r0 = __builtin_amdgcn_readfirstlane(out_row);
+        row_on = out_row - r0;
+        w_src = codes + (uint64_t)r0 * a.cols;
+        sc_src = scales + (uint64_t)r0 * blocks;
+        w_row = row_on * a.cols + 16u * kg;
+        w_row_odd = w_row - ((blocks & 1u) && kg >= 2u ? 32u : 0u);
+        sc_row = row_on * blocks;
+        y_dst = to;
+    };
+    auto aim_at = [&](uint32_t id) {
+        uint32_t of = 0; // 1 + the one of a.more
+#pragma unroll
+        for (uint32_t i = 0; i < LNG_Q8_MORE; ++i) of = i < a.n_more && id >= a.more[i].first_tile ? i + 1u : of;
+        if (of == 0) {
+            aim(a.codes, a.scales, a.y, a.rows, id);
+        } else {
+            const auto &m = a.more[of - 1u];
+            aim(m.codes, m.scales, m.y, m.rows, id - m.first_tile);
+        }
+    };
+    if constexpr (MANY) aim_at(tile);
+    else aim(a.codes, a.scales, a.y, a.rows, tile);
     float *s_unit = (float *)(s_mem + (pairs + 1u) * Q8ONE_PAIR);
     char *s_rest = s_mem + ((pairs + 1u) * (Q8ONE_PAIR + 8u) + 15u) / 16u * 16u;
 
@@ -601,14 +630,17 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
     ask(from);
     const float *any = (const float *)a.codes;
     float bias, held;
-    if constexpr (U > 1) {
-        bias = *(a.bias ? a.bias + out_row : any);
-        held = *(a.accumulate ? a.y + out_row : a.residual ? a.residual + out_row : any); // (never both)
-    } else {
-        if (a.bias) bias = a.bias[out_row];
-        if (a.accumulate) held = a.y[out_row];
-        if (a.residual) held = a.residual[out_row];
-    }
+    auto ask_added = [&] {
+        if constexpr (U > 1) {
+            bias = *(a.bias ? a.bias + out_row : any);
+            held = *(a.accumulate ? y_dst + out_row : a.residual ? a.residual + out_row : any); // (never both)
+        } else {
+            if (a.bias) bias = a.bias[out_row];
+            if (a.accumulate) held = y_dst[out_row];
+            if (a.residual) held = a.residual[out_row];
+        }
+    };
+    ask_added();
     Q8Prepared ready;
     if constexpr (PREPARE) ready.ask<true>(*prepare, which, 0, out_row, any);
     __builtin_amdgcn_sched_barrier(0);
@@ -675,79 +707,98 @@ __device__ __forceinline__ void q8_one_turns(const lng_k_q8 &a, uint32_t tile, c
     if constexpr (PREPARE) ready.place<true>(*prepare, which, 0, out_row);
     __syncthreads();
 
-    float y = 0.0f;
     const uint32_t some = s_finer[lane & (NW - 1u)];
     const i32x4 zero = {0, 0, 0, 0};
     const bool block_mine = ((j >> 2) & 1u) == (kg >> 1);
-    for (uint32_t base = from; base < to; base += 2u * U) {
-        if (base != from) ask(base);
-        const char *planes = s_mem + base * Q8ONE_PAIR + (j & 3u) * 64u + 16u * kg;
-        const char *first = block_mine && j < 8u ? planes : (const char *)s_zero;
-        const char *second = block_mine && j >= 8u ? planes + Q8ONE_PAIR : (const char *)s_zero;
-        i32x4 p[2 * U];
-        float unit[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (u == 0 || base + 2u * u < to) {
-                p[2 * u] = *(const i32x4 *)(first + 2u * u * Q8ONE_PAIR);
-                p[2 * u + 1] = *(const i32x4 *)(second + 2u * u * Q8ONE_PAIR);
-                unit[u] = s_unit[2u * base + 4u * u + kg];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (u == 0 || base + 2u * u < to) {
-                i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(p[2 * u], __builtin_bit_cast(i32x4, w[2 * u]), zero, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(p[2 * u + 1], __builtin_bit_cast(i32x4, w[2 * u + 1]), acc, 0, 0, 0);
-                float sum = __builtin_fmaf((float)acc[3], 256.0f, (float)acc[2]);
-                sum = __builtin_fmaf(sum, 256.0f, (float)acc[1]);
-                sum = __builtin_fmaf(sum, 256.0f, (float)acc[0]);
-                const uint32_t block = 2u * base + 4u * u + kg;
-                const bool used = block < 2u * to && block < blocks;
-                if constexpr (!BF16) {
-                    if (__builtin_amdgcn_ballot_w64(used && unit[u] < 0.0f)) {
-                        const char *rest = s_rest + (base + 2u * u) * Q8ONE_REST + (j & 3u) * 64u + 16u * kg;
-                        const i32x4 r0 = *(const i32x4 *)(block_mine && (j & 3u) < 2u && j < 8u ? rest : (const char *)s_zero);
-                        const i32x4 r1 = *(const i32x4 *)(block_mine && (j & 3u) < 2u && j >= 8u ? rest + Q8ONE_REST : (const char *)s_zero);
-                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(r0, __builtin_bit_cast(i32x4, w[2 * u]), zero, 0, 0, 0);
-                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(r1, __builtin_bit_cast(i32x4, w[2 * u + 1]), acc, 0, 0, 0);
-                        const float more = __builtin_fmaf((float)acc[1], 256.0f, (float)acc[0]);
-                        if (unit[u] < 0.0f) sum = __builtin_fmaf(more, 1.0f / (float)(1 << Q8WHOLE_REST), sum);
-                    }
+    for (uint32_t round = 0;; ++round) { // (!MANY: once)
+        float y = 0.0f;
+        for (uint32_t base = from; base < to; base += 2u * U) {
+            if (base != from) ask(base);
+            const char *planes = s_mem + base * Q8ONE_PAIR + (j & 3u) * 64u + 16u * kg;
+            const char *first = block_mine && j < 8u ? planes : (const char *)s_zero;
+            const char *second = block_mine && j >= 8u ? planes + Q8ONE_PAIR : (const char *)s_zero;
+            i32x4 p[2 * U];
+            float unit[U];
+    #pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (u == 0 || base + 2u * u < to) {
+                    p[2 * u] = *(const i32x4 *)(first + 2u * u * Q8ONE_PAIR);
+                    p[2 * u + 1] = *(const i32x4 *)(second + 2u * u * Q8ONE_PAIR);
+                    unit[u] = s_unit[2u * base + 4u * u + kg];
                 }
-                const float next = __builtin_fmaf(sum * f16_bits_to_f32(sc[u]), __builtin_fabsf(unit[u]), y);
-                y = used ? next : y;
+            }
+    #pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (u == 0 || base + 2u * u < to) {
+                    i32x4 acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(p[2 * u], __builtin_bit_cast(i32x4, w[2 * u]), zero, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(p[2 * u + 1], __builtin_bit_cast(i32x4, w[2 * u + 1]), acc, 0, 0, 0);
+                    float sum = __builtin_fmaf((float)acc[3], 256.0f, (float)acc[2]);
+                    sum = __builtin_fmaf(sum, 256.0f, (float)acc[1]);
+                    sum = __builtin_fmaf(sum, 256.0f, (float)acc[0]);
+                    const uint32_t block = 2u * base + 4u * u + kg;
+                    const bool used = block < 2u * to && block < blocks;
+                    if constexpr (!BF16) {
+                        if (__builtin_amdgcn_ballot_w64(used && unit[u] < 0.0f)) {
+                            const char *rest = s_rest + (base + 2u * u) * Q8ONE_REST + (j & 3u) * 64u + 16u * kg;
+                            const i32x4 r0 = *(const i32x4 *)(block_mine && (j & 3u) < 2u && j < 8u ? rest : (const char *)s_zero);
+                            const i32x4 r1 = *(const i32x4 *)(block_mine && (j & 3u) < 2u && j >= 8u ? rest + Q8ONE_REST : (const char *)s_zero);
+                            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(r0, __builtin_bit_cast(i32x4, w[2 * u]), zero, 0, 0, 0);
+                            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(r1, __builtin_bit_cast(i32x4, w[2 * u + 1]), acc, 0, 0, 0);
+                            const float more = __builtin_fmaf((float)acc[1], 256.0f, (float)acc[0]);
+                            if (unit[u] < 0.0f) sum = __builtin_fmaf(more, 1.0f / (float)(1 << Q8WHOLE_REST), sum);
+                        }
+                    }
+                    const float next = __builtin_fmaf(sum * f16_bits_to_f32(sc[u]), __builtin_fabsf(unit[u]), y);
+                    y = used ? next : y;
+                }
             }
         }
-    }
-    if (__builtin_amdgcn_ballot_w64(some != 0u)) { // uniform in the workgroup
-        for (uint32_t b = 2u * from; b < 2u * to; b += 64u) {
-            const bool more = b + lane < 2u * to && b + lane < blocks && s_unit[b + lane] < 0.0f;
-            for (uint64_t left = __builtin_amdgcn_ballot_w64(more); left; left &= left - 1u) {
-                const uint32_t block = b + (uint32_t)__builtin_ctzll(left);
-                const float rest = q8_one_rest<BF16>(a, block, normed, scale, -s_unit[block], w_src + row_on * a.cols, f16_bits_to_f32(sc_src[sc_row + block]));
-                if (kg == 0) y += rest;
+        if (__builtin_amdgcn_ballot_w64(some != 0u)) { // uniform in the workgroup
+            for (uint32_t b = 2u * from; b < 2u * to; b += 64u) {
+                const bool more = b + lane < 2u * to && b + lane < blocks && s_unit[b + lane] < 0.0f;
+                for (uint64_t left = __builtin_amdgcn_ballot_w64(more); left; left &= left - 1u) {
+                    const uint32_t block = b + (uint32_t)__builtin_ctzll(left);
+                    const float rest = q8_one_rest<BF16>(a, block, normed, scale, -s_unit[block], w_src + row_on * a.cols, f16_bits_to_f32(sc_src[sc_row + block]));
+                    if (kg == 0) y += rest;
+                }
             }
         }
-    }
-    s_red[wave][lane] = y;
-    __syncthreads();
-    if (wave != 0) return;
-    float sum = 0.0f;
+        float (&s_red)[NW][64] = lds.red[MANY ? round & 1u : 0u]; // (in turn: one may still be read when the other is written)
+        float *const to_y = y_dst;
+        const uint32_t to_row = out_row;
+        const bool writes = lane < 16u && row_mine;
+        const float bias_now = bias, held_now = held;
+        const bool again = MANY && tile + gridDim.x < a.tiles; // uniform
+        if constexpr (MANY) {
+            if (again) {
+                tile += gridDim.x;
+                aim_at(tile);
+                ask(from);
+                ask_added();
+            }
+        }
+        s_red[wave][lane] = y;
+        __syncthreads();
+        if (wave == (MANY ? round % NW : 0u)) {
+            float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NW; ++i) sum += s_red[i][lane];
-    const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
-    sum = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
-    const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
-    sum = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
-    if (a.bias) sum = sum + bias;
-    if (a.accumulate) sum = held + sum;
-    if (lane >= 16u || !row_mine) return;
-    a.y[out_row] = sum;
-    if (a.residual) a.residual[out_row] = held + sum;
-    if constexpr (PREPARE) {
-        const float there = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sum), 0x128, 0xf, 0xf, true)); // row_ror:8, 32 rows away
-        ready.store(*prepare, which, out_row, sum, there);
+            for (int i = 0; i < NW; ++i) sum += s_red[i][lane];
+            const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+            sum = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
+            const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+            sum = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
+            if (a.bias) sum = sum + bias_now;
+            if (a.accumulate) sum = held_now + sum;
+            if (writes) {
+                to_y[to_row] = sum;
+                if (a.residual) a.residual[to_row] = held_now + sum;
+                if constexpr (PREPARE) {
+                    const float there = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(sum), 0x128, 0xf, 0xf, true)); // row_ror:8, 32 rows away
+                    ready.store(*prepare, which, to_row, sum, there);
+                }
+            }
+        }
+        if (!again) return;
     }
 }
 
@@ -758,6 +809,22 @@ __device__ __forceinline__ void q8_one_body(const lng_k_q8 &a, uint32_t tile, ch
     else if (a.cols <= 256u * NW) q8_one_turns<BF16, NW, PREPARE, 2>(a, tile, s_mem, lds, prepare, which);
     else if (a.cols <= 320u * NW) q8_one_turns<BF16, NW, PREPARE, 3>(a, tile, s_mem, lds, prepare, which);
     else q8_one_turns<BF16, NW, PREPARE, 4>(a, tile, s_mem, lds, prepare, which);
+}
+
+// One position of more tiles than the device holds workgroups of. When each tile was a workgroup, the planes of x were made for
+// every one of them, 1 us that the codes of the next did not hide. us, f32 positions, the kernel before the integer one / a tile a
+// workgroup / so: 16,384 x 512 5.6 / 5.4 / 5.2, 65,536 x 1,024 20.4 / 22.0 / 15.4, x 2,880 35.7 / 37.5 / 35.2, x 4,096 50.0 / 55.7 / 50.5;
+// with the norm 6.7 / 6.6 / 5.9, 23.8 / 28.1 / 16.2, 39.2 / 43.2 / 35.5, 52.0 / 60.7 / 51.3. 150,000 x 4,096 105 / 119 / 109, x 2,880 74.5 / 79.1 /
+// 76.3 (with the norm 109 / 130 / 110, 81 / 93 / 77).
+// As many tiles to each workgroup, one grid apart: a run of neighbours to each is 5 to 8 % slower, workgroups of 2 to 9 tiles each up
+// to 45 %. Three twos of pairs in flight where they are all of a turn (24,576 x 2,880 16.7 with two, 15.3); more (9 % slower at
+// 4,096 columns, and f32 keeps registers in memory) or a third workgroup in a unit (1 % slower) read no faster.
+template <bool BF16, int NW>
+__device__ __forceinline__ void q8_tall_body(const lng_k_q8 &a, char *s_mem) {
+    __shared__ Q8OneLds<NW, 2> lds;
+    if (a.cols <= 128u * NW) q8_one_turns<BF16, NW, false, 1, true>(a, blockIdx.x, s_mem, lds);
+    else if (a.cols <= 256u * NW || a.cols > 384u * NW) q8_one_turns<BF16, NW, false, 2, true>(a, blockIdx.x, s_mem, lds);
+    else q8_one_turns<BF16, NW, false, 3, true>(a, blockIdx.x, s_mem, lds);
 }
 
 // 2 to 16 f32 positions of 2,048 to 4,096 columns in one dispatch, with the RMS norm if norm_w is set: x goes through the matrix
@@ -984,6 +1051,14 @@ Q8_FEW(lng_q8_few_bf16, q8_few_body, Q8F_BF16, 8)
 Q8_FEW(lng_q8_few_f32, q8_few_body, Q8F_F32, 8)
 Q8_FEW(lng_q8_one, q8_one_body, false, 8)
 Q8_FEW(lng_q8_one_bf16, q8_one_body, true, 8)
+
+#define Q8_TALL(name, bf16, nw) \
+    extern "C" __global__ __launch_bounds__(64 * nw, nw / 2) void name(lng_k_q8 a) { \
+        extern __shared__ __attribute__((aligned(16))) char s_mem[]; \
+        q8_tall_body<bf16, nw>(a, s_mem); \
+    }
+Q8_TALL(lng_q8_tall, false, 8)
+Q8_TALL(lng_q8_tall_bf16, true, 8)
 
 // q, k and v with the preparation of attention after them.
 #define Q8_FEW_PREPARE(name, body, what, nw) \

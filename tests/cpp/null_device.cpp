@@ -248,6 +248,26 @@ static void products_and_their_kernels() {
     CHECK(lng_hip_batch_dispatches(f.batch) == 3);
     const std::vector<std::string> names = run();
     CHECK((names == std::vector<std::string>{"lng_q8_frag_x", "lng_q8_mid_r32p32", "lng_q8_split_x", "lng_q8_tiled"}));
+    // one position: past as many tiles of 16 rows as the device holds workgroups, each workgroup takes several
+    const struct { uint64_t rows, cols; bool bf16; const char *kernel; uint32_t grid, tile, tiles; } ones[] = {
+        {8192, 96, false, "lng_q8_one", 512, 16, 512}, {8193, 96, false, "lng_q8_tall", 512, 16, 513}, {65536, 96, true, "lng_q8_tall_bf16", 512, 16, 4096},
+        {2880, 2880, true, "lng_q8_one_bf16", 240, 12, 240}, {4096, 12288, false, "lng_q8_one", 256, 16, 256}, {4097, 12288, false, "lng_q8_tall", 256, 16, 257}};
+    for (const auto &w : ones) {
+        const lng_slice x{2, 0, w.cols * (w.bf16 ? 2u : 4u)}, y{3, 0, w.rows * 4};
+        CHECK((w.bf16 ? lng_hip_gemm_q8_0_bf16 : lng_hip_gemm_q8_0)(f.batch, lng_slice{0, 0, w.rows * w.cols}, lng_slice{1, 0, w.rows * w.cols / 16}, x, y, w.rows, w.cols, 1, w.cols, w.rows) == LNG_OK);
+        CHECK(lng_hip_batch_commit(f.batch, nullptr, nullptr) == LNG_OK && lng_hip_batch_wait(f.batch, nullptr) == LNG_OK);
+        const std::vector<std::string> names = launched();
+        const char *name = nullptr;
+        unsigned grid[3], block[3];
+        const void *args = nullptr;
+        size_t size = 0;
+        CHECK(names == std::vector<std::string>{w.kernel} && lng_null_launch(0, &name, grid, block, &args, &size) == 0 && size == sizeof(lng_k_q8));
+        const lng_k_q8 *a = (const lng_k_q8 *)args;
+        if (grid[0] != w.grid || a->one_rows != w.tile || a->tiles != w.tiles) fprintf(stderr, "%llu x %llu: %u workgroups, %u tiles of %u\n", (unsigned long long)w.rows, (unsigned long long)w.cols, grid[0], a->tiles, a->one_rows);
+        CHECK(grid[0] == w.grid && a->one_rows == w.tile && a->tiles == w.tiles && block[0] == 512);
+        lng_null_clear();
+        f.rebatch();
+    }
     // 2 to 31 positions: f32 ones are split by the product itself where that is less than a dispatch before it
     typedef std::vector<std::string> Names;
     auto few = [&](uint64_t rows, uint64_t cols, uint64_t n, bool normed) {

@@ -629,6 +629,67 @@ def test_one_position_at_the_edges_of_what_is_in_flight(gpu, rows, cols, bf16):
     assert (np.abs(got - elements @ exact) <= (17 + cols / 1024) * 2.0**-24 * (np.abs(elements) @ np.abs(exact)) + 2.0**-30 * largest).all()
 
 
+@pytest.mark.parametrize("kind", ["f32", "norm", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(8193, 32), (9001, 96), (12290, 1024), (16400, 1056), (8195, 2080), (8200, 3104), (8210, 4128), (4100, 12288)])
+def test_one_position_of_many_rows(gpu, rows, cols, kind):
+    """More tiles than the device holds workgroups: each workgroup takes several, the last of them fewer rows; every number of pairs in
+    flight, one workgroup a unit too (12,288 columns). Bit for bit what parts of the matrix give that are a workgroup to a tile - an
+    output's sum knows nothing of the other rows - with values far apart in every block; and within the reference's bound (glue.rs:171)
+    of float64."""
+    from tests.helpers import from_bf16_bits, to_bf16_bits
+    codes, bits, elements = q8_test_matrix(rows, cols, 91)
+    x = xorshift_values(38, cols).astype(np.float32)
+    x[5::32] *= np.float32(2.0**28)
+    x[9::64] *= np.float32(2.0**-14)
+    xin = (to_bf16_bits(x) if kind == "bf16" else x).reshape(1, cols)
+    w = xorshift_values(39, cols).astype(np.float32) + 1.0 if kind == "norm" else None
+    got = _product(gpu, codes, bits, xin, rows, cols, 1, w)[0]
+    step = 2000
+    for at in range(0, rows, step):
+        part = min(step, rows - at)
+        assert np.array_equal(got[at:at + part], _product(gpu, codes[at * cols:][:part * cols], bits[at * cols // 32:][:part * cols // 32], xin, part, cols, 1, w)[0])
+    exact = (from_bf16_bits(xin) if kind == "bf16" else xin)[0].astype(np.float64)
+    if kind == "norm":
+        exact = exact / np.sqrt((exact * exact).mean() + 1e-5) * w
+    want = elements @ exact
+    assert np.abs(got - want).max() / np.abs(want).max() < 1e-5
+
+
+def test_one_position_of_many_rows_in_several_matrices_and_added(gpu):
+    """Several matrices whose tiles together are more than the device holds workgroups, and one such with bias and residual: bit for bit
+    each matrix alone, and the sums of the separate dispatches."""
+    cols, shapes = 288, [5003, 64, 4200]
+    mats = [q8_test_matrix(r, cols, 92 + i) for i, r in enumerate(shapes)]
+    x = xorshift_values(46, cols).astype(np.float32).reshape(1, cols)
+    bufs = [gpu.upload(x)] + [gpu.upload(a) for m in mats for a in m[:2]] + [gpu.buffer(4 * sum(shapes))]
+    bufs[-1].fill(0xFF)
+    batch = gpu.batch(bufs)
+    starts = [0] + list(np.cumsum(shapes))
+    batch.gemm_q8_0_many([((C.Slice(1 + 2 * i, 0, r * cols), C.Slice(2 + 2 * i, 0, r * cols // 16)), C.Slice(7, 4 * int(starts[i]), 4 * r), r)
+                          for i, r in enumerate(shapes)], C.Slice(0, 0, cols * 4), cols, 1, cols)
+    done = batch.run()
+    assert not isinstance(done.gpu_time, Exception), done.gpu_time
+    got = bufs[-1].read(np.float32)
+    batch.drop()
+    for b in bufs:
+        b.free()
+    for i, r in enumerate(shapes):
+        assert np.array_equal(got[starts[i]:starts[i + 1]], _product(gpu, mats[i][0], mats[i][1], x, r, cols, 1)[0])
+    rows = 9001
+    codes, bits, _ = q8_test_matrix(rows, cols, 96)
+    bias, h = xorshift_values(47, rows).astype(np.float32), xorshift_values(48, rows).astype(np.float32)
+    y = _product(gpu, codes, bits, x, rows, cols, 1)[0]
+    bufs = [gpu.upload(a) for a in (codes, bits, x, bias, h)]
+    batch = gpu.batch(bufs)
+    batch.gemm_q8_0_residual((C.Slice(0, 0, rows * cols), C.Slice(1, 0, rows * cols // 16)), C.Slice(2, 0, cols * 4), C.Slice(3, 0, rows * 4), C.Slice(4, 0, rows * 4), rows, cols, 1, (cols, rows))
+    done = batch.run()
+    assert not isinstance(done.gpu_time, Exception), done.gpu_time
+    assert np.array_equal(bufs[4].read(np.float32), h + (y + bias))
+    batch.drop()
+    for b in bufs:
+        b.free()
+
+
 @pytest.mark.parametrize("rows,cols,n", [(4098, 2048, 2), (4100, 2080, 16), (5120, 2880, 9), (5121, 3104, 3), (8192, 4096, 16), (8150, 4064, 15), (7000, 2048, 3)])
 def test_positions_split_by_the_product_itself(gpu, rows, cols, n):
     """2 to 16 f32 positions of more rows than compute units have 16 for, one dispatch with and without the RMS norm: workgroups of 18

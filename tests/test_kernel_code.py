@@ -43,3 +43,15 @@ def test_products_of_few_positions_ask_for_all_before_they_wait(kernels):
         early = [] if "prepare" in name else [line for line in code[name][:loads[7]] if re.match(r"s_waitcnt.*vmcnt", line)]
         assert not early, "%s waits for memory before it has asked for its first eight loads of 16 bytes" % name
         assert scratch[name] == 0, "%s keeps %d bytes a lane in memory" % (name, scratch[name])
+
+
+def test_products_of_one_position_and_many_rows(kernels):
+    """lng_q8_tall*, which ask for fewer at once and for the next tile's before the sums of one."""
+    code, scratch = kernels
+    names = [n for n in code if re.fullmatch(r"lng_q8_tall\w*", n)]
+    assert sorted(names) == ["lng_q8_tall", "lng_q8_tall_bf16"]
+    for name in names:
+        loads = [i for i, line in enumerate(code[name]) if line.startswith("global_load_dwordx4")]
+        waited = [i for i in loads if re.match(r"s_waitcnt vmcnt\(0\)", code[name][i + 1])]
+        assert len(loads) >= 24 and len(waited) <= 1, "%s waits for %d of its %d loads of 16 bytes one by one" % (name, len(waited), len(loads))
+        assert scratch[name] == 0, "%s keeps %d bytes a lane in memory" % (name, scratch[name])
