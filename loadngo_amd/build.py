@@ -58,22 +58,21 @@ def build(verbose=False):
     return LIB
 
 
-RECORD = os.path.join(HERE, "_record.so")
-
-
 def build_record(verbose=False):
-    """csrc/lng_record.cpp, the short way from compute.py into the library; without Python's headers compute.py does
-    without it."""
-    include = sysconfig.get_paths()["include"]
-    if not os.path.exists(os.path.join(include, "Python.h")):
-        if os.path.exists(RECORD):
-            os.remove(RECORD)  # of an older build: may not fit the library any more
+    """csrc/lng_record.cpp, the short way from compute.py into the library, under the name that this Python alone imports;
+    without Python's headers compute.py does without it."""
+    for name in os.listdir(HERE):
+        if name.startswith("_record.") and name.endswith(".so"):
+            os.remove(os.path.join(HERE, name))  # of an older build or another Python: may not fit the library any more
+    paths = sysconfig.get_paths()
+    if not os.path.exists(os.path.join(paths["include"], "Python.h")):
         return None
-    out = _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-Wextra", "-Wno-cast-function-type", "-I" + include,
-                os.path.join(CSRC, "lng_record.cpp"), "-o", RECORD])
+    record = os.path.join(HERE, "_record" + sysconfig.get_config_var("EXT_SUFFIX"))
+    out = _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-Wextra", "-Wno-cast-function-type", "-I" + paths["include"],
+                os.path.join(CSRC, "lng_record.cpp"), "-o", record])
     if verbose and out:
         print(out)
-    return RECORD
+    return record
 
 
 NULL_LIB = os.path.join(HERE, "liblng_hip_null.so")

@@ -4,6 +4,7 @@ null device, in a process of its own (a process binds one library)."""
 import os
 import subprocess
 import sys
+import sysconfig
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "loadngo_amd", "csrc")
@@ -172,3 +173,14 @@ def test_the_short_way_and_ctypes_make_the_same_calls(tmp_path):
     assert run.returncode == 0, run.stdout[-4000:]
     first, second, _ = run.stdout.split("--\n")
     assert first == second, run.stdout
+
+
+def test_the_extension_is_named_for_the_python_it_was_built_for(tmp_path, monkeypatch):
+    """One without a tag would be imported by any Python, whatever its objects look like."""
+    from loadngo_amd import build
+    (tmp_path / "_record.so").write_bytes(b"of an older build")
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    made = build.build_record()
+    assert [p.name for p in tmp_path.iterdir()] == ["_record" + sysconfig.get_config_var("EXT_SUFFIX")] == [os.path.basename(made)]
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})  # without headers: none, and none left
+    assert build.build_record() is None and list(tmp_path.iterdir()) == []
