@@ -28,6 +28,7 @@
 #include <random>
 #include <string>
 #include <thread>
+#include <tuple>
 #include <vector>
 
 #include "../../include/lng_hip.h"
@@ -284,6 +285,12 @@ static void products_and_their_kernels() {
         CHECK(few(2048, 512, 31, normed) == Names{"lng_q8_few_f32"});
         CHECK((few(2880, 2880, 31, normed) == Names{"lng_q8_norm_frag", "lng_q8_few"}));
         CHECK((few(4096, 2880, 31, normed) == Names{"lng_q8_norm_frag", "lng_q8_mid_r32p32"}));
+        // 2 to 16 positions of 2,048 to 4,096 columns and more rows than a workgroup of 16 a unit takes, up to 32
+        const Names planes{"lng_q8_norm_frag", "lng_q8_few"}, split{"lng_q8_few_split"};
+        CHECK(few(4096, 2880, 16, normed) == planes && few(4097, 2880, 16, normed) == split && few(8192, 2880, 16, normed) == split && few(8193, 2880, 16, normed) == planes);
+        CHECK(few(5120, 2016, 16, normed) == planes && few(5120, 2048, 16, normed) == split && few(5120, 4096, 16, normed) == split && few(5120, 4128, 16, normed) == planes);
+        CHECK((few(5120, 2880, 17, normed) == Names{"lng_q8_norm_frag", "lng_q8_mid_r32p32"}) && few(5120, 2880, 2, normed) == split);
+        CHECK(few(8192, 2880, 4, normed) == split && few(8192, 2880, 3, normed) == (normed ? split : Names{"lng_q8_few_f32"}));
     }
     lng_null_clear();
 }
@@ -303,7 +310,7 @@ template <typename A> static bool launch_args(size_t i, const char *prefix, A *a
 // Sequences of a block's dispatches that a commit makes one kernel of, and sequences that only look alike.
 static void fused_sequences() {
     typedef std::vector<std::string> Names;
-    Fixture f(9, 6 << 20);
+    Fixture f(9, 12 << 20);
     auto run = [&]() {
         CHECK(lng_hip_batch_commit(f.batch, nullptr, nullptr) == LNG_OK && lng_hip_batch_wait(f.batch, nullptr) == LNG_OK);
         return launched();
@@ -405,13 +412,26 @@ static void fused_sequences() {
         again();
     }
 
+    for (const auto &w : {std::make_tuple(4u, 4112u, 2048u, "lng_q8_few_split"), std::make_tuple(1u, 9000u, 96u, "lng_q8_tall")}) {
+        const uint64_t n = std::get<0>(w), rows = std::get<1>(w), cols = std::get<2>(w), len = n * rows * 4;
+        const lng_slice y{5, 0, len}, bias{2, 0, rows * 4}, h{6, 0, len};
+        CHECK(lng_hip_gemm_q8_0(f.batch, lng_slice{3, 0, rows * cols}, lng_slice{4, 0, rows * cols / 16}, lng_slice{0, 0, n * cols * 4}, y, rows, cols, n, cols, rows) == LNG_OK);
+        CHECK(lng_hip_add_rows(f.batch, y, bias, 0, n, rows) == LNG_OK && lng_hip_add_rows(f.batch, h, y, rows, n, rows) == LNG_OK);
+        lng_k_q8 a{};
+        CHECK(run() == Names{std::get<3>(w)} && launch_args(0, "lng_q8", &a) && a.bias && a.residual && a.residual != a.y && !a.accumulate);
+        again();
+    }
+
     // ---- the q, k and v projections + the preparation of attention ----
-    struct Case { uint64_t n, cols, rotary; bool normed, one_item; const char *kind; Names names; };
+    struct Case { uint64_t n, cols, rotary; bool normed, one_item; const char *kind; Names names; uint64_t heads = 6, kv = 2; };
     const Case cases[] = {
         {1, 96, 64, true, true, "", {"lng_q8_one_prepare"}},
         {4, 96, 64, true, false, "", {"lng_q8_few_f32_prepare"}},
         {16, 96, 64, false, true, "", {"lng_q8_few_f32_prepare"}},
         {4, 2880, 64, true, false, "", {"lng_q8_norm_frag", "lng_q8_few_prepare"}},
+        {2, 2048, 64, true, false, "", {"lng_q8_few_split_prepare"}, 64, 8},
+        {16, 2048, 64, false, true, "", {"lng_q8_few_split_prepare"}, 64, 8},
+        {1, 96, 64, true, true, "", {"lng_q8_one_prepare"}, 112, 16}, // (more tiles than the device holds workgroups: one to each all the same)
         {17, 96, 64, true, false, "", {"lng_q8_few_f32", "lng_prepare"}},
         {4, 96, 32, true, false, "", {"lng_q8_few_f32", "lng_prepare"}},
         {4, 96, 64, true, false, "backwards", {"lng_q8_few_f32", "lng_prepare"}},
@@ -421,7 +441,7 @@ static void fused_sequences() {
         {4, 96, 64, true, false, "biases over v", {"lng_q8_few_f32", "lng_prepare"}},
     };
     for (const Case &c : cases) {
-        const uint64_t heads = 6, kv = 2, qw = heads * 64, kw = kv * 64, n = c.n, slots = 24;
+        const uint64_t heads = c.heads, kv = c.kv, qw = heads * 64, kw = kv * 64, n = c.n, slots = 24;
         const std::string kind = c.kind;
         const uint64_t k_at = kind == "swapped" ? n * kw * 4 : 0, v_at = kind == "swapped" ? 0 : n * kw * 4;
         const lng_slice x{0, 0, n * c.cols * 4}, norm{2, 0, c.cols * 4};
@@ -456,6 +476,8 @@ static void fused_sequences() {
         if (names.back().find("_prepare") != std::string::npos && names.back().rfind("lng_q8", 0) == 0) {
             lng_k_q8_prepare both{};
             CHECK(launch_args(names.size() - 1, "lng_q8", &both) && both.q8.n == n && both.q8.n_more == 2 && both.prepare.heads == heads && both.prepare.kv_heads == kv);
+            unsigned grid = 0;
+            CHECK(launch_args(names.size() - 1, "lng_q8", &both, &grid) && (!both.q8.one_rows || (grid == both.q8.tiles && both.q8.one_rows % 2 == 0)));
             CHECK((both.prepare.items == nullptr) == (items.size() == 1) && both.prepare.q_bias && both.prepare.k_bias && both.prepare.v_bias);
         }
         again();
@@ -674,6 +696,40 @@ static void allocation_failures() {
     }
     CHECK(lng_hip_attention_grouped(batch, q, k, v, o, nullptr, &s, LNG_BF16) == LNG_OK);
     CHECK(lng_hip_batch_dispatches(batch) == 1);
+    // f32 rows of 257 to 512 positions do without the partials when there is no memory for them, one row and a table; longer ones and
+    // wider heads are refused
+    const struct { uint64_t ctx, dim; bool whole; } rows_of[] = {{257, 64, true}, {300, 64, true}, {512, 64, true}, {513, 64, false}, {600, 128, false}};
+    for (const auto &w : rows_of) {
+        for (const bool table : {false, true}) {
+            for (size_t nth = 1; nth <= 3; ++nth) { // the counters, the partial outputs, the (max, sum) pairs (after the table itself)
+                Fixture f(4, 4 << 20);
+                const uint64_t heads = 16, kv = 2, len = heads * w.dim * 4, cache = w.ctx * kv * w.dim * 4;
+                const lng_grouped_shape one = shape(1, w.ctx - 1, heads, kv, w.dim, LNG_WINDOW_FULL, w.ctx, 0.125f);
+                lng_decode_item items[2]{};
+                for (int i = 0; i < 2; ++i) {
+                    items[i].q_offset = items[i].out_offset = i * len, items[i].k_offset = items[i].v_offset = i * cache;
+                    items[i].sinks_offset = LNG_NO_SINKS, items[i].start = w.ctx - 1 - i, items[i].window = LNG_WINDOW_FULL, items[i].slots = w.ctx;
+                }
+                auto record = [&] {
+                    return table ? lng_hip_attention_decode_batched(f.batch, 0, 1, 2, 3, LNG_NO_SINKS, items, 2, heads, kv, w.dim, 0.125f, LNG_F32)
+                                 : lng_hip_attention_grouped(f.batch, lng_slice{0, 0, len}, lng_slice{1, 0, cache}, lng_slice{2, 0, cache}, lng_slice{3, 0, len}, nullptr, &one, LNG_F32);
+                };
+                lng_null_clear();
+                lng_null_fail_malloc_after(nth + table);
+                const int rc = record();
+                lng_null_fail_malloc_after(0);
+                CHECK(rc == (w.whole ? LNG_OK : LNG_ERR_ALLOC) && lng_hip_batch_dispatches(f.batch) == (w.whole ? 1u : 0u));
+                if (!w.whole) CHECK(record() == LNG_OK);
+                CHECK(lng_hip_batch_commit(f.batch, nullptr, nullptr) == LNG_OK && lng_hip_batch_wait(f.batch, nullptr) == LNG_OK);
+                lng_k_attn a{};
+                unsigned grid = 0;
+                CHECK(launched().size() == (w.whole ? 1u : 2u) && launch_args(0, "lng_decode_f32", &a, &grid));
+                if (w.whole) CHECK(launched()[0] == "lng_decode_f32_d64" && a.chunk == 512 && a.n_chunks == 1 && grid == (table ? 2 : 1) * kv);
+                else CHECK(a.n_chunks > 1);
+            }
+        }
+    }
+    lng_null_clear();
     // Q8_0 products of few positions do without the planes of their positions when there is no memory for them (17 to 31, which
     // prefer lng_q8_mid, ask a second time, which succeeds here)
     for (const uint64_t n : {16, 31}) {

@@ -99,7 +99,8 @@ def test_norm_at_the_edges_of_its_words(gpu, d, stride):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("n,rows,cols", [(1, 48, 96), (7, 33, 64), (17, 48, 96), (32, 64, 96), (77, 100, 64), (200, 192, 96), (1290, 260, 64)])
+@pytest.mark.parametrize("n,rows,cols", [(1, 48, 96), (7, 33, 64), (17, 48, 96), (32, 64, 96), (77, 100, 64), (200, 192, 96), (1290, 260, 64),
+                                         (2, 4112, 2048), (16, 5121, 2912), (1, 8201, 96)])
 def test_bias_and_residual_in_the_product(gpu, n, rows, cols, bf16):
     """Each kind of product with bias and residual, bias or residual alone, and the sequences that only look alike: hidden
     rows over the positions, over the codes or over the bias, a residual of another width, the bias added twice, y with gaps,
@@ -160,14 +161,18 @@ def test_bias_and_residual_in_the_product(gpu, n, rows, cols, bf16):
     (1, True, 64, 64, True, True, "", 2880, 6, 2), (16, False, 64, 64, True, True, "", 2880, 6, 2), (5, False, 64, 64, True, False, "", 2880, 6, 2),
     (1, True, 64, 64, True, True, "", 352, 64, 8), (16, True, 64, 64, False, False, "", 352, 64, 8), (1, True, 64, 64, False, False, "", 4160, 2, 1),
     (7, False, 64, 64, True, False, "", 4160, 2, 1), (1, True, 64, 64, True, True, "", 12288, 2, 1), (3, False, 64, 64, True, True, "", 12288, 2, 1),
-    (6, False, 64, 64, True, False, "", 16416, 2, 1), (9, False, 64, 64, True, True, "", 512, 6, 2), (16, False, 64, 64, True, False, "", 544, 6, 2)])
+    (6, False, 64, 64, True, False, "", 16416, 2, 1), (9, False, 64, 64, True, True, "", 512, 6, 2), (16, False, 64, 64, True, False, "", 544, 6, 2),
+    # more rows than a workgroup of 16 a unit takes: tiles of 18 to 32 rows, across heads
+    (2, False, 64, 64, True, True, "", 2880, 64, 8), (5, True, 64, 64, True, True, "", 2880, 64, 8), (16, False, 64, 64, False, True, "", 2880, 64, 8),
+    (16, True, 64, 64, True, False, "", 2912, 56, 7), (2, False, 64, 64, False, False, "", 4096, 64, 8), (5, False, 64, 64, True, True, "", 4064, 66, 11),
+    (16, False, 64, 64, True, True, "", 4096, 96, 16), (9, True, 64, 64, True, True, "", 2048, 66, 1), (1, True, 64, 64, True, True, "", 96, 112, 16)])
 def test_projections_and_preparation_in_one_kernel(gpu, n, one_item, dim, rotary, bias, normed, kind, cols, heads, kv_heads, dtype):
     """q, k and v of up to 16 positions with the preparation after them: tables of items and one item, rings that wrap, with
     and without biases and norm; and what stays apart: more positions, other widths, items in another order than the rows, k
     and v the other way round, a rotation table in rows that q is written to, prepared queries where x is. Columns: fewer
     pairs of blocks than wavefronts, several pairs a wavefront, more than one turn of 4,096, a block left over, scales that
-    wait in LDS in more than 64 words a row or do not fit there; positions split by the product itself and before it. The
-    products and the prepared rows against float64, too."""
+    wait in LDS in more than 64 words a row or do not fit there; positions split by the product itself, in tiles of 16 rows and of more,
+    and before it. The products and the prepared rows against float64, too."""
     slots, eps = 24, 1e-5
     qw, kw, es = heads * dim, kv_heads * dim, 4 if dtype == C.F32 else 2
     elements = []

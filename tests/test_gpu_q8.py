@@ -717,3 +717,38 @@ def test_positions_split_by_the_product_itself(gpu, rows, cols, n):
         assert (np.abs(got - want).max(1) < 1e-5 * np.abs(want).max(1)).all()
     for b in bufs:
         b.free()
+
+
+@pytest.mark.parametrize("normed", [False, True])
+@pytest.mark.parametrize("n,cols", [(1, 2880), (2, 2880), (9, 2080), (16, 2880), (16, 4096)])
+def test_a_few_positions_together_and_alone(gpu, n, cols, normed):
+    """q, k and v in one dispatch, whose rows together decide on the kernel, and each alone. Without a norm bit for bit. With one the
+    kernel for many rows multiplies what the norm's weights give and scales the finished sum: both within 2^-17 of float64 for each
+    term - two bf16 values hold 2^-18 of each, which leaves as much for the f32 sums of 128 blocks - so neither is the less exact."""
+    shapes = [4096, 512, 520]
+    mats = [q8_test_matrix(rows, cols, 21 + i) for i, rows in enumerate(shapes)]
+    x, w = xorshift_values(49, n * cols).reshape(n, cols).astype(np.float32), 1 + 0.2 * xorshift_values(50, cols).astype(np.float32)
+    eps, starts = 1e-5, [0] + list(np.cumsum(shapes) * n * 4)
+    bufs = [gpu.upload(x), gpu.upload(w)] + [gpu.upload(a) for m in mats for a in m[:2]] + [gpu.buffer(int(starts[-1]))]
+    bufs[-1].fill(0xFF)
+    batch = gpu.batch(bufs)
+    many = [((C.Slice(2 + 2 * i, 0, r * cols), C.Slice(3 + 2 * i, 0, r * cols // 16)), C.Slice(8, int(starts[i]), 4 * n * r), r) for i, r in enumerate(shapes)]
+    xs = C.Slice(0, 0, x.nbytes)
+    batch.gemm_q8_0_many_normed(many, xs, (C.Slice(1, 0, w.nbytes), eps), cols, n, cols) if normed else batch.gemm_q8_0_many(many, xs, cols, n, cols)
+    done = batch.run()
+    assert not isinstance(done.gpu_time, Exception), done.gpu_time
+    raw = bufs[-1].read(np.float32)
+    batch.drop()
+    for b in bufs:
+        b.free()
+    xd = x.astype(np.float64)
+    if normed:
+        xd = xd / np.sqrt((xd * xd).mean(axis=1, keepdims=True) + eps) * w
+    for i, rows in enumerate(shapes):
+        together = raw[starts[i] // 4:starts[i + 1] // 4].reshape(n, rows)
+        alone = _product(gpu, mats[i][0], mats[i][1], x, rows, cols, n, w if normed else None)
+        if not normed:
+            assert np.array_equal(together, alone)
+        want, terms = xd @ mats[i][2].T, np.abs(xd) @ np.abs(mats[i][2]).T
+        for got in (together, alone):
+            assert (np.abs(got - want) <= 2.0**-17 * terms).all(), np.max(np.abs(got - want) / terms) * 2.0**17
