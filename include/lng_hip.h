@@ -370,8 +370,9 @@ int lng_hip_gemm_q8_0_many(lng_batch *batch, const lng_q8_matrix *matrices, size
 
 /* The same with the RMS norm of the positions folded in (no counterpart in the reference, which copies the
  * hidden state, normalises the copy in place and then multiplies: gpu.rs:712-732): y_i[p] = W_i x'[p] with
- * x'[p][c] = (x[p][c] / sqrt(mean_c(x[p]^2) + eps)) * norm_w[c], the arithmetic of lng_hip_rmsnorm_rows; x is
- * left as it is. norm_w holds cols f32 on a 16-byte boundary. For decoding only: fewer than 32 positions of up
+ * x'[p][c] = (x[p][c] / sqrt(mean_c(x[p]^2) + eps)) * norm_w[c]; x is left as it is. Where the factor 1 / sqrt(..) goes in
+ * depends on the sizes and on the rows of all matrices together: before the product, as lng_hip_rmsnorm_rows has it, or (2 to 16
+ * positions of many rows) on the finished sum. Both are as exact, but a matrix alone and among others may differ in the last bits. norm_w holds cols f32 on a 16-byte boundary. For decoding only: fewer than 32 positions of up
  * to 12288 columns (refused otherwise: prompt passes are bound by the matrix unit and take the separate calls). */
 int lng_hip_gemm_q8_0_many_normed(lng_batch *batch, const lng_q8_matrix *matrices, size_t n_matrices, lng_slice x,
                                   lng_slice norm_w, float eps, uint64_t cols, uint64_t n, uint64_t x_stride);

@@ -586,9 +586,11 @@ DecodePlan plan_decode(lng_gpu *g, const lng_k_row *rows, size_t n, uint64_t t_u
     chunk = std::max<uint64_t>(chunk, ((longest + LNG_MAX_CHUNKS - 1) / LNG_MAX_CHUNKS + 127) / 128 * 128);
     // Short runs (a 128-token window seen from its 32-aligned start is up to 159 positions) stay whole: two
     // chunks would mean partials, arrival counters and a merge for five tiles of work.
-    // f32, whose tiles take twice the bytes and eight times the matrix instructions, past 256 positions only where the pairs
-    // fill the device: 300 and 500 positions whole and in chunks with a merge, us, 1 sequence 10.1, 13.9 and 9.0, 9.1, 4 sequences
-    // 10.9, 14.4 and 9.5, 9.7, 16 sequences 14.0, 18.8 and 14.1, 16.0, 30 sequences 15.6, 20.8 and 21, 24.5.
+    // f32, whose tiles take twice the bytes and eight times the matrix instructions, past 256 positions only from a quarter as many
+    // pairs as units on, up to which chunks are faster at every length (16 sequences would gain at 500 positions, not at 300; 30
+    // lose): 300 and 500 positions whole and in chunks with a merge, us, 1 sequence 10.1, 13.9 and 9.0, 9.1, 4 sequences 10.9, 14.4 and
+    // 9.5, 9.7, 16 sequences 14.0, 18.8 and 14.1, 16.0, 30 sequences 15.6, 20.8 and 21, 24.5. (8 sequences, in a batch of such, 257,
+    // 300, 384, 512 positions 10.3, 10.3, 11.0, 13.6 whole, 9.2 to 9.3 in chunks.)
     if (longest <= (in_f32 && 4 * pairs <= g->cus ? 256u : 512u)) chunk = std::max<uint64_t>(chunk, (longest + 127) / 128 * 128);
     p.chunk = (uint32_t)chunk;
     p.n_chunks = (uint32_t)((longest + chunk - 1) / chunk);
@@ -2290,7 +2292,8 @@ unsigned q8_one_rows(const lng_gpu *g, const lng_k_q8 &a, uint64_t held) {
 }
 
 // Rows of a workgroup of lng_q8_few_split; 0: not for it. It is for matrices whose tiles of 16 rows would leave some compute units
-// with two workgroups, each reading all of x: as many rows, dealt out evenly, as make it one (only one fits).
+// with two workgroups, each reading all of x: as many rows, dealt out evenly, as make it one (only one fits). Its wavefronts hold up
+// to 4,096 columns in one turn; below 2,048, where it is not measured, the planes stay.
 unsigned q8_few_split_rows(const lng_gpu *g, const lng_k_q8 &a) {
     if (a.n < 2 || a.n > 16 || a.cols < 2048 || a.cols > 4096) return 0;
     for (unsigned t = 16; t <= 32; t += 2) { // (even: lng_q8_few_split_prepare takes pairs of rows)
@@ -2301,8 +2304,8 @@ unsigned q8_few_split_rows(const lng_gpu *g, const lng_k_q8 &a) {
     return 0;
 }
 
-// Fewer than 32 positions: bound by reading the matrix, in tiles of 16 rows. One position splits (and normalises) x in
-// the kernel, whose LDS holds up to 48 KB of it; more go through the planes of q8_record_frag or are split by every workgroup.
+// Fewer than 32 positions: bound by reading the matrix, in tiles of 16 rows. One position makes x (normalised) whole numbers in
+// the kernel, whose LDS holds up to 48 KB of x; more go through the planes of q8_record_frag or are split by every workgroup.
 // `a` may name further matrices of the same dispatch (first_tile in tiles of 16 rows).
 int q8_record_few(lng_batch *b, lng_k_q8 a, uint64_t row_tiles, bool x_bf16) {
     const uint64_t blocks = a.cols / 32, groups = (a.n + 15) / 16;

@@ -1,5 +1,5 @@
 // Q8_0 products of fewer than 32 positions (17 to 31 of matrices of many rows share lng_q8_mid's tiles): lng_q8_norm_frag,
-// lng_q8_few*, lng_q8_one*. (Included by lng_kernels.hip after lng_q8_mid.h; see there for how a product goes through the matrix unit.)
+// lng_q8_few*, lng_q8_one*, lng_q8_tall*. (Included by lng_kernels.hip after lng_q8_mid.h; see there for how a product goes through the matrix unit.)
 
 // x[n][x_stride] f32 as the A operands of lng_q8_few and lng_q8_mid, RMS-normalised on the way if norm_w is set
 // (x / sqrt(mean(x^2) + eps) * w): one workgroup per position, lng_q8_frag_x's layout. Rows that pad n to whole groups
@@ -392,9 +392,10 @@ __device__ __forceinline__ void q8_few_body(const lng_k_q8 &a, uint32_t tile, ch
 // infinities, and NaN where the code is 0, as in the other products.
 // Bound by memory and by what lies before and after it: 1 us until all loads are on their way, a round trip, the matrix at the
 // rate of the whole device (15.7 MB: 2.6 us), 0.8 us of sums and their way through LDS, a dispatch's start and end. In a token
-// through 24 blocks (kernel trace): 5,120 x 2,880 with norm and preparation 9.1 us -> 7.6, 2,880 x 4,096 with bias and residual
-// 7.2 -> 5.5 from bf16, 7.3 -> 5.2 from f32; of which the whole numbers 9.1 -> 7.8 and 7.2 -> 5.9 (the sums of 4,096 columns took
-// a wavefront 1.55 us, now 0.5), tiles of 10 to 14 rows and x before the codes the rest.
+// through 24 blocks (kernel trace; as two bf16 planes on the other unit / so / with the planes of the rest): 5,120 x 2,880 with norm
+// and preparation 9.1 us / 7.6 / 8.2, 2,880 x 4,096 with bias and residual from bf16 7.2 / 5.5 / 5.9, from f32 7.3 / 5.2 / 6.1. Of the
+// gain the whole numbers 9.1 -> 7.8 and 7.2 -> 5.9 (the sums of 4,096 columns took a wavefront 1.55 us, now 0.5), tiles of 10 to 14
+// rows and x before the codes the rest.
 #define Q8WHOLE_REST 15
 struct Q8Whole { // eight columns, a quarter of a block; the other three are in the neighbouring lanes
     uint2 plane[4];
@@ -828,14 +829,15 @@ __device__ __forceinline__ void q8_tall_body(const lng_k_q8 &a, char *s_mem) {
 }
 
 // 2 to 16 f32 positions of 2,048 to 4,096 columns in one dispatch, with the RMS norm if norm_w is set: x goes through the matrix
-// unit as it is (times the norm's weights), its squares are added up on the way and each position's scale multiplies the result.
+// unit as it is (times the norm's weights), its squares are added up on the way and each position's scale multiplies the result (as
+// exact as normalising it first: two bf16 values hold as much of a number at any size).
 // So there is no dispatch of planes before it and x is read once: eight lanes to a position's 128 bytes of a block, split, and
 // turned into operand order through LDS that only this wavefront uses. x is most of what a workgroup reads (16 positions of 2,880
 // columns: 184 KB beside 46 KB of codes for 16 rows), so a workgroup takes up to 32 rows, NT runs of 16, and has a compute unit
 // to itself: all its loads of a turn but the last pairs' x are on their way at once.
 // With planes made by a dispatch before it and tiles of 16 rows / so, us, 16 positions: 5,120 x 2,880 12.4 / 10.9 with the norm,
 // 11.9 / 11.1 without, 4,112 x 4,096 15.7 / 13.1 and 15.1 / 13.4, 8,192 x 2,048 11.3 / 10.6 and 10.7 / 10.4; in a decoding step of
-// sixteen sequences (kernel trace, preparation included) 4.7 + 11.3 / 12.9. As many rows as have a unit each with one workgroup
+// sixteen sequences (kernel trace, preparation included) 4.7 + 11.4 / 13.0 to 13.5. As many rows as have a unit each with one workgroup
 // of 16 gain nothing (2,880 x 4,096 10.9 / 10.8).
 // U: pairs of blocks of a wavefront (2,880 columns: five or six of 6; up to 4,096: 8).
 template <int U, bool PREPARE>
